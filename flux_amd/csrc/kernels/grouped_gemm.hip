@@ -1,6 +1,6 @@
 // Grouped GEMM entry point: argument checks, choice between the MFMA kernel and the generic kernel, and
 // the generic kernel itself.  The MFMA kernel lives in grouped_gemm_kernel.hpp.
-#include "grouped_gemm.hpp"
+#include "grouped_gemm_stream.hpp"
 
 namespace fluxmi {
 namespace {
@@ -214,7 +214,9 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   // CUs left to other work of the caller (Flux's sm_margin): the persistent kernel launches fewer workgroups.
   cus = cus - args->cu_margin > 1 ? cus - args->cu_margin : 1;
 
-  if (mfma) {
+  if (mfma && grouped_gemm_stream_takes(p, args->dtype)) {
+    launch_grouped_gemm_stream(p, args->dtype, s);
+  } else if (mfma) {
     // Upper bound of the tile count: never launch more workgroups than tiles.
     const int64_t tiles_n = (args->n + BN - 1) / BN * ngroups;
     const int64_t max_tiles = (static_cast<int64_t>(args->max_rows) / BM + args->nexperts) * tiles_n;

@@ -1,0 +1,397 @@
+// Grouped GEMM for few rows per expert (decoding, small batches): D[r,:] = scale(r,:) * A[gather(r),:] @ B[e(r)]^T.
+//
+// Bound by HBM: every weight is read once and used for a handful of rows.  What that needs is bytes in flight on every
+// compute unit all the time (about 50 KB each to cover the memory latency at the card's read rate), not operand reuse,
+// so the shape of this kernel is the opposite of the macro-tile kernel's (grouped_gemm_kernel.hpp):
+//
+//  * A workgroup computes 16 * NB columns of up to 16 * MBMAX rows of one expert over the whole of K; its waves split K
+//    between them by 128-byte lines (wave w takes lines w, w + WAVES, ...), so that the workgroup reads each row of
+//    weights front to back.  The partial sums meet in LDS at the end and are added in wave order (same bits every run).
+//  * Operands go from memory straight into registers, eight whole 128-byte lines per load instruction, non-temporally for the
+//    weights.  A read-only probe of this access (0.94 GB, rows of 2 to 28 KiB): whole lines 6.7-7.1 TB/s non-temporally and
+//    6.1-6.6 with ordinary loads; the MFMA fragment layout itself (16 rows x 64 bytes per instruction, the two halves of a
+//    line in two instructions) 4.9-5.5 and 5.9-6.5; 1 KiB of one row per instruction 3.3-6.7.  Two loads become two
+//    fragments by exchanging lanes 8..15 of every 16 with lanes 0..7 (three register moves per four bytes and lane).
+//  * No barriers and no waits between waves in the loop; a ring of DEPTH lines per wave is in flight (128 KiB of weights per
+//    compute unit), several workgroups share a compute unit.
+//  * Rows beyond the expert's last repeat it (their lanes hit the same lines) and are not stored; bytes past the end of K
+//    are out-of-range buffer loads, which return zeros.
+//  * The items (expert, column tile, row chunk) are numbered with the row chunks of one column tile next to each other,
+//    and each XCD takes a contiguous eighth of them: weights that several chunks share are fetched into one L2.
+//
+// Measured (us per launch, the macro-tile kernel in its place -> this one; weights at 6.5 TB/s in brackets), bf16 8 experts
+// 14336 x 4096: 2 rows 60 -> 41 [36], 74 rows 211 -> 143 [145], 192 rows 217 -> 165; 4096 x 14336: 2 rows 87 -> 42 [36], 74
+// rows 213 -> 148 [145]; 64 experts 1408 x 2048, 222 rows: 111 -> 60 [57]; fp8 32 experts 2048 x 7168, 296 rows: 95 -> 74
+// [72]; 7168 x 2048: 116 -> 88 [72]; block-scaled, the same two: 128 -> 75 and 159 -> 91.
+#include "grouped_gemm_stream.hpp"
+
+namespace fluxmi {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+enum class Elem { BF16, F16, FP8, FP8_BLOCKSCALED };
+constexpr bool is_fp8(Elem t) { return t == Elem::FP8 || t == Elem::FP8_BLOCKSCALED; }
+
+#if defined(__HIP_DEVICE_COMPILE__)
+
+constexpr uint32_t kOutOfRange = 0xfffffff0u;  // a byte offset past every buffer: the load returns zeros
+
+// Clamped like the macro-tile kernel's: negative counts are 0, rows past max_rows do not exist.
+struct WorkItem {
+  bool valid;
+  int e, row_base, expert_rows;
+  int m0, rows;  // this chunk: its first row in the expert, its row count
+  int nt;        // column tile, over all weight groups
+};
+
+template <int MBMAX>
+__device__ __forceinline__ int row_chunks(int rows) { return (rows + 16 * MBMAX - 1) / (16 * MBMAX); }
+
+// Work item -> (expert, row chunk, column tile).  One wave-wide pass over the splits counts the chunks, a second finds
+// the item; with up to 64 experts both work on the same registers.
+template <int MBMAX>
+__device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n) {
+  const int lane = threadIdx.x & 63;
+  auto load = [&](int e0, int &carry, int &begin, int &rows) {
+    const int ee = e0 + lane;
+    int r = ee < p.nexperts ? p.splits[ee] : 0;
+    if (r < 0) r = 0;
+    const int incl = wave_inclusive_scan(r);
+    begin = carry + incl - r;
+    int end = carry + incl;
+    if (begin > p.max_rows) begin = p.max_rows;
+    if (end > p.max_rows) end = p.max_rows;
+    rows = end - begin;
+    carry += __shfl(incl, 63, 64);
+  };
+  int carry = 0, begin = 0, rows = 0, total = 0;
+  for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
+    load(e0, carry, begin, rows);
+    total += __shfl(wave_inclusive_scan(row_chunks<MBMAX>(rows)), 63, 64);
+  }
+  // Workgroups are dealt to the eight XCDs round-robin.
+  const int items = total * tiles_n;
+  const int per_xcd = (items + 7) / 8;
+  const int i = blockIdx.x >> 3;
+  int item = (blockIdx.x & 7) * per_xcd + i;
+  WorkItem w = {false, 0, 0, 0, 0, 0, 0};
+  if (i >= per_xcd || item >= items) return w;
+  carry = 0;
+  for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
+    if (p.nexperts > 64) load(e0, carry, begin, rows);
+    const int chunks = row_chunks<MBMAX>(rows);
+    const int incl = wave_inclusive_scan(chunks) * tiles_n;
+    const uint64_t hit = __ballot(item < incl);
+    if (hit != 0) {
+      const int src = __ffsll(static_cast<unsigned long long>(hit)) - 1;
+      const int nchunks = __builtin_amdgcn_readlane(chunks, src);
+      const int local = item - (__builtin_amdgcn_readlane(incl, src) - nchunks * tiles_n);
+      const int all_rows = __builtin_amdgcn_readlane(rows, src);
+      w.valid = true;
+      w.e = e0 + src;
+      w.row_base = __builtin_amdgcn_readlane(begin, src);
+      w.nt = local / nchunks;
+      // An expert's 16-row blocks are shared out evenly over its chunks.
+      const int blocks = (all_rows + 15) >> 4, per = (blocks + nchunks - 1) / nchunks;
+      w.expert_rows = all_rows;
+      w.m0 = (local - w.nt * nchunks) * per * 16;
+      w.rows = all_rows - w.m0 < per * 16 ? all_rows - w.m0 : per * 16;
+      if (w.rows <= 0) w.valid = false;
+      return w;
+    }
+    item -= __builtin_amdgcn_readlane(incl, 63);
+  }
+  return w;
+}
+
+template <Elem T, int MB, int NB>
+struct Line {  // one 128-byte line of every row of the wave's operand blocks, as loaded
+  i32x4 w[NB][2], x[MB][2];
+  float as[MB], bs;
+};
+
+// Two loads of eight rows each (lane: row l & 7, chunk 2 * (l >> 4) + bit 3 of l) -> two MFMA fragments of the sixteen rows
+// (lane: row l & 15, chunks 2 * (l >> 4) and 2 * (l >> 4) + 1): the lanes with bit 3 set of the first change places with
+// the lanes with bit 3 clear of the second.
+__device__ __forceinline__ void to_fragments(i32x4 (&v)[2]) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int a = v[0][c], b = v[1][c];
+    v[0][c] = __builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false);  // row_ror:8 into lanes 8..15 of every 16
+    v[1][c] = __builtin_amdgcn_update_dpp(b, a, 0x128, 0xf, 0x3, false);  // ... into lanes 0..7
+  }
+}
+
+template <Elem T>
+__device__ __forceinline__ f32x4 mfma_line(const i32x4 (&w)[2], const i32x4 (&x)[2], f32x4 acc) {
+  if constexpr (is_fp8(T)) {
+    const i32x8 wa = {w[0][0], w[0][1], w[0][2], w[0][3], w[1][0], w[1][1], w[1][2], w[1][3]};
+    const i32x8 xa = {x[0][0], x[0][1], x[0][2], x[0][3], x[1][0], x[1][1], x[1][2], x[1][3]};
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wa, xa, acc, 0, 0, 0, 0, 0, 0);
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if constexpr (T == Elem::F16)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w[h]), __builtin_bit_cast(f16x8, x[h]), acc, 0, 0, 0);
+      else
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[h]), __builtin_bit_cast(bf16x8, x[h]), acc, 0, 0, 0);
+    }
+    return acc;
+  }
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, int64_t bytes) {
+  const uint32_t n = bytes > 0xffffffffll ? 0xffffffffu : static_cast<uint32_t>(bytes < 0 ? 0 : bytes);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, static_cast<int>(n), 0x00020000);
+}
+
+template <int AUX>
+__device__ __forceinline__ i32x4 load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) {
+  return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(voff), soff, AUX));
+}
+
+// 16 * MB rows x 16 * NB columns of one expert: partial sums of this wave's lines of K into acc.
+template <Elem T, int MB, int NB, int WAVES, int DEPTH>
+__device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkItem &t, int g, int n0, f32x4 (&acc)[MB][NB]) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t kbytes = static_cast<int64_t>(p.k) * (is_fp8(T) ? 1 : 2);
+  const int kb32 = static_cast<int>(kbytes);
+  // Lane l of a load fetches 16 bytes of row l & 7 of an eight-row block, chunk 2 * (l >> 4) + ((l >> 3) & 1) of the line.
+  const int cbyte = (lane >> 4) * 32 + ((lane >> 3) & 1) * 16;
+  const auto wr = buffer_of(p.b[g] + (static_cast<int64_t>(t.e) * p.n + n0) * kbytes, static_cast<int64_t>(p.n - n0) * kbytes);
+  const bool gathered = p.gather_a != nullptr;
+  const auto xr = gathered ? buffer_of(p.a, static_cast<int64_t>(p.a_rows) * kbytes)
+                           : buffer_of(p.a + static_cast<int64_t>(t.row_base + t.m0) * kbytes, static_cast<int64_t>(t.rows) * kbytes);
+  uint32_t woff[NB][2], xoff[MB][2];
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      int r = j * 16 + h * 8 + (lane & 7);
+      if (r > p.n - n0 - 1) r = p.n - n0 - 1;
+      woff[j][h] = static_cast<uint32_t>(r * kbytes) + cbyte;
+    }
+  auto source_row = [&](int r) {  // row of A that row r of the chunk reads (the last one again past the end)
+    if (r > t.rows - 1) r = t.rows - 1;
+    if (!gathered) return static_cast<int64_t>(r);
+    const int64_t arow = p.gather_a[t.row_base + t.m0 + r];
+    return arow < 0 ? 0 : (arow >= p.a_rows ? p.a_rows - 1 : arow);
+  };
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) xoff[i][h] = static_cast<uint32_t>(source_row(i * 16 + h * 8 + (lane & 7)) * kbytes) + cbyte;
+  __amdgpu_buffer_rsrc_t sr = xr;
+  uint32_t soff[MB];
+  int a_kstep = 0, b_base = 0, b_kstep = 0;
+  const int kblocks = p.k >> 7;
+  if constexpr (T == Elem::FP8_BLOCKSCALED) {
+    sr = buffer_of(p.a_scale, 0xffffffffll);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int r = i * 16 + (lane & 15);
+      const int64_t srow = source_row(r) + (gathered ? 0 : t.row_base + t.m0);
+      soff[i] = p.a_scale_layout == FLUXMI_ASCALE_BLOCK128
+                    ? static_cast<uint32_t>(((srow >> 7) * kblocks * 128 + (srow & 127)) * 4)
+                    : static_cast<uint32_t>((static_cast<int64_t>(t.row_base) * (kblocks - 1) + srow) * 4);
+    }
+    a_kstep = p.a_scale_layout == FLUXMI_ASCALE_BLOCK128 ? 512 : t.expert_rows * 4;
+    const int nb = n0 >> 7, nblocks = (p.n + 127) >> 7;
+    b_base = p.b_scale_layout == FLUXMI_BSCALE_N_K ? (t.e * nblocks + nb) * kblocks : t.e * kblocks * nblocks + nb;
+    b_kstep = p.b_scale_layout == FLUXMI_BSCALE_N_K ? 1 : nblocks;
+  }
+
+  Line<T, MB, NB> ring[DEPTH];
+  auto load_line = [&](Line<T, MB, NB> &l, int line) {
+    const int kb = line * 128;
+    const bool ok = kb + cbyte < kb32;
+    const int ks = kb < kb32 ? kb : 0;
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) l.w[j][h] = load16<2>(wr, ok ? woff[j][h] : kOutOfRange, ks);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) l.x[i][h] = load16<0>(xr, ok ? xoff[i][h] : kOutOfRange, ks);
+    if constexpr (T == Elem::FP8_BLOCKSCALED) {
+      const int kblk = line < kblocks ? line : 0;
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+        l.as[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(sr, static_cast<int>(soff[i]), kblk * a_kstep, 0));
+      l.bs = p.b_scale[b_base + kblk * b_kstep];
+    }
+  };
+  auto use_line = [&](Line<T, MB, NB> &l) {
+#pragma unroll
+    for (int j = 0; j < NB; ++j) to_fragments(l.w[j]);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) to_fragments(l.x[i]);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      if constexpr (T == Elem::FP8_BLOCKSCALED) {
+        const float s = l.as[i] * l.bs;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const f32x4 b = mfma_line<T>(l.w[j], l.x[i], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[i][j][v] = fmaf(b[v], s, acc[i][j][v]);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = mfma_line<T>(l.w[j], l.x[i], acc[i][j]);
+      }
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int lines = static_cast<int>((kbytes + 127) >> 7);
+  const int steps = (lines + WAVES - 1) / WAVES;
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    load_line(ring[d], d * WAVES + wave);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (int s = 0; s < steps; s += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      use_line(ring[d]);
+      __builtin_amdgcn_sched_barrier(0);
+      load_line(ring[d], (s + d + DEPTH) * WAVES + wave);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// Sum of the waves' partial sums, scaled, cast and stored.  A unit is one lane's four consecutive columns of one row.
+template <Elem T, int MB, int NB, int WAVES>
+__device__ __forceinline__ void finish_tile(const GemmParams &p, f32x4 *red, const WorkItem &t, int g, int n0, const f32x4 (&acc)[MB][NB]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) red[(wave * MB * NB + i * NB + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  const float tile_scale = p.scalar * (p.scalar_dev ? p.scalar_dev[0] : 1.f) * (p.alpha[g] ? p.alpha[g][t.e] : 1.f);
+  for (int u = threadIdx.x; u < MB * NB * 64; u += WAVES * 64) {
+    f32x4 v = red[u];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) v += red[w * MB * NB * 64 + u];
+    const int l = u & 63, b = u >> 6;
+    const int r = (b / NB) * 16 + (l & 15), col = n0 + (b % NB) * 16 + (l >> 4) * 4;
+    if (r >= t.rows || col >= p.n) continue;  // n % 4 == 0: the four columns are all in or all out
+    const int row = t.row_base + t.m0 + r;
+    const float rs = tile_scale * (p.row_scale ? p.row_scale[row] : 1.f);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      v[c] *= rs;
+      if (p.col_scale) v[c] *= p.col_scale[static_cast<int64_t>(t.e) * p.n + col + c];
+    }
+    int64_t drow = row;
+    if (p.scatter_d) {
+      drow = p.scatter_d[row];
+      if (drow < 0 || drow >= p.d_rows) continue;
+    }
+    const int64_t at = drow * p.n + col;
+    if (p.accumulate) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) unsafeAtomicAdd(static_cast<float *>(p.d[g]) + at + c, v[c]);
+    } else if (p.d_fp32) {
+      *reinterpret_cast<f32x4 *>(static_cast<float *>(p.d[g]) + at) = v;
+    } else {
+      u32x2 o;
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        o[c] = T == Elem::F16 ? static_cast<uint32_t>(float_to_f16_bits(v[2 * c])) | (static_cast<uint32_t>(float_to_f16_bits(v[2 * c + 1])) << 16)
+                              : static_cast<uint32_t>(float_to_bf16_bits(v[2 * c])) | (static_cast<uint32_t>(float_to_bf16_bits(v[2 * c + 1])) << 16);
+      *reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(p.d[g]) + at) = o;
+    }
+  }
+}
+
+template <Elem T, int MB, int NB, int WAVES, int DEPTH>
+__device__ __forceinline__ void run_tile(const GemmParams &p, f32x4 *red, const WorkItem &t, int g, int n0) {
+  f32x4 acc[MB][NB];
+  accumulate_tile<T, MB, NB, WAVES, DEPTH>(p, t, g, n0, acc);
+  finish_tile<T, MB, NB, WAVES>(p, red, t, g, n0, acc);
+}
+
+#endif  // __HIP_DEVICE_COMPILE__
+
+
+template <Elem T, int MBMAX, int NB, int WAVES, int DEPTH>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(MBMAX <= 2 ? 4 : 2)))
+void grouped_gemm_stream_kernel(const GemmParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ f32x4 red[WAVES * MBMAX * NB * 64];
+  const int tiles_n1 = (p.n + 16 * NB - 1) / (16 * NB);
+  const WorkItem t = locate<MBMAX>(p, tiles_n1 * p.ngroups);
+  if (!t.valid) return;
+  const int g = p.ngroups > 1 ? t.nt / tiles_n1 : 0;
+  const int n0 = (t.nt - g * tiles_n1) * (16 * NB);
+  if (MBMAX == 1 || t.rows <= 16) {
+    run_tile<T, 1, NB, WAVES, DEPTH>(p, red, t, g, n0);
+  } else if constexpr (MBMAX >= 2) {
+    if (MBMAX == 2 || t.rows <= 32) {
+      run_tile<T, 2, NB, WAVES, (DEPTH > 3 ? 3 : DEPTH)>(p, red, t, g, n0);
+    } else if constexpr (MBMAX >= 4) {
+      run_tile<T, 4, NB, WAVES, (DEPTH > 3 ? 3 : DEPTH)>(p, red, t, g, n0);
+    }
+  }
+#endif
+}
+
+// Most row chunks a launch can have: every expert that gets a row starts one, and `chunk` rows fill one.
+int64_t most_chunks(const GemmParams &p, int chunk) {
+  const int64_t active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
+  return active + (p.max_rows - active) / chunk;
+}
+
+template <Elem T, int MBMAX, int NB, int WAVES, int DEPTH>
+void launch(const GemmParams &p, hipStream_t s) {
+  const int64_t items = most_chunks(p, 16 * MBMAX) * ((p.n + 16 * NB - 1) / (16 * NB)) * p.ngroups;
+  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, MBMAX, NB, WAVES, DEPTH>), dim3(static_cast<unsigned>((items + 7) / 8 * 8)),
+                     dim3(WAVES * 64), 0, s, p);
+}
+
+// Which tile.  Columns per workgroup (NB): 64 reads the rows' own operand least often (its loads share the queue behind the
+// weights' with them: at 9 rows per expert 140 us against 159 for 32 columns, bf16 14336 x 4096), but takes two waves
+// per SIMD; 32 columns with four waves per SIMD is as fast or faster while there is hardly a row (2.5 rows per expert:
+// 108 against 114 us; 3.5 rows, 64 experts: 60 against 68), except block-scaled, whose scales do not fit its 128 registers (73
+// against 70).  Where 64-column tiles would leave compute units without work (512 of them fill the card) it is 32 columns, and
+// eight waves per workgroup if K is long enough to share (two experts, 4096 x 14336: 42 us, four waves 47, 64 columns 61; at K = 2048
+// bytes per row eight waves lose, 17 against 14 us).
+template <Elem T>
+void launch_by_shape(const GemmParams &p, hipStream_t s) {
+  const int64_t lines = (static_cast<int64_t>(p.k) * (is_fp8(T) ? 1 : 2) + 127) / 128;
+  const int64_t items = most_chunks(p, 64) * ((p.n + 63) / 64) * p.ngroups;
+  const bool few = items < 512;
+  if (few && lines >= 64) launch<T, 2, 2, 8, 2>(p, s);
+  else if (few || (T != Elem::FP8_BLOCKSCALED && p.max_rows <= 4 * p.nexperts)) launch<T, 2, 2, 4, 2>(p, s);
+  else launch<T, 4, 4, 4, 2>(p, s);
+}
+
+}  // namespace
+
+// Up to how many rows per expert this form is the faster one (the macro-tile kernel's time hardly depends on the rows while
+// they are few; this one's grows with them): bf16 14336 x 4096 at 24 / 32 / 50 rows 165 / 189 / 214 us against 217 / 219 / 221,
+// 64 experts at 19 / 37 rows 73 / 105 against 112 / 109; fp8 2048 x 7168 at 24 / 32 rows 85 / 95 against 97 / 97, 7168 x 2048
+// 105 / 128 against 118 / 118; block-scaled at 24 / 50 rows 109 / 197 against 124 / 129.
+bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
+  const int64_t rows = dtype == FLUXMI_FP8_E4M3 ? 24 : 40;
+  return p.max_rows <= rows * p.nexperts;
+}
+
+void launch_grouped_gemm_stream(const GemmParams &p, int dtype, hipStream_t s) {
+  if (p.a_scale != nullptr) launch_by_shape<Elem::FP8_BLOCKSCALED>(p, s);
+  else if (dtype == FLUXMI_FP8_E4M3) launch_by_shape<Elem::FP8>(p, s);
+  else if (dtype == FLUXMI_FP16) launch_by_shape<Elem::F16>(p, s);
+  else launch_by_shape<Elem::BF16>(p, s);
+}
+
+}  // namespace fluxmi

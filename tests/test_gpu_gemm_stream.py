@@ -1,0 +1,96 @@
+"""GPU parity of the weight-streaming form of the grouped GEMM (few rows per expert) at the edges of its tiles.
+
+Operands are small integers, so every product and every partial sum is a whole number below 2^24 and the fp32 result is the
+same in any order of summation: the outputs have to equal an int64 matmul exactly, no tolerance.  (`max_rows` at most 24
+rows per expert on average, fp8, or 40, bf16 / fp16, selects the form.)"""
+import pytest
+import torch
+
+from flux_amd import capi
+
+pytestmark = pytest.mark.gpu
+DT = {"bf16": torch.bfloat16, "f16": torch.float16, "fp8": torch.float8_e4m3fn}
+
+
+def small_ints(gen, *shape):
+    return torch.randint(-3, 4, shape, generator=gen)
+
+
+def expected(a, w, splits, rows_of=None):
+    out = torch.zeros(sum(splits), w.shape[1], dtype=torch.int64)
+    at = 0
+    for e, n in enumerate(splits):
+        src = a[at:at + n] if rows_of is None else a[rows_of[at:at + n].long()]
+        out[at:at + n] = src @ w[e].t()
+        at += n
+    return out
+
+
+# (splits, N, K): one row; a chunk of 16 and one more row; 64 rows and one more (two chunks); empty experts and more than 64
+# of them; column tiles cut off at 4 columns; K shorter than a line, ending inside one, and over many lines per wave.
+CASES = [
+    ([1], 4, 16), ([1, 0, 2], 64, 128), ([15, 16, 17], 100, 272), ([33, 0, 64, 65, 2], 132, 1040),
+    ([0] * 70 + [3, 1] + [0] * 8 + [9], 68, 400), ([7, 5], 1028, 8192 + 48), ([2, 3, 1, 4, 2, 0, 1, 5], 4224, 2064),
+    ([40, 1, 22, 30], 704, 176),
+]
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("splits,n,k", CASES)
+def test_stream_form_is_exact_on_integers(dtype, splits, n, k):
+    print(f"[case] stream gemm {dtype} splits={splits[:6]} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(n + k)
+    m, e = sum(splits), len(splits)
+    a, w = small_ints(g, m, k), small_ints(g, e, n, k)
+    ad, wd = a.to(torch.float32).to(DT[dtype]).cuda(), w.to(torch.float32).to(DT[dtype]).cuda()
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    ref = expected(a, w, splits)
+    got, kind = capi.grouped_gemm(ad, wd, sp, out_dtype=torch.float32, want_kind=True)
+    assert kind == 1
+    assert torch.equal(got.cpu().long(), ref)
+    # rows picked by a gather, results put elsewhere, every scale factor (powers of two) and a second weight tensor
+    perm = torch.randperm(m, generator=g).to(torch.int32)
+    row_scale = 2.0 ** torch.randint(-1, 2, (m,), generator=g)
+    alpha = 2.0 ** torch.randint(-1, 2, (e,), generator=g)
+    out = torch.full((m, n), -7.0, device="cuda")
+    capi.grouped_gemm(ad, wd, sp, out=out, gather_a=perm.cuda(), scatter_d=perm.flip(0).contiguous().cuda(),
+                      row_scale=row_scale.cuda(), alpha=alpha.cuda())
+    per_row = torch.repeat_interleave(alpha, torch.tensor(splits)) * row_scale
+    want = torch.empty(m, n, dtype=torch.float64)
+    want[perm.flip(0).long()] = expected(a, w, splits, perm).double() * per_row[:, None].double()
+    assert torch.equal(out.cpu().double(), want)
+    two = capi.grouped_gemm_multi(ad, [wd, wd.flip(0).contiguous()] if dtype != "fp8" else [wd, wd], sp, out_dtype=torch.float32)
+    assert torch.equal(two[0].cpu().long(), ref)
+    assert torch.equal(two[1].cpu().long(), expected(a, w.flip(0) if dtype != "fp8" else w, splits))
+
+
+@pytest.mark.parametrize("splits,n,k", [([1], 128, 128), ([16, 0, 17, 2], 256, 384), ([33, 31, 5], 384, 2048), ([2, 1], 132, 8192)])
+@pytest.mark.parametrize("a_layout", [capi.ASCALE_BLOCK128, capi.ASCALE_EXPERT_K_M])
+@pytest.mark.parametrize("b_layout", [capi.BSCALE_N_K, capi.BSCALE_K_N])
+def test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b_layout):
+    print(f"[case] stream gemm block-scaled splits={splits} n={n} k={k} layouts {a_layout} {b_layout}", flush=True)
+    g = torch.Generator().manual_seed(n + k)
+    m, e, kb, nb = sum(splits), len(splits), k // 128, (n + 127) // 128
+    a, w = small_ints(g, m, k), small_ints(g, e, n, k)
+    sa = 2.0 ** torch.randint(-1, 2, (m, kb), generator=g)
+    sb = 2.0 ** torch.randint(-1, 2, (e, nb, kb), generator=g)
+    if a_layout == capi.ASCALE_BLOCK128:
+        pad = torch.zeros((m + 127) // 128 * 128, kb)
+        pad[:m] = sa
+        sad = pad.view(-1, 128, kb).permute(0, 2, 1).contiguous()
+    else:
+        at, parts = 0, []
+        for r in splits:
+            parts.append(sa[at:at + r].t().contiguous().flatten())
+            at += r
+        sad = torch.cat(parts)
+    sbd = sb if b_layout == capi.BSCALE_N_K else sb.transpose(1, 2).contiguous()
+    got = capi.grouped_gemm_blockscale(a.float().to(DT["fp8"]).cuda(), w.float().to(DT["fp8"]).cuda(),
+                                       torch.tensor(splits, dtype=torch.int32, device="cuda"), sad.cuda(), sbd.cuda(), a_layout,
+                                       b_layout, out_dtype=torch.float32)
+    af = a.double() * torch.repeat_interleave(sa.double(), 128, dim=1)
+    wf = w.double() * torch.repeat_interleave(torch.repeat_interleave(sb.double(), 128, dim=1)[:, :n], 128, dim=2)
+    at = 0
+    for i, r in enumerate(splits):
+        assert torch.equal(got[at:at + r].cpu().double(), af[at:at + r] @ wf[i].t()), f"expert {i}"
+        at += r
