@@ -224,3 +224,22 @@ def test_block128_all_bit_patterns_both_directions():
         finite = np.repeat(np.isfinite(f).all(axis=2), 128, axis=1)  # per (row, block), spread over its columns
         assert np.array_equal(gq[finite], rq[finite])
         assert np.array_equal(got_s.cpu().numpy().view(np.uint32), rs.view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,cols", [
+    (127, 136), (129, 128), (136, 264), (255, 8), (272, 392), (383, 136), (1029, 1160), (1031, 1029)])
+def test_transposed_rows_at_any_alignment(rows, cols):
+    """The transposed copy where its rows start at any byte (rows not a multiple of 16, nor of anything) and tiles meet
+    inside cache lines; 90 tiles, no multiple of the eight XCDs: both block forms, bytes bit-exact."""
+    from flux_amd import capi
+    print(f"[case] quant transposed any alignment rows={rows} cols={cols}", flush=True)
+    rng = np.random.default_rng(rows * 41 + cols)
+    x = (rng.standard_normal((rows, cols)) * rng.uniform(1e-3, 50, size=(rows, 1))).astype(np.float32)
+    bits = to_bits(torch.from_numpy(x).to(torch.bfloat16))
+    xd = torch.from_numpy(bits.view(np.int16).copy()).view(torch.bfloat16).cuda()
+    rqt, rst = quant.quant_rows_c(np.ascontiguousarray(bits.T), 128, 0.0, True)
+    _, _, qt, st = capi.quant_e4m3_block128(xd, 0.0, True)
+    assert np.array_equal(qt.view(torch.uint8).cpu().numpy(), rqt) and np.array_equal(st.cpu().numpy(), rst)
+    rq, _ = quant.quant_square_c(bits)
+    q, _, qt, _ = run_square(bits, 0.0, True)
+    assert np.array_equal(q, rq) and np.array_equal(qt, rq.T)
