@@ -211,11 +211,11 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   hipStream_t s = static_cast<hipStream_t>(stream);
   int cus = fluxmi_device_cu_count();
   FLUXMI_REQUIRE(cus > 0, FLUXMI_ERR_HIP, "grouped_gemm: cannot query the device");
-  // CUs left to other work of the caller (Flux's sm_margin): the persistent kernel launches fewer workgroups.
+  // CUs left to other work of the caller (Flux's sm_margin): both MFMA forms launch fewer workgroups.
   cus = cus - args->cu_margin > 1 ? cus - args->cu_margin : 1;
 
   if (mfma && grouped_gemm_stream_takes(p, args->dtype)) {
-    launch_grouped_gemm_stream(p, args->dtype, s);
+    launch_grouped_gemm_stream(p, args->dtype, args->cu_margin > 0 ? cus : 0, s);
   } else if (mfma) {
     // Upper bound of the tile count: never launch more workgroups than tiles.
     const int64_t tiles_n = (args->n + BN - 1) / BN * ngroups;

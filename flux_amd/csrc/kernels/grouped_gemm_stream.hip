@@ -52,7 +52,7 @@ __device__ __forceinline__ int row_chunks(int rows) { return (rows + 16 * MBMAX 
 // Work item -> (expert, row chunk, column tile).  One wave-wide pass over the splits counts the chunks, a second finds
 // the item; with up to 64 experts both work on the same registers.
 template <int MBMAX>
-__device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n) {
+__device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n, int block) {
   const int lane = threadIdx.x & 63;
   auto load = [&](int e0, int &carry, int &begin, int &rows) {
     const int ee = e0 + lane;
@@ -74,8 +74,8 @@ __device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n) {
   // Workgroups are dealt to the eight XCDs round-robin.
   const int items = total * tiles_n;
   const int per_xcd = (items + 7) / 8;
-  const int i = blockIdx.x >> 3;
-  int item = (blockIdx.x & 7) * per_xcd + i;
+  const int i = block >> 3;
+  int item = (block & 7) * per_xcd + i;
   WorkItem w = {false, 0, 0, 0, 0, 0, 0};
   if (i >= per_xcd || item >= items) return w;
   carry = 0;
@@ -324,25 +324,33 @@ __device__ __forceinline__ void run_tile(const GemmParams &p, f32x4 *red, const 
 #endif  // __HIP_DEVICE_COMPILE__
 
 
-template <Elem T, int MBMAX, int NB, int WAVES, int DEPTH>
+// WALK: workgroups walk the `blocks` items with the grid's stride (a launch cut down to leave compute units free); otherwise
+// there is one workgroup per item.  A form of its own because the loop costs the other one up to ten spilled registers.
+template <Elem T, int MBMAX, int NB, int WAVES, int DEPTH, bool WALK>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(MBMAX <= 2 ? 4 : 2)))
-void grouped_gemm_stream_kernel(const GemmParams p) {
+void grouped_gemm_stream_kernel(const GemmParams p, const int blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
   __shared__ f32x4 red[WAVES * MBMAX * NB * 64];
   const int tiles_n1 = (p.n + 16 * NB - 1) / (16 * NB);
-  const WorkItem t = locate<MBMAX>(p, tiles_n1 * p.ngroups);
-  if (!t.valid) return;
-  const int g = p.ngroups > 1 ? t.nt / tiles_n1 : 0;
-  const int n0 = (t.nt - g * tiles_n1) * (16 * NB);
-  if (MBMAX == 1 || t.rows <= 16) {
-    run_tile<T, 1, NB, WAVES, DEPTH>(p, red, t, g, n0);
-  } else if constexpr (MBMAX >= 2) {
-    if (MBMAX == 2 || t.rows <= 32) {
-      run_tile<T, 2, NB, WAVES, (DEPTH > 3 ? 3 : DEPTH)>(p, red, t, g, n0);
-    } else if constexpr (MBMAX >= 4) {
-      run_tile<T, 4, NB, WAVES, (DEPTH > 3 ? 3 : DEPTH)>(p, red, t, g, n0);
+  int block = blockIdx.x;
+  do {
+    const WorkItem t = locate<MBMAX>(p, tiles_n1 * p.ngroups, block);
+    if (t.valid) {
+      const int g = p.ngroups > 1 ? t.nt / tiles_n1 : 0;
+      const int n0 = (t.nt - g * tiles_n1) * (16 * NB);
+      if (MBMAX == 1 || t.rows <= 16) {
+        run_tile<T, 1, NB, WAVES, DEPTH>(p, red, t, g, n0);
+      } else if constexpr (MBMAX >= 2) {
+        if (MBMAX == 2 || t.rows <= 32) {
+          run_tile<T, 2, NB, WAVES, (DEPTH > 3 ? 3 : DEPTH)>(p, red, t, g, n0);
+        } else if constexpr (MBMAX >= 4) {
+          run_tile<T, 4, NB, WAVES, (DEPTH > 3 ? 3 : DEPTH)>(p, red, t, g, n0);
+        }
+      }
     }
-  }
+    if constexpr (WALK) __syncthreads();  // `red` has been read before the next item's sums go into it
+    block += gridDim.x;
+  } while (WALK && block < blocks);
 #endif
 }
 
@@ -352,11 +360,21 @@ int64_t most_chunks(const GemmParams &p, int chunk) {
   return active + (p.max_rows - active) / chunk;
 }
 
+// With compute units to be left to other work (`cus` of them may be used; 0: all), no more workgroups than these hold at
+// once; each then walks several items, so the results do not change.
 template <Elem T, int MBMAX, int NB, int WAVES, int DEPTH>
-void launch(const GemmParams &p, hipStream_t s) {
+void launch(const GemmParams &p, int cus, hipStream_t s) {
   const int64_t items = most_chunks(p, 16 * MBMAX) * ((p.n + 16 * NB - 1) / (16 * NB)) * p.ngroups;
-  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, MBMAX, NB, WAVES, DEPTH>), dim3(static_cast<unsigned>((items + 7) / 8 * 8)),
-                     dim3(WAVES * 64), 0, s, p);
+  const int64_t blocks = (items + 7) / 8 * 8;
+  if (cus == 0) {
+    hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, MBMAX, NB, WAVES, DEPTH, false>), dim3(static_cast<unsigned>(blocks)),
+                       dim3(WAVES * 64), 0, s, p, static_cast<int>(blocks));
+    return;
+  }
+  constexpr int resident = (MBMAX <= 2 ? 16 : 8) / WAVES;  // waves a compute unit holds / waves per workgroup
+  const int64_t most = (static_cast<int64_t>(cus) * resident + 7) / 8 * 8;  // a multiple of the XCDs
+  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, MBMAX, NB, WAVES, DEPTH, true>), dim3(static_cast<unsigned>(blocks < most ? blocks : most)),
+                     dim3(WAVES * 64), 0, s, p, static_cast<int>(blocks));
 }
 
 // Which tile.  Columns per workgroup (NB): 64 reads the rows' own operand least often (its loads share the queue behind the
@@ -367,13 +385,13 @@ void launch(const GemmParams &p, hipStream_t s) {
 // eight waves per workgroup if K is long enough to share (two experts, 4096 x 14336: 42 us, four waves 47, 64 columns 61; at K = 2048
 // bytes per row eight waves lose, 17 against 14 us).
 template <Elem T>
-void launch_by_shape(const GemmParams &p, hipStream_t s) {
+void launch_by_shape(const GemmParams &p, int cus, hipStream_t s) {
   const int64_t lines = (static_cast<int64_t>(p.k) * (is_fp8(T) ? 1 : 2) + 127) / 128;
   const int64_t items = most_chunks(p, 64) * ((p.n + 63) / 64) * p.ngroups;
   const bool few = items < 512;
-  if (few && lines >= 64) launch<T, 2, 2, 8, 2>(p, s);
-  else if (few || (T != Elem::FP8_BLOCKSCALED && p.max_rows <= 4 * p.nexperts)) launch<T, 2, 2, 4, 2>(p, s);
-  else launch<T, 4, 4, 4, 2>(p, s);
+  if (few && lines >= 64) launch<T, 2, 2, 8, 2>(p, cus, s);
+  else if (few || (T != Elem::FP8_BLOCKSCALED && p.max_rows <= 4 * p.nexperts)) launch<T, 2, 2, 4, 2>(p, cus, s);
+  else launch<T, 4, 4, 4, 2>(p, cus, s);
 }
 
 }  // namespace
@@ -387,11 +405,11 @@ bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
   return p.max_rows <= rows * p.nexperts;
 }
 
-void launch_grouped_gemm_stream(const GemmParams &p, int dtype, hipStream_t s) {
-  if (p.a_scale != nullptr) launch_by_shape<Elem::FP8_BLOCKSCALED>(p, s);
-  else if (dtype == FLUXMI_FP8_E4M3) launch_by_shape<Elem::FP8>(p, s);
-  else if (dtype == FLUXMI_FP16) launch_by_shape<Elem::F16>(p, s);
-  else launch_by_shape<Elem::BF16>(p, s);
+void launch_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, hipStream_t s) {
+  if (p.a_scale != nullptr) launch_by_shape<Elem::FP8_BLOCKSCALED>(p, cus, s);
+  else if (dtype == FLUXMI_FP8_E4M3) launch_by_shape<Elem::FP8>(p, cus, s);
+  else if (dtype == FLUXMI_FP16) launch_by_shape<Elem::F16>(p, cus, s);
+  else launch_by_shape<Elem::BF16>(p, cus, s);
 }
 
 }  // namespace fluxmi

@@ -7,6 +7,7 @@ namespace fluxmi {
 
 // Whether a launch that the MFMA kernels can take goes to this form: few rows per expert on average.
 bool grouped_gemm_stream_takes(const GemmParams &p, int dtype);
-void launch_grouped_gemm_stream(const GemmParams &p, int dtype, hipStream_t s);
+// cus: compute units it may use, 0 for all of them.
+void launch_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, hipStream_t s);
 
 }  // namespace fluxmi

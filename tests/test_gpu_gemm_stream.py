@@ -94,3 +94,16 @@ def test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b
     for i, r in enumerate(splits):
         assert torch.equal(got[at:at + r].cpu().double(), af[at:at + r] @ wf[i].t()), f"expert {i}"
         at += r
+
+
+@pytest.mark.parametrize("margin", [1, 100, 255, 1000])
+@pytest.mark.parametrize("splits,n,k", [([2, 3, 1, 4, 2, 0, 1, 5], 4224, 2064), ([33, 0, 64, 65, 2], 4096, 528), ([1] * 80, 1028, 400)])
+def test_stream_form_leaves_compute_units_and_changes_no_bit(splits, n, k, margin):
+    """With `cu_margin` few workgroups walk all items (down to one compute unit's worth)."""
+    print(f"[case] stream gemm margin={margin} splits={splits[:6]} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(n + k)
+    a = torch.randn(sum(splits), k, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(len(splits), n, k, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    base = capi.grouped_gemm(a, w, sp)
+    assert torch.equal(capi.grouped_gemm(a, w, sp, cu_margin=margin), base)
