@@ -225,7 +225,7 @@ __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkI
       l.bs = p.b_scale[b_base + kblk * b_kstep];
     }
   };
-  auto use_line = [&](Line<T, MB, NB> &l) {
+  auto use_line = [&](Line<T, MB, NB> &l, int line) {
 #pragma unroll
     for (int j = 0; j < NB; ++j) to_fragments(l.w[j]);
 #pragma unroll
@@ -233,7 +233,8 @@ __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkI
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
       if constexpr (T == Elem::FP8_BLOCKSCALED) {
-        const float s = l.as[i] * l.bs;
+        // A line past K has zero operands and the scales of block 0, whose product may be infinite: 0 * inf is not 0.
+        const float s = line < kblocks ? l.as[i] * l.bs : 0.f;
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
           const f32x4 b = mfma_line<T>(l.w[j], l.x[i], f32x4{0.f, 0.f, 0.f, 0.f});
@@ -260,7 +261,7 @@ __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkI
   for (int s = 0; s < steps; s += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
-      use_line(ring[d]);
+      use_line(ring[d], (s + d) * WAVES + wave);
       __builtin_amdgcn_sched_barrier(0);
       load_line(ring[d], (s + d + DEPTH) * WAVES + wave);
       __builtin_amdgcn_sched_barrier(0);

@@ -96,6 +96,33 @@ def test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b
         at += r
 
 
+@pytest.mark.parametrize("kblocks,rows,n,experts", [(1, 3, 128, 1), (3, 3, 128, 1), (7, 3, 256, 2), (8, 3, 128, 1), (9, 3, 128, 1),
+                                                    (65, 3, 128, 1), (3, 7, 2176, 24), (9, 7, 2176, 24)])
+def test_stream_form_block_scaled_infinite_scales(kblocks, rows, n, experts):
+    """An infinite product of scales (each of them finite, or one infinite) makes a result infinite, not NaN, whatever K is
+    padded to inside the kernel.  Codes 1 ... 3, so every block's sum is positive; fp32 results, exact integers or +inf."""
+    print(f"[case] stream gemm infinite scales kblocks={kblocks} rows={rows} n={n} experts={experts}", flush=True)
+    k, m = kblocks * 128, rows * experts
+    g = torch.Generator().manual_seed(kblocks)
+    a, w = torch.randint(1, 4, (m, k), generator=g), torch.randint(1, 4, (experts, n, k), generator=g)
+    sa, sb = torch.ones(m, kblocks), torch.ones(experts, n // 128, kblocks)
+    sa[1::rows, 0], sb[:, 0, 0] = 2.0 ** 100, 2.0 ** 100  # each row 1 of an expert overflows in its first 128 columns
+    sa[2::rows, kblocks - 1] = float("inf")              # each row 2 is infinite everywhere
+    pad = torch.zeros((m + 127) // 128 * 128, kblocks)
+    pad[:m] = sa
+    got = capi.grouped_gemm_blockscale(a.float().to(DT["fp8"]).cuda(), w.float().to(DT["fp8"]).cuda(),
+                                       torch.full((experts,), rows, dtype=torch.int32, device="cuda"),
+                                       pad.view(-1, 128, kblocks).permute(0, 2, 1).contiguous().cuda(), sb.cuda(),
+                                       out_dtype=torch.float32).cpu()
+    blocks = torch.einsum("erkc,enkc->ernk", a.view(experts, rows, kblocks, 128).float(), w.view(experts, n, kblocks, 128).float())
+    scale = sa.view(experts, rows, 1, kblocks) * torch.repeat_interleave(sb, 128, dim=1).unsqueeze(1)  # fp32: overflows here
+    ref = (blocks * scale).sum(-1).view(m, n)
+    assert torch.isinf(ref[1, 0]) and torch.isinf(ref[2]).all() and torch.isfinite(ref[0]).all()
+    inf = torch.isinf(ref)
+    assert torch.equal(torch.isinf(got) & (got > 0), inf)
+    assert torch.allclose(got[~inf].double(), ref[~inf].double(), rtol=1e-5, atol=0)
+
+
 @pytest.mark.parametrize("margin", [1, 100, 255, 1000])
 @pytest.mark.parametrize("splits,n,k", [([2, 3, 1, 4, 2, 0, 1, 5], 4224, 2064), ([33, 0, 64, 65, 2], 4096, 528), ([1] * 80, 1028, 400)])
 def test_stream_form_leaves_compute_units_and_changes_no_bit(splits, n, k, margin):
