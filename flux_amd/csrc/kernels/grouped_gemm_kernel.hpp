@@ -150,12 +150,26 @@ __device__ __forceinline__ float sum_read(float a) {
   else return acc_read(a);
 }
 
-// Compile-time loop: f(integral_constant<int, I>) for I in [0, N).
-template <int I, int N, class F>
+// Compile-time loop: f(integral_constant<int, I>) for I in [FIRST, END).
+template <int FIRST, class F, int... I>
+__device__ __forceinline__ void static_for_seq(F &f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, FIRST + I>{}), ...);
+}
+template <int FIRST, int END, class F>
 __device__ __forceinline__ void static_for(F &&f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
+  if constexpr (FIRST < END) static_for_seq<FIRST>(f, std::make_integer_sequence<int, END - FIRST>{});
+}
+
+// Compile-time loop over the I in [0, N) with I * MUL / DIV == AT: what falls into slot AT when N things are spread over
+// N * MUL / DIV slots.  A loop over all N that drops the others inside f gives the same instructions, but leaves the compiler about
+// 100000 empty functions per translation unit to inline: nine tenths of the compile time (bf16: 24 minutes, 3 like this).
+template <int N, int MUL, int DIV, int AT, class F>
+__device__ __forceinline__ void static_for_slot(F &&f) {
+  if constexpr (MUL == 0) {  // a single slot
+    if constexpr (AT == 0) static_for<0, N>(f);
+  } else if constexpr (AT >= 0) {
+    constexpr int first = (AT * DIV + MUL - 1) / MUL, end = ((AT + 1) * DIV + MUL - 1) / MUL;
+    static_for<first, (end < N ? end : N)>(f);
   }
 }
 
@@ -884,37 +898,35 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *smem, co
     __builtin_amdgcn_sched_barrier(0);
     static_for<0, NM>([&](auto T) {
       constexpr int t = decltype(T)::value;
-      static_for<0, NR>([&](auto R) {
-        constexpr int r = decltype(R)::value;
-        if constexpr (r * RSPAN / NR == t) read_one(std::integral_constant<int, (u + 1) % STG>{}, R, xn, wn_);
-      });
+      static_for_slot<NR, RSPAN, NR, t>([&](auto R) { read_one(std::integral_constant<int, (u + 1) % STG>{}, R, xn, wn_); });
       // Loads of this slot first, M0 writes for the loads of the next slot after them: a whole fill placed
       // here (fill_one writes M0 itself) must not come between another fill's M0 write and its load.
-      static_for<0, 2 * LOADS>([&](auto D) {
+      // Fill d of the pair goes into slot d * 2 NM / (2 LOADS) + 1 of the pair's 2 NM (the last one's successor: slot 0).
+      constexpr int pair_t = t + (even ? 0 : NM);
+      static_for_slot<2 * LOADS, 2 * NM, 2 * LOADS, (pair_t + 2 * NM - 1) % (2 * NM)>([&](auto D) {
         constexpr int d = decltype(D)::value;
         constexpr int at = (d * (2 * NM) / (2 * LOADS) + 1) % (2 * NM);
-        if constexpr (at == t + (even ? 0 : NM)) {
-          if constexpr (guarded) {
-            constexpr int q = d >> 1, h = d & 1, slot = (e0 + LA + h) % STG;
-            const bool ok = c.fill_chunk * 16 < valid[h];
-            if constexpr (q < XLOADS) {
-              const uint8_t *src = ok ? xbase + gk[h] + xoff[q] : g_zero_page + lane * 16;
-              __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(xdst + slot * SB + q * 1024), 16, 0, 0);
-            } else {
-              const uint8_t *src = ok ? wbase + gk[h] + woff[q - XLOADS] : g_zero_page + lane * 16;
-              __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(wdst + slot * SB + (q - XLOADS) * 1024), 16, 0, W_AUX);
-            }
-          } else if constexpr (SPLIT_M0 && at % NM != 0)  // the slot before is in the same step: M0 was written there
-            fill_go(std::integral_constant<int, (d >> 1)>{}, kbase + (e0 + LA + (d & 1)) * KBYTES);
-          else
-            fill_one(std::integral_constant<int, (e0 + LA + (d & 1)) % STG>{}, std::integral_constant<int, (d >> 1)>{},
-                     kbase + (e0 + LA + (d & 1)) * KBYTES);
-        }
+        static_assert(at == pair_t);
+        if constexpr (guarded) {
+          constexpr int q = d >> 1, h = d & 1, slot = (e0 + LA + h) % STG;
+          const bool ok = c.fill_chunk * 16 < valid[h];
+          if constexpr (q < XLOADS) {
+            const uint8_t *src = ok ? xbase + gk[h] + xoff[q] : g_zero_page + lane * 16;
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(xdst + slot * SB + q * 1024), 16, 0, 0);
+          } else {
+            const uint8_t *src = ok ? wbase + gk[h] + woff[q - XLOADS] : g_zero_page + lane * 16;
+            __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(wdst + slot * SB + (q - XLOADS) * 1024), 16, 0, W_AUX);
+          }
+        } else if constexpr (SPLIT_M0 && at % NM != 0)  // the slot before is in the same step: M0 was written there
+          fill_go(std::integral_constant<int, (d >> 1)>{}, kbase + (e0 + LA + (d & 1)) * KBYTES);
+        else
+          fill_one(std::integral_constant<int, (e0 + LA + (d & 1)) % STG>{}, std::integral_constant<int, (d >> 1)>{},
+                   kbase + (e0 + LA + (d & 1)) * KBYTES);
       });
-      static_for<0, 2 * LOADS>([&](auto D) {
+      static_for_slot<2 * LOADS, 2 * NM, 2 * LOADS, pair_t>([&](auto D) {
         constexpr int d = decltype(D)::value;
         constexpr int at = (d * (2 * NM) / (2 * LOADS) + 1) % (2 * NM);
-        if constexpr (!guarded && SPLIT_M0 && at % NM != 0 && at - 1 == t + (even ? 0 : NM))
+        if constexpr (!guarded && SPLIT_M0 && at % NM != 0)
           fill_m0(std::integral_constant<int, (e0 + LA + (d & 1)) % STG>{}, std::integral_constant<int, (d >> 1)>{});
       });
       mfma_slot<ELT, MBK, NBK>(t, xc, wc, acc);
@@ -1130,30 +1142,24 @@ __device__ __forceinline__ void gemm_tile_lines(const GemmParams &p, uint8_t *sm
     __builtin_amdgcn_sched_barrier(0);
     static_for<0, NM>([&](auto T) {
       constexpr int t = decltype(T)::value;
-      static_for<0, NR>([&](auto R) {
-        constexpr int r = decltype(R)::value;
-        if constexpr (r * RSPAN / NR == t) read_one(std::integral_constant<int, u + 1>{}, R, xn, wn_);
-      });
-      static_for<0, NF>([&](auto Q) {
-        constexpr int q = decltype(Q)::value;
-        if constexpr (guarded) {
-          if constexpr (q * NM / NF == t) {
+      static_for_slot<NR, RSPAN, NR, t>([&](auto R) { read_one(std::integral_constant<int, u + 1>{}, R, xn, wn_); });
+      if constexpr (SPLIT) {
+        static_for_slot<NF, NM, NF, t - 1>([&](auto Q) { fill_go(IsW{}, Q, kbyte); });
+        static_for_slot<NF, NM, NF, t>([&](auto Q) { fill_m0(IsW{}, std::integral_constant<int, fslot>{}, Q); });
+      } else {
+        static_for_slot<NF, NM, NF, t>([&](auto Q) {
+          if constexpr (guarded) {
+            constexpr int q = decltype(Q)::value;
             uint32_t off;
             if constexpr (even) off = woff[q];
             else off = xoff[q];
             const uint8_t *src = c.lfill_byte[q & 1] < valid ? gbase + off : g_zero_page + c.lane * 16;
             __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)((even ? wdst : xdst) + fslot * UB + q * 1024), 16, 0, 0);
+          } else {
+            fill_one(IsW{}, std::integral_constant<int, fslot>{}, Q, kbyte);
           }
-        } else if constexpr (SPLIT) {
-          if constexpr (q * NM / NF + 1 == t) fill_go(IsW{}, Q, kbyte);
-        } else {
-          if constexpr (q * NM / NF == t) fill_one(IsW{}, std::integral_constant<int, fslot>{}, Q, kbyte);
-        }
-      });
-      static_for<0, NF>([&](auto Q) {
-        constexpr int q = decltype(Q)::value;
-        if constexpr (SPLIT && q * NM / NF == t) fill_m0(IsW{}, std::integral_constant<int, fslot>{}, Q);
-      });
+        });
+      }
       mfma_slot<ELT, MBK, NBK>(t, xc, wc, acc);
       __builtin_amdgcn_sched_barrier(0);
     });
@@ -1421,10 +1427,7 @@ __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8
       constexpr int b = (tt >> 2) * 2 + (tt & 1), h = (tt >> 1) & 1;
       if constexpr (tt < NBLK) {
         // first half: the fills of pair kb + 2
-        static_for<0, PAIRF>([&](auto Q) {
-          constexpr int q = decltype(Q)::value;
-          if constexpr (q * NBLK / PAIRF == tt) fill(std::integral_constant<int, (u + 2) % NSTG>{}, Q, kb + 2);
-        });
+        static_for_slot<PAIRF, NBLK, PAIRF, tt>([&](auto Q) { fill(std::integral_constant<int, (u + 2) % NSTG>{}, Q, kb + 2); });
       } else {
         if constexpr (tt == NBLK) {
           // pair kb + 1 has landed (everything but the fills just issued), for every wave's share
@@ -1432,10 +1435,7 @@ __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8
           __builtin_amdgcn_s_barrier();
           __builtin_amdgcn_sched_barrier(0);
         }
-        static_for<0, NREADS>([&](auto R) {
-          constexpr int r = decltype(R)::value;
-          if constexpr (r * NBLK / NREADS == tt - NBLK) read_one(std::integral_constant<int, (u + 1) % NSTG>{}, R, nxt, snxt);
-        });
+        static_for_slot<NREADS, NBLK, NREADS, tt - NBLK>([&](auto R) { read_one(std::integral_constant<int, (u + 1) % NSTG>{}, R, nxt, snxt); });
       }
       if constexpr (h == 0) blk[b] = mfma(cur, b / NBK, b % NBK, 0, Acc{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f});
       else blk[b] = mfma(cur, b / NBK, b % NBK, 1, blk[b]);
