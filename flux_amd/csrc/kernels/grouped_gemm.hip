@@ -111,15 +111,22 @@ extern "C" size_t fluxmi_grouped_gemm_workspace_bytes(const fluxmi_grouped_gemm_
 namespace fluxmi {
 namespace {
 
-// dry_run: check the arguments and report which kernel would run (1 MFMA, 0 generic) without launching.
-// accumulate_rows > 0: D is fp32 with that many rows and results are added to it atomically.
 struct BlockScales {
   const float *a_scale = nullptr, *b_scale = nullptr;
   int32_t a_layout = 0, b_layout = 0;
 };
 
+// What a launch would be, without launching it; cus: the compute units of the device it is asked for.
+struct DryRun {
+  int cus = 0;
+  bool stream = false, macro = false;
+  StreamPlan plan = {};
+};
+
+// dry_run: check the arguments and report which kernel would run (1 MFMA, 0 generic) without launching.
+// accumulate_rows > 0: D is fp32 with that many rows and results are added to it atomically.
 int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const void *const *b, void *const *d,
-                     const float *const *alpha, void *stream, bool dry_run = false, int32_t accumulate_rows = 0,
+                     const float *const *alpha, void *stream, DryRun *dry_run = nullptr, int32_t accumulate_rows = 0,
                      const BlockScales *bs = nullptr) {
   FLUXMI_REQUIRE(args != nullptr, FLUXMI_ERR_INVALID_ARG, "grouped_gemm: null args");
   FLUXMI_REQUIRE(args->dtype == FLUXMI_BF16 || args->dtype == FLUXMI_FP8_E4M3 || args->dtype == FLUXMI_FP16, FLUXMI_ERR_INVALID_ARG,
@@ -207,16 +214,27 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   p.raster_rows = args->raster_rows > 0 ? args->raster_rows : 8;
   p.sched_flags = args->sched_flags;
 
-  if (dry_run) return mfma ? 1 : 0;
+  const bool stream_form = mfma && grouped_gemm_stream_takes(p, args->dtype);
+  const bool macro = mfma && (!stream_form || args->max_rows > kStreamRows);
+  p.stream_rows = stream_form && macro ? kStreamRows : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  int cus = fluxmi_device_cu_count();
-  FLUXMI_REQUIRE(cus > 0, FLUXMI_ERR_HIP, "grouped_gemm: cannot query the device");
+  int cus = dry_run ? dry_run->cus : fluxmi_device_cu_count();
+  FLUXMI_REQUIRE(cus > 0 || dry_run, FLUXMI_ERR_HIP, "grouped_gemm: cannot query the device");
   // CUs left to other work of the caller (Flux's sm_margin): both MFMA forms launch fewer workgroups.
   cus = cus - args->cu_margin > 1 ? cus - args->cu_margin : 1;
+  const StreamPlan plan = stream_form ? plan_grouped_gemm_stream(p, args->dtype, cus, args->cu_margin > 0) : StreamPlan{};
+  if (dry_run) {
+    dry_run->stream = stream_form;
+    dry_run->macro = macro;
+    dry_run->plan = plan;
+    return mfma ? 1 : 0;
+  }
 
-  if (mfma && grouped_gemm_stream_takes(p, args->dtype)) {
-    launch_grouped_gemm_stream(p, args->dtype, args->cu_margin > 0 ? cus : 0, s);
-  } else if (mfma) {
+  if (stream_form) {
+    const int rc = launch_grouped_gemm_stream(p, args->dtype, plan, s);
+    if (rc != FLUXMI_OK) return rc;
+  }
+  if (macro) {
     // Upper bound of the tile count: never launch more workgroups than tiles.
     const int64_t tiles_n = (args->n + BN - 1) / BN * ngroups;
     const int64_t max_tiles = (static_cast<int64_t>(args->max_rows) / BM + args->nexperts) * tiles_n;
@@ -237,7 +255,8 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
                    : args->dtype == FLUXMI_FP16 ? launch_grouped_gemm_f16(p, grid, s)  // the half-line form only
                                                 : (lines ? launch_grouped_gemm_fp8_lines(p, grid, s) : launch_grouped_gemm_fp8(p, grid, s));
     if (rc != FLUXMI_OK) return rc;
-  } else {
+  }
+  if (!mfma) {
     const int grid = cus * 8;
     for (int g = 0; g < ngroups; ++g) {
       if (args->dtype != FLUXMI_FP8_E4M3)
@@ -323,7 +342,7 @@ extern "C" int fluxmi_grouped_gemm_topk_reduce(const fluxmi_grouped_gemm_args *a
   const void *b = a.b;
   void *d = workspace;
   const float *alpha = a.alpha;
-  const int rc = run_grouped_gemm(&a, 1, &b, &d, &alpha, stream, false, ntokens);
+  const int rc = run_grouped_gemm(&a, 1, &b, &d, &alpha, stream, nullptr, ntokens);
   if (rc != FLUXMI_OK) return rc;
   if (args->dtype == FLUXMI_FP16)
     hipLaunchKernelGGL(cast_f32x4_half_kernel<true>, dim3(grid), dim3(256), 0, s, static_cast<const float4 *>(workspace),
@@ -347,7 +366,7 @@ extern "C" int fluxmi_grouped_gemm_blockscale(const fluxmi_grouped_gemm_args *ar
   const void *b = args->b;
   void *d = args->d;
   const float *alpha = args->alpha;
-  return fluxmi::run_grouped_gemm(args, 1, &b, &d, &alpha, stream, false, 0, &bs);
+  return fluxmi::run_grouped_gemm(args, 1, &b, &d, &alpha, stream, nullptr, 0, &bs);
 }
 
 extern "C" int fluxmi_grouped_gemm_kernel_kind(const fluxmi_grouped_gemm_args *args) {
@@ -355,7 +374,41 @@ extern "C" int fluxmi_grouped_gemm_kernel_kind(const fluxmi_grouped_gemm_args *a
   const void *b = args->b;
   void *d = args->d;
   const float *alpha = args->alpha;
-  return fluxmi::run_grouped_gemm(args, 1, &b, &d, &alpha, nullptr, /*dry_run=*/true);
+  fluxmi::DryRun dry;
+  return fluxmi::run_grouped_gemm(args, 1, &b, &d, &alpha, nullptr, &dry);
+}
+
+extern "C" int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
+                                               const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_launch_info *info) {
+  using namespace fluxmi;
+  FLUXMI_REQUIRE(args != nullptr && info != nullptr, FLUXMI_ERR_INVALID_ARG, "grouped_gemm_launch_info: null args / info");
+  FLUXMI_REQUIRE(cu_count >= 1, FLUXMI_ERR_INVALID_ARG, "grouped_gemm_launch_info: cu_count must be positive");
+  FLUXMI_REQUIRE(ngroups >= 1 && ngroups <= kMaxWeightGroups, FLUXMI_ERR_UNSUPPORTED, "grouped_gemm_launch_info: ngroups=%d outside [1,%d]",
+                 ngroups, kMaxWeightGroups);
+  const void *b[kMaxWeightGroups];
+  void *d[kMaxWeightGroups];
+  const float *alpha[kMaxWeightGroups];
+  for (int g = 0; g < kMaxWeightGroups; ++g) b[g] = args->b, d[g] = args->d, alpha[g] = args->alpha;
+  BlockScales bs;
+  bs.a_scale = bs.b_scale = a_scale;
+  DryRun dry;
+  dry.cus = cu_count;
+  *info = fluxmi_gemm_launch_info{};
+  const int kind = run_grouped_gemm(args, ngroups, b, d, alpha, nullptr, &dry, 0, a_scale != nullptr ? &bs : nullptr);
+  if (kind < 0) return kind;
+  info->form = kind == 0 ? FLUXMI_GEMM_GENERIC : (!dry.stream ? FLUXMI_GEMM_MACRO_TILES : (dry.macro ? FLUXMI_GEMM_BY_SPLITS : FLUXMI_GEMM_STREAM));
+  if (info->form == FLUXMI_GEMM_BY_SPLITS && splits_host != nullptr) {
+    info->form = FLUXMI_GEMM_STREAM;
+    for (int e = 0; e < args->nexperts; ++e)
+      if (splits_host[e] > kStreamRows) info->form = FLUXMI_GEMM_MACRO_TILES;
+  }
+  if (dry.stream) {
+    info->stream_cols = dry.plan.cols;
+    info->stream_waves = dry.plan.waves;
+    info->stream_workgroups = static_cast<int32_t>(dry.plan.workgroups);
+    info->stream_lds_bytes = dry.plan.lds_bytes;
+  }
+  return FLUXMI_OK;
 }
 
 extern "C" int fluxmi_grouped_gemm_multi(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const void *const *b,

@@ -92,6 +92,9 @@ struct GemmParams {
   int32_t b_scale_layout;  // FLUXMI_BSCALE_*
   int32_t half_is_f16;     // 2-byte operands and outputs are fp16, not bf16 (read by the generic kernel; the MFMA
                            // kernel is built once per 16-bit type)
+  // > 0: the streaming form and the macro tiles are both launched; the first computes the launch if no expert has more
+  // rows than this, the second if one has, and the other returns at once.  0: the launched one computes it.
+  int32_t stream_rows;
 };
 
 

@@ -4,7 +4,7 @@
 // compute unit all the time (about 50 KB each to cover the memory latency at the card's read rate), not operand reuse,
 // so the shape of this kernel is the opposite of the macro-tile kernel's (grouped_gemm_kernel.hpp):
 //
-//  * A workgroup computes 16 * NB columns of up to 16 * MBMAX rows of one expert over the whole of K; its waves split K
+//  * A workgroup computes 16 * NB columns of all rows of one expert, 32 at most, over the whole of K; its waves split K
 //    between them by 128-byte lines (wave w takes lines w, w + WAVES, ...), so that the workgroup reads each row of
 //    weights front to back.  The partial sums meet in LDS at the end and are added in wave order (same bits every run).
 //  * Operands go from memory straight into registers, eight whole 128-byte lines per load instruction, non-temporally for the
@@ -12,17 +12,26 @@
 //    6.1-6.6 with ordinary loads; the MFMA fragment layout itself (16 rows x 64 bytes per instruction, the two halves of a
 //    line in two instructions) 4.9-5.5 and 5.9-6.5; 1 KiB of one row per instruction 3.3-6.7.  Two loads become two
 //    fragments by exchanging lanes 8..15 of every 16 with lanes 0..7 (three register moves per four bytes and lane).
-//  * No barriers and no waits between waves in the loop; a ring of DEPTH lines per wave is in flight (128 KiB of weights per
+//  * No barriers and no waits between waves in the loop; a ring of two lines per wave is in flight (128 KiB of weights per
 //    compute unit), several workgroups share a compute unit.
 //  * Rows beyond the expert's last repeat it (their lanes hit the same lines) and are not stored; bytes past the end of K
 //    are out-of-range buffer loads, which return zeros.
-//  * The items (expert, column tile, row chunk) are numbered with the row chunks of one column tile next to each other,
-//    and each XCD takes a contiguous eighth of them: weights that several chunks share are fetched into one L2.
+//  * The items (expert that has rows, column tile) are numbered expert by expert and each XCD takes a contiguous eighth of
+//    them, so that the rows of an expert are fetched into few L2s.
 //
-// Measured (us per launch, the macro-tile kernel in its place -> this one; weights at 6.5 TB/s in brackets), bf16 8 experts
-// 14336 x 4096: 2 rows 60 -> 41 [36], 74 rows 211 -> 143 [145], 192 rows 217 -> 165; 4096 x 14336: 2 rows 87 -> 42 [36], 74
-// rows 213 -> 148 [145]; 64 experts 1408 x 2048, 222 rows: 111 -> 60 [57]; fp8 32 experts 2048 x 7168, 296 rows: 95 -> 74
-// [72]; 7168 x 2048: 116 -> 88 [72]; block-scaled, the same two: 128 -> 75 and 159 -> 91.
+// Why 32 rows.  Every weight is then read once, every item takes about the same time, and the XCDs' contiguous shares are even
+// whatever the routing is.  With chunks of up to 64 rows and any number of chunks per expert a skewed routing left one XCD with the
+// long items, and a busy expert's weights were read once per chunk: us per launch, this form with chunks / the macro tiles, fp8 32
+// experts 7168 x 2048, 768 rows: Zipf (exponent 1.2) 165 / 115, all on eight experts 72 / 33, all on one 62 / 24; bf16 8
+// experts 14336 x 4096, 320 rows on two 174 / 68; block-scaled 7168 x 2048, 512 rows Zipf 214 / 153.  Launches that
+// have such an expert run on the macro tiles (GemmParams::stream_rows), at the price of a launch that returns at once: 2 to 3 us
+// when this form computes the launch, 3 to 10 when the macro tiles do.
+//
+// Measured (us per launch, the macro tiles -> this form; weights at 6.5 TB/s in brackets), even splits, bf16 8 experts 14336 x
+// 4096: 64 rows 216 -> 138 [145], 128 rows 216 -> 141, 256 rows 218 -> 165; 4096 x 14336: 64 rows 212 -> 145 [145], 256 rows
+// 218 -> 165; 64 experts 1408 x 2048, 256 rows: 113 -> 57 [57], 2048 rows 116 -> 78; fp8 32 experts 2048 x 7168, 256 rows:
+// 94 -> 72 [72], 768 rows 96 -> 82; 7168 x 2048: 115 -> 80 [72] and 118 -> 98; block-scaled, the same four: 123 -> 74,
+// 125 -> 83, 148 -> 85 and 152 -> 104.
 #include "grouped_gemm_stream.hpp"
 
 namespace fluxmi {
@@ -40,68 +49,54 @@ constexpr uint32_t kOutOfRange = 0xfffffff0u;  // a byte offset past every buffe
 
 // Clamped like the macro-tile kernel's: negative counts are 0, rows past max_rows do not exist.
 struct WorkItem {
-  bool valid;
-  int e, row_base, expert_rows;
-  int m0, rows;  // this chunk: its first row in the expert, its row count
-  int nt;        // column tile, over all weight groups
+  int e, row_base, rows;  // the expert, its first row, its row count (0: there is no such item)
+  int nt;                 // column tile, over all weight groups
 };
 
-template <int MBMAX>
-__device__ __forceinline__ int row_chunks(int rows) { return (rows + 16 * MBMAX - 1) / (16 * MBMAX); }
-
-// Work item -> (expert, row chunk, column tile).  One wave-wide pass over the splits counts the chunks, a second finds
-// the item; with up to 64 experts both work on the same registers.
-template <int MBMAX>
+// Work item -> (expert that has rows, column tile).  One wave-wide pass over the splits counts the experts with rows, a second
+// finds the item's; with up to 64 experts both work on the same registers.
 __device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n, int block) {
   const int lane = threadIdx.x & 63;
+  uint64_t above = 0;
   auto load = [&](int e0, int &carry, int &begin, int &rows) {
     const int ee = e0 + lane;
     int r = ee < p.nexperts ? p.splits[ee] : 0;
     if (r < 0) r = 0;
+    above |= __ballot(r > p.stream_rows);
     const int incl = wave_inclusive_scan(r);
     begin = carry + incl - r;
     int end = carry + incl;
     if (begin > p.max_rows) begin = p.max_rows;
     if (end > p.max_rows) end = p.max_rows;
     rows = end - begin;
-    carry += __shfl(incl, 63, 64);
+    carry += __builtin_amdgcn_readlane(incl, 63);
+    return __ballot(rows > 0);
   };
-  int carry = 0, begin = 0, rows = 0, total = 0;
+  int carry = 0, begin = 0, rows = 0, active = 0;
+  uint64_t some = 0;
   for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
-    load(e0, carry, begin, rows);
-    total += __shfl(wave_inclusive_scan(row_chunks<MBMAX>(rows)), 63, 64);
+    some = load(e0, carry, begin, rows);
+    active += __popcll(some);
   }
+  WorkItem w = {0, 0, 0, 0};
+  if (p.stream_rows > 0 && above != 0) return w;  // the macro tiles run this launch
   // Workgroups are dealt to the eight XCDs round-robin.
-  const int items = total * tiles_n;
-  const int per_xcd = (items + 7) / 8;
-  const int i = block >> 3;
-  int item = (block & 7) * per_xcd + i;
-  WorkItem w = {false, 0, 0, 0, 0, 0, 0};
+  const int items = active * tiles_n, per_xcd = (items + 7) / 8, i = block >> 3, item = (block & 7) * per_xcd + i;
   if (i >= per_xcd || item >= items) return w;
+  int nth = item / tiles_n;
+  w.nt = item - nth * tiles_n;
   carry = 0;
   for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
-    if (p.nexperts > 64) load(e0, carry, begin, rows);
-    const int chunks = row_chunks<MBMAX>(rows);
-    const int incl = wave_inclusive_scan(chunks) * tiles_n;
-    const uint64_t hit = __ballot(item < incl);
-    if (hit != 0) {
-      const int src = __ffsll(static_cast<unsigned long long>(hit)) - 1;
-      const int nchunks = __builtin_amdgcn_readlane(chunks, src);
-      const int local = item - (__builtin_amdgcn_readlane(incl, src) - nchunks * tiles_n);
-      const int all_rows = __builtin_amdgcn_readlane(rows, src);
-      w.valid = true;
+    if (p.nexperts > 64) some = load(e0, carry, begin, rows);
+    const int here = __popcll(some);
+    if (nth < here) {
+      const int src = __ffsll(static_cast<unsigned long long>(__ballot(rows > 0 && popc_below_lane(some) == nth))) - 1;
       w.e = e0 + src;
       w.row_base = __builtin_amdgcn_readlane(begin, src);
-      w.nt = local / nchunks;
-      // An expert's 16-row blocks are shared out evenly over its chunks.
-      const int blocks = (all_rows + 15) >> 4, per = (blocks + nchunks - 1) / nchunks;
-      w.expert_rows = all_rows;
-      w.m0 = (local - w.nt * nchunks) * per * 16;
-      w.rows = all_rows - w.m0 < per * 16 ? all_rows - w.m0 : per * 16;
-      if (w.rows <= 0) w.valid = false;
+      w.rows = __builtin_amdgcn_readlane(rows, src);
       return w;
     }
-    item -= __builtin_amdgcn_readlane(incl, 63);
+    nth -= here;
   }
   return w;
 }
@@ -153,7 +148,7 @@ __device__ __forceinline__ i32x4 load16(__amdgpu_buffer_rsrc_t r, uint32_t voff,
 }
 
 // 16 * MB rows x 16 * NB columns of one expert: partial sums of this wave's lines of K into acc.
-template <Elem T, int MB, int NB, int WAVES, int DEPTH>
+template <Elem T, int MB, int NB, int WAVES>
 __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkItem &t, int g, int n0, f32x4 (&acc)[MB][NB]) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -164,7 +159,7 @@ __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkI
   const auto wr = buffer_of(p.b[g] + (static_cast<int64_t>(t.e) * p.n + n0) * kbytes, static_cast<int64_t>(p.n - n0) * kbytes);
   const bool gathered = p.gather_a != nullptr;
   const auto xr = gathered ? buffer_of(p.a, static_cast<int64_t>(p.a_rows) * kbytes)
-                           : buffer_of(p.a + static_cast<int64_t>(t.row_base + t.m0) * kbytes, static_cast<int64_t>(t.rows) * kbytes);
+                           : buffer_of(p.a + static_cast<int64_t>(t.row_base) * kbytes, static_cast<int64_t>(t.rows) * kbytes);
   uint32_t woff[NB][2], xoff[MB][2];
 #pragma unroll
   for (int j = 0; j < NB; ++j)
@@ -177,7 +172,7 @@ __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkI
   auto source_row = [&](int r) {  // row of A that row r of the chunk reads (the last one again past the end)
     if (r > t.rows - 1) r = t.rows - 1;
     if (!gathered) return static_cast<int64_t>(r);
-    const int64_t arow = p.gather_a[t.row_base + t.m0 + r];
+    const int64_t arow = p.gather_a[t.row_base + r];
     return arow < 0 ? 0 : (arow >= p.a_rows ? p.a_rows - 1 : arow);
   };
 #pragma unroll
@@ -193,17 +188,18 @@ __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkI
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
       const int r = i * 16 + (lane & 15);
-      const int64_t srow = source_row(r) + (gathered ? 0 : t.row_base + t.m0);
+      const int64_t srow = source_row(r) + (gathered ? 0 : t.row_base);
       soff[i] = p.a_scale_layout == FLUXMI_ASCALE_BLOCK128
                     ? static_cast<uint32_t>(((srow >> 7) * kblocks * 128 + (srow & 127)) * 4)
                     : static_cast<uint32_t>((static_cast<int64_t>(t.row_base) * (kblocks - 1) + srow) * 4);
     }
-    a_kstep = p.a_scale_layout == FLUXMI_ASCALE_BLOCK128 ? 512 : t.expert_rows * 4;
+    a_kstep = p.a_scale_layout == FLUXMI_ASCALE_BLOCK128 ? 512 : t.rows * 4;
     const int nb = n0 >> 7, nblocks = (p.n + 127) >> 7;
     b_base = p.b_scale_layout == FLUXMI_BSCALE_N_K ? (t.e * nblocks + nb) * kblocks : t.e * kblocks * nblocks + nb;
     b_kstep = p.b_scale_layout == FLUXMI_BSCALE_N_K ? 1 : nblocks;
   }
 
+  constexpr int DEPTH = 2;
   Line<T, MB, NB> ring[DEPTH];
   auto load_line = [&](Line<T, MB, NB> &l, int line) {
     const int kb = line * 128;
@@ -286,7 +282,7 @@ __device__ __forceinline__ void finish_tile(const GemmParams &p, f32x4 *red, con
     const int l = u & 63, b = u >> 6;
     const int r = (b / NB) * 16 + (l & 15), col = n0 + (b % NB) * 16 + (l >> 4) * 4;
     if (r >= t.rows || col >= p.n) continue;  // n % 4 == 0: the four columns are all in or all out
-    const int row = t.row_base + t.m0 + r;
+    const int row = t.row_base + r;
     const float rs = tile_scale * (p.row_scale ? p.row_scale[row] : 1.f);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -315,39 +311,32 @@ __device__ __forceinline__ void finish_tile(const GemmParams &p, f32x4 *red, con
   }
 }
 
-template <Elem T, int MB, int NB, int WAVES, int DEPTH>
+template <Elem T, int MB, int NB, int WAVES>
 __device__ __forceinline__ void run_tile(const GemmParams &p, f32x4 *red, const WorkItem &t, int g, int n0) {
   f32x4 acc[MB][NB];
-  accumulate_tile<T, MB, NB, WAVES, DEPTH>(p, t, g, n0, acc);
+  accumulate_tile<T, MB, NB, WAVES>(p, t, g, n0, acc);
   finish_tile<T, MB, NB, WAVES>(p, red, t, g, n0, acc);
 }
 
 #endif  // __HIP_DEVICE_COMPILE__
 
 
-// WALK: workgroups walk the `blocks` items with the grid's stride (a launch cut down to leave compute units free); otherwise
-// there is one workgroup per item.  A form of its own because the loop costs the other one up to ten spilled registers.
-template <Elem T, int MBMAX, int NB, int WAVES, int DEPTH, bool WALK>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(MBMAX <= 2 ? 4 : 2)))
+// WALK: workgroups walk the `blocks` items with the grid's stride; otherwise there is one workgroup per item.
+// A form of its own because the loop costs registers (27 to 34 of the 64-column forms; the 32-column ones spill one, block-scaled nine).
+template <Elem T, int NB, int WAVES, bool WALK>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(NB <= 2 ? 4 : 2)))
 void grouped_gemm_stream_kernel(const GemmParams p, const int blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ f32x4 red[WAVES * MBMAX * NB * 64];
+  __shared__ f32x4 red[WAVES * 2 * NB * 64];
   const int tiles_n1 = (p.n + 16 * NB - 1) / (16 * NB);
   int block = blockIdx.x;
   do {
-    const WorkItem t = locate<MBMAX>(p, tiles_n1 * p.ngroups, block);
-    if (t.valid) {
+    const WorkItem t = locate(p, tiles_n1 * p.ngroups, block);
+    if (t.rows > 0) {
       const int g = p.ngroups > 1 ? t.nt / tiles_n1 : 0;
       const int n0 = (t.nt - g * tiles_n1) * (16 * NB);
-      if (MBMAX == 1 || t.rows <= 16) {
-        run_tile<T, 1, NB, WAVES, DEPTH>(p, red, t, g, n0);
-      } else if constexpr (MBMAX >= 2) {
-        if (MBMAX == 2 || t.rows <= 32) {
-          run_tile<T, 2, NB, WAVES, (DEPTH > 3 ? 3 : DEPTH)>(p, red, t, g, n0);
-        } else if constexpr (MBMAX >= 4) {
-          run_tile<T, 4, NB, WAVES, (DEPTH > 3 ? 3 : DEPTH)>(p, red, t, g, n0);
-        }
-      }
+      if (t.rows <= 16) run_tile<T, 1, NB, WAVES>(p, red, t, g, n0);
+      else run_tile<T, 2, NB, WAVES>(p, red, t, g, n0);
     }
     if constexpr (WALK) __syncthreads();  // `red` has been read before the next item's sums go into it
     block += gridDim.x;
@@ -355,62 +344,70 @@ void grouped_gemm_stream_kernel(const GemmParams p, const int blocks) {
 #endif
 }
 
-// Most row chunks a launch can have: every expert that gets a row starts one, and `chunk` rows fill one.
-int64_t most_chunks(const GemmParams &p, int chunk) {
+// Most items a launch can have: every expert that gets a row is one per column tile of 16 * nb.
+int64_t most_items(const GemmParams &p, int ngroups, int nb) {
   const int64_t active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
-  return active + (p.max_rows - active) / chunk;
+  return active * ((p.n + 16 * nb - 1) / (16 * nb)) * ngroups;
 }
 
-// With compute units to be left to other work (`cus` of them may be used; 0: all), no more workgroups than these hold at
-// once; each then walks several items, so the results do not change.
-template <Elem T, int MBMAX, int NB, int WAVES, int DEPTH>
-void launch(const GemmParams &p, int cus, hipStream_t s) {
-  const int64_t items = most_chunks(p, 16 * MBMAX) * ((p.n + 16 * NB - 1) / (16 * NB)) * p.ngroups;
-  const int64_t blocks = (items + 7) / 8 * 8;
-  if (cus == 0) {
-    hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, MBMAX, NB, WAVES, DEPTH, false>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(WAVES * 64), 0, s, p, static_cast<int>(blocks));
-    return;
+template <Elem T, int NB, int WAVES>
+int launch(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
+  if (!plan.walk) {
+    hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, false>), dim3(plan.workgroups), dim3(WAVES * 64), 0, s, p, plan.blocks);
+    return FLUXMI_OK;
   }
-  constexpr int resident = (MBMAX <= 2 ? 16 : 8) / WAVES;  // waves a compute unit holds / waves per workgroup
-  const int64_t most = (static_cast<int64_t>(cus) * resident + 7) / 8 * 8;  // a multiple of the XCDs
-  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, MBMAX, NB, WAVES, DEPTH, true>), dim3(static_cast<unsigned>(blocks < most ? blocks : most)),
-                     dim3(WAVES * 64), 0, s, p, static_cast<int>(blocks));
+  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, true>), dim3(plan.workgroups), dim3(WAVES * 64), 0, s, p, plan.blocks);
+  return FLUXMI_OK;
 }
 
-// Which tile.  Columns per workgroup (NB): 64 reads the rows' own operand least often (its loads share the queue behind the
-// weights' with them: at 9 rows per expert 140 us against 159 for 32 columns, bf16 14336 x 4096), but takes two waves
-// per SIMD; 32 columns with four waves per SIMD is as fast or faster while there is hardly a row (2.5 rows per expert:
-// 108 against 114 us; 3.5 rows, 64 experts: 60 against 68), except block-scaled, whose scales do not fit its 128 registers (73
-// against 70).  Where 64-column tiles would leave compute units without work (512 of them fill the card) it is 32 columns, and
-// eight waves per workgroup if K is long enough to share (two experts, 4096 x 14336: 42 us, four waves 47, 64 columns 61; at K = 2048
-// bytes per row eight waves lose, 17 against 14 us).
 template <Elem T>
-void launch_by_shape(const GemmParams &p, int cus, hipStream_t s) {
-  const int64_t lines = (static_cast<int64_t>(p.k) * (is_fp8(T) ? 1 : 2) + 127) / 128;
-  const int64_t items = most_chunks(p, 64) * ((p.n + 63) / 64) * p.ngroups;
-  const bool few = items < 512;
-  if (few && lines >= 64) launch<T, 2, 2, 8, 2>(p, cus, s);
-  else if (few || (T != Elem::FP8_BLOCKSCALED && p.max_rows <= 4 * p.nexperts)) launch<T, 2, 2, 4, 2>(p, cus, s);
-  else launch<T, 4, 4, 4, 2>(p, cus, s);
+int launch_by_plan(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
+  if (plan.waves == 8) return launch<T, 2, 8>(p, plan, s);
+  if (plan.cols == 32) return launch<T, 2, 4>(p, plan, s);
+  return launch<T, 4, 4>(p, plan, s);
 }
 
 }  // namespace
 
-// Up to how many rows per expert this form is the faster one (the macro-tile kernel's time hardly depends on the rows while
-// they are few; this one's grows with them): bf16 14336 x 4096 at 24 / 32 / 50 rows 165 / 189 / 214 us against 217 / 219 / 221,
-// 64 experts at 19 / 37 rows 73 / 105 against 112 / 109; fp8 2048 x 7168 at 24 / 32 rows 85 / 95 against 97 / 97, 7168 x 2048
-// 105 / 128 against 118 / 118; block-scaled at 24 / 50 rows 109 / 197 against 124 / 129.
+// Up to how many rows per expert on average this form is the faster one on even splits (the macro tiles' time hardly depends on
+// the rows while they are few; this one's grows with them): 16-bit at 32 rows 165 / 218 us on the two 8-expert shapes above,
+// 78 / 116 and 80 / 92 on 64 experts of 1408 x 2048 and 2048 x 1408, 12 / 19 on 8 of 2048 x 1024; fp8 at 24 rows 82 / 96 and 98 /
+// 118, at 32 an earlier build 95 / 97 and 128 / 118; block-scaled at 24 rows 83 / 125 and 104 / 152.
 bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
-  const int64_t rows = dtype == FLUXMI_FP8_E4M3 ? 24 : 40;
+  const int64_t rows = dtype == FLUXMI_FP8_E4M3 ? 24 : kStreamRows;
   return p.max_rows <= rows * p.nexperts;
 }
 
-void launch_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, hipStream_t s) {
-  if (p.a_scale != nullptr) launch_by_shape<Elem::FP8_BLOCKSCALED>(p, cus, s);
-  else if (dtype == FLUXMI_FP8_E4M3) launch_by_shape<Elem::FP8>(p, cus, s);
-  else if (dtype == FLUXMI_FP16) launch_by_shape<Elem::F16>(p, cus, s);
-  else launch_by_shape<Elem::BF16>(p, cus, s);
+// Columns per workgroup: 64 reads the rows' own operand least often (its loads share the queue behind the weights' with them), but
+// takes two waves per SIMD; 32 columns with four waves per SIMD is as fast or faster on most shapes while there is hardly a row (us at
+// 2 rows per expert, 32 / 64 columns: bf16 4096 x 14336 140 / 143, 64 experts of 1408 x 2048 59 / 66, fp8 7168 x 2048
+// 77 / 80; not on 8 experts of 14336 x 4096, 158 / 136).  Block-scaled launches differ by 1 to 4 us either way and take 64.  Where
+// 64-column tiles would leave compute units without work (512 of them fill the card) it is 32 columns, and eight waves per
+// workgroup if K is long enough to share (two experts, 4096 x 14336: 42 us, four waves 47, 64 columns 61; at K = 2048 bytes per row
+// eight waves lose, 17 against 14 us).
+// With compute units to be left to other work no more workgroups than the others hold at once are launched and each walks
+// several items, so the results do not change.
+StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, bool leave_cus) {
+  StreamPlan plan;
+  const int64_t lines = (static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2) + 127) / 128;
+  const bool few = most_items(p, p.ngroups, 4) < 512;
+  plan.waves = few && lines >= 64 ? 8 : 4;
+  plan.cols = few || (p.a_scale == nullptr && p.max_rows <= 4 * p.nexperts) ? 32 : 64;
+  const int64_t blocks = (most_items(p, p.ngroups, plan.cols / 16) + 7) / 8 * 8;
+  plan.blocks = static_cast<int>(blocks);
+  plan.walk = leave_cus;
+  const int resident = (plan.cols == 32 ? 16 : 8) / plan.waves;  // waves a compute unit holds / waves per workgroup
+  const int64_t most = (static_cast<int64_t>(cus) * resident + 7) / 8 * 8;  // a multiple of the XCDs
+  plan.workgroups = static_cast<unsigned>(plan.walk && blocks > most ? most : blocks);
+  plan.lds_bytes = plan.waves * 2 * (plan.cols / 16) * 1024;
+  return plan;
+}
+
+int launch_grouped_gemm_stream(const GemmParams &p, int dtype, const StreamPlan &plan, hipStream_t s) {
+  if (p.a_scale != nullptr) return launch_by_plan<Elem::FP8_BLOCKSCALED>(p, plan, s);
+  if (dtype == FLUXMI_FP8_E4M3) return launch_by_plan<Elem::FP8>(p, plan, s);
+  if (dtype == FLUXMI_FP16) return launch_by_plan<Elem::F16>(p, plan, s);
+  return launch_by_plan<Elem::BF16>(p, plan, s);
 }
 
 }  // namespace fluxmi

@@ -160,6 +160,25 @@ int fluxmi_grouped_gemm(const fluxmi_grouped_gemm_args *args, void *workspace,
  * shapes only); callers use this to assert they are not on the generic kernel. */
 int fluxmi_grouped_gemm_kernel_kind(const fluxmi_grouped_gemm_args *args);
 
+/* Which form of the MFMA kernels a launch takes and how the streaming form is launched.  Host only: nothing is
+ * launched, no device is needed, and pointers in `args` are only looked at for their alignment (b and d stand for every
+ * weight group).  a_scale: non-NULL for fluxmi_grouped_gemm_blockscale with MFMA-kernel layouts.  splits_host: host copy of
+ * args->splits, or NULL.  cu_count: compute units of the device asked about.  Returns FLUXMI_OK or the status the call
+ * itself would return. */
+#define FLUXMI_GEMM_GENERIC 0
+#define FLUXMI_GEMM_MACRO_TILES 1
+#define FLUXMI_GEMM_STREAM 2    /* few rows per expert: weights streamed into MFMA registers */
+#define FLUXMI_GEMM_BY_SPLITS 3 /* 2 if no expert has more than 32 rows, else 1; decided on the device from `splits` */
+typedef struct fluxmi_gemm_launch_info {
+  int32_t form;              /* FLUXMI_GEMM_* */
+  int32_t stream_cols;       /* the streaming form: columns per workgroup, */
+  int32_t stream_waves;      /* waves per workgroup (K is split over them), */
+  int32_t stream_workgroups; /* workgroups launched, */
+  int32_t stream_lds_bytes;  /* LDS per workgroup; all 0 for the other forms */
+} fluxmi_gemm_launch_info;
+int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
+                                    const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_launch_info *info);
+
 /* ------------------------------------------------------------------------------------------------
  * Top-k reduction fused into the grouped GEMM's epilogue (layer1 in one pass, no [M, N] intermediate):
  *

@@ -1,0 +1,28 @@
+"""Which form of the MFMA kernels a grouped GEMM takes, and how the streaming form is launched (host code only, no GPU)."""
+import pytest
+import torch
+
+from flux_amd import capi
+
+BF16, F16, FP8 = torch.bfloat16, torch.float16, torch.float8_e4m3fn
+
+
+@pytest.mark.parametrize("dtype,block_scaled,line", [(BF16, False, 32), (F16, False, 32), (FP8, False, 24), (FP8, True, 24)])
+def test_form_by_rows(dtype, block_scaled, line):
+    def form(rows, splits=None):
+        return capi.gemm_launch_info(dtype, 8, rows, 4096, 1024, block_scaled=block_scaled, splits=splits).form
+
+    assert form(1) == form(32) == capi.GEMM_STREAM  # no expert can have more than 32 rows
+    assert form(33) == form(8 * line) == capi.GEMM_BY_SPLITS
+    assert form(8 * line + 1) == form(100000) == capi.GEMM_MACRO_TILES
+    assert form(80, [32, 0, 10, 0, 0, 30, 8, 0]) == capi.GEMM_STREAM
+    assert form(80, [33, 0, 10, 0, 0, 30, 7, 0]) == capi.GEMM_MACRO_TILES  # one expert has too many
+    assert form(80, [80, -5, 0, 0, 0, 0, 0, 0]) == capi.GEMM_MACRO_TILES
+
+
+def test_generic_shapes_have_no_streaming_form():
+    assert capi.gemm_launch_info(BF16, 8, 16, 4096, 1023).form == capi.GEMM_GENERIC
+    with pytest.raises(RuntimeError, match="cu_count"):
+        capi.gemm_launch_info(BF16, 8, 16, 4096, 1024, cu_count=0)
+    with pytest.raises(RuntimeError, match="ngroups"):
+        capi.gemm_launch_info(BF16, 8, 16, 4096, 1024, ngroups=5)

@@ -96,6 +96,49 @@ def test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b
         at += r
 
 
+# The 64-column form: more than four rows per expert on average (block-scaled: any) and at least 512 column tiles in all.  One block
+# and two blocks of 16 rows, rows that do not fill them; columns cut off at 4; K that ends inside a line and numbers of lines that
+# four waves with two lines in flight do not divide; more than 64 experts.
+WIDE = [([32, 0, 31, 17, 16, 1, 2, 9], 4164, 272), ([32, 32, 32, 32, 5, 0, 31, 20], 4096, 1040), ([17] * 70 + [0, 32, 1], 516, 2064 + 16)]
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("splits,n,k", WIDE)
+def test_stream_form_64_columns(dtype, splits, n, k):
+    info = capi.gemm_launch_info(DT[dtype], len(splits), sum(splits), n, k, splits=splits)
+    assert (info.form, info.stream_cols) == (capi.GEMM_STREAM, 64)
+    test_stream_form_is_exact_on_integers(dtype, splits, n, k)
+
+
+@pytest.mark.parametrize("splits,n,k", [([32, 0, 31, 17, 16, 1, 2, 9], 4160, 384), ([3] * 70 + [0, 32, 1], 516, 1152)])
+@pytest.mark.parametrize("a_layout", [capi.ASCALE_BLOCK128, capi.ASCALE_EXPERT_K_M])
+@pytest.mark.parametrize("b_layout", [capi.BSCALE_N_K, capi.BSCALE_K_N])
+def test_stream_form_64_columns_block_scaled(splits, n, k, a_layout, b_layout):
+    info = capi.gemm_launch_info(DT["fp8"], len(splits), sum(splits), n, k, splits=splits, block_scaled=True)
+    assert (info.form, info.stream_cols) == (capi.GEMM_STREAM, 64)
+    test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b_layout)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("splits,form", [([32, 7, 0, 20, 32, 1], 2), ([33, 7, 0, 20, 31, 1], 1), ([0, 0, 0, 0, 0, 90], 1),
+                                         ([1] * 70 + [33], 1), ([1] * 70 + [32], 2), ([9, 3, 0, 20], 2)])
+def test_one_form_computes_a_launch(dtype, splits, form):
+    """Which form runs is decided on the device; every result is computed, and added to a sum, exactly once."""
+    print(f"[case] form by splits {dtype} {splits[-6:]}", flush=True)
+    n, k, m, e = 260, 272, sum(splits), len(splits)
+    assert capi.gemm_launch_info(DT[dtype], e, m, n, k, splits=splits).form == form
+    g = torch.Generator().manual_seed(m)
+    a, w = small_ints(g, m, k), small_ints(g, e, n, k)
+    ad, wd = a.float().to(DT[dtype]).cuda(), w.float().to(DT[dtype]).cuda()
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    ref = expected(a, w, splits)
+    assert torch.equal(capi.grouped_gemm(ad, wd, sp, out_dtype=torch.float32).cpu().long(), ref)
+    token = torch.randint(0, m // 2 + 1, (m,), generator=g).to(torch.int32)
+    sums = torch.zeros(m // 2 + 1, n, dtype=torch.int64).index_add_(0, token.long(), ref)
+    out = capi.grouped_gemm_topk_reduce(ad, wd, sp, token.cuda(), m // 2 + 1)
+    assert torch.equal(out.cpu(), sums.float().to(out.dtype))
+
+
 @pytest.mark.parametrize("kblocks,rows,n,experts", [(1, 3, 128, 1), (3, 3, 128, 1), (7, 3, 256, 2), (8, 3, 128, 1), (9, 3, 128, 1),
                                                     (65, 3, 128, 1), (3, 7, 2176, 24), (9, 7, 2176, 24)])
 def test_stream_form_block_scaled_infinite_scales(kblocks, rows, n, experts):
