@@ -362,7 +362,7 @@ int launch(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
 
 template <Elem T>
 int launch_by_plan(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
-  if (plan.waves == 8) return launch<T, 2, 8>(p, plan, s);
+  if (plan.waves == 8) return plan.cols == 32 ? launch<T, 2, 8>(p, plan, s) : launch<T, 4, 8>(p, plan, s);
   if (plan.cols == 32) return launch<T, 2, 4>(p, plan, s);
   return launch<T, 4, 4>(p, plan, s);
 }
@@ -391,7 +391,7 @@ StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, boo
   StreamPlan plan;
   const int64_t lines = (static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2) + 127) / 128;
   const bool few = most_items(p, p.ngroups, 4) < 512;
-  plan.waves = few && lines >= 64 ? 8 : 4;
+  plan.waves = most_items(p, 1, 4) < 512 && lines >= 64 ? 8 : 4;  // of one weight group: a launch of several has its bits
   plan.cols = few || (p.a_scale == nullptr && p.max_rows <= 4 * p.nexperts) ? 32 : 64;
   const int64_t blocks = (most_items(p, p.ngroups, plan.cols / 16) + 7) / 8 * 8;
   plan.blocks = static_cast<int>(blocks);

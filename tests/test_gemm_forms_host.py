@@ -26,3 +26,13 @@ def test_generic_shapes_have_no_streaming_form():
         capi.gemm_launch_info(BF16, 8, 16, 4096, 1024, cu_count=0)
     with pytest.raises(RuntimeError, match="ngroups"):
         capi.gemm_launch_info(BF16, 8, 16, 4096, 1024, ngroups=5)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16, FP8])
+@pytest.mark.parametrize("experts,rows,n,k", [(8, 74, 2048, 4096), (8, 20, 2048, 8192), (64, 90, 400, 8192), (1, 8, 16384, 8192), (16, 200, 1408, 2048)])
+def test_weight_groups_do_not_change_how_k_is_split(dtype, experts, rows, n, k):
+    """A launch of several weight groups adds K up in the order of a launch per group: the same number of waves."""
+    alone = capi.gemm_launch_info(dtype, experts, rows, n, k)
+    for groups in (2, 3, 4):
+        together = capi.gemm_launch_info(dtype, experts, rows, n, k, ngroups=groups)
+        assert (together.form, together.stream_waves) == (alone.form, alone.stream_waves)

@@ -139,6 +139,21 @@ def test_one_form_computes_a_launch(dtype, splits, form):
     assert torch.equal(out.cpu(), sums.float().to(out.dtype))
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+@pytest.mark.parametrize("splits,n,k", [([9, 10, 8, 11, 7, 9, 10, 10], 2048, 4096), ([2, 0, 3, 1], 4100, 8192 + 16)])
+def test_stream_form_weight_groups_have_the_bits_of_one_launch_each(dtype, splits, n, k):
+    """One group alone is less than 512 column tiles, the groups together are more."""
+    print(f"[case] stream gemm groups {dtype} splits={splits} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(n + k)
+    x = torch.randn(sum(splits), k, generator=g).to(DT[dtype]).cuda()
+    ws = [(torch.randn(len(splits), n, k, generator=g) * 0.05).to(DT[dtype]).cuda() for _ in range(4)]
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    alone = [capi.grouped_gemm(x, w, sp, out_dtype=torch.float32) for w in ws]
+    for groups in (2, 3, 4):
+        for got, want in zip(capi.grouped_gemm_multi(x, ws[:groups], sp, out_dtype=torch.float32), alone):
+            assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("kblocks,rows,n,experts", [(1, 3, 128, 1), (3, 3, 128, 1), (7, 3, 256, 2), (8, 3, 128, 1), (9, 3, 128, 1),
                                                     (65, 3, 128, 1), (3, 7, 2176, 24), (9, 7, 2176, 24)])
 def test_stream_form_block_scaled_infinite_scales(kblocks, rows, n, experts):
