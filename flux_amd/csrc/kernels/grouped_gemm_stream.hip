@@ -149,9 +149,8 @@ __device__ __forceinline__ i32x4 load16(__amdgpu_buffer_rsrc_t r, uint32_t voff,
 
 // 16 * MB rows x 16 * NB columns of one expert: partial sums of this wave's lines of K into acc.
 template <Elem T, int MB, int NB, int WAVES>
-__device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkItem &t, int g, int n0, f32x4 (&acc)[MB][NB]) {
+__device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkItem &t, int g, int n0, int wave, f32x4 (&acc)[MB][NB]) {
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t kbytes = static_cast<int64_t>(p.k) * (is_fp8(T) ? 1 : 2);
   const int kb32 = static_cast<int>(kbytes);
   // Lane l of a load fetches 16 bytes of row l & 7 of an eight-row block, chunk 2 * (l >> 4) + ((l >> 3) & 1) of the line.
@@ -265,17 +264,24 @@ __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkI
   }
 }
 
-// Sum of the waves' partial sums, scaled, cast and stored.  A unit is one lane's four consecutive columns of one row.
+// Partial sums of one wave's lines of K to LDS.
 template <Elem T, int MB, int NB, int WAVES>
-__device__ __forceinline__ void finish_tile(const GemmParams &p, f32x4 *red, const WorkItem &t, int g, int n0, const f32x4 (&acc)[MB][NB]) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+__device__ __forceinline__ void partial_sums(const GemmParams &p, f32x4 *red, const WorkItem &t, int g, int n0, int wave) {
+  f32x4 acc[MB][NB];
+  accumulate_tile<T, MB, NB, WAVES>(p, t, g, n0, wave, acc);
+  const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) red[(wave * MB * NB + i * NB + j) * 64 + lane] = acc[i][j];
-  __syncthreads();
+}
+
+// Sum of the waves' partial sums, scaled, cast and stored.  A unit is one lane's four consecutive columns of one row.
+template <Elem T, int MB, int NB, int WAVES>
+__device__ __forceinline__ void finish_tile(const GemmParams &p, const f32x4 *red, const WorkItem &t, int g, int n0, int wave) {
+  const int lane = threadIdx.x & 63;
   const float tile_scale = p.scalar * (p.scalar_dev ? p.scalar_dev[0] : 1.f) * (p.alpha[g] ? p.alpha[g][t.e] : 1.f);
-  for (int u = threadIdx.x; u < MB * NB * 64; u += WAVES * 64) {
+  for (int u = wave * 64 + lane; u < MB * NB * 64; u += WAVES * 64) {
     f32x4 v = red[u];
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) v += red[w * MB * NB * 64 + u];
@@ -311,35 +317,39 @@ __device__ __forceinline__ void finish_tile(const GemmParams &p, f32x4 *red, con
   }
 }
 
-template <Elem T, int MB, int NB, int WAVES>
-__device__ __forceinline__ void run_tile(const GemmParams &p, f32x4 *red, const WorkItem &t, int g, int n0) {
-  f32x4 acc[MB][NB];
-  accumulate_tile<T, MB, NB, WAVES>(p, t, g, n0, acc);
-  finish_tile<T, MB, NB, WAVES>(p, red, t, g, n0, acc);
-}
-
 #endif  // __HIP_DEVICE_COMPILE__
 
 
-// WALK: workgroups walk the `blocks` items with the grid's stride; otherwise there is one workgroup per item.
-// A form of its own because the loop costs registers (27 to 34 of the 64-column forms; the 32-column ones spill one, block-scaled nine).
+// WALK: a workgroup per compute unit that walks the `blocks` items with the grid's stride, as many at a time as the unit holds
+// workgroups of the other form (its teams of WAVES waves); otherwise one workgroup per item.  Two forms because the loop costs registers.
+constexpr int unit_waves(int nb) { return nb <= 2 ? 16 : 8; }  // what the registers of a compute unit hold
 template <Elem T, int NB, int WAVES, bool WALK>
-__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(NB <= 2 ? 4 : 2)))
+__global__ __launch_bounds__(WALK ? unit_waves(NB) * 64 : WAVES * 64) __attribute__((amdgpu_waves_per_eu(unit_waves(NB) / 4)))
 void grouped_gemm_stream_kernel(const GemmParams p, const int blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ f32x4 red[WAVES * 2 * NB * 64];
+  constexpr int TEAMS = WALK ? unit_waves(NB) / WAVES : 1;
+  constexpr int TEAM_SUMS = WAVES * 2 * NB * 64;
+  __shared__ f32x4 red_all[TEAMS * TEAM_SUMS];
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int team = TEAMS > 1 ? wave_all / WAVES : 0, wave = TEAMS > 1 ? wave_all % WAVES : wave_all;
+  f32x4 *const red = red_all + team * TEAM_SUMS;
   const int tiles_n1 = (p.n + 16 * NB - 1) / (16 * NB);
+  const int stride = static_cast<int>(gridDim.x);
   int block = blockIdx.x;
   do {
-    const WorkItem t = locate(p, tiles_n1 * p.ngroups, block);
-    if (t.rows > 0) {
-      const int g = p.ngroups > 1 ? t.nt / tiles_n1 : 0;
-      const int n0 = (t.nt - g * tiles_n1) * (16 * NB);
-      if (t.rows <= 16) run_tile<T, 1, NB, WAVES>(p, red, t, g, n0);
-      else run_tile<T, 2, NB, WAVES>(p, red, t, g, n0);
+    const WorkItem t = locate(p, tiles_n1 * p.ngroups, block + team * stride);
+    const int g = p.ngroups > 1 ? t.nt / tiles_n1 : 0;
+    const int n0 = (t.nt - g * tiles_n1) * (16 * NB);
+    if constexpr (!WALK) {
+      if (t.rows == 0) return;
     }
-    if constexpr (WALK) __syncthreads();  // `red` has been read before the next item's sums go into it
-    block += gridDim.x;
+    if (t.rows > 16) partial_sums<T, 2, NB, WAVES>(p, red, t, g, n0, wave);
+    else if (t.rows > 0) partial_sums<T, 1, NB, WAVES>(p, red, t, g, n0, wave);
+    __syncthreads();
+    if (t.rows > 16) finish_tile<T, 2, NB, WAVES>(p, red, t, g, n0, wave);
+    else if (t.rows > 0) finish_tile<T, 1, NB, WAVES>(p, red, t, g, n0, wave);
+    if constexpr (WALK) __syncthreads();  // the sums have been read before the next items' go there
+    block += TEAMS * stride;
   } while (WALK && block < blocks);
 #endif
 }
@@ -350,21 +360,26 @@ int64_t most_items(const GemmParams &p, int ngroups, int nb) {
   return active * ((p.n + 16 * nb - 1) / (16 * nb)) * ngroups;
 }
 
+// A walking workgroup's sums take 64 KiB of LDS; with what it asks for on top that is more than half of a compute unit's
+// 160 KiB, so no unit takes two of them and N workgroups occupy N units.
+constexpr int kWalkSums = 64 * 1024, kWalkExtra = 32 * 1024;
+
 template <Elem T, int NB, int WAVES>
-int launch(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
+void launch(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
   if (!plan.walk) {
     hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, false>), dim3(plan.workgroups), dim3(WAVES * 64), 0, s, p, plan.blocks);
-    return FLUXMI_OK;
+    return;
   }
-  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, true>), dim3(plan.workgroups), dim3(WAVES * 64), 0, s, p, plan.blocks);
-  return FLUXMI_OK;
+  static_assert(unit_waves(NB) * 2 * NB * 1024 == kWalkSums, "LDS of the walking form");
+  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, true>), dim3(plan.workgroups), dim3(unit_waves(NB) * 64), kWalkExtra, s, p, plan.blocks);
 }
 
 template <Elem T>
-int launch_by_plan(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
-  if (plan.waves == 8) return plan.cols == 32 ? launch<T, 2, 8>(p, plan, s) : launch<T, 4, 8>(p, plan, s);
-  if (plan.cols == 32) return launch<T, 2, 4>(p, plan, s);
-  return launch<T, 4, 4>(p, plan, s);
+void launch_by_plan(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
+  if (plan.waves == 8 && plan.cols == 32) launch<T, 2, 8>(p, plan, s);
+  else if (plan.waves == 8) launch<T, 4, 8>(p, plan, s);
+  else if (plan.cols == 32) launch<T, 2, 4>(p, plan, s);
+  else launch<T, 4, 4>(p, plan, s);
 }
 
 }  // namespace
@@ -385,8 +400,11 @@ bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
 // 64-column tiles would leave compute units without work (512 of them fill the card) it is 32 columns, and eight waves per
 // workgroup if K is long enough to share (two experts, 4096 x 14336: 42 us, four waves 47, 64 columns 61; at K = 2048 bytes per row
 // eight waves lose, 17 against 14 us).
-// With compute units to be left to other work no more workgroups than the others hold at once are launched and each walks
-// several items, so the results do not change.
+// With compute units to be left to other work there is one workgroup for each of the others, which walks several items; the results
+// do not change, which is why a margin does not choose the macro tiles either where those are faster.  us at a margin of 8 / 64 / 128
+// / 224 of 256 units, this form and the macro tiles: bf16 8 experts 14336 x 4096, 74 rows 162 / 185 / 255 / 995 and 215 / 238 / 268 /
+// 773; fp8 32 experts 7168 x 2048, 400 rows 97 / 118 / 168 / 642 and 111 / 120 / 147 / 500 (a unit alone streams 30 GB/s here; a
+// ring of three or four lines in place of two changed nothing).
 StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, bool leave_cus) {
   StreamPlan plan;
   const int64_t lines = (static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2) + 127) / 128;
@@ -396,18 +414,17 @@ StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, boo
   const int64_t blocks = (most_items(p, p.ngroups, plan.cols / 16) + 7) / 8 * 8;
   plan.blocks = static_cast<int>(blocks);
   plan.walk = leave_cus;
-  const int resident = (plan.cols == 32 ? 16 : 8) / plan.waves;  // waves a compute unit holds / waves per workgroup
-  const int64_t most = (static_cast<int64_t>(cus) * resident + 7) / 8 * 8;  // a multiple of the XCDs
+  const int64_t most = cus >= 8 ? cus / 8 * 8 : cus;  // whole rounds over the XCDs where there are enough units
   plan.workgroups = static_cast<unsigned>(plan.walk && blocks > most ? most : blocks);
-  plan.lds_bytes = plan.waves * 2 * (plan.cols / 16) * 1024;
+  plan.lds_bytes = plan.walk ? kWalkSums + kWalkExtra : plan.waves * 2 * (plan.cols / 16) * 1024;
   return plan;
 }
 
-int launch_grouped_gemm_stream(const GemmParams &p, int dtype, const StreamPlan &plan, hipStream_t s) {
-  if (p.a_scale != nullptr) return launch_by_plan<Elem::FP8_BLOCKSCALED>(p, plan, s);
-  if (dtype == FLUXMI_FP8_E4M3) return launch_by_plan<Elem::FP8>(p, plan, s);
-  if (dtype == FLUXMI_FP16) return launch_by_plan<Elem::F16>(p, plan, s);
-  return launch_by_plan<Elem::BF16>(p, plan, s);
+void launch_grouped_gemm_stream(const GemmParams &p, int dtype, const StreamPlan &plan, hipStream_t s) {
+  if (p.a_scale != nullptr) launch_by_plan<Elem::FP8_BLOCKSCALED>(p, plan, s);
+  else if (dtype == FLUXMI_FP8_E4M3) launch_by_plan<Elem::FP8>(p, plan, s);
+  else if (dtype == FLUXMI_FP16) launch_by_plan<Elem::F16>(p, plan, s);
+  else launch_by_plan<Elem::BF16>(p, plan, s);
 }
 
 }  // namespace fluxmi

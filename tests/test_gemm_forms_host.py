@@ -36,3 +36,16 @@ def test_weight_groups_do_not_change_how_k_is_split(dtype, experts, rows, n, k):
     for groups in (2, 3, 4):
         together = capi.gemm_launch_info(dtype, experts, rows, n, k, ngroups=groups)
         assert (together.form, together.stream_waves) == (alone.form, alone.stream_waves)
+
+
+@pytest.mark.parametrize("dtype,block_scaled", [(BF16, False), (FP8, False), (FP8, True)])
+@pytest.mark.parametrize("experts,rows,n,k", [(8, 16, 4224, 2064 - 16), (8, 180, 14336, 4096), (32, 400, 7168, 2048), (4, 8, 1024, 8192)])
+@pytest.mark.parametrize("margin", [1, 100, 249, 255, 1000])
+def test_margin_leaves_whole_compute_units(dtype, block_scaled, experts, rows, n, k, margin):
+    """With a margin every workgroup has a compute unit for itself (more than half of its 160 KiB of LDS), and there are no more
+    of them than units that may be used."""
+    info = capi.gemm_launch_info(dtype, experts, rows, n, k, block_scaled=block_scaled, cu_margin=margin)
+    assert 80 * 1024 < info.stream_lds_bytes <= 160 * 1024
+    assert 1 <= info.stream_workgroups <= max(1, 256 - margin)
+    free = capi.gemm_launch_info(dtype, experts, rows, n, k, block_scaled=block_scaled)
+    assert (free.form, free.stream_cols, free.stream_waves) == (info.form, info.stream_cols, info.stream_waves)  # same bits

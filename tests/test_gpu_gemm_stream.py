@@ -3,6 +3,8 @@
 Operands are small integers, so every product and every partial sum is a whole number below 2^24 and the fp32 result is the
 same in any order of summation: the outputs have to equal an int64 matmul exactly, no tolerance.  (`max_rows` at most 24
 rows per expert on average, fp8, or 40, bf16 / fp16, selects the form.)"""
+import ctypes
+
 import pytest
 import torch
 
@@ -192,3 +194,26 @@ def test_stream_form_leaves_compute_units_and_changes_no_bit(splits, n, k, margi
     sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
     base = capi.grouped_gemm(a, w, sp)
     assert torch.equal(capi.grouped_gemm(a, w, sp, cu_margin=margin), base)
+
+
+@pytest.mark.parametrize("margin", [1, 249, 1000])
+@pytest.mark.parametrize("dtype,splits,n,k", [("fp8", [32, 0, 31, 17, 16, 1, 2, 9], 4164, 272), ("f16", [32, 0, 31, 17, 16, 1, 2, 9], 4164, 272),
+                                              ("bf16", [7, 33, 2], 516, 1040), ("fp8", [5, 0, 2], 516, 8192), ("bs", [32, 0, 31, 17, 16, 1, 2, 9], 4160, 384),
+                                              ("bs", [3, 1], 260, 8192)])
+def test_margin_changes_no_bit_of_any_form(dtype, splits, n, k, margin):
+    print(f"[case] stream gemm margin={margin} {dtype} splits={splits} n={n} k={k}", flush=True)
+    g = torch.Generator().manual_seed(n + k)
+    m, e = sum(splits), len(splits)
+    td = DT["fp8" if dtype == "bs" else dtype]
+    a = torch.randn(m, k, generator=g).to(td).cuda()
+    w = (torch.randn(e, n, k, generator=g) * 0.05).to(td).cuda()
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    if dtype != "bs":
+        assert torch.equal(capi.grouped_gemm(a, w, sp, cu_margin=margin), capi.grouped_gemm(a, w, sp))
+        return
+    sa = torch.rand((m + 127) // 128, k // 128, 128, generator=g).cuda()
+    sb = torch.rand(e, (n + 127) // 128, k // 128, generator=g).cuda()
+    args, out = capi._gemm_args(a, w, sp, None, None, None, None, None, None, 1.0, None, None, torch.float32, margin, 0, 0)
+    capi._check(capi.load().fluxmi_grouped_gemm_blockscale(ctypes.byref(args), capi._ptr(sa), capi.ASCALE_BLOCK128, capi._ptr(sb),
+                                                           capi.BSCALE_N_K, capi._stream()), "fluxmi_grouped_gemm_blockscale")
+    assert torch.equal(out, capi.grouped_gemm_blockscale(a, w, sp, sa, sb, out_dtype=torch.float32))
