@@ -387,10 +387,11 @@ void launch_by_plan(const GemmParams &p, const StreamPlan &plan, hipStream_t s) 
 // Up to how many rows per expert on average this form is the faster one on even splits (the macro tiles' time hardly depends on
 // the rows while they are few; this one's grows with them): 16-bit at 32 rows 165 / 218 us on the two 8-expert shapes above,
 // 78 / 116 and 80 / 92 on 64 experts of 1408 x 2048 and 2048 x 1408, 12 / 19 on 8 of 2048 x 1024; fp8 at 24 rows 82 / 96 and 98 /
-// 118, at 32 an earlier build 95 / 97 and 128 / 118; block-scaled at 24 rows 83 / 125 and 104 / 152.
+// 118, at 32 an earlier build 95 / 97 and 128 / 118; block-scaled at 24 rows 83 / 125 and 104 / 152.  Items are numbered with ints
+// (for the most weight groups a launch can have, so that their number does not choose the form).
 bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
   const int64_t rows = dtype == FLUXMI_FP8_E4M3 ? 24 : kStreamRows;
-  return p.max_rows <= rows * p.nexperts;
+  return p.max_rows <= rows * p.nexperts && most_items(p, kMaxWeightGroups, 2) < (int64_t{1} << 31) - (1 << 20);
 }
 
 // Columns per workgroup: 64 reads the rows' own operand least often (its loads share the queue behind the weights' with them), but
@@ -413,7 +414,7 @@ StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, boo
   plan.cols = few || (p.a_scale == nullptr && p.max_rows <= 4 * p.nexperts) ? 32 : 64;
   const int64_t blocks = (most_items(p, p.ngroups, plan.cols / 16) + 7) / 8 * 8;
   plan.blocks = static_cast<int>(blocks);
-  plan.walk = leave_cus;
+  plan.walk = leave_cus || blocks * plan.waves * 64 > 0xffffffffll;  // a launch has less than 2^32 threads
   const int64_t most = cus >= 8 ? cus / 8 * 8 : cus;  // whole rounds over the XCDs where there are enough units
   plan.workgroups = static_cast<unsigned>(plan.walk && blocks > most ? most : blocks);
   plan.lds_bytes = plan.walk ? kWalkSums + kWalkExtra : plan.waves * 2 * (plan.cols / 16) * 1024;

@@ -49,3 +49,17 @@ def test_margin_leaves_whole_compute_units(dtype, block_scaled, experts, rows, n
     assert 1 <= info.stream_workgroups <= max(1, 256 - margin)
     free = capi.gemm_launch_info(dtype, experts, rows, n, k, block_scaled=block_scaled)
     assert (free.form, free.stream_cols, free.stream_waves) == (info.form, info.stream_cols, info.stream_waves)  # same bits
+
+
+@pytest.mark.parametrize("dtype,k,block_scaled", [(BF16, 8, False), (FP8, 16, False), (FP8, 128, True)])
+@pytest.mark.parametrize("groups", [1, 4])
+def test_a_launch_stays_below_the_grid_limit(dtype, k, block_scaled, groups):
+    """2^32 threads are more than a launch may have: workgroups then walk the items.  Beyond what an int numbers the macro tiles run."""
+    if block_scaled and groups > 1:
+        return
+    for experts, n in ((1024, 1 << 18), (1024, 1 << 20), (700, (1 << 20) + 4), (4, 1 << 24)):
+        info = capi.gemm_launch_info(dtype, experts, experts, n, k, ngroups=groups, block_scaled=block_scaled)
+        assert info.form in (capi.GEMM_STREAM, capi.GEMM_BY_SPLITS)
+        assert 1 <= info.stream_workgroups <= ((1 << 32) - 1) // (info.stream_waves * 64)
+    assert capi.gemm_launch_info(dtype, 1024, 1024, 1 << 20, k, block_scaled=block_scaled).stream_workgroups == 256
+    assert capi.gemm_launch_info(dtype, 1024, 1024, 1 << 24, k, block_scaled=block_scaled).form == capi.GEMM_MACRO_TILES
