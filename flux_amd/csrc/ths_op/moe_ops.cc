@@ -47,9 +47,6 @@ GemmShapeKey shape_key(const fluxmi_grouped_gemm_args &args, int32_t ngroups) {
     if (err_ != hipSuccess) throw std::runtime_error(std::string(#expr " failed: ") + hipGetErrorString(err_)); \
   } while (0)
 
-// Times `run` (one whole forward) under every candidate schedule on the current stream, 5 warm-up and 10
-// timed calls each like the reference's profiling loops (gemm_grouped_v3_ag_scatter.cc:540-590), records
-// them in `ctx` and registers the fastest for `key`.
 // Mean time in ms of one call of `run` on the current stream: 5 warm-up and 10 timed calls.
 template <class F>
 float time_calls(F &&run) {
@@ -76,13 +73,40 @@ float time_calls(F &&run) {
   return ms / kIters;
 }
 
+// Times `run` (one whole forward) under every candidate schedule on the current stream, 5 warm-up and 10
+// timed calls each like the reference's profiling loops (gemm_grouped_v3_ag_scatter.cc:540-590), records
+// them in `ctx` and registers the fastest for `key`.  `args`: the launch that `run` makes; splits: its row counts on the host.  The
+// schedules are the macro tiles'; where the streaming form runs the launch they are all one, and only the default is timed.
 template <class F>
-void profile_schedules(const GemmShapeKey &key, ProfilingContext *ctx, F &&run) {
+void profile_schedules(const GemmShapeKey &key, ProfilingContext *ctx, const fluxmi_grouped_gemm_args &args, const torch::Tensor &splits,
+                       F &&run) {
+  fluxmi_gemm_launch_info info;
+  check_status(fluxmi_grouped_gemm_launch_info(&args, key.ngroups, nullptr, splits.data_ptr<int32_t>(), fluxmi_device_cu_count(), &info),
+               "fluxmi_grouped_gemm_launch_info");
   for (const GemmLaunchTuning &cand : gemm_tuning_candidates()) {
     ScopedTuningOverride scope(&cand);
     ctx->add(key, cand, time_calls(run));
+    if (info.form == FLUXMI_GEMM_STREAM) break;
   }
   TuningTable::instance().add(key, ctx->record_best(key));
+}
+
+// What decides the form of a launch: sizes, and the pointers for their alignment.
+fluxmi_grouped_gemm_args launch_of(const GemmShapeKey &key, const torch::Tensor &a, const torch::Tensor &b, void *d, const int32_t *gather_a,
+                                   const torch::Tensor &splits) {
+  fluxmi_grouped_gemm_args args{};
+  args.dtype = key.dtype;
+  args.nexperts = key.nexperts;
+  args.max_rows = key.max_rows;
+  args.n = key.n;
+  args.k = key.k;
+  args.a_rows = static_cast<int32_t>(a.size(0));
+  args.a = a.data_ptr();
+  args.b = b.data_ptr();
+  args.d = d;
+  args.splits = splits.data_ptr<int32_t>();
+  args.gather_a = gather_a;
+  return args;
 }
 }  // namespace
 
@@ -272,7 +296,7 @@ torch::Tensor GemmGroupedV3AGScatter::profiling(torch::Tensor inputs_shard, torc
     return forward(inputs_shard, weights, splits_gpu, scatter_index, output_scale, outputs_buf, allgather_output,
                    fast_accum, sm_margin);
   };
-  run();  // argument checks before anything is timed
+  const torch::Tensor out = run();  // argument checks before anything is timed
   GemmShapeKey key;
   key.dtype = to_fluxmi_dtype(moe_args_.input_dtype);
   key.nexperts = moe_args_.nexperts;
@@ -280,7 +304,10 @@ torch::Tensor GemmGroupedV3AGScatter::profiling(torch::Tensor inputs_shard, torc
   key.k = moe_args_.hidden;
   key.max_rows = static_cast<int32_t>(inputs_shard.size(0) * moe_args_.topk);
   key.ngroups = 1;
-  if (key.max_rows > 0) profile_schedules(key, ctx, run);
+  if (key.max_rows > 0) {
+    const torch::Tensor splits = splits_gpu.cpu();
+    profile_schedules(key, ctx, launch_of(key, inputs_shard, weights, out.data_ptr(), gather_index_.data_ptr<int32_t>(), splits), splits, run);
+  }
   return run();  // with the schedule just registered
 }
 
@@ -485,7 +512,10 @@ torch::Tensor GemmGroupedV3GatherRS::profiling(
   if (key.max_rows > 0) {
     {
       ScopedReduceOverride twopass(fused_mode_ == 0 ? 2 : 0);  // an earlier record must not switch forms mid-sweep
-      profile_schedules(key, ctx, run);
+      const torch::Tensor splits = splits_cpu.contiguous();
+      fluxmi_grouped_gemm_args args = launch_of(key, input, weight, inter_[0].data_ptr(), nullptr, splits);
+      args.d_fp32 = inter_fp32_ ? 1 : 0;
+      profile_schedules(key, ctx, args, splits, run);
     }
     // With the fastest schedule registered: the other form of the reduction (atomic adds in the GEMM's epilogue
     // instead of GEMM + gather-reduce kernel), when this op could run either.  Its time ranks among the two-pass

@@ -2,8 +2,9 @@
 // records (PyTuningRecord / load_tuning_record, src/ths_op/ths_op.cc:208-216), its ProfilingContext
 // (include/flux/ths_op/ths_op.h:64-113, src/ths_op/ths_op.cc:217-320) and its TuningConfigRegistry.
 // The reference's records pick one of its generated kernel variants; here a record picks the tile
-// schedule of the one persistent kernel (height of the raster groups, whether the last round is cut into
-// pieces, whether an expert's last row tile may run half height).  No choice changes a result bit.
+// schedule of the persistent macro-tile kernel (height of the raster groups, whether the last round is cut into
+// pieces, whether an expert's last row tile may run half height).  No choice changes a result bit.  Launches that the
+// streaming form computes (few rows per expert) have no such schedule: a record changes nothing there.
 #pragma once
 #include <cstdint>
 #include <map>

@@ -301,6 +301,34 @@ def test_profiling_registers_a_schedule_and_keeps_results(c1):
     m.clear_tuning_records()
 
 
+@pytest.mark.parametrize("cnt,timed", [([9, 0, 30, 32, 5, 1, 0, 3], 1), ([0, 0, 40, 32, 5, 1, 0, 2], 5)])
+def test_profiling_times_one_schedule_where_none_has_an_effect(cnt, timed):
+    """With at most 32 rows in every expert the streaming form computes the launch, whatever the schedule; with more the macro
+    tiles do, and all schedules are timed."""
+    m = flux_amd.flux_ths_pybind
+    m.clear_tuning_records()
+    g = torch.Generator().manual_seed(3)
+    e, h, f, t, k = len(cnt), 256, 512, sum(cnt) // 2, 2
+    x = torch.randn(t, h, generator=g).to(torch.bfloat16).cuda()
+    w1 = (torch.randn(e, f, h, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    w2 = (torch.randn(e, h, f, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    splits = torch.tensor(cnt, dtype=torch.int32)
+    scatter = torch.randperm(t * k, generator=g).to(torch.int32).view(t, k).cuda()
+    op0 = flux_amd.GemmGroupedV3AGScatter(flux_amd.DistEnvTPWithEP(None, 1, None), flux_amd.MoeArguments(t, h, f, e, k, torch.bfloat16))
+    op1 = flux_amd.GemmGroupedV3GatherRS(e, t * k, h, k, 0, 1, 1, 1)
+    for fused in (0, 1):  # layer0; layer1, whose other form of the reduction is timed as well
+        ctx = flux_amd.ProfilingContext("few rows")
+        if fused == 0:
+            y = op0.forward(x, w1, splits.cuda(), scatter)
+            assert torch.equal(op0.profiling(x, w1, splits.cuda(), scatter, prof_ctx=ctx), y)
+        else:
+            op1.profiling(y, w2, splits, scatter.view(-1), prof_ctx=ctx)
+        assert ctx.get_latest_prof_result().count("TopK=") == min(5, timed + fused)
+        rec = ctx.get_latest_record()
+        assert timed > 1 or (rec.raster_rows, rec.sched_flags) == (8, 0)
+    m.clear_tuning_records()
+
+
 @pytest.mark.parametrize("raster_rows,flags,margin", [(4, 0, 0), (16, 1, 0), (8, 2, 0), (1, 3, 0), (8, 0, 40), (8, 0, 255),
                                                        (8, 0, 1000), (8, 4, 0), (8, 8, 0), (2, 9, 5)])
 def test_tile_schedules_and_cu_margin_do_not_change_a_bit(raster_rows, flags, margin):
