@@ -1,5 +1,6 @@
-// Grouped GEMM entry point: argument checks, choice between the MFMA kernel and the generic kernel, and
-// the generic kernel itself.  The MFMA kernel lives in grouped_gemm_kernel.hpp.
+// Grouped GEMM entry point: argument checks, choice between the MFMA kernels and the generic kernel, and
+// the generic kernel itself.  The MFMA kernels are the macro tiles (grouped_gemm_kernel.hpp) and, for few rows per
+// expert, the streaming form (grouped_gemm_stream.hip).
 #include "grouped_gemm_stream.hpp"
 
 namespace fluxmi {
@@ -216,7 +217,7 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
 
   const bool stream_form = mfma && grouped_gemm_stream_takes(p, args->dtype);
   const bool macro = mfma && (!stream_form || args->max_rows > kStreamRows);
-  p.stream_rows = stream_form && macro ? kStreamRows : 0;
+  p.by_splits = stream_form && macro ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   int cus = dry_run ? dry_run->cus : fluxmi_device_cu_count();
   FLUXMI_REQUIRE(cus > 0 || dry_run, FLUXMI_ERR_HIP, "grouped_gemm: cannot query the device");
@@ -395,9 +396,14 @@ extern "C" int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *a
   if (kind < 0) return kind;
   info->form = kind == 0 ? FLUXMI_GEMM_GENERIC : (!dry.stream ? FLUXMI_GEMM_MACRO_TILES : (dry.macro ? FLUXMI_GEMM_BY_SPLITS : FLUXMI_GEMM_STREAM));
   if (info->form == FLUXMI_GEMM_BY_SPLITS && splits_host != nullptr) {
-    info->form = FLUXMI_GEMM_STREAM;
-    for (int e = 0; e < args->nexperts; ++e)
-      if (splits_host[e] > kStreamRows) info->form = FLUXMI_GEMM_MACRO_TILES;
+    int left = args->max_rows, chunks = 0, active = 0;
+    for (int e = 0; e < args->nexperts; ++e) {
+      const int rows = splits_host[e] < 0 ? 0 : (splits_host[e] < left ? splits_host[e] : left);
+      left -= rows;
+      active += rows > 0 ? 1 : 0;
+      chunks += (rows + kStreamRows - 1) / kStreamRows;
+    }
+    info->form = chunks <= stream_chunks_limit(active) ? FLUXMI_GEMM_STREAM : FLUXMI_GEMM_MACRO_TILES;
   }
   if (dry.stream) {
     info->stream_cols = dry.plan.cols;

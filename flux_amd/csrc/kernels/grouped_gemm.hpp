@@ -92,10 +92,16 @@ struct GemmParams {
   int32_t b_scale_layout;  // FLUXMI_BSCALE_*
   int32_t half_is_f16;     // 2-byte operands and outputs are fp16, not bf16 (read by the generic kernel; the MFMA
                            // kernel is built once per 16-bit type)
-  // > 0: the streaming form and the macro tiles are both launched; the first computes the launch if no expert has more
-  // rows than this, the second if one has, and the other returns at once.  0: the launched one computes it.
-  int32_t stream_rows;
+  // 1: the streaming form and the macro tiles are both launched; `splits` says which of them computes the launch
+  // (stream_chunks_limit) and the other returns at once.  0: the launched one computes it.
+  int32_t by_splits;
 };
+
+// Rows of a work item of the streaming form: two 16-row MFMA blocks.  An expert with more is several items per column tile.
+constexpr int kStreamRows = 32;
+
+// Most chunks of up to kStreamRows rows that the streaming form computes in a launch in which `active` experts have rows.
+__host__ __device__ inline int stream_chunks_limit(int active) { return active + (active >= 16 ? active / 4 : 0); }
 
 
 // One launcher per element type, each in a translation unit of its own (the kernel is a long compile).

@@ -1588,16 +1588,19 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
   int total_tiles = 0, skinny_experts = 0;
   {
     int row_carry = 0, acc_tiles = 0, acc_cand = 0;
-    uint64_t above = 0;
+    int chunks = 0, active = 0;  // for launches that the streaming form may compute
     for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
       const int ee = e0 + lane;
       int rows = ee < p.nexperts ? p.splits[ee] : 0;
       if (rows < 0) rows = 0;
-      above |= __ballot(rows > p.stream_rows);
       const int incl = wave_inclusive_scan(rows);
       int begin = row_carry + incl - rows, end = row_carry + incl;
       if (begin > p.max_rows) begin = p.max_rows;
       if (end > p.max_rows) end = p.max_rows;
+      if (p.by_splits) {
+        active += __popcll(__ballot(end > begin));
+        chunks += __builtin_amdgcn_readlane(wave_inclusive_scan((end - begin + kStreamRows - 1) / kStreamRows), 63);
+      }
       int tiles = ((end - begin + BM - 1) / BM) * tiles_n;
       int cand = (end > begin && ((end - begin - 1) & (BM - 1)) < 64) ? 1 : 0;
 #pragma unroll
@@ -1609,7 +1612,7 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
       acc_cand += cand;
       row_carry += __shfl(incl, 63, 64);
     }
-    if (p.stream_rows > 0 && above == 0) return;  // the streaming form runs this launch
+    if (p.by_splits && chunks <= stream_chunks_limit(active)) return;  // the streaming form runs this launch
     total_tiles = __builtin_amdgcn_readfirstlane(acc_tiles);
     skinny_experts = __builtin_amdgcn_readfirstlane(acc_cand);
   }

@@ -4,7 +4,7 @@
 // compute unit all the time (about 50 KB each to cover the memory latency at the card's read rate), not operand reuse,
 // so the shape of this kernel is the opposite of the macro-tile kernel's (grouped_gemm_kernel.hpp):
 //
-//  * A workgroup computes 16 * NB columns of all rows of one expert, 32 at most, over the whole of K; its waves split K
+//  * A workgroup computes 16 * NB columns of up to 32 rows of one expert over the whole of K; its waves split K
 //    between them by 128-byte lines (wave w takes lines w, w + WAVES, ...), so that the workgroup reads each row of
 //    weights front to back.  The partial sums meet in LDS at the end and are added in wave order (same bits every run).
 //  * Operands go from memory straight into registers, eight whole 128-byte lines per load instruction, non-temporally for the
@@ -16,16 +16,20 @@
 //    compute unit), several workgroups share a compute unit.
 //  * Rows beyond the expert's last repeat it (their lanes hit the same lines) and are not stored; bytes past the end of K
 //    are out-of-range buffer loads, which return zeros.
-//  * The items (expert that has rows, column tile) are numbered expert by expert and each XCD takes a contiguous eighth of
-//    them, so that the rows of an expert are fetched into few L2s.
+//  * The items (expert, column tile, chunk of 32 rows) are numbered with the chunks of one column tile next to each other, and
+//    each XCD takes a contiguous eighth of them: weights that several chunks share and the rows of an expert are fetched into
+//    few L2s.
 //
-// Why 32 rows.  Every weight is then read once, every item takes about the same time, and the XCDs' contiguous shares are even
-// whatever the routing is.  With chunks of up to 64 rows and any number of chunks per expert a skewed routing left one XCD with the
-// long items, and a busy expert's weights were read once per chunk: us per launch, this form with chunks / the macro tiles, fp8 32
-// experts 7168 x 2048, 768 rows: Zipf (exponent 1.2) 165 / 115, all on eight experts 72 / 33, all on one 62 / 24; bf16 8
-// experts 14336 x 4096, 320 rows on two 174 / 68; block-scaled 7168 x 2048, 512 rows Zipf 214 / 153.  Launches that
-// have such an expert run on the macro tiles (GemmParams::stream_rows), at the price of a launch that returns at once: 2 to 3 us
-// when this form computes the launch, 3 to 10 when the macro tiles do.
+// Which launches.  Where (nearly) every expert's rows are one chunk, every weight is read once, the items take about the same
+// time and the XCDs' shares are even.  The form once took any splits with few rows on average, in chunks of up to 64 rows: under
+// a skewed routing one XCD had the long items and a busy expert's weights were read once per chunk.  So launches in which an
+// expert can have more than one chunk are launched in both forms and the splits decide (stream_chunks_limit): this form up to a
+// quarter more chunks than experts with rows, and none more with under 16 experts, where one more can be a whole round of the
+// card (8 experts 4096 x 14336, 10 chunks 241 us, macro tiles 219).  The launch that returns at once costs 2 to 4 us when it is
+// the macro tiles' and 3 to 10 when it is this form's.  us per launch, any splits / now / macro tiles: Zipf (exponent 1.2), fp8 32
+// experts 7168 x 2048, 512 and 768 rows 154 / 124 / 125 and 165 / 124 / 115; block-scaled, 256 and 512 rows 175 / 117 / 156 and
+// 214 / 129 / 159; bf16 64 experts 1408 x 2048, 512 rows 90 / 87 / 123; all 768 rows on eight of the 32 72 / 42 / 33, on
+// one 62 / 34 / 24.
 //
 // Measured (us per launch, the macro tiles -> this form; weights at 6.5 TB/s in brackets), even splits, bf16 8 experts 14336 x
 // 4096: 64 rows 216 -> 138 [145], 128 rows 216 -> 141, 256 rows 218 -> 165; 4096 x 14336: 64 rows 212 -> 145 [145], 256 rows
@@ -49,54 +53,55 @@ constexpr uint32_t kOutOfRange = 0xfffffff0u;  // a byte offset past every buffe
 
 // Clamped like the macro-tile kernel's: negative counts are 0, rows past max_rows do not exist.
 struct WorkItem {
-  int e, row_base, rows;  // the expert, its first row, its row count (0: there is no such item)
-  int nt;                 // column tile, over all weight groups
+  int e, expert_base, expert_rows;  // the expert, its first row, its row count
+  int row_base, rows;               // the item's rows (0: there is no such item)
+  int nt;                           // column tile, over all weight groups
 };
 
-// Work item -> (expert that has rows, column tile).  One wave-wide pass over the splits counts the experts with rows, a second
+// Work item -> (expert, chunk of its rows, column tile).  One wave-wide pass over the splits counts the chunks, a second
 // finds the item's; with up to 64 experts both work on the same registers.
 __device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n, int block) {
   const int lane = threadIdx.x & 63;
-  uint64_t above = 0;
-  auto load = [&](int e0, int &carry, int &begin, int &rows) {
+  int begin, rows, chunks_end;  // this lane's expert of the 64 looked at
+  auto load = [&](int e0, int &row_carry, int &chunk_carry) {
     const int ee = e0 + lane;
     int r = ee < p.nexperts ? p.splits[ee] : 0;
     if (r < 0) r = 0;
-    above |= __ballot(r > p.stream_rows);
     const int incl = wave_inclusive_scan(r);
-    begin = carry + incl - r;
-    int end = carry + incl;
+    begin = row_carry + incl - r;
+    int end = row_carry + incl;
     if (begin > p.max_rows) begin = p.max_rows;
     if (end > p.max_rows) end = p.max_rows;
     rows = end - begin;
-    carry += __builtin_amdgcn_readlane(incl, 63);
-    return __ballot(rows > 0);
+    row_carry += __builtin_amdgcn_readlane(incl, 63);
+    chunks_end = chunk_carry + wave_inclusive_scan((rows + kStreamRows - 1) / kStreamRows);
+    chunk_carry = __builtin_amdgcn_readlane(chunks_end, 63);
+    return __popcll(__ballot(rows > 0));
   };
-  int carry = 0, begin = 0, rows = 0, active = 0;
-  uint64_t some = 0;
-  for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
-    some = load(e0, carry, begin, rows);
-    active += __popcll(some);
-  }
-  WorkItem w = {0, 0, 0, 0};
-  if (p.stream_rows > 0 && above != 0) return w;  // the macro tiles run this launch
+  int row_carry = 0, total = 0, active = 0;
+  for (int e0 = 0; e0 < p.nexperts; e0 += 64) active += load(e0, row_carry, total);
+  WorkItem w = {0, 0, 0, 0, 0, 0};
+  if (p.by_splits && total > stream_chunks_limit(active)) return w;  // the macro tiles run this launch
   // Workgroups are dealt to the eight XCDs round-robin.
-  const int items = active * tiles_n, per_xcd = (items + 7) / 8, i = block >> 3, item = (block & 7) * per_xcd + i;
+  const int items = total * tiles_n, per_xcd = (items + 7) / 8, i = block >> 3, item = (block & 7) * per_xcd + i;
   if (i >= per_xcd || item >= items) return w;
-  int nth = item / tiles_n;
-  w.nt = item - nth * tiles_n;
-  carry = 0;
+  int row_carry2 = 0, chunk_carry2 = 0;
   for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
-    if (p.nexperts > 64) some = load(e0, carry, begin, rows);
-    const int here = __popcll(some);
-    if (nth < here) {
-      const int src = __ffsll(static_cast<unsigned long long>(__ballot(rows > 0 && popc_below_lane(some) == nth))) - 1;
+    if (p.nexperts > 64) load(e0, row_carry2, chunk_carry2);
+    const uint64_t hit = __ballot(item < chunks_end * tiles_n);
+    if (hit != 0) {
+      const int src = __ffsll(static_cast<unsigned long long>(hit)) - 1;
       w.e = e0 + src;
-      w.row_base = __builtin_amdgcn_readlane(begin, src);
-      w.rows = __builtin_amdgcn_readlane(rows, src);
+      w.expert_base = __builtin_amdgcn_readlane(begin, src);
+      w.expert_rows = __builtin_amdgcn_readlane(rows, src);
+      const int chunks = (w.expert_rows + kStreamRows - 1) / kStreamRows;
+      const int local = item - (__builtin_amdgcn_readlane(chunks_end, src) - chunks) * tiles_n;
+      w.nt = local / chunks;
+      const int first = (local - w.nt * chunks) * kStreamRows;
+      w.row_base = w.expert_base + first;
+      w.rows = w.expert_rows - first < kStreamRows ? w.expert_rows - first : kStreamRows;
       return w;
     }
-    nth -= here;
   }
   return w;
 }
@@ -190,9 +195,9 @@ __device__ __forceinline__ void accumulate_tile(const GemmParams &p, const WorkI
       const int64_t srow = source_row(r) + (gathered ? 0 : t.row_base);
       soff[i] = p.a_scale_layout == FLUXMI_ASCALE_BLOCK128
                     ? static_cast<uint32_t>(((srow >> 7) * kblocks * 128 + (srow & 127)) * 4)
-                    : static_cast<uint32_t>((static_cast<int64_t>(t.row_base) * (kblocks - 1) + srow) * 4);
+                    : static_cast<uint32_t>((static_cast<int64_t>(t.expert_base) * (kblocks - 1) + srow) * 4);
     }
-    a_kstep = p.a_scale_layout == FLUXMI_ASCALE_BLOCK128 ? 512 : t.rows * 4;
+    a_kstep = p.a_scale_layout == FLUXMI_ASCALE_BLOCK128 ? 512 : t.expert_rows * 4;
     const int nb = n0 >> 7, nblocks = (p.n + 127) >> 7;
     b_base = p.b_scale_layout == FLUXMI_BSCALE_N_K ? (t.e * nblocks + nb) * kblocks : t.e * kblocks * nblocks + nb;
     b_kstep = p.b_scale_layout == FLUXMI_BSCALE_N_K ? 1 : nblocks;
@@ -321,7 +326,8 @@ __device__ __forceinline__ void finish_tile(const GemmParams &p, const f32x4 *re
 
 
 // WALK: a workgroup per compute unit that walks the `blocks` items with the grid's stride, as many at a time as the unit holds
-// workgroups of the other form (its teams of WAVES waves); otherwise one workgroup per item.  Two forms because the loop costs registers.
+// workgroups of the other form (its teams of WAVES waves); otherwise one workgroup per item.  Two forms because the loop costs
+// registers (the 32-column fp8 and block-scaled ones spill 4 to 9 with it).
 constexpr int unit_waves(int nb) { return nb <= 2 ? 16 : 8; }  // what the registers of a compute unit hold
 template <Elem T, int NB, int WAVES, bool WALK>
 __global__ __launch_bounds__(WALK ? unit_waves(NB) * 64 : WAVES * 64) __attribute__((amdgpu_waves_per_eu(unit_waves(NB) / 4)))
@@ -354,10 +360,16 @@ void grouped_gemm_stream_kernel(const GemmParams p, const int blocks) {
 #endif
 }
 
-// Most items a launch can have: every expert that gets a row is one per column tile of 16 * nb.
-int64_t most_items(const GemmParams &p, int ngroups, int nb) {
+// Items of a launch in which every expert that can get rows is one per column tile of 16 * nb, and the most items a launch of
+// this form can have.
+int64_t one_chunk_items(const GemmParams &p, int ngroups, int nb) {
   const int64_t active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
   return active * ((p.n + 16 * nb - 1) / (16 * nb)) * ngroups;
+}
+int64_t most_items(const GemmParams &p, int ngroups, int nb) {
+  const int active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
+  const int chunks = active + (p.max_rows - active) / kStreamRows, limit = stream_chunks_limit(active);
+  return static_cast<int64_t>(chunks < limit ? chunks : limit) * ((p.n + 16 * nb - 1) / (16 * nb)) * ngroups;
 }
 
 // A walking workgroup's sums take 64 KiB of LDS; with what it asks for on top that is more than half of a compute unit's
@@ -409,8 +421,8 @@ bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
 StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, bool leave_cus) {
   StreamPlan plan;
   const int64_t lines = (static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2) + 127) / 128;
-  const bool few = most_items(p, p.ngroups, 4) < 512;
-  plan.waves = most_items(p, 1, 4) < 512 && lines >= 64 ? 8 : 4;  // of one weight group: a launch of several has its bits
+  const bool few = one_chunk_items(p, p.ngroups, 4) < 512;
+  plan.waves = one_chunk_items(p, 1, 4) < 512 && lines >= 64 ? 8 : 4;  // of one weight group: a launch of several has its bits
   plan.cols = few || (p.a_scale == nullptr && p.max_rows <= 4 * p.nexperts) ? 32 : 64;
   const int64_t blocks = (most_items(p, p.ngroups, plan.cols / 16) + 7) / 8 * 8;
   plan.blocks = static_cast<int>(blocks);

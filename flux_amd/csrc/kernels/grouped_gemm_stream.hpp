@@ -5,9 +5,6 @@
 
 namespace fluxmi {
 
-// Rows an expert may have in this form: two 16-row MFMA blocks, so that each weight is read once and by one workgroup.
-constexpr int kStreamRows = 32;
-
 struct StreamPlan {
   int cols, waves;      // columns per workgroup; waves that split K
   int blocks;           // items the launch is numbered for
@@ -17,8 +14,8 @@ struct StreamPlan {
 };
 
 // Whether a launch that the MFMA kernels can take may go to this form: few rows per expert on average.  With more than
-// kStreamRows rows in the launch one expert can have more than this form takes; which form runs is then decided on the
-// device (GemmParams::stream_rows).
+// kStreamRows rows in the launch an expert can have several chunks; which form runs is then decided on the device
+// (GemmParams::by_splits).
 bool grouped_gemm_stream_takes(const GemmParams &p, int dtype);
 // cus: compute units the launch may use; leave_cus: the others are to be left to other work.
 StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, bool leave_cus);

@@ -114,6 +114,7 @@ int fluxmi_moe_gather_index(const int32_t *scatter_index, int32_t nrows, int32_t
  *   - N % 4 == 0; a, b 16-byte aligned; d 8-byte (bf16) / 16-byte (fp32) aligned; col_scale 16-byte aligned;
  *   - one expert's weights below 4 GiB (N * K * element size), and with `gather_a`: a_rows > 0 and the whole
  *     of A below 4 GiB (its rows are addressed with 32-bit byte offsets).
+ * With few rows per expert it has a second form that streams the weights (fluxmi_grouped_gemm_launch_info).
  * Any other shape runs a generic kernel (one thread per output element, roughly 100 times slower, meant for
  * correctness only).  fluxmi_grouped_gemm_kernel_kind() tells which of the two a call would take.
  * ---------------------------------------------------------------------------------------------- */
@@ -169,7 +170,7 @@ int fluxmi_grouped_gemm_kernel_kind(const fluxmi_grouped_gemm_args *args);
 #define FLUXMI_GEMM_GENERIC 0
 #define FLUXMI_GEMM_MACRO_TILES 1
 #define FLUXMI_GEMM_STREAM 2    /* few rows per expert: weights streamed into MFMA registers */
-#define FLUXMI_GEMM_BY_SPLITS 3 /* 2 if no expert has more than 32 rows, else 1; decided on the device from `splits` */
+#define FLUXMI_GEMM_BY_SPLITS 3 /* 2 or 1, decided on the device from `splits`: 2 while few experts have more than 32 rows */
 typedef struct fluxmi_gemm_launch_info {
   int32_t form;              /* FLUXMI_GEMM_* */
   int32_t stream_cols;       /* the streaming form: columns per workgroup, */

@@ -12,12 +12,23 @@ def test_form_by_rows(dtype, block_scaled, line):
     def form(rows, splits=None):
         return capi.gemm_launch_info(dtype, 8, rows, 4096, 1024, block_scaled=block_scaled, splits=splits).form
 
-    assert form(1) == form(32) == capi.GEMM_STREAM  # no expert can have more than 32 rows
+    assert form(1) == form(32) == capi.GEMM_STREAM  # no expert can have more than one chunk of 32 rows
     assert form(33) == form(8 * line) == capi.GEMM_BY_SPLITS
     assert form(8 * line + 1) == form(100000) == capi.GEMM_MACRO_TILES
+    # under 16 experts with rows: one chunk each
     assert form(80, [32, 0, 10, 0, 0, 30, 8, 0]) == capi.GEMM_STREAM
-    assert form(80, [33, 0, 10, 0, 0, 30, 7, 0]) == capi.GEMM_MACRO_TILES  # one expert has too many
+    assert form(80, [33, 0, 10, 0, 0, 29, 8, 0]) == capi.GEMM_MACRO_TILES
     assert form(80, [80, -5, 0, 0, 0, 0, 0, 0]) == capi.GEMM_MACRO_TILES
+    # counts past max_rows do not exist
+    assert form(40, [20, 20, 400, 0, 0, 0, 0, 0]) == capi.GEMM_STREAM
+
+    # from 16 on a quarter more chunks of 32 rows than experts with rows
+    def form_of(splits):
+        return capi.gemm_launch_info(dtype, len(splits), 200, 4096, 1024, block_scaled=block_scaled, splits=splits).form
+
+    assert form_of([33] * 4 + [0] * 5 + [3] * 12) == form_of([129] + [0] * 5 + [3] * 15) == capi.GEMM_STREAM
+    assert form_of([33] * 5 + [0] * 5 + [2] * 11) == form_of([129, 33] + [0] * 5 + [2] * 14) == capi.GEMM_MACRO_TILES
+    assert form_of([33] + [0] * 5 + [3] * 14) == capi.GEMM_MACRO_TILES  # 15 experts with rows
 
 
 def test_generic_shapes_have_no_streaming_form():

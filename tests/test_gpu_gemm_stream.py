@@ -1,8 +1,8 @@
 """GPU parity of the weight-streaming form of the grouped GEMM (few rows per expert) at the edges of its tiles.
 
 Operands are small integers, so every product and every partial sum is a whole number below 2^24 and the fp32 result is the
-same in any order of summation: the outputs have to equal an int64 matmul exactly, no tolerance.  (`max_rows` at most 24
-rows per expert on average, fp8, or 40, bf16 / fp16, selects the form.)"""
+same in any order of summation: the outputs have to equal an int64 matmul exactly, no tolerance.  The form computes launches
+of up to 24 (fp8) or 32 rows per expert on average in which few experts have more than 32 rows; `gemm_launch_info` tells."""
 import ctypes
 
 import pytest
@@ -28,8 +28,9 @@ def expected(a, w, splits, rows_of=None):
     return out
 
 
-# (splits, N, K): one row; a chunk of 16 and one more row; 64 rows and one more (two chunks); empty experts and more than 64
-# of them; column tiles cut off at 4 columns; K shorter than a line, ending inside one, and over many lines per wave.
+# (splits, N, K), all of them on 32-column tiles: one row; 15, 16 and 17 rows; empty experts and more than 64 of them; column tiles
+# cut off at 4 columns; K shorter than a line, ending inside one, and over many lines per wave (eight waves).  The macro tiles
+# compute the cases with an expert of more than 32 rows: same results where the two forms meet.
 CASES = [
     ([1], 4, 16), ([1, 0, 2], 64, 128), ([15, 16, 17], 100, 272), ([33, 0, 64, 65, 2], 132, 1040),
     ([0] * 70 + [3, 1] + [0] * 8 + [9], 68, 400), ([7, 5], 1028, 8192 + 48), ([2, 3, 1, 4, 2, 0, 1, 5], 4224, 2064),
@@ -99,9 +100,10 @@ def test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b
 
 
 # The 64-column form: more than four rows per expert on average (block-scaled: any) and at least 512 column tiles in all.  One block
-# and two blocks of 16 rows, rows that do not fill them; columns cut off at 4; K that ends inside a line and numbers of lines that
+# and two blocks of 16 rows, rows that do not fill them, experts of several chunks of 32 rows; columns cut off at 4; K that ends inside a line and numbers of lines that
 # four waves with two lines in flight do not divide; more than 64 experts.
-WIDE = [([32, 0, 31, 17, 16, 1, 2, 9], 4164, 272), ([32, 32, 32, 32, 5, 0, 31, 20], 4096, 1040), ([17] * 70 + [0, 32, 1], 516, 2064 + 16)]
+WIDE = [([32, 0, 31, 17, 16, 1, 2, 9], 4164, 272), ([32, 32, 32, 32, 5, 0, 31, 20], 4096, 1040), ([17] * 70 + [0, 32, 1], 516, 2064 + 16),
+        ([65, 7, 9, 5, 3, 30, 1, 8, 2, 64, 17] + [2] * 8, 2052, 400), ([3] * 66 + [70, 33, 0, 96], 580, 272)]
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
@@ -112,7 +114,8 @@ def test_stream_form_64_columns(dtype, splits, n, k):
     test_stream_form_is_exact_on_integers(dtype, splits, n, k)
 
 
-@pytest.mark.parametrize("splits,n,k", [([32, 0, 31, 17, 16, 1, 2, 9], 4160, 384), ([3] * 70 + [0, 32, 1], 516, 1152)])
+@pytest.mark.parametrize("splits,n,k", [([32, 0, 31, 17, 16, 1, 2, 9], 4160, 384), ([3] * 70 + [0, 32, 1], 516, 1152),
+                                        ([65, 7, 9, 5, 3, 30, 1, 8, 2, 64, 17] + [2] * 8, 2052, 384), ([3] * 66 + [70, 33, 0, 96], 580, 256)])
 @pytest.mark.parametrize("a_layout", [capi.ASCALE_BLOCK128, capi.ASCALE_EXPERT_K_M])
 @pytest.mark.parametrize("b_layout", [capi.BSCALE_N_K, capi.BSCALE_K_N])
 def test_stream_form_64_columns_block_scaled(splits, n, k, a_layout, b_layout):
@@ -122,8 +125,9 @@ def test_stream_form_64_columns_block_scaled(splits, n, k, a_layout, b_layout):
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
-@pytest.mark.parametrize("splits,form", [([32, 7, 0, 20, 32, 1], 2), ([33, 7, 0, 20, 31, 1], 1), ([0, 0, 0, 0, 0, 90], 1),
-                                         ([1] * 70 + [33], 1), ([1] * 70 + [32], 2), ([9, 3, 0, 20], 2)])
+@pytest.mark.parametrize("splits,form", [([32, 7, 0, 20, 32, 1], 2), ([33, 7, 0, 20, 31, 1], 1), ([33] * 4 + [0, 1] + [3] * 12, 2),
+                                         ([33] * 5 + [0, 1] + [3] * 10, 1), ([130, 0] + [2] * 15, 2), ([0, 0, 0, 0, 0, 90], 1), ([1] * 70 + [600], 1),
+                                         ([1] * 70 + [90, 64, 33], 2), ([9, 3, 0, 20], 2)])
 def test_one_form_computes_a_launch(dtype, splits, form):
     """Which form runs is decided on the device; every result is computed, and added to a sum, exactly once."""
     print(f"[case] form by splits {dtype} {splits[-6:]}", flush=True)
@@ -139,6 +143,26 @@ def test_one_form_computes_a_launch(dtype, splits, form):
     sums = torch.zeros(m // 2 + 1, n, dtype=torch.int64).index_add_(0, token.long(), ref)
     out = capi.grouped_gemm_topk_reduce(ad, wd, sp, token.cuda(), m // 2 + 1)
     assert torch.equal(out.cpu(), sums.float().to(out.dtype))
+
+
+def test_form_follows_the_splits_of_each_replay():
+    """A captured launch holds both forms; every replay runs the one that its row counts ask for, as an eager call does."""
+    g = torch.Generator().manual_seed(7)
+    x = torch.randn(90, 400, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(6, 516, 400, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    sp, out = torch.zeros(6, dtype=torch.int32, device="cuda"), torch.zeros(90, 516, device="cuda")
+    capi.grouped_gemm(x, w, sp, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        capi.grouped_gemm(x, w, sp, out=out)
+    for splits in ([32, 0, 8, 20, 30, 0], [33, 0, 7, 20, 30, 0], [15] * 6, [0, 0, 90, 0, 0, 0], [32, 0, 8, 20, 30, 0]):
+        sp.copy_(torch.tensor(splits, dtype=torch.int32))
+        want = capi.grouped_gemm(x, w, sp, out_dtype=torch.float32)
+        out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp8"])
@@ -186,7 +210,7 @@ def test_stream_form_block_scaled_infinite_scales(kblocks, rows, n, experts):
 @pytest.mark.parametrize("margin", [1, 100, 255, 1000])
 @pytest.mark.parametrize("splits,n,k", [([2, 3, 1, 4, 2, 0, 1, 5], 4224, 2064), ([33, 0, 64, 65, 2], 4096, 528), ([1] * 80, 1028, 400)])
 def test_stream_form_leaves_compute_units_and_changes_no_bit(splits, n, k, margin):
-    """With `cu_margin` few workgroups walk all items (down to one compute unit's worth)."""
+    """With `cu_margin` few workgroups walk all items (down to one workgroup); the second case is the macro tiles'."""
     print(f"[case] stream gemm margin={margin} splits={splits[:6]} n={n} k={k}", flush=True)
     g = torch.Generator().manual_seed(n + k)
     a = torch.randn(sum(splits), k, generator=g).to(torch.bfloat16).cuda()
