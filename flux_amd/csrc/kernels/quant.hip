@@ -156,8 +156,8 @@ __global__ __launch_bounds__(256) void quant_row_long_kernel(const uint16_t *__r
 }
 
 // ---- one scale per (row, 128-column block) -----------------------------------------------------
-// 16 consecutive lanes own one block (16 vectors of 8 elements); the amax reduction is four xor
-// shuffles inside that lane group.
+// 16 consecutive lanes own one block (16 vectors of 8 elements); the amax reduction is four DPP moves
+// inside that lane group.
 template <int THREADS_PER_ROW>
 __global__ __launch_bounds__(256) void quant_block128_kernel(const uint16_t *__restrict__ x,
                                                              int64_t rows, int32_t nvec,
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(256) void quant_square_kernel(const uint16_t *__res
 // row cg and passes the scale to the 16 lanes with a DPP broadcast, the first two waves do the columns and pass theirs through
 // LDS.  (Every lane used to divide for all its eight rows and eight columns: 32 divisions a lane instead of
 // four were a third of the kernel.)
-// Measured, both outputs: 11000 x 7168 186 -> 56 us (5.6 TB/s, what a copy reaches), 4096 x 7168 36.8 -> 24.4, 1000 x 2048 15 -> 7;
+// Measured, both outputs: 11000 x 7168 186 -> 56 us (5.6 TB/s; a copy of as many bytes takes 53 to 61 us), 4096 x 7168 36.8 -> 24.4, 1000 x 2048 15 -> 7;
 // without the transposed output 16384 x 7168 64.5 -> 60.3, 16384 x 2048 22.6 -> 19.0.  104 registers, four waves per SIMD: held to
 // 96 or 80 the compiler spills (70 and 109 us).
 // Scales are stored as [ceil(rows/128)][ceil(cols/128)][128] (row inside its block fastest), the
