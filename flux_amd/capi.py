@@ -28,7 +28,7 @@ EXPORTS = (
     "fluxmi_moe_route_sort_workspace_bytes", "fluxmi_moe_route_sort", "fluxmi_moe_gather_index",
     "fluxmi_moe_route_sort_static_max_bytes", "fluxmi_moe_route_sort_static_init", "fluxmi_moe_route_sort_static",
     "fluxmi_grouped_gemm_workspace_bytes", "fluxmi_grouped_gemm", "fluxmi_grouped_gemm_kernel_kind",
-    "fluxmi_grouped_gemm_launch_info",
+    "fluxmi_grouped_gemm_launch_info", "fluxmi_grouped_gemm_panel_info",
     "fluxmi_grouped_gemm_multi", "fluxmi_grouped_gemm_topk_reduce_workspace_bytes",
     "fluxmi_grouped_gemm_topk_reduce", "fluxmi_grouped_gemm_blockscale",
     "fluxmi_topk_gather_reduce", "fluxmi_quant_e4m3_rowwise", "fluxmi_quant_e4m3_square",
@@ -52,6 +52,10 @@ class GroupedGemmArgs(ctypes.Structure):
 
 class GemmLaunchInfo(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int32) for n in ("form", "stream_cols", "stream_waves", "stream_workgroups", "stream_lds_bytes")]
+
+
+class GemmPanelInfo(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("cols", "chunk_rows", "workgroups", "lds_bytes", "macro_tiles_too", "computes")]
 
 
 def lib_path():
@@ -83,6 +87,7 @@ def load():
     lib.fluxmi_grouped_gemm_kernel_kind.argtypes = [ctypes.POINTER(GroupedGemmArgs)]
     lib.fluxmi_grouped_gemm_launch_info.argtypes = [ctypes.POINTER(GroupedGemmArgs), i32, vp, vp, i32,
                                                     ctypes.POINTER(GemmLaunchInfo)]
+    lib.fluxmi_grouped_gemm_panel_info.argtypes = [ctypes.POINTER(GroupedGemmArgs), i32, vp, vp, i32, ctypes.POINTER(GemmPanelInfo)]
     lib.fluxmi_grouped_gemm_topk_reduce_workspace_bytes.restype = sz
     lib.fluxmi_grouped_gemm_topk_reduce_workspace_bytes.argtypes = [i32, i32]
     lib.fluxmi_grouped_gemm_topk_reduce.argtypes = [ctypes.POINTER(GroupedGemmArgs), vp, i32, vp, vp, sz, vp]
@@ -238,16 +243,18 @@ GEMM_GENERIC, GEMM_MACRO_TILES, GEMM_STREAM, GEMM_BY_SPLITS = 0, 1, 2, 3
 
 
 def gemm_launch_info(dtype, nexperts, max_rows, n, k, ngroups=1, block_scaled=False, splits=None, cu_count=256, cu_margin=0,
-                     gathered=False, sched_flags=0, raster_rows=0):
-    """The form a grouped GEMM with aligned operands takes (fluxmi_grouped_gemm_launch_info); needs no GPU."""
+                     gathered=False, sched_flags=0, raster_rows=0, panel=False):
+    """The form a grouped GEMM with aligned operands takes (fluxmi_grouped_gemm_launch_info; with `panel` the
+    fluxmi_grouped_gemm_panel_info of it); needs no GPU."""
     aligned = ctypes.c_void_p(4096)
     args = GroupedGemmArgs(dtype=_DTYPES[dtype], nexperts=nexperts, max_rows=max_rows, n=n, k=k, a_rows=max_rows, a=aligned,
                            b=aligned, d=aligned, splits=aligned, gather_a=aligned if gathered else None, scalar_scale=1.0,
                            cu_margin=cu_margin, sched_flags=sched_flags, raster_rows=raster_rows)
-    info = GemmLaunchInfo()
+    info = GemmPanelInfo() if panel else GemmLaunchInfo()
+    call = load().fluxmi_grouped_gemm_panel_info if panel else load().fluxmi_grouped_gemm_launch_info
     host = None if splits is None else (ctypes.c_int32 * nexperts)(*splits)
-    _check(load().fluxmi_grouped_gemm_launch_info(ctypes.byref(args), ngroups, aligned if block_scaled else None, host, cu_count,
-                                                  ctypes.byref(info)), "fluxmi_grouped_gemm_launch_info")
+    _check(call(ctypes.byref(args), ngroups, aligned if block_scaled else None, host, cu_count, ctypes.byref(info)),
+           "fluxmi_grouped_gemm_panel_info" if panel else "fluxmi_grouped_gemm_launch_info")
     return info
 
 

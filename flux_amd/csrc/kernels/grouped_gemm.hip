@@ -1,6 +1,7 @@
 // Grouped GEMM entry point: argument checks, choice between the MFMA kernels and the generic kernel, and
 // the generic kernel itself.  The MFMA kernels are the macro tiles (grouped_gemm_kernel.hpp) and, for few rows per
 // expert, the streaming form (grouped_gemm_stream.hip).
+#include "grouped_gemm_panel.hpp"
 #include "grouped_gemm_stream.hpp"
 
 namespace fluxmi {
@@ -122,6 +123,7 @@ struct DryRun {
   int cus = 0;
   bool stream = false, macro = false;
   StreamPlan plan = {};
+  PanelPlan panel = {};
 };
 
 // dry_run: check the arguments and report which kernel would run (1 MFMA, 0 generic) without launching.
@@ -216,22 +218,32 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   p.sched_flags = args->sched_flags;
 
   const bool stream_form = mfma && grouped_gemm_stream_takes(p, args->dtype);
-  const bool macro = mfma && (!stream_form || args->max_rows > kStreamRows);
-  p.by_splits = stream_form && macro ? 1 : 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  p.by_splits = 0;
   int cus = dry_run ? dry_run->cus : fluxmi_device_cu_count();
   FLUXMI_REQUIRE(cus > 0 || dry_run, FLUXMI_ERR_HIP, "grouped_gemm: cannot query the device");
   // CUs left to other work of the caller (Flux's sm_margin): both MFMA forms launch fewer workgroups.
   cus = cus - args->cu_margin > 1 ? cus - args->cu_margin : 1;
-  const StreamPlan plan = stream_form ? plan_grouped_gemm_stream(p, args->dtype, cus, args->cu_margin > 0) : StreamPlan{};
+  const bool leave_cus = args->cu_margin > 0;
+  PanelPlan panel = {};
+  if (mfma) panel = plan_panel(p, args->dtype, stream_form, cus, leave_cus);
+  const StreamPlan plan = stream_form && panel.cols == 0 ? plan_grouped_gemm_stream(p, args->dtype, cus, leave_cus) : StreamPlan{};
+  const bool macro = mfma && !panel.any_splits && (!stream_form || args->max_rows > kStreamRows);
+  if (macro) p.by_splits = panel.cols != 0 ? panel.chunk_rows : (stream_form ? kStreamRows : 0);
   if (dry_run) {
     dry_run->stream = stream_form;
     dry_run->macro = macro;
     dry_run->plan = plan;
+    dry_run->panel = panel;
     return mfma ? 1 : 0;
   }
 
-  if (stream_form) launch_grouped_gemm_stream(p, args->dtype, plan, s);
+  if (panel.cols != 0) {
+    const int rc = launch_grouped_gemm_panel(p, args->dtype, panel, s);
+    if (rc != FLUXMI_OK) return rc;
+  } else if (stream_form) {
+    launch_grouped_gemm_stream(p, args->dtype, plan, s);
+  }
   if (macro) {
     // Upper bound of the tile count: never launch more workgroups than tiles.
     const int64_t tiles_n = (args->n + BN - 1) / BN * ngroups;
@@ -376,10 +388,23 @@ extern "C" int fluxmi_grouped_gemm_kernel_kind(const fluxmi_grouped_gemm_args *a
   return fluxmi::run_grouped_gemm(args, 1, &b, &d, &alpha, nullptr, &dry);
 }
 
-extern "C" int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
-                                               const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_launch_info *info) {
-  using namespace fluxmi;
-  FLUXMI_REQUIRE(args != nullptr && info != nullptr, FLUXMI_ERR_INVALID_ARG, "grouped_gemm_launch_info: null args / info");
+namespace fluxmi {
+namespace {
+
+// Whether a form for few rows per expert, with chunks of chunk_rows rows, computes a launch with these splits.
+bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, int chunk_rows) {
+  int left = args->max_rows, chunks = 0, active = 0;
+  for (int e = 0; e < args->nexperts; ++e) {
+    const int rows = splits_host[e] < 0 ? 0 : (splits_host[e] < left ? splits_host[e] : left);
+    left -= rows;
+    active += rows > 0 ? 1 : 0;
+    chunks += (rows + chunk_rows - 1) / chunk_rows;
+  }
+  return chunks <= stream_chunks_limit(active, chunk_rows);
+}
+
+// The dry run of a launch of ngroups weight groups that all look like args->b / d / alpha.
+int describe_launch(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale, int32_t cu_count, DryRun &dry) {
   FLUXMI_REQUIRE(cu_count >= 1, FLUXMI_ERR_INVALID_ARG, "grouped_gemm_launch_info: cu_count must be positive");
   FLUXMI_REQUIRE(ngroups >= 1 && ngroups <= kMaxWeightGroups, FLUXMI_ERR_UNSUPPORTED, "grouped_gemm_launch_info: ngroups=%d outside [1,%d]",
                  ngroups, kMaxWeightGroups);
@@ -389,28 +414,53 @@ extern "C" int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *a
   for (int g = 0; g < kMaxWeightGroups; ++g) b[g] = args->b, d[g] = args->d, alpha[g] = args->alpha;
   BlockScales bs;
   bs.a_scale = bs.b_scale = a_scale;
-  DryRun dry;
   dry.cus = cu_count;
+  return run_grouped_gemm(args, ngroups, b, d, alpha, nullptr, &dry, 0, a_scale != nullptr ? &bs : nullptr);
+}
+
+}  // namespace
+}  // namespace fluxmi
+
+extern "C" int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
+                                               const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_launch_info *info) {
+  using namespace fluxmi;
+  FLUXMI_REQUIRE(args != nullptr && info != nullptr, FLUXMI_ERR_INVALID_ARG, "grouped_gemm_launch_info: null args / info");
   *info = fluxmi_gemm_launch_info{};
-  const int kind = run_grouped_gemm(args, ngroups, b, d, alpha, nullptr, &dry, 0, a_scale != nullptr ? &bs : nullptr);
+  DryRun dry;
+  const int kind = describe_launch(args, ngroups, a_scale, cu_count, dry);
   if (kind < 0) return kind;
-  info->form = kind == 0 ? FLUXMI_GEMM_GENERIC : (!dry.stream ? FLUXMI_GEMM_MACRO_TILES : (dry.macro ? FLUXMI_GEMM_BY_SPLITS : FLUXMI_GEMM_STREAM));
-  if (info->form == FLUXMI_GEMM_BY_SPLITS && splits_host != nullptr) {
-    int left = args->max_rows, chunks = 0, active = 0;
-    for (int e = 0; e < args->nexperts; ++e) {
-      const int rows = splits_host[e] < 0 ? 0 : (splits_host[e] < left ? splits_host[e] : left);
-      left -= rows;
-      active += rows > 0 ? 1 : 0;
-      chunks += (rows + kStreamRows - 1) / kStreamRows;
-    }
-    info->form = chunks <= stream_chunks_limit(active) ? FLUXMI_GEMM_STREAM : FLUXMI_GEMM_MACRO_TILES;
-  }
-  if (dry.stream) {
+  info->form = kind == 0 ? FLUXMI_GEMM_GENERIC : (!dry.stream ? FLUXMI_GEMM_MACRO_TILES : (args->max_rows > kStreamRows ? FLUXMI_GEMM_BY_SPLITS : FLUXMI_GEMM_STREAM));
+  if (info->form == FLUXMI_GEMM_BY_SPLITS && splits_host != nullptr)
+    info->form = few_chunks(args, splits_host, kStreamRows) ? FLUXMI_GEMM_STREAM : FLUXMI_GEMM_MACRO_TILES;
+  if (dry.stream && dry.panel.cols != 0) {
+    info->stream_cols = dry.panel.cols;
+    info->stream_waves = 4;
+    info->stream_workgroups = static_cast<int32_t>(dry.panel.workgroups);
+    info->stream_lds_bytes = dry.panel.lds_bytes;
+  } else if (dry.stream) {
     info->stream_cols = dry.plan.cols;
     info->stream_waves = dry.plan.waves;
     info->stream_workgroups = static_cast<int32_t>(dry.plan.workgroups);
     info->stream_lds_bytes = dry.plan.lds_bytes;
   }
+  return FLUXMI_OK;
+}
+
+extern "C" int fluxmi_grouped_gemm_panel_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
+                                              const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_panel_info *info) {
+  using namespace fluxmi;
+  FLUXMI_REQUIRE(args != nullptr && info != nullptr, FLUXMI_ERR_INVALID_ARG, "grouped_gemm_panel_info: null args / info");
+  *info = fluxmi_gemm_panel_info{};
+  DryRun dry;
+  const int kind = describe_launch(args, ngroups, a_scale, cu_count, dry);
+  if (kind < 0) return kind;
+  if (kind == 0 || dry.panel.cols == 0) return FLUXMI_OK;
+  info->cols = dry.panel.cols;
+  info->chunk_rows = dry.panel.chunk_rows;
+  info->workgroups = static_cast<int32_t>(dry.panel.workgroups);
+  info->lds_bytes = dry.panel.lds_bytes;
+  info->macro_tiles_too = dry.macro ? 1 : 0;
+  info->computes = !dry.macro || (splits_host != nullptr && few_chunks(args, splits_host, dry.panel.chunk_rows)) ? 1 : 0;
   return FLUXMI_OK;
 }
 

@@ -92,17 +92,24 @@ struct GemmParams {
   int32_t b_scale_layout;  // FLUXMI_BSCALE_*
   int32_t half_is_f16;     // 2-byte operands and outputs are fp16, not bf16 (read by the generic kernel; the MFMA
                            // kernel is built once per 16-bit type)
-  // 1: the streaming form and the macro tiles are both launched; `splits` says which of them computes the launch
-  // (stream_chunks_limit) and the other returns at once.  0: the launched one computes it.
+  // Not 0: a form for few rows per expert, whose items are chunks of up to this many rows (a power of two), and the macro tiles are both launched;
+  // `splits` says which of them computes the launch (stream_chunks_limit) and the other returns at once.  0: the launched one
+  // computes it.
   int32_t by_splits;
 };
 
 // Rows of a work item of the streaming form: two 16-row MFMA blocks.  An expert with more is several items per column tile.
 constexpr int kStreamRows = 32;
 
-// Most chunks of up to kStreamRows rows that the streaming form computes in a launch in which `active` experts have rows.
-__host__ __device__ inline int stream_chunks_limit(int active) { return active + (active >= 16 ? active / 4 : 0); }
-
+// Most chunks of up to chunk_rows rows that a form for few rows per expert computes in a launch in which `active` experts have
+// rows: it reads an expert's weights once per chunk, and the items of a launch take about the same time each.  Chunks of 32 rows:
+// one per expert, from 16 experts on a quarter more (one more of few can be a whole round of the card: 8 experts 4096 x 14336, 10
+// chunks 241 us, macro tiles 219).  Longer ones: an eighth and one more (Zipf with exponent 1.2, us, panel and macro tiles: bf16 8
+// experts 14336 x 4096, 64 rows per expert on average, 9 chunks 196 / 225; a layer of 65 experts 5760 x 1792 at 38 rows, a quarter
+// more chunks than experts 646 / 619; all rows on one of 8 experts 95 / 47).
+__host__ __device__ inline int stream_chunks_limit(int active, int chunk_rows) {
+  return chunk_rows <= kStreamRows ? active + (active >= 16 ? active / 4 : 0) : active + active / 8 + 1;
+}
 
 // One launcher per element type, each in a translation unit of its own (the kernel is a long compile).
 int launch_grouped_gemm_bf16(const GemmParams &p, int grid, hipStream_t s);

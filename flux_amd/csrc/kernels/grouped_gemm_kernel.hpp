@@ -1588,7 +1588,7 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
   int total_tiles = 0, skinny_experts = 0;
   {
     int row_carry = 0, acc_tiles = 0, acc_cand = 0;
-    int chunks = 0, active = 0;  // for launches that the streaming form may compute
+    int chunks = 0, active = 0;  // for launches that a form for few rows per expert may compute
     for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
       const int ee = e0 + lane;
       int rows = ee < p.nexperts ? p.splits[ee] : 0;
@@ -1599,7 +1599,7 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
       if (end > p.max_rows) end = p.max_rows;
       if (p.by_splits) {
         active += __popcll(__ballot(end > begin));
-        chunks += __builtin_amdgcn_readlane(wave_inclusive_scan((end - begin + kStreamRows - 1) / kStreamRows), 63);
+        chunks += __builtin_amdgcn_readlane(wave_inclusive_scan((end - begin + p.by_splits - 1) >> (31 - __builtin_clz(p.by_splits))), 63);
       }
       int tiles = ((end - begin + BM - 1) / BM) * tiles_n;
       int cand = (end > begin && ((end - begin - 1) & (BM - 1)) < 64) ? 1 : 0;
@@ -1612,7 +1612,7 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
       acc_cand += cand;
       row_carry += __shfl(incl, 63, 64);
     }
-    if (p.by_splits && chunks <= stream_chunks_limit(active)) return;  // the streaming form runs this launch
+    if (p.by_splits && chunks <= stream_chunks_limit(active, p.by_splits)) return;  // the other form runs this launch
     total_tiles = __builtin_amdgcn_readfirstlane(acc_tiles);
     skinny_experts = __builtin_amdgcn_readfirstlane(acc_cand);
   }

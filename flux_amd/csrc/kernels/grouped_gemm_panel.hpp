@@ -1,0 +1,24 @@
+// Launcher of the panel forms of the grouped GEMM (grouped_gemm_panel.hip).
+#pragma once
+
+#include "grouped_gemm.hpp"
+
+namespace fluxmi {
+
+// cols == 0: the launch is not for these forms.
+struct PanelPlan {
+  int cols;             // columns per workgroup: 64 or 128 (weights through LDS), 256 (weights through registers)
+  int chunk_rows;       // most rows of a work item: 32, 64 or 128
+  bool pairs;           // 64 columns, 32 rows: lines of K are asked for in pairs
+  int blocks;           // items the launch is numbered for
+  unsigned workgroups;  // workgroups launched; fewer than `blocks`: each walks several items
+  bool walk;
+  bool any_splits;      // computes every distribution of the rows; otherwise only those with few chunks (stream_chunks_limit)
+  int lds_bytes;        // per workgroup
+};
+
+// few_rows: the launch has few enough rows for the streaming form.
+PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, bool leave_cus);
+int launch_grouped_gemm_panel(const GemmParams &p, int dtype, const PanelPlan &plan, hipStream_t s);
+
+}  // namespace fluxmi

@@ -36,121 +36,18 @@
 // 218 -> 165; 64 experts 1408 x 2048, 256 rows: 113 -> 57 [57], 2048 rows 116 -> 78; fp8 32 experts 2048 x 7168, 256 rows:
 // 94 -> 72 [72], 768 rows 96 -> 82; 7168 x 2048: 115 -> 80 [72] and 118 -> 98; block-scaled, the same four: 123 -> 74,
 // 125 -> 83, 148 -> 85 and 152 -> 104.
-#include "grouped_gemm_stream.hpp"
+#include "grouped_gemm_rows.hpp"
 
 namespace fluxmi {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-enum class Elem { BF16, F16, FP8, FP8_BLOCKSCALED };
-constexpr bool is_fp8(Elem t) { return t == Elem::FP8 || t == Elem::FP8_BLOCKSCALED; }
-
 #if defined(__HIP_DEVICE_COMPILE__)
-
-constexpr uint32_t kOutOfRange = 0xfffffff0u;  // a byte offset past every buffer: the load returns zeros
-
-// Clamped like the macro-tile kernel's: negative counts are 0, rows past max_rows do not exist.
-struct WorkItem {
-  int e, expert_base, expert_rows;  // the expert, its first row, its row count
-  int row_base, rows;               // the item's rows (0: there is no such item)
-  int nt;                           // column tile, over all weight groups
-};
-
-// Work item -> (expert, chunk of its rows, column tile).  One wave-wide pass over the splits counts the chunks, a second
-// finds the item's; with up to 64 experts both work on the same registers.
-__device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n, int block) {
-  const int lane = threadIdx.x & 63;
-  int begin, rows, chunks_end;  // this lane's expert of the 64 looked at
-  auto load = [&](int e0, int &row_carry, int &chunk_carry) {
-    const int ee = e0 + lane;
-    int r = ee < p.nexperts ? p.splits[ee] : 0;
-    if (r < 0) r = 0;
-    const int incl = wave_inclusive_scan(r);
-    begin = row_carry + incl - r;
-    int end = row_carry + incl;
-    if (begin > p.max_rows) begin = p.max_rows;
-    if (end > p.max_rows) end = p.max_rows;
-    rows = end - begin;
-    row_carry += __builtin_amdgcn_readlane(incl, 63);
-    chunks_end = chunk_carry + wave_inclusive_scan((rows + kStreamRows - 1) / kStreamRows);
-    chunk_carry = __builtin_amdgcn_readlane(chunks_end, 63);
-    return __popcll(__ballot(rows > 0));
-  };
-  int row_carry = 0, total = 0, active = 0;
-  for (int e0 = 0; e0 < p.nexperts; e0 += 64) active += load(e0, row_carry, total);
-  WorkItem w = {0, 0, 0, 0, 0, 0};
-  if (p.by_splits && total > stream_chunks_limit(active)) return w;  // the macro tiles run this launch
-  // Workgroups are dealt to the eight XCDs round-robin.
-  const int items = total * tiles_n, per_xcd = (items + 7) / 8, i = block >> 3, item = (block & 7) * per_xcd + i;
-  if (i >= per_xcd || item >= items) return w;
-  int row_carry2 = 0, chunk_carry2 = 0;
-  for (int e0 = 0; e0 < p.nexperts; e0 += 64) {
-    if (p.nexperts > 64) load(e0, row_carry2, chunk_carry2);
-    const uint64_t hit = __ballot(item < chunks_end * tiles_n);
-    if (hit != 0) {
-      const int src = __ffsll(static_cast<unsigned long long>(hit)) - 1;
-      w.e = e0 + src;
-      w.expert_base = __builtin_amdgcn_readlane(begin, src);
-      w.expert_rows = __builtin_amdgcn_readlane(rows, src);
-      const int chunks = (w.expert_rows + kStreamRows - 1) / kStreamRows;
-      const int local = item - (__builtin_amdgcn_readlane(chunks_end, src) - chunks) * tiles_n;
-      w.nt = local / chunks;
-      const int first = (local - w.nt * chunks) * kStreamRows;
-      w.row_base = w.expert_base + first;
-      w.rows = w.expert_rows - first < kStreamRows ? w.expert_rows - first : kStreamRows;
-      return w;
-    }
-  }
-  return w;
-}
 
 template <Elem T, int MB, int NB>
 struct Line {  // one 128-byte line of every row of the wave's operand blocks, as loaded
   i32x4 w[NB][2], x[MB][2];
   float as[MB], bs;
 };
-
-// Two loads of eight rows each (lane: row l & 7, chunk 2 * (l >> 4) + bit 3 of l) -> two MFMA fragments of the sixteen rows
-// (lane: row l & 15, chunks 2 * (l >> 4) and 2 * (l >> 4) + 1): the lanes with bit 3 set of the first change places with
-// the lanes with bit 3 clear of the second.
-__device__ __forceinline__ void to_fragments(i32x4 (&v)[2]) {
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int a = v[0][c], b = v[1][c];
-    v[0][c] = __builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false);  // row_ror:8 into lanes 8..15 of every 16
-    v[1][c] = __builtin_amdgcn_update_dpp(b, a, 0x128, 0xf, 0x3, false);  // ... into lanes 0..7
-  }
-}
-
-template <Elem T>
-__device__ __forceinline__ f32x4 mfma_line(const i32x4 (&w)[2], const i32x4 (&x)[2], f32x4 acc) {
-  if constexpr (is_fp8(T)) {
-    const i32x8 wa = {w[0][0], w[0][1], w[0][2], w[0][3], w[1][0], w[1][1], w[1][2], w[1][3]};
-    const i32x8 xa = {x[0][0], x[0][1], x[0][2], x[0][3], x[1][0], x[1][1], x[1][2], x[1][3]};
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wa, xa, acc, 0, 0, 0, 0, 0, 0);
-  } else {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if constexpr (T == Elem::F16)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w[h]), __builtin_bit_cast(f16x8, x[h]), acc, 0, 0, 0);
-      else
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[h]), __builtin_bit_cast(bf16x8, x[h]), acc, 0, 0, 0);
-    }
-    return acc;
-  }
-}
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, int64_t bytes) {
-  const uint32_t n = bytes > 0xffffffffll ? 0xffffffffu : static_cast<uint32_t>(bytes < 0 ? 0 : bytes);
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, static_cast<int>(n), 0x00020000);
-}
-
-template <int AUX>
-__device__ __forceinline__ i32x4 load16(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) {
-  return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(voff), soff, AUX));
-}
 
 // 16 * MB rows x 16 * NB columns of one expert: partial sums of this wave's lines of K into acc.
 template <Elem T, int MB, int NB, int WAVES>
@@ -343,7 +240,7 @@ void grouped_gemm_stream_kernel(const GemmParams p, const int blocks) {
   const int stride = static_cast<int>(gridDim.x);
   int block = blockIdx.x;
   do {
-    const WorkItem t = locate(p, tiles_n1 * p.ngroups, block + team * stride);
+    const WorkItem t = locate(p, tiles_n1 * p.ngroups, kStreamRows, block + team * stride);
     const int g = p.ngroups > 1 ? t.nt / tiles_n1 : 0;
     const int n0 = (t.nt - g * tiles_n1) * (16 * NB);
     if constexpr (!WALK) {
@@ -368,7 +265,7 @@ int64_t one_chunk_items(const GemmParams &p, int ngroups, int nb) {
 }
 int64_t most_items(const GemmParams &p, int ngroups, int nb) {
   const int active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
-  const int chunks = active + (p.max_rows - active) / kStreamRows, limit = stream_chunks_limit(active);
+  const int chunks = active + (p.max_rows - active) / kStreamRows, limit = stream_chunks_limit(active, kStreamRows);
   return static_cast<int64_t>(chunks < limit ? chunks : limit) * ((p.n + 16 * nb - 1) / (16 * nb)) * ngroups;
 }
 

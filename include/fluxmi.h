@@ -181,6 +181,20 @@ typedef struct fluxmi_gemm_launch_info {
 int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
                                     const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_launch_info *info);
 
+/* The panel tiles: what launches of up to about 96 rows per expert run on where the streaming form above is not the one that
+ * splits K over waves.  They compute FLUXMI_GEMM_STREAM launches with stream_waves == 4 and, with more rows per expert, launches
+ * that fluxmi_grouped_gemm_launch_info calls FLUXMI_GEMM_MACRO_TILES; arguments as there. */
+typedef struct fluxmi_gemm_panel_info {
+  int32_t cols;            /* columns per workgroup; 0 (and everything else 0): not for these tiles */
+  int32_t chunk_rows;      /* most rows of a work item; an expert with more is several */
+  int32_t workgroups;      /* workgroups launched */
+  int32_t lds_bytes;       /* LDS per workgroup */
+  int32_t macro_tiles_too; /* 1: the macro tiles are launched as well and the splits decide on the device which of the two computes */
+  int32_t computes;        /* 1: these tiles compute the launch (with macro_tiles_too: for splits_host; 0 without it) */
+} fluxmi_gemm_panel_info;
+int fluxmi_grouped_gemm_panel_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
+                                   const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_panel_info *info);
+
 /* ------------------------------------------------------------------------------------------------
  * Top-k reduction fused into the grouped GEMM's epilogue (layer1 in one pass, no [M, N] intermediate):
  *

@@ -1,0 +1,216 @@
+"""GPU parity of the panel tiles of the grouped GEMM (up to about 96 rows per expert) at the edges of their tiles.
+
+Operands are small integers and scales powers of two, so every product and every partial sum is a whole multiple of a power of two
+below 2^24 steps: the fp32 result is the same in any order of summation and has to equal a float64 matmul exactly, no tolerance."""
+import ctypes
+import random
+
+import pytest
+import torch
+
+from flux_amd import capi
+
+pytestmark = pytest.mark.gpu
+DT = {"bf16": torch.bfloat16, "f16": torch.float16, "fp8": torch.float8_e4m3fn, "bs": torch.float8_e4m3fn}
+
+
+def spread(lo, hi, experts, seed):
+    rng = random.Random(seed)
+    return [lo, hi] + [rng.randint(lo, hi) for _ in range(experts - 2)]
+
+
+# (name, splits, N, K, columns, rows of a chunk): every instance of the tiles, with chunks at both sides of 32, 64, 96 and 128 rows, empty
+# experts and more than 64 of them, columns cut off at 4 (the last wave's moved back, also past a whole wave), K shorter than a line,
+# ending inside one, and of as many lines as the rings have stages and more.
+CASES = [
+    ("64 columns, 32 rows", [32, 0, 31, 17, 16, 1, 2, 9], 4164, 272, 64, 32),
+    ("64 columns, 32 rows, lines in pairs", [32, 0, 31, 17, 16, 1, 2, 9], 4164, 3216, 64, 32),
+    ("128 columns, 32 rows", [1, 32, 16, 17] + [0] * 3 + [5] * 123, 1028, 144, 128, 32),
+    ("64 columns, 64 rows", [64, 65, 1, 0, 16, 97, 33, 130], 132, 272, 64, 64),
+    ("64 columns, 64 rows, all on one", [0, 0, 300, 0], 68, 16, 64, 64),
+    ("64 columns, 128 rows, small", [150, 129, 300, 1, 128], 132, 272, 64, 128),
+    ("128 columns, 64 rows", spread(1, 64, 70, 1), 580, 400, 128, 64),
+    ("256 columns", spread(33, 128, 70, 2), 1540, 400, 256, 128),
+    ("256 columns, short K", [64, 96, 128, 65, 97, 48] + [50] * 64, 1540, 48, 256, 128),
+    ("128 columns, 128 rows", spread(1, 128, 24, 3), 1412, 1040, 128, 128),
+    ("64 columns, 128 rows", [32, 33, 64, 65, 96, 97, 128, 0], 1092, 8192 + 16, 64, 128),
+]
+
+
+def made(splits, n, k, dtype, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    m, e = sum(splits), len(splits)
+    a = torch.randint(-3, 4, (m, k), generator=g, device="cuda").float()
+    w = torch.randint(-3, 4, (e, n, k), generator=g, device="cuda").float()
+    return a, w, torch.tensor(splits, dtype=torch.int32, device="cuda"), g
+
+
+def product(a, w, splits):
+    out, at = [], 0
+    for e, r in enumerate(splits):
+        out.append(a[at:at + r].double() @ w[e].double().t().contiguous())
+        at += r
+    return torch.cat(out)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("name,splits,n,k,cols,chunk", CASES, ids=[c[0] for c in CASES])
+def test_panel_tiles_are_exact_on_integers(name, splits, n, k, cols, chunk, dtype):
+    print(f"[case] panel gemm {dtype} {name} n={n} k={k}", flush=True)
+    m, e = sum(splits), len(splits)
+    info = capi.gemm_launch_info(DT[dtype], e, m, n, k, splits=splits, panel=True)
+    if dtype != "fp8" or name != "64 columns, 128 rows":  # (fp8: half the bytes, so the small launches' 64 rows)
+        assert (info.cols, info.chunk_rows, info.computes) == (cols, chunk, 1)
+    a, w, sp, g = made(splits, n, k, dtype, n + k)
+    ad, wd = a.to(DT[dtype]), w.to(DT[dtype])
+    assert torch.equal(capi.grouped_gemm(ad, wd, sp, out_dtype=torch.float32).double(), product(a, w, splits))
+    # rows picked by a gather, results put elsewhere, every scale factor, a second weight tensor, margins
+    perm = torch.randperm(m, generator=g, device="cuda").to(torch.int32)
+    to = perm.flip(0).contiguous()
+    row_scale = 2.0 ** torch.randint(-1, 2, (m,), generator=g, device="cuda").float()
+    col_scale = 2.0 ** torch.randint(-1, 2, (e, n), generator=g, device="cuda").float()
+    alpha = 2.0 ** torch.randint(-1, 2, (e,), generator=g, device="cuda").float()
+    expert = torch.repeat_interleave(torch.arange(e, device="cuda"), sp.long())
+    want = torch.empty(m, n, dtype=torch.float64, device="cuda")
+    want[to.long()] = product(a[perm.long()], w, splits) * (alpha[expert] * row_scale).double()[:, None] * col_scale[expert].double()
+    for margin in (0, 40, 250, 1000):
+        out = torch.full((m, n), -7.0, device="cuda")
+        capi.grouped_gemm(ad, wd, sp, out=out, gather_a=perm, scatter_d=to, row_scale=row_scale, col_scale=col_scale, alpha=alpha, cu_margin=margin)
+        assert torch.equal(out.double(), want), f"margin {margin}"
+    two = capi.grouped_gemm_multi(ad, [wd, wd.flip(0).contiguous()] if dtype != "fp8" else [wd, wd], sp, out_dtype=torch.float32)
+    assert torch.equal(two[0].double(), product(a, w, splits))
+    assert torch.equal(two[1].double(), product(a, w.flip(0) if dtype != "fp8" else w, splits))
+    # added to sums: every result once
+    token = torch.randint(0, m // 2 + 1, (m,), generator=g, device="cuda")
+    sums = torch.zeros(m // 2 + 1, n, dtype=torch.float64, device="cuda").index_add_(0, token, product(a, w, splits))
+    assert torch.equal(capi.grouped_gemm_topk_reduce(ad, wd, sp, token.to(torch.int32), m // 2 + 1), sums.float().to(capi._half_out(ad.dtype)))
+
+
+BLOCK_SCALED = [
+    ("64 columns, 32 rows", [32, 0, 31, 17, 16, 1, 2, 9], 4160, 384, 64, 32),
+    ("64 columns, 32 rows, lines in pairs", [32, 0, 31, 17, 16, 1, 2, 9], 4160, 6272, 64, 32),
+    ("128 columns, 32 rows", [1, 32, 16, 17] + [0] * 3 + [5] * 123, 1088, 256, 128, 32),
+    ("64 columns, 64 rows", [64, 65, 1, 0, 16, 97, 33, 130], 192, 384, 64, 64),
+    ("128 columns, 64 rows", spread(1, 64, 70, 1), 640, 640, 128, 64),
+    ("128 columns, 128 rows", spread(1, 128, 24, 3), 1408, 1152, 128, 128),
+    ("64 columns, 128 rows", [32, 33, 64, 65, 96, 97, 128, 0], 1088, 8192, 64, 128),
+]
+
+
+def block_scales(m, e, n, k, splits, a_layout, b_layout, g):
+    kb, nb = k // 128, (n + 127) // 128
+    sa = 2.0 ** torch.randint(-1, 2, (m, kb), generator=g, device="cuda").float()
+    sb = 2.0 ** torch.randint(-1, 2, (e, nb, kb), generator=g, device="cuda").float()
+    if a_layout == capi.ASCALE_BLOCK128:
+        pad = torch.zeros((m + 127) // 128 * 128, kb, device="cuda")
+        pad[:m] = sa
+        sad = pad.view(-1, 128, kb).permute(0, 2, 1).contiguous()
+    else:
+        at, parts = 0, []
+        for r in splits:
+            parts.append(sa[at:at + r].t().contiguous().flatten())
+            at += r
+        sad = torch.cat(parts)
+    return sa, sb, sad, (sb if b_layout == capi.BSCALE_N_K else sb.transpose(1, 2).contiguous())
+
+
+@pytest.mark.parametrize("name,splits,n,k,cols,chunk", BLOCK_SCALED, ids=[c[0] for c in BLOCK_SCALED])
+@pytest.mark.parametrize("a_layout", [capi.ASCALE_BLOCK128, capi.ASCALE_EXPERT_K_M])
+@pytest.mark.parametrize("b_layout", [capi.BSCALE_N_K, capi.BSCALE_K_N])
+def test_panel_tiles_block_scaled_are_exact_on_integers(name, splits, n, k, cols, chunk, a_layout, b_layout):
+    print(f"[case] panel gemm block-scaled {name} n={n} k={k} layouts {a_layout} {b_layout}", flush=True)
+    m, e = sum(splits), len(splits)
+    info = capi.gemm_launch_info(DT["bs"], e, m, n, k, splits=splits, panel=True, block_scaled=True)
+    if name != "64 columns, 128 rows":
+        assert (info.cols, info.chunk_rows, info.computes) == (cols, chunk, 1)
+    a, w, sp, g = made(splits, n, k, "fp8", n + k)
+    sa, sb, sad, sbd = block_scales(m, e, n, k, splits, a_layout, b_layout, g)
+    af = a * torch.repeat_interleave(sa, 128, dim=1)
+    wf = w * torch.repeat_interleave(torch.repeat_interleave(sb, 128, dim=1)[:, :n], 128, dim=2)
+    want = product(af, wf, splits)
+    ad, wd = a.to(DT["bs"]), w.to(DT["bs"])
+    assert torch.equal(capi.grouped_gemm_blockscale(ad, wd, sp, sad, sbd, a_layout, b_layout, out_dtype=torch.float32).double(), want)
+    if a_layout == capi.ASCALE_BLOCK128:  # rows, and their scales, picked by a gather
+        perm = torch.randperm(m, generator=g, device="cuda").to(torch.int32)
+        got = capi.grouped_gemm_blockscale(ad, wd, sp, sad, sbd, a_layout, b_layout, out_dtype=torch.float32, gather_a=perm)
+        assert torch.equal(got.double(), product(af[perm.long()], wf, splits))
+    for margin in (40, 1000):
+        args, out = capi._gemm_args(ad, wd, sp, None, None, None, None, None, None, 1.0, None, None, torch.float32, margin, 0, 0)
+        capi._check(capi.load().fluxmi_grouped_gemm_blockscale(ctypes.byref(args), capi._ptr(sad), a_layout, capi._ptr(sbd), b_layout, capi._stream()),
+                    "fluxmi_grouped_gemm_blockscale")
+        assert torch.equal(out.double(), want), f"margin {margin}"
+
+
+@pytest.mark.parametrize("kblocks,rows,n,experts", [(1, 40, 128, 4), (2, 40, 640, 70), (3, 70, 1408, 24), (9, 90, 192, 3), (17, 5, 2176, 24), (49, 5, 2176, 24)])
+def test_panel_tiles_infinite_scales(kblocks, rows, n, experts):
+    """An infinite product of scales makes a result infinite, not NaN, whatever K is padded to inside the kernel."""
+    print(f"[case] panel gemm infinite scales kblocks={kblocks} rows={rows} n={n} experts={experts}", flush=True)
+    k, m = kblocks * 128, rows * experts
+    assert capi.gemm_launch_info(DT["bs"], experts, m, n, k, panel=True, block_scaled=True).cols > 0
+    g = torch.Generator(device="cuda").manual_seed(kblocks)
+    a, w = (torch.randint(1, 4, s, generator=g, device="cuda").float() for s in ((m, k), (experts, n, k)))
+    sa, sb = torch.ones(m, kblocks, device="cuda"), torch.ones(experts, (n + 127) // 128, kblocks, device="cuda")
+    sa[1::rows, 0], sb[:, 0, 0] = 2.0 ** 100, 2.0 ** 100  # row 1 of an expert overflows in its first 128 columns
+    sa[2::rows, kblocks - 1] = float("inf")              # row 2 is infinite everywhere
+    pad = torch.zeros((m + 127) // 128 * 128, kblocks, device="cuda")
+    pad[:m] = sa
+    got = capi.grouped_gemm_blockscale(a.to(DT["bs"]), w.to(DT["bs"]), torch.full((experts,), rows, dtype=torch.int32, device="cuda"),
+                                       pad.view(-1, 128, kblocks).permute(0, 2, 1).contiguous(), sb, out_dtype=torch.float32)
+    assert not torch.isnan(got).any()
+    inf = torch.zeros(experts, rows, n, dtype=torch.bool, device="cuda")
+    inf[:, 1, :128] = True
+    inf[:, 2] = True
+    assert torch.equal(torch.isinf(got) & (got > 0), inf.view(m, n))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("name,splits,n,k,cols,chunk", CASES, ids=[c[0] for c in CASES])
+def test_panel_tiles_have_the_bits_of_the_macro_tiles(name, splits, n, k, cols, chunk, dtype):
+    """16-bit operands: the same rows among so many others that the macro tiles compute the launch."""
+    print(f"[case] panel gemm bits {dtype} {name} n={n} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    more = [r + 200 for r in splits]
+    assert capi.gemm_launch_info(DT[dtype], len(splits), sum(more), n, k, panel=True).cols == 0
+    x = torch.randn(sum(more), k, generator=g, device="cuda").to(DT[dtype])
+    w = (torch.randn(len(splits), n, k, generator=g, device="cuda") * 0.05).to(DT[dtype])
+    starts = torch.tensor([0] + more).cumsum(0)[:-1]
+    rows = torch.cat([torch.arange(s, s + r) for s, r in zip(starts.tolist(), splits)]).cuda()
+    many = capi.grouped_gemm(x, w, torch.tensor(more, dtype=torch.int32, device="cuda"), out_dtype=torch.float32)
+    few = capi.grouped_gemm(x[rows], w, torch.tensor(splits, dtype=torch.int32, device="cuda"), out_dtype=torch.float32)
+    assert torch.equal(few, many[rows])
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp8", "bs"])
+@pytest.mark.parametrize("splits,computes", [([129] + [40] * 15 + [30] * 8, 1), ([600, 600] + [10] * 22, 0), ([64] * 5 + [0] * 19, 1)])
+def test_splits_choose_between_panel_and_macro_tiles(dtype, splits, computes):
+    """Both are launched; every result is computed, and added to a sum, exactly once, also by a captured launch whose splits change."""
+    n, k, m, e = 1408, 1152, sum(splits), len(splits)
+    print(f"[case] panel gemm by splits {dtype} {splits[:3]}", flush=True)
+    rows = 24 * 60  # on average, whatever the splits
+    info = capi.gemm_launch_info(DT[dtype], e, rows, n, k, splits=splits, panel=True, block_scaled=dtype == "bs")
+    assert (info.macro_tiles_too, info.computes) == (1, computes)
+    a, w, sp, g = made(splits, n, k, dtype, m)
+    a = torch.cat([a, a.new_zeros(rows - m, k)])
+    ad, wd = a.to(DT[dtype]), w.to(DT[dtype])
+    want = product(a, w, splits)
+    if dtype == "bs":
+        sad, sbd = torch.ones((rows + 127) // 128, k // 128, 128, device="cuda"), torch.ones(e, n // 128, k // 128, device="cuda")
+        run = lambda out: capi.grouped_gemm_blockscale(ad, wd, sp, sad, sbd, out=out)
+    else:
+        run = lambda out: capi.grouped_gemm(ad, wd, sp, out=out)
+        token = torch.randint(0, m // 2 + 1, (rows,), generator=g, device="cuda")
+        sums = torch.zeros(m // 2 + 1, n, dtype=torch.float64, device="cuda").index_add_(0, token[:m], want)
+        got = capi.grouped_gemm_topk_reduce(ad, wd, sp, token.to(torch.int32), m // 2 + 1)
+        assert torch.equal(got, sums.float().to(got.dtype))
+    out = torch.full((rows, n), -1.0, device="cuda")
+    run(out)
+    assert torch.equal(out[:m].double(), want) and bool((out[m:] == -1).all())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(out)
+    for s in (splits, [0] * (e - 1) + [300], [20] * e, splits):
+        sp.copy_(torch.tensor(s, dtype=torch.int32))
+        out.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:sum(s)].double(), product(a, w, s)) and bool((out[sum(s):] == -1).all())
