@@ -126,11 +126,31 @@ struct DryRun {
   PanelPlan panel = {};
 };
 
+// Whether a form for few rows per expert, with chunks of chunk_rows rows, computes a launch with these splits.
+bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, int chunk_rows) {
+  int left = args->max_rows, chunks = 0, active = 0;
+  for (int e = 0; e < args->nexperts; ++e) {
+    const int rows = splits_host[e] < 0 ? 0 : (splits_host[e] < left ? splits_host[e] : left);
+    left -= rows;
+    active += rows > 0 ? 1 : 0;
+    chunks += (rows + chunk_rows - 1) / chunk_rows;
+  }
+  return chunks <= stream_chunks_limit(active, chunk_rows);
+}
+
+// Row counts that are known on the host, and a second factor per row.
+struct HostSplits {
+  const int32_t *splits;
+  const float *row_scale2;
+};
+
 // dry_run: check the arguments and report which kernel would run (1 MFMA, 0 generic) without launching.
 // accumulate_rows > 0: D is fp32 with that many rows and results are added to it atomically.
+// host: the launch is made for these row counts, one kernel.  Without args->splits that takes a form for few rows per expert that
+// computes them; returns 1 if it was launched, otherwise 0.
 int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const void *const *b, void *const *d,
                      const float *const *alpha, void *stream, DryRun *dry_run = nullptr, int32_t accumulate_rows = 0,
-                     const BlockScales *bs = nullptr) {
+                     const BlockScales *bs = nullptr, const HostSplits *host = nullptr) {
   FLUXMI_REQUIRE(args != nullptr, FLUXMI_ERR_INVALID_ARG, "grouped_gemm: null args");
   FLUXMI_REQUIRE(args->dtype == FLUXMI_BF16 || args->dtype == FLUXMI_FP8_E4M3 || args->dtype == FLUXMI_FP16, FLUXMI_ERR_INVALID_ARG,
                  "grouped_gemm: unknown dtype %d", args->dtype);
@@ -146,9 +166,9 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
                  args->k);
   FLUXMI_REQUIRE(ngroups >= 1 && ngroups <= kMaxWeightGroups, FLUXMI_ERR_UNSUPPORTED,
                  "grouped_gemm: ngroups=%d outside [1,%d]", ngroups, kMaxWeightGroups);
-  if (args->max_rows == 0 || args->n == 0) return dry_run ? 1 : FLUXMI_OK;
+  if (args->max_rows == 0 || args->n == 0) return dry_run || host ? 1 : FLUXMI_OK;
   FLUXMI_REQUIRE(args->k >= 1, FLUXMI_ERR_UNSUPPORTED, "grouped_gemm: k must be positive");
-  FLUXMI_REQUIRE(args->a && args->splits && b && d, FLUXMI_ERR_INVALID_ARG, "grouped_gemm: null a / b / d / splits");
+  FLUXMI_REQUIRE(args->a && (args->splits || host) && b && d, FLUXMI_ERR_INVALID_ARG, "grouped_gemm: null a / b / d / splits");
 
   GemmParams p;
   bool mfma = true;
@@ -238,13 +258,32 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
     return mfma ? 1 : 0;
   }
 
-  if (panel.cols != 0) {
-    const int rc = launch_grouped_gemm_panel(p, args->dtype, panel, s);
-    if (rc != FLUXMI_OK) return rc;
-  } else if (stream_form) {
-    launch_grouped_gemm_stream(p, args->dtype, plan, s);
+  FewRowsArgs few;
+  few.count = 0;
+  few.row_scale2 = nullptr;
+  bool run_few = panel.cols != 0 || stream_form, run_macro = macro;
+  if (host != nullptr) {
+    const bool computes = run_few && (!macro || few_chunks(args, host->splits, p.by_splits));
+    p.by_splits = 0;
+    if (computes && args->nexperts <= kArgSplits) {
+      run_macro = false;
+      few.row_scale2 = host->row_scale2;
+      few.count = args->nexperts;
+      for (int e = 0; e < args->nexperts; ++e) few.splits[e] = host->splits[e];
+    } else {
+      if (args->splits == nullptr) return 0;
+      FLUXMI_REQUIRE(host->row_scale2 == nullptr, FLUXMI_ERR_UNSUPPORTED, "grouped_gemm_host_splits: row_scale2 with splits on the device");
+      run_few = computes;
+      run_macro = macro && !computes;
+    }
   }
-  if (macro) {
+  if (run_few && panel.cols != 0) {
+    const int rc = launch_grouped_gemm_panel(p, few, args->dtype, panel, s);
+    if (rc != FLUXMI_OK) return rc;
+  } else if (run_few) {
+    launch_grouped_gemm_stream(p, few, args->dtype, plan, s);
+  }
+  if (run_macro) {
     // Upper bound of the tile count: never launch more workgroups than tiles.
     const int64_t tiles_n = (args->n + BN - 1) / BN * ngroups;
     const int64_t max_tiles = (static_cast<int64_t>(args->max_rows) / BM + args->nexperts) * tiles_n;
@@ -276,7 +315,7 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
     }
   }
   FLUXMI_HIP_CHECK(hipGetLastError());
-  return FLUXMI_OK;
+  return host != nullptr ? 1 : FLUXMI_OK;
 }
 
 }  // namespace
@@ -379,6 +418,22 @@ extern "C" int fluxmi_grouped_gemm_blockscale(const fluxmi_grouped_gemm_args *ar
   return fluxmi::run_grouped_gemm(args, 1, &b, &d, &alpha, stream, nullptr, 0, &bs);
 }
 
+extern "C" int fluxmi_grouped_gemm_host_splits(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, const float *row_scale2,
+                                               const float *a_scale, int32_t a_scale_layout, const float *b_scale, int32_t b_scale_layout,
+                                               void *stream) {
+  FLUXMI_REQUIRE(args != nullptr && splits_host != nullptr, FLUXMI_ERR_INVALID_ARG, "grouped_gemm_host_splits: null args / splits");
+  fluxmi::BlockScales bs;
+  bs.a_scale = a_scale;
+  bs.b_scale = b_scale;
+  bs.a_layout = a_scale_layout;
+  bs.b_layout = b_scale_layout;
+  const fluxmi::HostSplits host = {splits_host, row_scale2};
+  const void *b = args->b;
+  void *d = args->d;
+  const float *alpha = args->alpha;
+  return fluxmi::run_grouped_gemm(args, 1, &b, &d, &alpha, stream, nullptr, 0, a_scale != nullptr || b_scale != nullptr ? &bs : nullptr, &host);
+}
+
 extern "C" int fluxmi_grouped_gemm_kernel_kind(const fluxmi_grouped_gemm_args *args) {
   FLUXMI_REQUIRE(args != nullptr, FLUXMI_ERR_INVALID_ARG, "grouped_gemm: null args");
   const void *b = args->b;
@@ -390,18 +445,6 @@ extern "C" int fluxmi_grouped_gemm_kernel_kind(const fluxmi_grouped_gemm_args *a
 
 namespace fluxmi {
 namespace {
-
-// Whether a form for few rows per expert, with chunks of chunk_rows rows, computes a launch with these splits.
-bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, int chunk_rows) {
-  int left = args->max_rows, chunks = 0, active = 0;
-  for (int e = 0; e < args->nexperts; ++e) {
-    const int rows = splits_host[e] < 0 ? 0 : (splits_host[e] < left ? splits_host[e] : left);
-    left -= rows;
-    active += rows > 0 ? 1 : 0;
-    chunks += (rows + chunk_rows - 1) / chunk_rows;
-  }
-  return chunks <= stream_chunks_limit(active, chunk_rows);
-}
 
 // The dry run of a launch of ngroups weight groups that all look like args->b / d / alpha.
 int describe_launch(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale, int32_t cu_count, DryRun &dry) {

@@ -98,6 +98,15 @@ struct GemmParams {
   int32_t by_splits;
 };
 
+// What a launch of a form for few rows per expert may carry besides GemmParams.  The first argument of those kernels, so that a lane
+// can index the row counts where they lie in the argument segment.
+constexpr int kArgSplits = 128;
+struct FewRowsArgs {
+  const float *row_scale2;      // a second factor per row, or null
+  int32_t count;                // 0: the row counts are GemmParams::splits
+  int32_t splits[kArgSplits];   // known on the host: no copy to the device, and only the kernel that they call for is launched
+};
+
 // Rows of a work item of the streaming form: two 16-row MFMA blocks.  An expert with more is several items per column tile.
 constexpr int kStreamRows = 32;
 

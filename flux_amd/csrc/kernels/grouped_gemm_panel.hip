@@ -131,7 +131,7 @@ __device__ __forceinline__ void multiply(const i32x4 (&w)[NB][2], const i32x4 (&
 
 // Scale, cast and store: a lane holds four consecutive columns of one row per block.
 template <Elem T, int MB, int NB>
-__device__ __forceinline__ void store(const GemmParams &p, const WorkItem &t, int g, const Columns &c, const f32x4 (&acc)[MB][NB]) {
+__device__ __forceinline__ void store(const GemmParams &p, const FewRowsArgs &few, const WorkItem &t, int g, const Columns &c, const f32x4 (&acc)[MB][NB]) {
   const int lane = threadIdx.x & 63;
   const float tile_scale = p.scalar * (p.scalar_dev ? p.scalar_dev[0] : 1.f) * (p.alpha[g] ? p.alpha[g][t.e] : 1.f);
 #pragma unroll
@@ -139,7 +139,7 @@ __device__ __forceinline__ void store(const GemmParams &p, const WorkItem &t, in
     const int r = i * 16 + (lane & 15);
     if (r >= t.rows) continue;
     const int row = t.row_base + r;
-    const float rs = tile_scale * (p.row_scale ? p.row_scale[row] : 1.f);
+    const float rs = row_factor(p, few, tile_scale, row);
     int64_t drow = row;
     if (p.scatter_d) {
       drow = p.scatter_d[row];
@@ -200,7 +200,7 @@ __device__ __forceinline__ void zero(f32x4 *acc) {
 // STEP: lines that are asked for together, waited for and computed.  Two halve the waits, and neighbouring lines of a row are
 // fetched one after the other (64 columns, bf16 8 experts 14336 x 4096, 8 rows each: 142 us line by line, 136 in pairs).
 template <Elem T, int MB, int NB, int DEPTH, int STEP>
-__device__ __forceinline__ void lds_tile(const GemmParams &p, uint8_t *smem, const WorkItem &t, int g, int n0, int wave) {
+__device__ __forceinline__ void lds_tile(const GemmParams &p, const FewRowsArgs &few, uint8_t *smem, const WorkItem &t, int g, int n0, int wave) {
   typedef Rows<T, MB> X;
   constexpr bool BS = X::BS;
   constexpr int WF = 2 * NB, PER_STEP = (X::FILLS + WF) * STEP, STEPS = DEPTH / STEP;  // vector-memory instructions per wave and step
@@ -292,12 +292,12 @@ __device__ __forceinline__ void lds_tile(const GemmParams &p, uint8_t *smem, con
     step = step == STEPS - 1 ? 0 : step + 1;
   }
   FLUXMI_VMCNT(0);  // no fill may reach LDS after the workgroup has ended (or its next item has begun)
-  store<T, MB, NB>(p, t, g, c, acc);
+  store<T, MB, NB>(p, few, t, g, c, acc);
 }
 
 // 16 * MB rows x 64 * NB columns, weights through registers, two lines ahead; the rows' ring has a stage more.  Not block-scaled.
 template <Elem T, int MB, int NB>
-__device__ __forceinline__ void register_tile(const GemmParams &p, uint8_t *smem, const WorkItem &t, int g, int n0, int wave) {
+__device__ __forceinline__ void register_tile(const GemmParams &p, const FewRowsArgs &few, uint8_t *smem, const WorkItem &t, int g, int n0, int wave) {
   typedef Rows<T, MB> X;
   static_assert(!X::BS, "no registers left for block scales");
   constexpr int DEPTH = 2, GB = 2, GROUPS = MB / GB, STAGE = X::BYTES, PER_LINE = X::FILLS + 2 * NB;
@@ -365,7 +365,7 @@ __device__ __forceinline__ void register_tile(const GemmParams &p, uint8_t *smem
     }
   }
   FLUXMI_VMCNT(0);
-  store<T, MB, NB>(p, t, g, c, acc);
+  store<T, MB, NB>(p, few, t, g, c, acc);
 }
 
 #endif  // __HIP_DEVICE_COMPILE__
@@ -381,7 +381,7 @@ constexpr int lds_bytes() {
 
 template <Elem T, int CH, int NB, int DEPTH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-void grouped_gemm_panel_kernel(const GemmParams p, const int blocks) {
+void grouped_gemm_panel_kernel(const FewRowsArgs few, const GemmParams p, const int blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -395,8 +395,8 @@ void grouped_gemm_panel_kernel(const GemmParams p, const int blocks) {
       auto tile = [&](auto BLOCKS) {
         constexpr int mb = decltype(BLOCKS)::value;
         if constexpr (mb <= CH) {
-          if constexpr (DEPTH > 0) lds_tile<T, mb, NB, DEPTH, DEPTH == 6 ? 2 : 1>(p, smem, t, g, n0, wave);
-          else register_tile<T, mb, NB>(p, smem, t, g, n0, wave);
+          if constexpr (DEPTH > 0) lds_tile<T, mb, NB, DEPTH, DEPTH == 6 ? 2 : 1>(p, few, smem, t, g, n0, wave);
+          else register_tile<T, mb, NB>(p, few, smem, t, g, n0, wave);
         }
       };
       if (CH == 2 && t.rows <= 16) tile(std::integral_constant<int, CH == 2 ? 1 : 2>{});
@@ -414,12 +414,12 @@ void grouped_gemm_panel_kernel(const GemmParams p, const int blocks) {
 }
 
 template <Elem T, int CH, int NB, int DEPTH>
-int launch(const GemmParams &p, const PanelPlan &plan, hipStream_t s) {
+int launch(const GemmParams &p, const FewRowsArgs &few, const PanelPlan &plan, hipStream_t s) {
   static std::atomic<uint64_t> done{0};
   const void *kernel = reinterpret_cast<const void *>(grouped_gemm_panel_kernel<T, CH, NB, DEPTH>);
   const int rc = ensure_dynamic_lds(kernel, kCuLds, done);
   if (rc != FLUXMI_OK) return rc;
-  hipLaunchKernelGGL((grouped_gemm_panel_kernel<T, CH, NB, DEPTH>), dim3(plan.workgroups), dim3(256), plan.lds_bytes, s, p, plan.blocks);
+  hipLaunchKernelGGL((grouped_gemm_panel_kernel<T, CH, NB, DEPTH>), dim3(plan.workgroups), dim3(256), plan.lds_bytes, s, few, p, plan.blocks);
   return FLUXMI_OK;
 }
 
@@ -428,13 +428,13 @@ template <Elem T>
 constexpr int kDepth32 = T == Elem::FP8_BLOCKSCALED ? 3 : 4;
 
 template <Elem T>
-int launch_by_plan(const GemmParams &p, const PanelPlan &plan, hipStream_t s) {
+int launch_by_plan(const GemmParams &p, const FewRowsArgs &few, const PanelPlan &plan, hipStream_t s) {
   const int blocks16 = plan.chunk_rows / 16;
   if constexpr (T != Elem::FP8_BLOCKSCALED)
-    if (plan.cols == 256) return launch<T, 8, 4, 0>(p, plan, s);
-  if (plan.cols == 128) return blocks16 <= 2 ? launch<T, 2, 2, kDepth32<T>>(p, plan, s) : (blocks16 <= 4 ? launch<T, 4, 2, 3>(p, plan, s) : launch<T, 8, 2, 3>(p, plan, s));
-  if (blocks16 <= 2 && plan.pairs) return launch<T, 2, 1, 6>(p, plan, s);
-  return blocks16 <= 2 ? launch<T, 2, 1, 4>(p, plan, s) : (blocks16 <= 4 ? launch<T, 4, 1, 4>(p, plan, s) : launch<T, 8, 1, 3>(p, plan, s));
+    if (plan.cols == 256) return launch<T, 8, 4, 0>(p, few, plan, s);
+  if (plan.cols == 128) return blocks16 <= 2 ? launch<T, 2, 2, kDepth32<T>>(p, few, plan, s) : (blocks16 <= 4 ? launch<T, 4, 2, 3>(p, few, plan, s) : launch<T, 8, 2, 3>(p, few, plan, s));
+  if (blocks16 <= 2 && plan.pairs) return launch<T, 2, 1, 6>(p, few, plan, s);
+  return blocks16 <= 2 ? launch<T, 2, 1, 4>(p, few, plan, s) : (blocks16 <= 4 ? launch<T, 4, 1, 4>(p, few, plan, s) : launch<T, 8, 1, 3>(p, few, plan, s));
 }
 
 template <Elem T>
@@ -536,11 +536,11 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
   return plan;
 }
 
-int launch_grouped_gemm_panel(const GemmParams &p, int dtype, const PanelPlan &plan, hipStream_t s) {
-  if (p.a_scale != nullptr) return launch_by_plan<Elem::FP8_BLOCKSCALED>(p, plan, s);
-  if (dtype == FLUXMI_FP8_E4M3) return launch_by_plan<Elem::FP8>(p, plan, s);
-  if (dtype == FLUXMI_FP16) return launch_by_plan<Elem::F16>(p, plan, s);
-  return launch_by_plan<Elem::BF16>(p, plan, s);
+int launch_grouped_gemm_panel(const GemmParams &p, const FewRowsArgs &few, int dtype, const PanelPlan &plan, hipStream_t s) {
+  if (p.a_scale != nullptr) return launch_by_plan<Elem::FP8_BLOCKSCALED>(p, few, plan, s);
+  if (dtype == FLUXMI_FP8_E4M3) return launch_by_plan<Elem::FP8>(p, few, plan, s);
+  if (dtype == FLUXMI_FP16) return launch_by_plan<Elem::F16>(p, few, plan, s);
+  return launch_by_plan<Elem::BF16>(p, few, plan, s);
 }
 
 }  // namespace fluxmi

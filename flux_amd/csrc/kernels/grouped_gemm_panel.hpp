@@ -19,6 +19,6 @@ struct PanelPlan {
 
 // few_rows: the launch has few enough rows for the streaming form.
 PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, bool leave_cus);
-int launch_grouped_gemm_panel(const GemmParams &p, int dtype, const PanelPlan &plan, hipStream_t s);
+int launch_grouped_gemm_panel(const GemmParams &p, const FewRowsArgs &few, int dtype, const PanelPlan &plan, hipStream_t s);
 
 }  // namespace fluxmi

@@ -23,15 +23,26 @@ struct WorkItem {
   int nt;                           // column tile, over all weight groups
 };
 
+typedef const __attribute__((address_space(4))) FewRowsArgs *ArgSegment;
+
+// Scale of output row `row`, the tile's included.
+__device__ __forceinline__ float row_factor(const GemmParams &p, const FewRowsArgs &f, float tile_scale, int row) {
+  float s = p.row_scale ? p.row_scale[row] : 1.f;
+  if (f.row_scale2) s *= f.row_scale2[row];
+  return tile_scale * s;
+}
+
 // Work item -> (expert, chunk of its rows, column tile); a chunk is at most chunk_rows rows (a power of two, 16 or more), and the chunks of
 // an expert are about equally long.  One wave-wide pass over the splits counts the chunks, a second finds the item's; with up to
 // 64 experts both work on the same registers.
 __device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n, int chunk_rows, int block) {
   const int lane = threadIdx.x & 63;
   int begin, rows, chunks_end;  // this lane's expert of the 64 looked at
+  const ArgSegment args = (ArgSegment)__builtin_amdgcn_kernarg_segment_ptr();
   auto load = [&](int e0, int &row_carry, int &chunk_carry) {
     const int ee = e0 + lane;
-    int r = ee < p.nexperts ? p.splits[ee] : 0;
+    int r = 0;
+    if (ee < p.nexperts) r = args->count > 0 ? args->splits[ee] : p.splits[ee];
     if (r < 0) r = 0;
     const int incl = wave_inclusive_scan(r);
     begin = row_carry + incl - r;

@@ -180,7 +180,7 @@ __device__ __forceinline__ void partial_sums(const GemmParams &p, f32x4 *red, co
 
 // Sum of the waves' partial sums, scaled, cast and stored.  A unit is one lane's four consecutive columns of one row.
 template <Elem T, int MB, int NB, int WAVES>
-__device__ __forceinline__ void finish_tile(const GemmParams &p, const f32x4 *red, const WorkItem &t, int g, int n0, int wave) {
+__device__ __forceinline__ void finish_tile(const GemmParams &p, const FewRowsArgs &few, const f32x4 *red, const WorkItem &t, int g, int n0, int wave) {
   const int lane = threadIdx.x & 63;
   const float tile_scale = p.scalar * (p.scalar_dev ? p.scalar_dev[0] : 1.f) * (p.alpha[g] ? p.alpha[g][t.e] : 1.f);
   for (int u = wave * 64 + lane; u < MB * NB * 64; u += WAVES * 64) {
@@ -191,7 +191,7 @@ __device__ __forceinline__ void finish_tile(const GemmParams &p, const f32x4 *re
     const int r = (b / NB) * 16 + (l & 15), col = n0 + (b % NB) * 16 + (l >> 4) * 4;
     if (r >= t.rows || col >= p.n) continue;  // n % 4 == 0: the four columns are all in or all out
     const int row = t.row_base + r;
-    const float rs = tile_scale * (p.row_scale ? p.row_scale[row] : 1.f);
+    const float rs = row_factor(p, few, tile_scale, row);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       v[c] *= rs;
@@ -228,7 +228,7 @@ __device__ __forceinline__ void finish_tile(const GemmParams &p, const f32x4 *re
 constexpr int unit_waves(int nb) { return nb <= 2 ? 16 : 8; }  // what the registers of a compute unit hold
 template <Elem T, int NB, int WAVES, bool WALK>
 __global__ __launch_bounds__(WALK ? unit_waves(NB) * 64 : WAVES * 64) __attribute__((amdgpu_waves_per_eu(unit_waves(NB) / 4)))
-void grouped_gemm_stream_kernel(const GemmParams p, const int blocks) {
+void grouped_gemm_stream_kernel(const FewRowsArgs few, const GemmParams p, const int blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int TEAMS = WALK ? unit_waves(NB) / WAVES : 1;
   constexpr int TEAM_SUMS = WAVES * 2 * NB * 64;
@@ -249,8 +249,8 @@ void grouped_gemm_stream_kernel(const GemmParams p, const int blocks) {
     if (t.rows > 16) partial_sums<T, 2, NB, WAVES>(p, red, t, g, n0, wave);
     else if (t.rows > 0) partial_sums<T, 1, NB, WAVES>(p, red, t, g, n0, wave);
     __syncthreads();
-    if (t.rows > 16) finish_tile<T, 2, NB, WAVES>(p, red, t, g, n0, wave);
-    else if (t.rows > 0) finish_tile<T, 1, NB, WAVES>(p, red, t, g, n0, wave);
+    if (t.rows > 16) finish_tile<T, 2, NB, WAVES>(p, few, red, t, g, n0, wave);
+    else if (t.rows > 0) finish_tile<T, 1, NB, WAVES>(p, few, red, t, g, n0, wave);
     if constexpr (WALK) __syncthreads();  // the sums have been read before the next items' go there
     block += TEAMS * stride;
   } while (WALK && block < blocks);
@@ -274,21 +274,21 @@ int64_t most_items(const GemmParams &p, int ngroups, int nb) {
 constexpr int kWalkSums = 64 * 1024, kWalkExtra = 32 * 1024;
 
 template <Elem T, int NB, int WAVES>
-void launch(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
+void launch(const GemmParams &p, const FewRowsArgs &few, const StreamPlan &plan, hipStream_t s) {
   if (!plan.walk) {
-    hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, false>), dim3(plan.workgroups), dim3(WAVES * 64), 0, s, p, plan.blocks);
+    hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, false>), dim3(plan.workgroups), dim3(WAVES * 64), 0, s, few, p, plan.blocks);
     return;
   }
   static_assert(unit_waves(NB) * 2 * NB * 1024 == kWalkSums, "LDS of the walking form");
-  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, true>), dim3(plan.workgroups), dim3(unit_waves(NB) * 64), kWalkExtra, s, p, plan.blocks);
+  hipLaunchKernelGGL((grouped_gemm_stream_kernel<T, NB, WAVES, true>), dim3(plan.workgroups), dim3(unit_waves(NB) * 64), kWalkExtra, s, few, p, plan.blocks);
 }
 
 template <Elem T>
-void launch_by_plan(const GemmParams &p, const StreamPlan &plan, hipStream_t s) {
-  if (plan.waves == 8 && plan.cols == 32) launch<T, 2, 8>(p, plan, s);
-  else if (plan.waves == 8) launch<T, 4, 8>(p, plan, s);
-  else if (plan.cols == 32) launch<T, 2, 4>(p, plan, s);
-  else launch<T, 4, 4>(p, plan, s);
+void launch_by_plan(const GemmParams &p, const FewRowsArgs &few, const StreamPlan &plan, hipStream_t s) {
+  if (plan.waves == 8 && plan.cols == 32) launch<T, 2, 8>(p, few, plan, s);
+  else if (plan.waves == 8) launch<T, 4, 8>(p, few, plan, s);
+  else if (plan.cols == 32) launch<T, 2, 4>(p, few, plan, s);
+  else launch<T, 4, 4>(p, few, plan, s);
 }
 
 }  // namespace
@@ -330,11 +330,11 @@ StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, boo
   return plan;
 }
 
-void launch_grouped_gemm_stream(const GemmParams &p, int dtype, const StreamPlan &plan, hipStream_t s) {
-  if (p.a_scale != nullptr) launch_by_plan<Elem::FP8_BLOCKSCALED>(p, plan, s);
-  else if (dtype == FLUXMI_FP8_E4M3) launch_by_plan<Elem::FP8>(p, plan, s);
-  else if (dtype == FLUXMI_FP16) launch_by_plan<Elem::F16>(p, plan, s);
-  else launch_by_plan<Elem::BF16>(p, plan, s);
+void launch_grouped_gemm_stream(const GemmParams &p, const FewRowsArgs &few, int dtype, const StreamPlan &plan, hipStream_t s) {
+  if (p.a_scale != nullptr) launch_by_plan<Elem::FP8_BLOCKSCALED>(p, few, plan, s);
+  else if (dtype == FLUXMI_FP8_E4M3) launch_by_plan<Elem::FP8>(p, few, plan, s);
+  else if (dtype == FLUXMI_FP16) launch_by_plan<Elem::F16>(p, few, plan, s);
+  else launch_by_plan<Elem::BF16>(p, few, plan, s);
 }
 
 }  // namespace fluxmi

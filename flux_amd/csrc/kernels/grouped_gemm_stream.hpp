@@ -19,6 +19,6 @@ struct StreamPlan {
 bool grouped_gemm_stream_takes(const GemmParams &p, int dtype);
 // cus: compute units the launch may use; leave_cus: the others are to be left to other work.
 StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, bool leave_cus);
-void launch_grouped_gemm_stream(const GemmParams &p, int dtype, const StreamPlan &plan, hipStream_t s);
+void launch_grouped_gemm_stream(const GemmParams &p, const FewRowsArgs &few, int dtype, const StreamPlan &plan, hipStream_t s);
 
 }  // namespace fluxmi

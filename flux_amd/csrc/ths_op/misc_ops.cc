@@ -170,7 +170,7 @@ static torch::Tensor blockscale_run(const torch::Tensor &input, const torch::Ten
     out = torch::empty({m, n}, input.options().dtype(out_dtype));
   }
   if (m == 0) return out;
-  torch::Tensor splits_dev = splits_cpu.to(at::kInt).to(input.device(), /*non_blocking=*/true);
+  const torch::Tensor splits_host = splits_cpu.to(at::kInt).contiguous();
   fluxmi_grouped_gemm_args args{};
   args.dtype = FLUXMI_FP8_E4M3;
   args.nexperts = static_cast<int32_t>(e);
@@ -181,9 +181,16 @@ static torch::Tensor blockscale_run(const torch::Tensor &input, const torch::Ten
   args.a = input.data_ptr();
   args.b = weight3.data_ptr();
   args.d = out.data_ptr();
-  args.splits = splits_dev.data_ptr<int32_t>();
   args.scalar_scale = 1.0f;
   args.d_fp32 = out_dtype == at::kFloat ? 1 : 0;
+  auto one_kernel = [&]() {
+    return run_host_splits(args, splits_host.data_ptr<int32_t>(), nullptr, input_scale.data_ptr<float>(), a_layout,
+                           weight_scale.data_ptr<float>(), b_layout);
+  };
+  if (one_kernel()) return out;
+  const torch::Tensor splits_dev = splits_host.to(input.device(), /*non_blocking=*/true);
+  args.splits = splits_dev.data_ptr<int32_t>();
+  if (one_kernel()) return out;
   check_status(fluxmi_grouped_gemm_blockscale(&args, input_scale.data_ptr<float>(), a_layout,
                                               weight_scale.data_ptr<float>(), b_layout, current_stream()),
                "fluxmi_grouped_gemm_blockscale");

@@ -122,10 +122,10 @@ void apply_launch_tuning(fluxmi_grouped_gemm_args &args, int32_t ngroups, int64_
   }
 }
 
-void run_grouped_gemm(const torch::Tensor &a, const torch::Tensor &b, const torch::Tensor &splits_dev,
-                      torch::Tensor &d, const int32_t *gather_a, int64_t max_rows, const float *alpha,
-                      const float *row_scale, const float *col_scale, const float *scalar_dev,
-                      int64_t sm_margin) {
+namespace {
+fluxmi_grouped_gemm_args gemm_args(const torch::Tensor &a, const torch::Tensor &b, const int32_t *splits_dev, const torch::Tensor &d,
+                                   const int32_t *gather_a, int64_t max_rows, const float *alpha, const float *row_scale,
+                                   const float *col_scale, const float *scalar_dev, int64_t sm_margin) {
   fluxmi_grouped_gemm_args args{};
   args.dtype = to_fluxmi_dtype(a.scalar_type());
   args.nexperts = static_cast<int32_t>(b.size(0));
@@ -136,7 +136,7 @@ void run_grouped_gemm(const torch::Tensor &a, const torch::Tensor &b, const torc
   args.a = a.data_ptr();
   args.b = b.data_ptr();
   args.d = d.data_ptr();
-  args.splits = splits_dev.data_ptr<int32_t>();
+  args.splits = splits_dev;
   args.gather_a = gather_a;
   args.scatter_d = nullptr;
   args.alpha = alpha;
@@ -146,7 +146,18 @@ void run_grouped_gemm(const torch::Tensor &a, const torch::Tensor &b, const torc
   args.d_fp32 = d.scalar_type() == at::ScalarType::Float ? 1 : 0;
   args.scalar_scale_dev = scalar_dev;
   apply_launch_tuning(args, 1, sm_margin);
-  check_status(fluxmi_grouped_gemm(&args, nullptr, 0, current_stream()), "fluxmi_grouped_gemm");
+  return args;
+}
+}  // namespace
+
+bool run_host_splits(const fluxmi_grouped_gemm_args &args, const int32_t *splits_host, const float *row_scale2, const float *a_scale,
+                     int32_t a_layout, const float *b_scale, int32_t b_layout) {
+  hipStream_t stream = static_cast<hipStream_t>(current_stream());
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+  const int rc = fluxmi_grouped_gemm_host_splits(&args, splits_host, row_scale2, a_scale, a_layout, b_scale, b_layout, stream);
+  if (rc < 0) check_status(rc, "fluxmi_grouped_gemm_host_splits");
+  return rc == 1;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -392,7 +403,12 @@ torch::Tensor GemmGroupedV3GatherRS::forward_impl(
   const bool f16 = st == at::ScalarType::Half;
   torch::Tensor out = torch::empty({ntokens, n_dim_}, inputs[0].options().dtype(moe_output_dtype(st)));
   if (global_m == 0) return out;
-  splits_dev_.copy_(splits_cpu.contiguous(), /*non_blocking=*/true);
+  const torch::Tensor splits_host = splits_cpu.contiguous();
+  bool splits_on_device = false;
+  auto splits_to_device = [&]() {
+    if (!splits_on_device) splits_dev_.copy_(splits_host, /*non_blocking=*/true);
+    splits_on_device = true;
+  };
 
   // One input group and an fp32 scratch at hand: the reduction may run in the GEMM's epilogue.  It does when
   // FLUX_AMD_LAYER1_REDUCE=fused asks for it, or when profiling() found it faster for this shape (a tuning record
@@ -416,8 +432,8 @@ torch::Tensor GemmGroupedV3GatherRS::forward_impl(
   const bool fused = want_fused && groups == 1 && inter_fp32_;
   std::vector<const void *> group_ptrs;
   for (size_t g = 0; g < groups; ++g) {
-    const float *alpha = nullptr, *row = nullptr, *col = nullptr, *scalar = nullptr;
-    torch::Tensor row_holder;
+    const float *alpha = nullptr, *col = nullptr, *scalar = nullptr;
+    const float *row_factors[2] = {nullptr, nullptr};
     if (weight_scale.has_value()) {
       const auto &ws = weight_scale->at(g);
       if (ws.numel() == num_experts_) alpha = ws.data_ptr<float>();
@@ -426,15 +442,30 @@ torch::Tensor GemmGroupedV3GatherRS::forward_impl(
     }
     if (output_vec_scale.has_value()) {
       TORCH_CHECK(output_vec_scale->at(g).numel() == m, "output_vec_scale must be [M]");
-      row_holder = output_vec_scale->at(g);
+      row_factors[0] = output_vec_scale->at(g).data_ptr<float>();
     }
     if (input_scale.has_value()) {
       const auto &is = input_scale->at(g);
       if (is.numel() == 1) scalar = is.data_ptr<float>();
-      else if (is.numel() == m) row_holder = row_holder.defined() ? row_holder * is.reshape({m}) : is;
+      else if (is.numel() == m) row_factors[row_factors[0] != nullptr ? 1 : 0] = is.data_ptr<float>();
       else TORCH_CHECK(false, "input_scale must be [1] or [M]");
     }
-    if (row_holder.defined()) row = row_holder.data_ptr<float>();
+    // With few rows per expert one kernel takes the row counts and both factors of a row as they are.
+    if (!fused) {
+      const fluxmi_grouped_gemm_args args = gemm_args(inputs[g], weights[g], nullptr, inter_[g], nullptr, m, alpha, row_factors[0], col, scalar,
+                                                      sm_margin);
+      if (run_host_splits(args, splits_host.data_ptr<int32_t>(), row_factors[1])) {
+        group_ptrs.push_back(inter_[g].data_ptr());
+        continue;
+      }
+    }
+    splits_to_device();
+    torch::Tensor row_holder;  // the product of the two factors
+    const float *row = row_factors[0];
+    if (row_factors[1] != nullptr) {
+      row_holder = output_vec_scale->at(g).reshape({m}) * input_scale->at(g).reshape({m});
+      row = row_holder.data_ptr<float>();
+    }
     if (fused) {
       token_of_row_.fill_(-1);  // sorted rows that no routing entry names are skipped by the epilogue
       check_status(fluxmi_moe_gather_index(routing_idx.data_ptr<int32_t>(), static_cast<int32_t>(global_m),
@@ -464,7 +495,10 @@ torch::Tensor GemmGroupedV3GatherRS::forward_impl(
       if (with_stream_sync) c10::hip::getCurrentHIPStream().synchronize();
       return out;
     }
-    run_grouped_gemm(inputs[g], weights[g], splits_dev_, inter_[g], nullptr, m, alpha, row, col, scalar, sm_margin);
+    const fluxmi_grouped_gemm_args args = gemm_args(inputs[g], weights[g], splits_dev_.data_ptr<int32_t>(), inter_[g], nullptr, m, alpha, row, col,
+                                                    scalar, sm_margin);
+    if (!run_host_splits(args, splits_host.data_ptr<int32_t>(), nullptr))
+      check_status(fluxmi_grouped_gemm(&args, nullptr, 0, current_stream()), "fluxmi_grouped_gemm");
     group_ptrs.push_back(inter_[g].data_ptr());
   }
   check_status(fluxmi_topk_gather_reduce(group_ptrs.data(), static_cast<int32_t>(groups), (inter_fp32_ ? 1 : 0) | (f16 ? 2 : 0),
@@ -567,8 +601,14 @@ torch::Tensor GemmGroupedV3::forward(torch::Tensor input, torch::Tensor splits_c
               weight_.size(0));
   torch::Tensor out = torch::empty({input.size(0), weight_.size(1)}, input.options().dtype(moe_output_dtype(input.scalar_type())));
   if (input.size(0) == 0) return out;
-  torch::Tensor splits_dev = splits_cpu.to(at::kInt).to(input.device(), /*non_blocking=*/true);
-  run_grouped_gemm(input, weight_, splits_dev, out, nullptr, input.size(0), nullptr, nullptr, nullptr, nullptr, 0);
+  const torch::Tensor splits_host = splits_cpu.to(at::kInt).contiguous();
+  fluxmi_grouped_gemm_args args = gemm_args(input, weight_, nullptr, out, nullptr, input.size(0), nullptr, nullptr, nullptr, nullptr, 0);
+  const bool on_host = !splits_host.is_cuda();
+  if (on_host && run_host_splits(args, splits_host.data_ptr<int32_t>(), nullptr)) return out;
+  const torch::Tensor splits_dev = splits_host.to(input.device(), /*non_blocking=*/true);
+  args.splits = splits_dev.data_ptr<int32_t>();
+  if (on_host && run_host_splits(args, splits_host.data_ptr<int32_t>(), nullptr)) return out;
+  check_status(fluxmi_grouped_gemm(&args, nullptr, 0, current_stream()), "fluxmi_grouped_gemm");
   return out;
 }
 

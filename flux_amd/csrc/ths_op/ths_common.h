@@ -71,10 +71,11 @@ struct DistEnvTPWithEP {  // include/flux/ths_op/ths_op.h:117-130; only world si
   }
 };
 
-// Filled grouped-GEMM argument block (everything on the current stream).
-void run_grouped_gemm(const torch::Tensor &a, const torch::Tensor &b, const torch::Tensor &splits_dev,
-                      torch::Tensor &d, const int32_t *gather_a, int64_t max_rows, const float *alpha,
-                      const float *row_scale, const float *col_scale, const float *scalar_dev, int64_t sm_margin);
+// The GEMM of `args` for row counts known on the host: one kernel is launched.  With args.splits unset that takes a form for few rows
+// per expert, with the counts in its arguments and no copy to the device.  False: nothing was launched, and always while the current
+// stream is being captured (a replay reads the counts again from where the copy reads them).
+bool run_host_splits(const fluxmi_grouped_gemm_args &args, const int32_t *splits_host, const float *row_scale2,
+                     const float *a_scale = nullptr, int32_t a_layout = 0, const float *b_scale = nullptr, int32_t b_layout = 0);
 
 // Launch tuning of a grouped GEMM: CUs to leave free (Flux's sm_margin) and the tile schedule registered
 // for the problem's shape, if any.

@@ -162,6 +162,18 @@ int fluxmi_grouped_gemm(const fluxmi_grouped_gemm_args *args, void *workspace,
  * shapes only); callers use this to assert they are not on the generic kernel. */
 int fluxmi_grouped_gemm_kernel_kind(const fluxmi_grouped_gemm_args *args);
 
+/* fluxmi_grouped_gemm (with a_scale / b_scale: fluxmi_grouped_gemm_blockscale) for row counts that are known on the host: one kernel
+ * is launched, the one that they call for, where the ordinary call may launch two and let the device choose; same bits.
+ * Without args->splits the counts go into the kernel's arguments, which takes a form for few rows per expert that computes them and
+ * at most 128 experts: returns 1 if it was launched, 0 if not (nothing was then; copy the counts to the device and call again with
+ * args->splits).  With args->splits: returns 1.  A negative result is the status of the ordinary call.  splits_host: [nexperts], equal
+ * to args->splits, read before the call returns.  row_scale2: device [max_rows] or NULL, a second factor per row (multiplied with
+ * row_scale first), only without args->splits.  A captured launch keeps the choice, and without args->splits the counts, of the
+ * capture. */
+int fluxmi_grouped_gemm_host_splits(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, const float *row_scale2,
+                                    const float *a_scale, int32_t a_scale_layout, const float *b_scale, int32_t b_scale_layout,
+                                    void *stream);
+
 /* Which form of the MFMA kernels a launch takes and how the streaming form is launched.  Host only: nothing is
  * launched, no device is needed, and pointers in `args` are only looked at for their alignment (b and d stand for every
  * weight group).  a_scale: non-NULL for fluxmi_grouped_gemm_blockscale with MFMA-kernel layouts.  splits_host: host copy of

@@ -214,3 +214,37 @@ def test_splits_choose_between_panel_and_macro_tiles(dtype, splits, computes):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out[:sum(s)].double(), product(a, w, s)) and bool((out[sum(s):] == -1).all())
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp8", "bs"])
+@pytest.mark.parametrize("splits,n,k,done", [([7, 0, 30, 1], 1024, 8192, 1), ([12, 3, 9, 20, 17, 0, 31, 8], 4160, 384, 1), ([70, 64, 1, 0], 192, 256, 1),
+                                             ([-3, 20, 600, 5], 192, 256, 1), ([129] + [40] * 15 + [30] * 8, 1408, 1152, 1),
+                                             ([600, 600] + [10] * 22, 1408, 1152, 0), ([300, 200], 1024, 1024, 0), ([4] * 129, 1024, 384, 0)])
+def test_row_counts_known_on_the_host(dtype, splits, n, k, done):
+    """One kernel with the counts in its arguments has the bits of the ordinary call; otherwise nothing is launched."""
+    print(f"[case] host splits {dtype} {splits[:4]} n={n} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    m, e = sum(max(0, r) for r in splits), len(splits)
+    x = torch.randn(m, k, generator=g, device="cuda").to(DT[dtype])
+    w = (torch.randn(e, n, k, generator=g, device="cuda") * 0.05).to(DT[dtype])
+    sa = torch.rand((m + 127) // 128, k // 128, 128, generator=g, device="cuda")
+    sb = torch.rand(e, (n + 127) // 128, k // 128, generator=g, device="cuda")
+    r1, r2 = (torch.rand(m, generator=g, device="cuda") + 0.5 for _ in range(2))
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    kw = {} if dtype == "bs" else {"row_scale": r1 * r2}
+    want = torch.full((m, n), -1.0, device="cuda")
+    if dtype == "bs": capi.grouped_gemm_blockscale(x, w, sp, sa, sb, out=want)
+    else: capi.grouped_gemm(x, w, sp, out=want, **kw)
+    args, out = capi._gemm_args(x, w, sp, None, None, None, None, None if dtype == "bs" else r1, None, 1.0, None, None, torch.float32, 0, 0, 0)
+    host, on_device = (ctypes.c_int32 * e)(*splits), args.splits
+    scales = [capi._ptr(sa), capi.ASCALE_BLOCK128, capi._ptr(sb), capi.BSCALE_N_K] if dtype == "bs" else [None, 0, None, 0]
+    call = lambda second: capi.load().fluxmi_grouped_gemm_host_splits(ctypes.byref(args), host, second, *scales, capi._stream())
+    args.splits = None
+    out.fill_(-1)
+    assert call(None if dtype == "bs" else capi._ptr(r2)) == done
+    assert torch.equal(out, want) if done else bool((out == -1).all())
+    args.splits, r12 = on_device, r1 * r2  # with the counts on the device as well
+    if dtype != "bs": args.row_scale = r12.data_ptr()
+    out.fill_(-1)
+    assert call(None) == 1
+    assert torch.equal(out, want)
