@@ -135,7 +135,7 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
     active += rows > 0 ? 1 : 0;
     chunks += (rows + chunk_rows - 1) / chunk_rows;
   }
-  return chunks <= stream_chunks_limit(active, chunk_rows);
+  return chunks <= stream_chunks_limit(active, chunk_rows, args->dtype == FLUXMI_FP8_E4M3);
 }
 
 // Row counts that are known on the host, and a second factor per row.

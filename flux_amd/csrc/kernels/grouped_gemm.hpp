@@ -113,11 +113,13 @@ constexpr int kStreamRows = 32;
 // Most chunks of up to chunk_rows rows that a form for few rows per expert computes in a launch in which `active` experts have
 // rows: it reads an expert's weights once per chunk, and the items of a launch take about the same time each.  Chunks of 32 rows:
 // one per expert, from 16 experts on a quarter more (one more of few can be a whole round of the card: 8 experts 4096 x 14336, 10
-// chunks 241 us, macro tiles 219).  Longer ones: an eighth and one more (Zipf with exponent 1.2, us, panel and macro tiles: bf16 8
-// experts 14336 x 4096, 64 rows per expert on average, 9 chunks 196 / 225; a layer of 65 experts 5760 x 1792 at 38 rows, a quarter
-// more chunks than experts 646 / 619; all rows on one of 8 experts 95 / 47).
-__host__ __device__ inline int stream_chunks_limit(int active, int chunk_rows) {
-  return chunk_rows <= kStreamRows ? active + (active >= 16 ? active / 4 : 0) : active + active / 8 + 1;
+// chunks 241 us, macro tiles 219).  Longer ones: an eighth and one more, in fp8 a sixteenth (Zipf with exponent 1.2, us, panel and
+// macro tiles: bf16 8 experts 14336 x 4096, 64 rows per expert on average, 9 chunks 196 / 225; a layer of 65 experts 5760 x 1792 at
+// 38 rows, a quarter more chunks than experts 646 / 619; all rows on one of 8 experts 95 / 47; fp8 layer of 49 experts 1024 x 1024 at
+// 41 rows 83 / 76; block-scaled 7 experts 6400 x 6912 at 61 rows, one more chunk 255 / 241).
+__host__ __device__ inline int stream_chunks_limit(int active, int chunk_rows, bool fp8) {
+  if (chunk_rows <= kStreamRows) return active + (active >= 16 ? active / 4 : 0);
+  return fp8 ? active + active / 16 : active + active / 8 + 1;
 }
 
 // One launcher per element type, each in a translation unit of its own (the kernel is a long compile).

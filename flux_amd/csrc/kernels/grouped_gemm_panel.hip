@@ -388,7 +388,7 @@ void grouped_gemm_panel_kernel(const FewRowsArgs few, const GemmParams p, const 
   const int tiles_n1 = (p.n + 64 * NB - 1) / (64 * NB);
   int block = blockIdx.x;
   while (true) {
-    const WorkItem t = locate(p, tiles_n1 * p.ngroups, 16 * CH, block);
+    const WorkItem t = locate<T>(p, tiles_n1 * p.ngroups, 16 * CH, block);
     if (t.rows > 0) {
       const int g = p.ngroups > 1 ? __builtin_amdgcn_readfirstlane(t.nt / tiles_n1) : 0;
       const int n0 = (t.nt - g * tiles_n1) * (64 * NB);
@@ -459,10 +459,10 @@ int64_t even_items(const GemmParams &p, int cols, int ngroups) {
   return active * ((p.n + cols - 1) / cols) * ngroups;
 }
 
-int64_t most_items(const GemmParams &p, int cols, int chunk_rows, bool any_splits, int ngroups) {
+int64_t most_items(const GemmParams &p, int dtype, int cols, int chunk_rows, bool any_splits, int ngroups) {
   const int active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
   int64_t chunks = active + (p.max_rows - active) / chunk_rows;
-  const int limit = stream_chunks_limit(active, chunk_rows);
+  const int limit = stream_chunks_limit(active, chunk_rows, dtype == FLUXMI_FP8_E4M3);
   if (!any_splits && chunks > limit) chunks = limit;
   return chunks * ((p.n + cols - 1) / cols) * ngroups;
 }
@@ -470,8 +470,8 @@ int64_t most_items(const GemmParams &p, int cols, int chunk_rows, bool any_split
 constexpr int64_t kMostItems = (int64_t{1} << 31) - (1 << 20);  // items are numbered with ints
 
 // Sizes of the launch of a plan whose columns and chunks are decided.
-void finish(const GemmParams &p, int cus, bool leave_cus, PanelPlan &plan) {
-  const int64_t blocks = (most_items(p, plan.cols, plan.chunk_rows, plan.any_splits, p.ngroups) + 7) / 8 * 8;
+void finish(const GemmParams &p, int dtype, int cus, bool leave_cus, PanelPlan &plan) {
+  const int64_t blocks = (most_items(p, dtype, plan.cols, plan.chunk_rows, plan.any_splits, p.ngroups) + 7) / 8 * 8;
   plan.blocks = static_cast<int>(blocks);
   plan.walk = leave_cus || blocks * 256 > 0x7fffffffll;
   const int64_t most = cus >= 8 ? cus / 8 * 8 : cus;  // whole rounds over the XCDs where there are enough units
@@ -531,8 +531,8 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
   } else {
     return plan;
   }
-  if (most_items(p, 64, plan.chunk_rows, plan.any_splits, kMaxWeightGroups) > kMostItems) return PanelPlan{};
-  finish(p, cus, leave_cus, plan);
+  if (most_items(p, dtype, 64, plan.chunk_rows, plan.any_splits, kMaxWeightGroups) > kMostItems) return PanelPlan{};
+  finish(p, dtype, cus, leave_cus, plan);
   return plan;
 }
 

@@ -240,7 +240,7 @@ void grouped_gemm_stream_kernel(const FewRowsArgs few, const GemmParams p, const
   const int stride = static_cast<int>(gridDim.x);
   int block = blockIdx.x;
   do {
-    const WorkItem t = locate(p, tiles_n1 * p.ngroups, kStreamRows, block + team * stride);
+    const WorkItem t = locate<T>(p, tiles_n1 * p.ngroups, kStreamRows, block + team * stride);
     const int g = p.ngroups > 1 ? t.nt / tiles_n1 : 0;
     const int n0 = (t.nt - g * tiles_n1) * (16 * NB);
     if constexpr (!WALK) {
@@ -265,7 +265,7 @@ int64_t one_chunk_items(const GemmParams &p, int ngroups, int nb) {
 }
 int64_t most_items(const GemmParams &p, int ngroups, int nb) {
   const int active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
-  const int chunks = active + (p.max_rows - active) / kStreamRows, limit = stream_chunks_limit(active, kStreamRows);
+  const int chunks = active + (p.max_rows - active) / kStreamRows, limit = stream_chunks_limit(active, kStreamRows, false);
   return static_cast<int64_t>(chunks < limit ? chunks : limit) * ((p.n + 16 * nb - 1) / (16 * nb)) * ngroups;
 }
 
