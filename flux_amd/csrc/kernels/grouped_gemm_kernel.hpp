@@ -1240,12 +1240,13 @@ __device__ __forceinline__ void gemm_tile_lines(const GemmParams &p, uint8_t *sm
   __builtin_amdgcn_s_barrier();  // the LDS windows are free again before the next tile's fills start
 }
 
-// Block-scaled fp8, one 256 x 128 piece: A carries one scale per row and 128 of K, B one per 128 x 128 block, and
-// the products of every 128 of K are added to the result with a_scale[row] * b_scale (the promotion).
+// Block-scaled fp8, one piece of 64 * MB rows (256; 128 or 64 for the last rows of an expert) x 128 columns: A carries one scale
+// per row and 128 of K, B one per 128 x 128 block, and the products of every 128 of K are added to the result with
+// a_scale[row] * b_scale (the promotion).
 //
 // The unit of the k loop is a pair of k-steps, i.e. one scale block: LDS rows hold 128 bytes of K, a ring stage is
-// 256 X rows + 128 W rows + the 256 row scales of the pair (49 KiB; three stages).  A wave computes its 128 x 64
-// quarter block by block: for each 32 x 32 block the two MFMAs of the pair (the first with C = 0), then
+// 64 * MB X rows + 128 W rows + their row scales of the pair (49 KiB for 256 rows; three stages).  A wave computes its
+// 32 * MB x 64 quarter block by block: for each 32 x 32 block the two MFMAs of the pair (the first with C = 0), then
 // main += block * scale — the block's sums live in vector registers for the length of three MFMAs and the promotion
 // is one v_fmac per element (sums kept in accumulation registers across a whole k-step would cost a register read
 // per element as well: with one wave per SIMD the vector ALU's time adds to the MFMA time).  Fragments of a whole
@@ -1255,16 +1256,17 @@ __device__ __forceinline__ void gemm_tile_lines(const GemmParams &p, uint8_t *sm
 //
 // A fill instruction covers 8 rows x 128 bytes (whole cache lines); chunk c of row r lies in 16-byte slot
 // c ^ ((r >> 1) & 7) of the row, which makes the 32-row fragment reads free of bank conflicts.
+template <int MB>
 __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8_t *smem, const TileCtx &c, const TileDesc &t) {
-  constexpr int XROWS = 256, WROWS = 128, ROWB = 128;
-  constexpr int XBYTES = XROWS * ROWB, WBYTES = WROWS * ROWB;  // 32 KiB, 16 KiB
-  constexpr int SCALE_OFF = XBYTES + WBYTES;                   // 256 floats
+  constexpr int XROWS = 64 * MB, WROWS = 128, ROWB = 128;
+  constexpr int XBYTES = XROWS * ROWB, WBYTES = WROWS * ROWB;  // 8 * MB KiB, 16 KiB
+  constexpr int SCALE_OFF = XBYTES + WBYTES;                   // XROWS floats
   constexpr int PSB = SCALE_OFF + 1024;                        // bytes of a stage
   constexpr int NSTG = 3;
   static_assert(NSTG * PSB <= LDS_BYTES, "three stages fit the LDS");
-  constexpr int XF = 8, WF = 4;          // fill instructions per wave and pair: X rows, W rows
+  constexpr int XF = 2 * MB, WF = 4;     // fill instructions per wave and pair: X rows, W rows
   constexpr int PAIRF = XF + WF + 1;     // ... with the scale fill
-  constexpr int MBK = 4, NBK = 2, NBLK = MBK * NBK;
+  constexpr int MBK = MB, NBK = 2, NBLK = MBK * NBK;
   typedef Geom<1>::Acc Acc;
   const int wave = c.wave, lane = c.lane, wm = c.wm, wn = c.wn;
   const int e = t.e, row_base = t.row_base, rows_e = t.rows_e, m0 = t.m0;
@@ -1285,7 +1287,7 @@ __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8
   uint32_t xoff[XF], woff[WF];
 #pragma unroll
   for (int j = 0; j < XF; ++j) {
-    int xr = m0 + 64 * wave + 8 * j + (lane >> 3);
+    int xr = m0 + 8 * XF * wave + 8 * j + (lane >> 3);
     if (xr > rows_e - 1) xr = rows_e - 1;
     if (xr < 0) xr = 0;
     int64_t arow = xr - m0;
@@ -1293,7 +1295,7 @@ __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8
       arow = p.gather_a[row_base + xr];
       if (p.a_rows > 0) arow = arow < 0 ? 0 : (arow >= p.a_rows ? p.a_rows - 1 : arow);
     }
-    const int chunk = (lane & 7) ^ ((4 * j + (lane >> 4)) & 7);
+    const int chunk = (lane & 7) ^ ((4 * j + (lane >> 4)) & 7);  // (8 * XF * wave is a multiple of 16)
     xoff[j] = static_cast<uint32_t>(arow * c.kbytes) + chunk * 16;
   }
 #pragma unroll
@@ -1303,12 +1305,13 @@ __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8
     const int chunk = (lane & 7) ^ ((4 * j + (lane >> 4)) & 7);
     woff[j] = static_cast<uint32_t>((wr - n0) * c.kbytes) + chunk * 16;
   }
-  // Scales: lane l of a wave fetches the scale of tile row 64 * wave + l.
+  // Scales: lane l of a wave fetches the scale of tile row 64 * wave + l (with fewer rows two or all waves the same ones).
+  const int srow0 = 64 * (wave & (MB - 1));
   const __amdgpu_buffer_rsrc_t as_rsrc = make_rsrc(reinterpret_cast<const uint8_t *>(pe->a_scale), 0xffffffffll);
   uint32_t as_voff;
   int as_kstep, bs_base, bs_kstep;
   {
-    int xr = m0 + 64 * wave + lane;
+    int xr = m0 + srow0 + lane;
     if (xr > rows_e - 1) xr = rows_e - 1;
     int64_t arow = row_base + xr;
     if (gathered) {
@@ -1343,7 +1346,7 @@ __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8
     constexpr int stage = decltype(STAGE)::value, q = decltype(Q)::value;
     const bool in = kb < kblocks;
     if constexpr (q == 0)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(in ? as_rsrc : zrsrc, (lds_ptr_t)(smem + stage * PSB + SCALE_OFF + wave * 256), 4,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(in ? as_rsrc : zrsrc, (lds_ptr_t)(smem + stage * PSB + SCALE_OFF + srow0 * 4), 4,
                                                static_cast<int>(in ? as_voff : static_cast<uint32_t>(lane * 4)),
                                                in ? kb * as_kstep : 0, 0, 0);
     else if constexpr (q <= XF)
@@ -1369,25 +1372,25 @@ __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8
       const int r = lane & 31, ch = 4 * h + 2 * (lane >> 5) + s2;
       roff[h][s2] = r * ROWB + ((ch ^ ((r >> 1) & 7)) << 4);
     }
-  const uint8_t *const xread = smem + wm * 128 * ROWB;
+  const uint8_t *const xread = smem + wm * (32 * MB) * ROWB;
   const uint8_t *const wread = smem + XBYTES + wn * 64 * ROWB;
-  const float *const sread = reinterpret_cast<const float *>(smem + SCALE_OFF) + wm * 128 + (lane & 31);
-  // Read number R (0 .. 25) of the pair in stage STAGE: 16 X chunks, 8 W chunks, then the row scales (2 x 2).
+  const float *const sread = reinterpret_cast<const float *>(smem + SCALE_OFF) + wm * (32 * MB) + (lane & 31);
+  // Read number R of the pair in stage STAGE: 4 * MB X chunks, 8 W chunks, then the row scales, two at a time.
   auto read_one = [&](auto STAGE, auto R, Frags &f, float (&sc)[MBK]) {
     constexpr int stage = decltype(STAGE)::value, r = decltype(R)::value;
-    if constexpr (r < 16) {
+    if constexpr (r < 4 * MB) {
       constexpr int i = r >> 2, h = (r >> 1) & 1, s2 = r & 1;
       f.x[i][h][s2] = *reinterpret_cast<const i32x4 *>(xread + stage * PSB + i * 32 * ROWB + roff[h][s2]);
-    } else if constexpr (r < 24) {
-      constexpr int j = (r - 16) >> 2, h = ((r - 16) >> 1) & 1, s2 = (r - 16) & 1;
+    } else if constexpr (r < 4 * MB + 8) {
+      constexpr int j = (r - 4 * MB) >> 2, h = ((r - 4 * MB) >> 1) & 1, s2 = (r - 4 * MB) & 1;
       f.w[j][h][s2] = *reinterpret_cast<const i32x4 *>(wread + stage * PSB + j * 32 * ROWB + roff[h][s2]);
     } else {
-      constexpr int i0 = (r - 24) * 2;
+      constexpr int i0 = (r - 4 * MB - 8) * 2;
       sc[i0] = sread[stage * (PSB / 4) + i0 * 32];
-      sc[i0 + 1] = sread[stage * (PSB / 4) + (i0 + 1) * 32];
+      if constexpr (i0 + 1 < MBK) sc[i0 + 1] = sread[stage * (PSB / 4) + (i0 + 1) * 32];
     }
   };
-  constexpr int NREADS = 26;
+  constexpr int NREADS = 4 * MB + 8 + (MB + 1) / 2;
 
   Acc main_acc[MBK][NBK];
 #pragma unroll
@@ -1484,21 +1487,21 @@ __device__ __forceinline__ void gemm_tile_blockscaled(const GemmParams &p, uint8
   FLUXMI_WAITCNT(0, 0);          // this wave's trailing fills have landed
   __builtin_amdgcn_s_barrier();  // ... and everybody else's; nobody reads the ring any more
   uint8_t *windows = smem + wave * 8192;  // one 8 KiB window per wave
-  const int wrow0 = m0 + wm * 128;
+  const int wrow0 = m0 + wm * (32 * MB);
   {
     const int wcol0 = n0 + wn * 64;
-    const bool full = wrow0 + 128 <= rows_e && wcol0 + 64 <= pe->n && pe->scatter_d == nullptr && pe->accumulate == 0;
+    const bool full = wrow0 + 32 * MB <= rows_e && wcol0 + 64 <= pe->n && pe->scatter_d == nullptr && pe->accumulate == 0;
     const bool out_f32 = pe->d_fp32 != 0;
     const bool scaled = !(c.scalar == 1.f && pe->alpha[g] == nullptr && pe->row_scale == nullptr && pe->col_scale == nullptr);
     if (full && !scaled) {
-      if (out_f32) store_tile<1, 4, 2, true, true, false, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
-      else store_tile<1, 4, 2, true, false, false, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
+      if (out_f32) store_tile<1, MB, 2, true, true, false, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
+      else store_tile<1, MB, 2, true, false, false, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
     } else if (full) {
-      if (out_f32) store_tile<1, 4, 2, true, true, true, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
-      else store_tile<1, 4, 2, true, false, true, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
+      if (out_f32) store_tile<1, MB, 2, true, true, true, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
+      else store_tile<1, MB, 2, true, false, true, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
     } else {
-      if (out_f32) store_tile<1, 4, 2, false, true, true, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
-      else store_tile<1, 4, 2, false, false, true, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
+      if (out_f32) store_tile<1, MB, 2, false, true, true, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
+      else store_tile<1, MB, 2, false, false, true, true>(windows, c, g, e, row_base, rows_e, wrow0, wcol0, main_acc);
     }
   }
   __builtin_amdgcn_s_barrier();  // the LDS windows are free again before the next tile's fills start
@@ -1744,7 +1747,12 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
     item += grid;
     const TileDesc next = locate(item);
     if constexpr (BS) {
-      if (cur.kind == 2) gemm_tile_blockscaled(p, smem, c, cur);
+      // The last row tile of an expert runs 128 or 64 rows high when that covers its rows (32 experts, 512 rows each on average,
+      // 2048 x 7168 318 -> 311 us and 7168 x 2048 364 -> 344; at 140 to 194 rows within 1 % either way).
+      const int left = half_tiles ? cur.rows_e - cur.m0 : BM;
+      if (cur.kind == 2 && left > 128) gemm_tile_blockscaled<4>(p, smem, c, cur);
+      else if (cur.kind == 2 && left > 64) gemm_tile_blockscaled<2>(p, smem, c, cur);
+      else if (cur.kind == 2) gemm_tile_blockscaled<1>(p, smem, c, cur);
     } else if constexpr (kLineFills) {
       if (cur.kind == 0) gemm_tile_lines<ELT, 4, 4>(p, smem, c, cur, next, pf);
       else if (cur.kind == 1) gemm_tile_lines<ELT, 2, 4>(p, smem, c, cur, next, pf);

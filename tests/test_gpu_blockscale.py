@@ -168,3 +168,33 @@ def test_blockscale_c5_shapes_quantised_on_the_gpu(layer):
     assert (num / den) ** 0.5 < 3e-2
     assert (num / den) ** 0.5 < 5e-3          # accumulation order and the bf16 rounding only
     assert (num_u / den) ** 0.5 < 6e-2        # e4m3 block quantisation against the unquantised product
+
+
+@pytest.mark.parametrize("k", [128, 256, 384, 896, 1664])
+@pytest.mark.parametrize("split,n", [([129, 192, 193, 64, 65, 128, 1, 320, 321, 384, 385, 255], 264), ([513, 576, 577, 640, 641], 136)])
+def test_blockscale_last_rows_of_an_expert(split, n, k):
+    """The last row tile is 64, 128 or 256 rows high: the sums of a row do not depend on which."""
+    from flux_amd import capi
+    print(f"[case] blockscale last rows {split} N={n} K={k}", flush=True)
+    g = torch.Generator().manual_seed(k + n)
+    rows, experts = sum(split), len(split)
+    qa = torch.randn(rows, k, generator=g).to(torch.float8_e4m3fn)
+    qw = torch.randn(experts, n, k, generator=g).to(torch.float8_e4m3fn)
+    sa = torch.rand(rows, k // 128, generator=g) + 0.5
+    sw = torch.rand(experts, (n + 127) // 128, k // 128, generator=g) + 0.5
+
+    def run(a, scale, counts):
+        counts = np.array(counts, dtype=np.int32)
+        return capi.grouped_gemm_blockscale(a.cuda(), qw.cuda(), torch.from_numpy(counts).cuda(), layers.a_scale_to_block128(scale).cuda(),
+                                            sw.cuda(), out_dtype=torch.float32).cpu()
+    out = run(qa, sa, split)
+    ref = layers.fp8_blockscale_grouped_gemm_fp32(qa, sa, qw, sw, np.array(split, dtype=np.int32))
+    assert torch.allclose(out, ref, rtol=1e-4, atol=2e-3 * k ** 0.5), float((out - ref).abs().max())
+    # the same rows as part of experts of whole 256-row tiles
+    whole = [(c + 255) // 256 * 256 for c in split]
+    at = torch.cat([torch.arange(c) + sum(whole[:e]) for e, c in enumerate(split)])
+    wide_a = torch.zeros(sum(whole), k, dtype=torch.uint8)
+    wide_a[at] = qa.view(torch.uint8)
+    wide_s = torch.ones(sum(whole), k // 128)
+    wide_s[at] = sa
+    assert torch.equal(run(wide_a.view(torch.float8_e4m3fn), wide_s, whole)[at], out)
