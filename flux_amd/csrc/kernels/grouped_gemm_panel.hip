@@ -4,7 +4,10 @@
 // 128 or 256 columns of one chunk over the whole of K; each wave has a quarter of the columns and all of the rows.
 //
 //  * K goes by lines of 128 bytes per row.  Every load instruction covers eight whole lines, weights non-temporally (a stream of such
-//    lines from HBM: 50 to 53 GB/s per compute unit alone and 26 with all of them, ordinary loads 45 and 20).
+//    lines from HBM: 50 to 53 GB/s per compute unit alone and 26 with all of them, ordinary loads 45 and 20).  Where rows do not
+//    start on lines (WHOLE false), each load covers parts of two lines and the next one wants the second again, which a
+//    non-temporal load has given up: ordinary loads there (whole passes, non-temporal -> ordinary, us: bf16 40 experts 3760 x 1456,
+//    80 rows each 311 -> 282, macro tiles 293; fp8 44 experts 5792 x 1680, 36 rows each 302 -> 269, macro tiles 299).
 //  * The rows' operand goes through LDS: the four waves fill one ring of lines for all (direct-to-LDS loads), one wait and one
 //    barrier per line.
 //  * The weights are used by one wave only.  64- and 128-column workgroups pass them through LDS too, each wave through a ring of its
@@ -197,9 +200,9 @@ __device__ __forceinline__ void zero(f32x4 *acc) {
 }
 
 // 16 * MB rows x 64 * NB columns, weights through LDS.  Ring of DEPTH stages: the rows' line, then a line of each wave's weights.
-// STEP: lines that are asked for together, waited for and computed.  Two halve the waits, and neighbouring lines of a row are
+// WHOLE: rows start on lines.  STEP: lines that are asked for together, waited for and computed.  Two halve the waits, and neighbouring lines of a row are
 // fetched one after the other (64 columns, bf16 8 experts 14336 x 4096, 8 rows each: 142 us line by line, 136 in pairs).
-template <Elem T, int MB, int NB, int DEPTH, int STEP>
+template <Elem T, int MB, int NB, int DEPTH, int STEP, bool WHOLE>
 __device__ __forceinline__ void lds_tile(const GemmParams &p, const FewRowsArgs &few, uint8_t *smem, const WorkItem &t, int g, int n0, int wave) {
   typedef Rows<T, MB> X;
   constexpr bool BS = X::BS;
@@ -238,7 +241,7 @@ __device__ __forceinline__ void lds_tile(const GemmParams &p, const FewRowsArgs 
 #pragma unroll
       for (int u = 0; u < STEP; ++u) {
         const uint8_t *src = kb + u * 128 + wbyte[j & 1] < kb32 ? b + u * 128 + j * 8 * kbytes + woff[j & 1] : g_zero_line + lane * 16;
-        __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(at + u * STAGE + X::BYTES + X::SCALES + wave * WBYTES + j * 1024), 16, 0, 2);
+        __builtin_amdgcn_global_load_lds((gbl_ptr_t)src, (lds_ptr_t)(at + u * STAGE + X::BYTES + X::SCALES + wave * WBYTES + j * 1024), 16, 0, WHOLE ? 2 : 0);
       }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -296,7 +299,7 @@ __device__ __forceinline__ void lds_tile(const GemmParams &p, const FewRowsArgs 
 }
 
 // 16 * MB rows x 64 * NB columns, weights through registers, two lines ahead; the rows' ring has a stage more.  Not block-scaled.
-template <Elem T, int MB, int NB>
+template <Elem T, int MB, int NB, bool WHOLE>
 __device__ __forceinline__ void register_tile(const GemmParams &p, const FewRowsArgs &few, uint8_t *smem, const WorkItem &t, int g, int n0, int wave) {
   typedef Rows<T, MB> X;
   static_assert(!X::BS, "no registers left for block scales");
@@ -319,7 +322,7 @@ __device__ __forceinline__ void register_tile(const GemmParams &p, const FewRows
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) v[j][h] = load16<2>(wr, off, static_cast<int>(ks + (2 * j + h) * 8u * static_cast<uint32_t>(kb32)));
+      for (int h = 0; h < 2; ++h) v[j][h] = load16<WHOLE ? 2 : 0>(wr, off, static_cast<int>(ks + (2 * j + h) * 8u * static_cast<uint32_t>(kb32)));
   };
   f32x4 acc[MB][NB];
   zero<MB * NB>(&acc[0][0]);
@@ -379,7 +382,7 @@ constexpr int lds_bytes() {
   return DEPTH > 0 ? DEPTH * (CH * 2048 + scales + NB * 8192) : 3 * CH * 2048;
 }
 
-template <Elem T, int CH, int NB, int DEPTH>
+template <Elem T, int CH, int NB, int DEPTH, bool WHOLE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void grouped_gemm_panel_kernel(const FewRowsArgs few, const GemmParams p, const int blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -395,8 +398,8 @@ void grouped_gemm_panel_kernel(const FewRowsArgs few, const GemmParams p, const 
       auto tile = [&](auto BLOCKS) {
         constexpr int mb = decltype(BLOCKS)::value;
         if constexpr (mb <= CH) {
-          if constexpr (DEPTH > 0) lds_tile<T, mb, NB, DEPTH, DEPTH == 6 ? 2 : 1>(p, few, smem, t, g, n0, wave);
-          else register_tile<T, mb, NB>(p, few, smem, t, g, n0, wave);
+          if constexpr (DEPTH > 0) lds_tile<T, mb, NB, DEPTH, DEPTH == 6 ? 2 : 1, WHOLE>(p, few, smem, t, g, n0, wave);
+          else register_tile<T, mb, NB, WHOLE>(p, few, smem, t, g, n0, wave);
         }
       };
       if (CH == 2 && t.rows <= 16) tile(std::integral_constant<int, CH == 2 ? 1 : 2>{});
@@ -413,14 +416,27 @@ void grouped_gemm_panel_kernel(const FewRowsArgs few, const GemmParams p, const 
 #endif
 }
 
-template <Elem T, int CH, int NB, int DEPTH>
-int launch(const GemmParams &p, const FewRowsArgs &few, const PanelPlan &plan, hipStream_t s) {
+template <Elem T, int CH, int NB, int DEPTH, bool WHOLE>
+int launch_tiles(const GemmParams &p, const FewRowsArgs &few, const PanelPlan &plan, hipStream_t s) {
   static std::atomic<uint64_t> done{0};
-  const void *kernel = reinterpret_cast<const void *>(grouped_gemm_panel_kernel<T, CH, NB, DEPTH>);
+  const void *kernel = reinterpret_cast<const void *>(grouped_gemm_panel_kernel<T, CH, NB, DEPTH, WHOLE>);
   const int rc = ensure_dynamic_lds(kernel, kCuLds, done);
   if (rc != FLUXMI_OK) return rc;
-  hipLaunchKernelGGL((grouped_gemm_panel_kernel<T, CH, NB, DEPTH>), dim3(plan.workgroups), dim3(256), plan.lds_bytes, s, few, p, plan.blocks);
+  hipLaunchKernelGGL((grouped_gemm_panel_kernel<T, CH, NB, DEPTH, WHOLE>), dim3(plan.workgroups), dim3(256), plan.lds_bytes, s, few, p, plan.blocks);
   return FLUXMI_OK;
+}
+
+// Whether every row of the weights starts on a line of 128 bytes.
+bool whole_lines(const GemmParams &p, int elt) {
+  uint64_t bits = static_cast<uint64_t>(p.k) * elt;
+  for (int g = 0; g < p.ngroups; ++g) bits |= reinterpret_cast<uintptr_t>(p.b[g]);
+  return bits % 128 == 0;
+}
+
+template <Elem T, int CH, int NB, int DEPTH>
+int launch(const GemmParams &p, const FewRowsArgs &few, const PanelPlan &plan, hipStream_t s) {
+  if (whole_lines(p, is_fp8(T) ? 1 : 2)) return launch_tiles<T, CH, NB, DEPTH, true>(p, few, plan, s);
+  return launch_tiles<T, CH, NB, DEPTH, false>(p, few, plan, s);
 }
 
 // Stages of the ring for 128 columns and 32 rows: four fill half of a compute unit's LDS exactly; with scales three do.

@@ -180,6 +180,22 @@ def test_panel_tiles_have_the_bits_of_the_macro_tiles(name, splits, n, k, cols, 
     assert torch.equal(few, many[rows])
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("name,splits,n,k,cols,chunk", CASES, ids=[c[0] for c in CASES])
+def test_panel_tiles_same_bits_where_weights_do_not_start_on_lines(name, splits, n, k, cols, chunk, dtype):
+    """The cache policy of the weights' loads follows their alignment to 128 bytes; results do not."""
+    a, w, sp, _ = made(splits, n, k, dtype, n + k)
+    ad, wd = a.to(DT[dtype]), w.to(DT[dtype])
+    raw = wd.view(torch.uint8).reshape(-1)
+    store = torch.empty(raw.numel() + 128, dtype=torch.uint8, device="cuda")
+    store[16:16 + raw.numel()] = raw
+    moved = store[16:16 + raw.numel()].view(DT[dtype]).view(wd.shape)
+    assert moved.data_ptr() % 128 == 16 and moved.is_contiguous()
+    want = capi.grouped_gemm(ad, wd, sp, out_dtype=torch.float32)
+    assert torch.equal(capi.grouped_gemm(ad, moved, sp, out_dtype=torch.float32), want)
+    assert torch.equal(want.double(), product(a, w, splits))
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp8", "bs"])
 @pytest.mark.parametrize("splits,computes", [([129] + [40] * 15 + [30] * 8, 1), ([600, 600] + [10] * 22, 0), ([64] * 5 + [0] * 19, 1)])
 def test_splits_choose_between_panel_and_macro_tiles(dtype, splits, computes):
