@@ -16,8 +16,12 @@
 //    then holds the rows' ring alone, and two workgroups with 128 rows share a compute unit.  What both do is keep about 64 KiB
 //    of weights in flight per unit; more does not help (16 KiB 26 GB/s, 32 KiB 44, 64 KiB 52, 128 KiB 52 through LDS, but 30 with 32
 //    register loads outstanding per wave).
-//  * A result is summed over K in one wave, in ascending lines, with the bits of the macro tiles for 16-bit operands (the same
-//    MFMAs over the same 32 elements).  Columns per workgroup, chunks, weight groups and cu_margin do not change it.
+//  * A result is summed over K in one wave.  In launches of few rows per expert, which the streaming form takes as well, it is the sum
+//    of as many partial sums as that form has waves, line l of K in sum l % SUMS, added in ascending order: the bits of the streaming
+//    form, so the choice between the two is free to follow the time.  One chain over K loses precision there (fp32 results
+//    against float64, one chain / four sums: bf16 K = 4096 4.0e-7 / 1.9e-7, K = 14336 7.7e-7 / 3.7e-7; the sums are registers that were
+//    free).  With more rows it is one chain in ascending lines, the macro tiles' order and for 16-bit operands their bits (the same
+//    MFMAs over the same 32 elements).  Columns per workgroup, chunks, weight groups and cu_margin do not change a bit.
 //  * A wave whose columns would end past N takes the last ones instead and stores only those that are its own; rows past the
 //    chunk's last repeat it and are not stored; bytes past the end of K are zeros (of a page of zeros, or buffer loads out of range).
 #include "grouped_gemm_panel.hpp"
@@ -107,11 +111,12 @@ struct Rows {
   }
 };
 
-// Byte offset of this lane's fragment half h inside a block of sixteen rows of a line.  16-bit: MFMA h takes the chunks 4h .. 4h + 3,
-// a lane one of them; fp8: one MFMA takes them all, a lane two.
-template <Elem T>
+// Byte offset of this lane's fragment half h inside a block of sixteen rows of a line.  fp8: one MFMA takes all eight chunks, a lane two
+// neighbours.  16-bit: MFMA h takes four of them, 4h .. 4h + 3 as the macro tiles do (one chain over K) or every second one as the
+// streaming form does (several sums).
+template <Elem T, int SUMS>
 __device__ __forceinline__ int fragment_offset(int lane, int h) {
-  const int r = lane & 15, c = is_fp8(T) ? 2 * (lane >> 4) + h : (lane >> 4) + 4 * h;
+  const int r = lane & 15, c = is_fp8(T) || SUMS > 1 ? 2 * (lane >> 4) + h : (lane >> 4) + 4 * h;
   return r * 128 + ((c ^ ((r >> 1) & 7)) << 4);
 }
 
@@ -202,12 +207,15 @@ __device__ __forceinline__ void zero(f32x4 *acc) {
 // 16 * MB rows x 64 * NB columns, weights through LDS.  Ring of DEPTH stages: the rows' line, then a line of each wave's weights.
 // WHOLE: rows start on lines.  STEP: lines that are asked for together, waited for and computed.  Two halve the waits, and neighbouring lines of a row are
 // fetched one after the other (64 columns, bf16 8 experts 14336 x 4096, 8 rows each: 142 us line by line, 136 in pairs).
-template <Elem T, int MB, int NB, int DEPTH, int STEP, bool WHOLE>
+// SUMS: partial sums of a result, line l belongs to sum l % SUMS.
+template <Elem T, int MB, int NB, int DEPTH, int STEP, int SUMS, bool WHOLE>
 __device__ __forceinline__ void lds_tile(const GemmParams &p, const FewRowsArgs &few, uint8_t *smem, const WorkItem &t, int g, int n0, int wave) {
   typedef Rows<T, MB> X;
   constexpr bool BS = X::BS;
   constexpr int WF = 2 * NB, PER_STEP = (X::FILLS + WF) * STEP, STEPS = DEPTH / STEP;  // vector-memory instructions per wave and step
   constexpr int WBYTES = 16 * NB * 128, STAGE = X::BYTES + X::SCALES + 4 * WBYTES;
+  constexpr int UNROLL = SUMS > STEP ? SUMS / STEP : 1;  // steps until a line's sum is that of the first one again
+  static_assert(SUMS == 1 || SUMS % STEP == 0, "a step starts at the same sum in every round");
   static_assert(DEPTH % STEP == 0 && STEPS >= 3, "a step computed, a step waited for, a step under way");
   const int lane = threadIdx.x & 63;
   const int64_t kbytes = static_cast<int64_t>(p.k) * (is_fp8(T) ? 1 : 2);
@@ -245,10 +253,10 @@ __device__ __forceinline__ void lds_tile(const GemmParams &p, const FewRowsArgs 
       }
     __builtin_amdgcn_sched_barrier(0);
   };
-  f32x4 acc[MB][NB];
-  zero<MB * NB>(&acc[0][0]);
-  const int foff[2] = {fragment_offset<T>(lane, 0), fragment_offset<T>(lane, 1)};
-  auto compute = [&](const uint8_t *sx, float bs) {
+  f32x4 acc[SUMS][MB][NB];
+  zero<SUMS * MB * NB>(&acc[0][0][0]);
+  const int foff[2] = {fragment_offset<T, SUMS>(lane, 0), fragment_offset<T, SUMS>(lane, 1)};
+  auto compute = [&](const uint8_t *sx, float bs, f32x4 (&sum)[MB][NB]) {
     const uint8_t *const sw = sx + X::BYTES + X::SCALES + wave * WBYTES;
     i32x4 w[NB][2], xf[2][1][2];
 #pragma unroll
@@ -270,7 +278,11 @@ __device__ __forceinline__ void lds_tile(const GemmParams &p, const FewRowsArgs 
       }
       __builtin_amdgcn_sched_barrier(0);
       const float s[1] = {BS ? as[i] : 1.f};
-      multiply<T, 1, NB>(w, xf[i & 1], s, &acc[i]);
+      multiply<T, 1, NB>(w, xf[i & 1], s, &sum[i]);
+      if constexpr (BS) {  // added here: sunk towards the next use of this sum, they keep products alive (308 spilled registers)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) asm volatile("" : "+v"(sum[i][j]));
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -278,24 +290,35 @@ __device__ __forceinline__ void lds_tile(const GemmParams &p, const FewRowsArgs 
 #pragma unroll
   for (int d = 0; d < STEPS - 1; ++d) fill(d, d * STEP);
   int step = 0;
-  for (int line = 0; line < lines; line += STEP) {
-    FLUXMI_VMCNT((STEPS - 2) * PER_STEP);  // these lines have landed for this wave's share
-    __builtin_amdgcn_s_barrier();          // ... and for everybody's; nobody reads the lines before them any more
-    __builtin_amdgcn_sched_barrier(0);
-    fill(step == 0 ? STEPS - 1 : step - 1, line + (STEPS - 1) * STEP);
+  for (int line = 0; line < lines;) {
 #pragma unroll
-    for (int u = 0; u < STEP; ++u) {
-      float bs = 1.f;
-      if constexpr (BS) {
-        bs = line + u < lines ? bs_next[u] : 0.f;  // past K the rows' scales are zeros, and 0 * inf is not 0
-        bs_next[u] = ws(line + STEP + u);
+    for (int q = 0; q < UNROLL; ++q) {
+      if (q > 0 && line >= lines) break;
+      FLUXMI_VMCNT((STEPS - 2) * PER_STEP);  // these lines have landed for this wave's share
+      __builtin_amdgcn_s_barrier();          // ... and for everybody's; nobody reads the lines before them any more
+      __builtin_amdgcn_sched_barrier(0);
+      fill(step == 0 ? STEPS - 1 : step - 1, line + (STEPS - 1) * STEP);
+#pragma unroll
+      for (int u = 0; u < STEP; ++u) {
+        float bs = 1.f;
+        if constexpr (BS) {
+          bs = line + u < lines ? bs_next[u] : 0.f;  // past K the rows' scales are zeros, and 0 * inf is not 0
+          bs_next[u] = ws(line + STEP + u);
+        }
+        compute(smem + (step * STEP + u) * STAGE, bs, acc[(q * STEP + u) % SUMS]);
       }
-      compute(smem + (step * STEP + u) * STAGE, bs);
+      line += STEP;
+      step = step == STEPS - 1 ? 0 : step + 1;
     }
-    step = step == STEPS - 1 ? 0 : step + 1;
   }
   FLUXMI_VMCNT(0);  // no fill may reach LDS after the workgroup has ended (or its next item has begun)
-  store<T, MB, NB>(p, few, t, g, c, acc);
+#pragma unroll
+  for (int u = 1; u < SUMS; ++u)
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[0][i][j] += acc[u][i][j];
+  store<T, MB, NB>(p, few, t, g, c, acc[0]);
 }
 
 // 16 * MB rows x 64 * NB columns, weights through registers, two lines ahead; the rows' ring has a stage more.  Not block-scaled.
@@ -326,7 +349,7 @@ __device__ __forceinline__ void register_tile(const GemmParams &p, const FewRows
   };
   f32x4 acc[MB][NB];
   zero<MB * NB>(&acc[0][0]);
-  const int foff[2] = {fragment_offset<T>(lane, 0), fragment_offset<T>(lane, 1)};
+  const int foff[2] = {fragment_offset<T, 1>(lane, 0), fragment_offset<T, 1>(lane, 1)};
   i32x4 xf[2][GB][2];
   auto read_x = [&](i32x4 (&v)[GB][2], const uint8_t *sx, int grp) {
 #pragma unroll
@@ -382,7 +405,7 @@ constexpr int lds_bytes() {
   return DEPTH > 0 ? DEPTH * (CH * 2048 + scales + NB * 8192) : 3 * CH * 2048;
 }
 
-template <Elem T, int CH, int NB, int DEPTH, bool WHOLE>
+template <Elem T, int CH, int NB, int DEPTH, int SUMS, bool WHOLE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void grouped_gemm_panel_kernel(const FewRowsArgs few, const GemmParams p, const int blocks) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -398,7 +421,7 @@ void grouped_gemm_panel_kernel(const FewRowsArgs few, const GemmParams p, const 
       auto tile = [&](auto BLOCKS) {
         constexpr int mb = decltype(BLOCKS)::value;
         if constexpr (mb <= CH) {
-          if constexpr (DEPTH > 0) lds_tile<T, mb, NB, DEPTH, DEPTH == 6 ? 2 : 1, WHOLE>(p, few, smem, t, g, n0, wave);
+          if constexpr (DEPTH > 0) lds_tile<T, mb, NB, DEPTH, DEPTH == 6 ? 2 : 1, SUMS, WHOLE>(p, few, smem, t, g, n0, wave);
           else register_tile<T, mb, NB, WHOLE>(p, few, smem, t, g, n0, wave);
         }
       };
@@ -416,13 +439,13 @@ void grouped_gemm_panel_kernel(const FewRowsArgs few, const GemmParams p, const 
 #endif
 }
 
-template <Elem T, int CH, int NB, int DEPTH, bool WHOLE>
+template <Elem T, int CH, int NB, int DEPTH, int SUMS, bool WHOLE>
 int launch_tiles(const GemmParams &p, const FewRowsArgs &few, const PanelPlan &plan, hipStream_t s) {
   static std::atomic<uint64_t> done{0};
-  const void *kernel = reinterpret_cast<const void *>(grouped_gemm_panel_kernel<T, CH, NB, DEPTH, WHOLE>);
+  const void *kernel = reinterpret_cast<const void *>(grouped_gemm_panel_kernel<T, CH, NB, DEPTH, SUMS, WHOLE>);
   const int rc = ensure_dynamic_lds(kernel, kCuLds, done);
   if (rc != FLUXMI_OK) return rc;
-  hipLaunchKernelGGL((grouped_gemm_panel_kernel<T, CH, NB, DEPTH, WHOLE>), dim3(plan.workgroups), dim3(256), plan.lds_bytes, s, few, p, plan.blocks);
+  hipLaunchKernelGGL((grouped_gemm_panel_kernel<T, CH, NB, DEPTH, SUMS, WHOLE>), dim3(plan.workgroups), dim3(256), plan.lds_bytes, s, few, p, plan.blocks);
   return FLUXMI_OK;
 }
 
@@ -433,10 +456,10 @@ bool whole_lines(const GemmParams &p, int elt) {
   return bits % 128 == 0;
 }
 
-template <Elem T, int CH, int NB, int DEPTH>
+template <Elem T, int CH, int NB, int DEPTH, int SUMS>
 int launch(const GemmParams &p, const FewRowsArgs &few, const PanelPlan &plan, hipStream_t s) {
-  if (whole_lines(p, is_fp8(T) ? 1 : 2)) return launch_tiles<T, CH, NB, DEPTH, true>(p, few, plan, s);
-  return launch_tiles<T, CH, NB, DEPTH, false>(p, few, plan, s);
+  if (whole_lines(p, is_fp8(T) ? 1 : 2)) return launch_tiles<T, CH, NB, DEPTH, SUMS, true>(p, few, plan, s);
+  return launch_tiles<T, CH, NB, DEPTH, SUMS, false>(p, few, plan, s);
 }
 
 // Stages of the ring for 128 columns and 32 rows: four fill half of a compute unit's LDS exactly; with scales three do.
@@ -445,12 +468,17 @@ constexpr int kDepth32 = T == Elem::FP8_BLOCKSCALED ? 3 : 4;
 
 template <Elem T>
 int launch_by_plan(const GemmParams &p, const FewRowsArgs &few, const PanelPlan &plan, hipStream_t s) {
-  const int blocks16 = plan.chunk_rows / 16;
   if constexpr (T != Elem::FP8_BLOCKSCALED)
-    if (plan.cols == 256) return launch<T, 8, 4, 0>(p, few, plan, s);
-  if (plan.cols == 128) return blocks16 <= 2 ? launch<T, 2, 2, kDepth32<T>>(p, few, plan, s) : (blocks16 <= 4 ? launch<T, 4, 2, 3>(p, few, plan, s) : launch<T, 8, 2, 3>(p, few, plan, s));
-  if (blocks16 <= 2 && plan.pairs) return launch<T, 2, 1, 6>(p, few, plan, s);
-  return blocks16 <= 2 ? launch<T, 2, 1, 4>(p, few, plan, s) : (blocks16 <= 4 ? launch<T, 4, 1, 4>(p, few, plan, s) : launch<T, 8, 1, 3>(p, few, plan, s));
+    if (plan.cols == 256) return launch<T, 8, 4, 0, 1>(p, few, plan, s);
+  const bool wide = plan.cols == 128;
+  if (plan.chunk_rows == 128) return wide ? launch<T, 8, 2, 3, 1>(p, few, plan, s) : launch<T, 8, 1, 3, 1>(p, few, plan, s);
+  if (plan.chunk_rows == 32) {  // always few rows, and four sums
+    if (wide) return launch<T, 2, 2, kDepth32<T>, 4>(p, few, plan, s);
+    return plan.pairs ? launch<T, 2, 1, 6, 4>(p, few, plan, s) : launch<T, 2, 1, 4, 4>(p, few, plan, s);
+  }
+  if (wide) return plan.sums == 4 ? launch<T, 4, 2, 3, 4>(p, few, plan, s) : launch<T, 4, 2, 3, 1>(p, few, plan, s);
+  return plan.sums == 8 ? launch<T, 4, 1, 4, 8>(p, few, plan, s)
+                        : (plan.sums == 4 ? launch<T, 4, 1, 4, 4>(p, few, plan, s) : launch<T, 4, 1, 4, 1>(p, few, plan, s));
 }
 
 template <Elem T>
@@ -500,8 +528,7 @@ void finish(const GemmParams &p, int dtype, int cus, bool leave_cus, PanelPlan &
 }  // namespace
 
 // Rules by rows per expert on average (R), items and bytes of the weights; us are bf16 unless they say otherwise, before (streaming
-// form or macro tiles) -> these tiles.  What the rules look at belongs to one weight group where it chooses between forms whose bits
-// differ, and not to the margin.
+// form or macro tiles) -> these tiles.  The sums of a result follow from the launch of one weight group, whatever its margin.
 PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, bool leave_cus) {
   PanelPlan plan = {};
   const int64_t line_count = (row_bytes(p, dtype) + 127) / 128, items64 = even_items(p, 64, 1);
@@ -509,14 +536,15 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
   const bool small = items64 <= 512 && static_cast<int64_t>(p.nexperts) * p.n * row_bytes(p, dtype) <= (64 << 20);
   const bool long_k = line_count >= 48, many_items = even_items(p, 128, p.ngroups) >= 1024;
   if (!shape_ok(p, dtype)) return plan;
+  plan.sums = few_rows ? stream_waves(p, dtype) : 1;
   // Hardly a row: the streaming form (64 experts 2816 x 2048, R 1: 78 against 86; fp8 32 experts 2048 x 7168 46 against 50).
-  if (few_rows && at_most(4)) return plan;
+  if (few_rows && at_most(4)) return PanelPlan{};
   // Few columns and long K: the streaming form splits K over eight waves (8 rows on 8 experts 4096 x 14336: 77 against 82).
-  if (few_rows && at_most(16) && items64 < 512 && line_count >= 64) return plan;
+  if (few_rows && at_most(16) && items64 < 512 && line_count >= 64) return PanelPlan{};
   // 128 columns of rows that lie a multiple of 4 KiB apart, all of them read at the same line: few memory channels at a time.  The
   // streaming form's waves are at different lines (64 experts 2816 x 2048, R 8: 115 against 118, fp8 4096 117 against 126; K = 2112
   // 126 against 119, K = 1984 114 against 113).
-  if (few_rows && at_most(16) && many_items && !long_k && row_bytes(p, dtype) % 4096 == 0) return plan;
+  if (few_rows && at_most(16) && many_items && !long_k && row_bytes(p, dtype) % 4096 == 0) return PanelPlan{};
   if (small && at_most(192)) {
     // Weights that fit the Infinity Cache in few items: latency counts, so many workgroups, and no second launch whatever the splits
     // (the macro tiles that return at once cost 5).  8 experts of 2048 x 1024, R 16 / 64 / 128: 14.4 -> 11.9, 23 -> 13, 34 -> 20; of
@@ -545,7 +573,7 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
     plan.cols = even_items(p, 256, p.ngroups) >= 384 && p.a_scale == nullptr && !leave_cus ? 256 : (even_items(p, 128, p.ngroups) >= 192 ? 128 : 64);
     plan.chunk_rows = 128;
   } else {
-    return plan;
+    return PanelPlan{};
   }
   if (most_items(p, dtype, 64, plan.chunk_rows, plan.any_splits, kMaxWeightGroups) > kMostItems) return PanelPlan{};
   finish(p, dtype, cus, leave_cus, plan);

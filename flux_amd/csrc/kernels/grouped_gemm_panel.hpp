@@ -9,6 +9,7 @@ namespace fluxmi {
 struct PanelPlan {
   int cols;             // columns per workgroup: 64 or 128 (weights through LDS), 256 (weights through registers)
   int chunk_rows;       // most rows of a work item: 32, 64 or 128
+  int sums;             // partial sums of a result over K: 4 or 8 (few rows per expert, the streaming form's bits), 1
   bool pairs;           // 64 columns, 32 rows: lines of K are asked for in pairs
   int blocks;           // items the launch is numbered for
   unsigned workgroups;  // workgroups launched; fewer than `blocks`: each walks several items

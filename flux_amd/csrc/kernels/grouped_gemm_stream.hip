@@ -315,11 +315,15 @@ bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
 // / 224 of 256 units, this form and the macro tiles: bf16 8 experts 14336 x 4096, 74 rows 162 / 185 / 255 / 995 and 215 / 238 / 268 /
 // 773; fp8 32 experts 7168 x 2048, 400 rows 97 / 118 / 168 / 642 and 111 / 120 / 147 / 500 (a unit alone streams 30 GB/s here; a
 // ring of three or four lines in place of two changed nothing).
+int stream_waves(const GemmParams &p, int dtype) {
+  const int64_t lines = (static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2) + 127) / 128;
+  return one_chunk_items(p, 1, 4) < 512 && lines >= 64 ? 8 : 4;
+}
+
 StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, bool leave_cus) {
   StreamPlan plan;
-  const int64_t lines = (static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2) + 127) / 128;
   const bool few = one_chunk_items(p, p.ngroups, 4) < 512;
-  plan.waves = one_chunk_items(p, 1, 4) < 512 && lines >= 64 ? 8 : 4;  // of one weight group: a launch of several has its bits
+  plan.waves = stream_waves(p, dtype);
   plan.cols = few || (p.a_scale == nullptr && p.max_rows <= 4 * p.nexperts) ? 32 : 64;
   const int64_t blocks = (most_items(p, p.ngroups, plan.cols / 16) + 7) / 8 * 8;
   plan.blocks = static_cast<int>(blocks);

@@ -163,8 +163,11 @@ def test_panel_tiles_infinite_scales(kblocks, rows, n, experts):
     assert torch.equal(torch.isinf(got) & (got > 0), inf.view(m, n))
 
 
+MORE_ROWS = [c for c in CASES if sum(c[1]) > 32 * len(c[1])]  # (with fewer rows they have the streaming form's bits, below)
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
-@pytest.mark.parametrize("name,splits,n,k,cols,chunk", CASES, ids=[c[0] for c in CASES])
+@pytest.mark.parametrize("name,splits,n,k,cols,chunk", MORE_ROWS, ids=[c[0] for c in MORE_ROWS])
 def test_panel_tiles_have_the_bits_of_the_macro_tiles(name, splits, n, k, cols, chunk, dtype):
     """16-bit operands: the same rows among so many others that the macro tiles compute the launch."""
     print(f"[case] panel gemm bits {dtype} {name} n={n} k={k}", flush=True)
@@ -178,6 +181,76 @@ def test_panel_tiles_have_the_bits_of_the_macro_tiles(name, splits, n, k, cols, 
     many = capi.grouped_gemm(x, w, torch.tensor(more, dtype=torch.int32, device="cuda"), out_dtype=torch.float32)
     few = capi.grouped_gemm(x[rows], w, torch.tensor(splits, dtype=torch.int32, device="cuda"), out_dtype=torch.float32)
     assert torch.equal(few, many[rows])
+
+
+# (name, splits, N, bytes of K, columns, rows of a chunk, waves over which the streaming form splits K): launches of few rows per
+# expert, which both forms take.  Numbers of lines that four and eight sums do not divide.
+FEW_ROWS = [
+    ("64 columns, 32 rows", [32, 0, 31, 17, 16, 1, 2, 9], 4164, 544, 64, 32, 4),
+    ("64 columns, 32 rows, lines in pairs", [32, 0, 31, 17, 16, 1, 2, 9], 4164, 6432, 64, 32, 4),
+    ("128 columns, 32 rows", [1, 32, 16, 17] + [0] * 3 + [5] * 123, 1028, 800, 128, 32, 4),
+    ("64 columns, 64 rows", [20, 32, 17, 26], 192, 2080, 64, 64, 4),
+    ("128 columns, 64 rows", [20] * 62 + [17, 32], 2052, 800, 128, 64, 4),
+    ("64 columns, 64 rows, eight sums, small", [20, 24, 28, 18], 192, 16416, 64, 64, 8),
+    ("64 columns, 64 rows, eight sums", [20, 24, 28, 18], 4096, 16416, 64, 64, 8),
+]
+
+
+def random_operands(splits, n, k, dtype, groups=1):
+    """x, w for each group, and run(rows, splits, weights): the fp32 results of these rows of x."""
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    m, e = sum(splits), len(splits)
+    x = torch.randn(m, k, generator=g, device="cuda").to(DT[dtype])
+    ws = [(torch.randn(e, n, k, generator=g, device="cuda") * (1.0 if dtype in ("fp8", "bs") else 0.05)).to(DT[dtype]) for _ in range(groups)]
+    sa = torch.rand(m, k // 128, generator=g, device="cuda") + 0.5
+    sb = torch.rand(e, (n + 127) // 128, k // 128, generator=g, device="cuda") + 0.5
+
+    def run(rows, counts, w):
+        sp = torch.tensor(counts, dtype=torch.int32, device="cuda")
+        if dtype != "bs":
+            return capi.grouped_gemm(x[rows], w, sp, out_dtype=torch.float32)
+        pad = torch.zeros((len(rows) + 127) // 128 * 128, k // 128, device="cuda")
+        pad[:len(rows)] = sa[rows]
+        return capi.grouped_gemm_blockscale(x[rows], w, sp, pad.view(-1, 128, k // 128).permute(0, 2, 1).contiguous(), sb, out_dtype=torch.float32)
+
+    return x, ws, run
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8", "bs"])
+@pytest.mark.parametrize("name,splits,n,kbytes,cols,chunk,waves", FEW_ROWS, ids=[c[0] for c in FEW_ROWS])
+def test_few_rows_have_the_bits_of_the_streaming_form(name, splits, n, kbytes, cols, chunk, waves, dtype):
+    """A result is the same sum of partial sums over K in both forms (one chain would be less precise): the rows, four of each expert at a
+    time, in launches that the streaming form computes."""
+    k = kbytes // (2 if dtype in ("bf16", "f16") else 1)
+    if dtype == "bs":
+        n, k = (n + 127) // 128 * 128, (k + 127) // 128 * 128
+    print(f"[case] panel gemm, streaming form's bits {dtype} {name} n={n} k={k}", flush=True)
+    m, e, bs = sum(splits), len(splits), dtype == "bs"
+    info = capi.gemm_launch_info(DT[dtype], e, m, n, k, splits=splits, panel=True, block_scaled=bs)
+    assert (info.cols, info.chunk_rows, info.computes) == (cols, chunk, 1)
+    _, (w,), run = random_operands(splits, n, k, dtype)
+    got = run(torch.arange(m, device="cuda"), splits, w)
+    starts = torch.tensor([0] + splits).cumsum(0).tolist()
+    for first in range(0, max(splits), 4):
+        counts = [max(0, min(4, r - first)) for r in splits]
+        rows = torch.cat([torch.arange(s + first, s + first + c) for s, c in zip(starts, counts)]).cuda()
+        assert capi.gemm_launch_info(DT[dtype], e, len(rows), n, k, panel=True, block_scaled=bs).cols == 0
+        part = capi.gemm_launch_info(DT[dtype], e, len(rows), n, k, splits=counts, block_scaled=bs)
+        assert (part.form, part.stream_waves) == (capi.GEMM_STREAM, waves)
+        assert torch.equal(got[rows], run(rows, counts, w)), f"rows {first} to {first + 3} of each expert"
+
+
+@pytest.mark.parametrize("dtype,splits,n,k", [("bf16", [9] * 64, 1408, 2048), ("bf16", [8] * 32, 2048, 2048), ("fp8", [9] * 64, 1408, 4096),
+                                              ("bf16", [20] * 32, 1024, 512), ("f16", [20, 24, 28, 18], 192, 8208)])
+def test_few_rows_several_weight_groups_have_the_bits_of_one_launch_each(dtype, splits, n, k):
+    """The number of weight groups may choose between panel tiles and the streaming form."""
+    print(f"[case] panel gemm groups {dtype} n={n} k={k}", flush=True)
+    x, ws, run = random_operands(splits, n, k, dtype, groups=4)
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    alone = [run(torch.arange(len(x), device="cuda"), splits, w) for w in ws]
+    for groups in (2, 3, 4):
+        for got, want in zip(capi.grouped_gemm_multi(x, ws[:groups], sp, out_dtype=torch.float32), alone):
+            assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
