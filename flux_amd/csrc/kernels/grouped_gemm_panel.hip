@@ -513,11 +513,18 @@ int64_t most_items(const GemmParams &p, int dtype, int cols, int chunk_rows, boo
 
 constexpr int64_t kMostItems = (int64_t{1} << 31) - (1 << 20);  // items are numbered with ints
 
+int64_t block_count(const GemmParams &p, int dtype, const PanelPlan &plan) {
+  return (most_items(p, dtype, plan.cols, plan.chunk_rows, plan.any_splits, p.ngroups) + 7) / 8 * 8;
+}
+
+// Whether the workgroups of a launch walk several items: compute units are to be left free, or it would have 2^31 threads and more.
+bool walks(int64_t blocks, bool leave_cus) { return leave_cus || blocks * 256 > 0x7fffffffll; }
+
 // Sizes of the launch of a plan whose columns and chunks are decided.
 void finish(const GemmParams &p, int dtype, int cus, bool leave_cus, PanelPlan &plan) {
-  const int64_t blocks = (most_items(p, dtype, plan.cols, plan.chunk_rows, plan.any_splits, p.ngroups) + 7) / 8 * 8;
+  const int64_t blocks = block_count(p, dtype, plan);
   plan.blocks = static_cast<int>(blocks);
-  plan.walk = leave_cus || blocks * 256 > 0x7fffffffll;
+  plan.walk = walks(blocks, leave_cus);
   const int64_t most = cus >= 8 ? cus / 8 * 8 : cus;  // whole rounds over the XCDs where there are enough units
   plan.workgroups = static_cast<unsigned>(plan.walk && blocks > most ? most : blocks);
   plan.lds_bytes = p.a_scale != nullptr ? lds_of<Elem::FP8_BLOCKSCALED>(plan) : lds_of<Elem::FP8>(plan);
@@ -569,9 +576,11 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
     // R 64: 8 experts 14336 x 4096 228 -> 176 (256 columns; 128: 198), 4096 x 14336 390 -> 165 (128 columns; 256: 315), 64 experts 2048
     // x 1408 100 -> 76, fp8 32 experts 7168 x 2048 125 -> 108, block-scaled 161 -> 143; R 88: 239 -> 185, 241 -> 172, 104 -> 85, 133 ->
     // 117, 164 -> 162.  R 128, where half of the experts have two chunks: 243 -> 268.  The 256-column form has no registers left for a
-    // loop over items or for block scales.
-    plan.cols = even_items(p, 256, p.ngroups) >= 384 && p.a_scale == nullptr && !leave_cus ? 256 : (even_items(p, 128, p.ngroups) >= 192 ? 128 : 64);
+    // loop over items, so it takes no launch that walks, nor for block scales.
     plan.chunk_rows = 128;
+    plan.cols = 256;
+    if (even_items(p, 256, p.ngroups) < 384 || p.a_scale != nullptr || walks(block_count(p, dtype, plan), leave_cus))
+      plan.cols = even_items(p, 128, p.ngroups) >= 192 ? 128 : 64;
   } else {
     return PanelPlan{};
   }

@@ -74,3 +74,21 @@ def test_a_launch_stays_below_the_grid_limit(dtype, k, block_scaled, groups):
         assert 1 <= info.stream_workgroups <= ((1 << 32) - 1) // (info.stream_waves * 64)
     assert capi.gemm_launch_info(dtype, 1024, 1024, 1 << 20, k, block_scaled=block_scaled).stream_workgroups == 256
     assert capi.gemm_launch_info(dtype, 1024, 1024, 1 << 24, k, block_scaled=block_scaled).form == capi.GEMM_MACRO_TILES
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16, FP8])
+@pytest.mark.parametrize("experts,rows,k", [(64, 64 * 64, 8), (1024, 1024 * 64, 8), (8, 8 * 90, 16)])
+def test_panel_tiles_of_256_columns_have_a_workgroup_per_item(dtype, experts, rows, k):
+    """That kernel computes one item per workgroup: where a launch cannot have that many, other tiles, which walk, take it."""
+    def info(n):
+        return capi.gemm_launch_info(dtype, experts, rows, n, k * (2 if dtype == FP8 else 1), panel=True)
+
+    for n in (2048 * 256, 1 << 21, 1 << 23, 1 << 25, 30000000, 1 << 28):
+        got = info(n)
+        if got.cols == 256:
+            assert got.workgroups >= experts * ((n + 255) // 256)
+        assert got.cols == 0 or 1 <= got.workgroups <= ((1 << 31) - 1) // 256
+    if (experts, dtype) == (64, BF16):  # 73 chunks of 128 rows at most: both sides of 2^31 threads
+        below, above = info(114912 * 256), info(114912 * 256 + 4)
+        assert (below.cols, below.workgroups) == (256, 73 * 114912)
+        assert (above.cols, above.workgroups) == (128, 256)
