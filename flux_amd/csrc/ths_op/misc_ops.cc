@@ -184,7 +184,7 @@ static torch::Tensor blockscale_run(const torch::Tensor &input, const torch::Ten
   args.scalar_scale = 1.0f;
   args.d_fp32 = out_dtype == at::kFloat ? 1 : 0;
   auto one_kernel = [&]() {
-    return run_host_splits(args, splits_host.data_ptr<int32_t>(), nullptr, input_scale.data_ptr<float>(), a_layout,
+    return run_host_splits(args, splits_host, nullptr, input_scale.data_ptr<float>(), a_layout,
                            weight_scale.data_ptr<float>(), b_layout);
   };
   if (one_kernel()) return out;

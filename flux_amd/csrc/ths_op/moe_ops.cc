@@ -150,12 +150,13 @@ fluxmi_grouped_gemm_args gemm_args(const torch::Tensor &a, const torch::Tensor &
 }
 }  // namespace
 
-bool run_host_splits(const fluxmi_grouped_gemm_args &args, const int32_t *splits_host, const float *row_scale2, const float *a_scale,
+bool run_host_splits(const fluxmi_grouped_gemm_args &args, const torch::Tensor &splits, const float *row_scale2, const float *a_scale,
                      int32_t a_layout, const float *b_scale, int32_t b_layout) {
   hipStream_t stream = static_cast<hipStream_t>(current_stream());
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
-  const int rc = fluxmi_grouped_gemm_host_splits(&args, splits_host, row_scale2, a_scale, a_layout, b_scale, b_layout, stream);
+  if (splits.is_cuda() || splits.is_pinned()) return false;
+  const int rc = fluxmi_grouped_gemm_host_splits(&args, splits.data_ptr<int32_t>(), row_scale2, a_scale, a_layout, b_scale, b_layout, stream);
   if (rc < 0) check_status(rc, "fluxmi_grouped_gemm_host_splits");
   return rc == 1;
 }
@@ -454,7 +455,7 @@ torch::Tensor GemmGroupedV3GatherRS::forward_impl(
     if (!fused) {
       const fluxmi_grouped_gemm_args args = gemm_args(inputs[g], weights[g], nullptr, inter_[g], nullptr, m, alpha, row_factors[0], col, scalar,
                                                       sm_margin);
-      if (run_host_splits(args, splits_host.data_ptr<int32_t>(), row_factors[1])) {
+      if (run_host_splits(args, splits_host, row_factors[1])) {
         group_ptrs.push_back(inter_[g].data_ptr());
         continue;
       }
@@ -497,7 +498,7 @@ torch::Tensor GemmGroupedV3GatherRS::forward_impl(
     }
     const fluxmi_grouped_gemm_args args = gemm_args(inputs[g], weights[g], splits_dev_.data_ptr<int32_t>(), inter_[g], nullptr, m, alpha, row, col,
                                                     scalar, sm_margin);
-    if (!run_host_splits(args, splits_host.data_ptr<int32_t>(), nullptr))
+    if (!run_host_splits(args, splits_host, nullptr))
       check_status(fluxmi_grouped_gemm(&args, nullptr, 0, current_stream()), "fluxmi_grouped_gemm");
     group_ptrs.push_back(inter_[g].data_ptr());
   }
@@ -603,11 +604,10 @@ torch::Tensor GemmGroupedV3::forward(torch::Tensor input, torch::Tensor splits_c
   if (input.size(0) == 0) return out;
   const torch::Tensor splits_host = splits_cpu.to(at::kInt).contiguous();
   fluxmi_grouped_gemm_args args = gemm_args(input, weight_, nullptr, out, nullptr, input.size(0), nullptr, nullptr, nullptr, nullptr, 0);
-  const bool on_host = !splits_host.is_cuda();
-  if (on_host && run_host_splits(args, splits_host.data_ptr<int32_t>(), nullptr)) return out;
+  if (run_host_splits(args, splits_host, nullptr)) return out;
   const torch::Tensor splits_dev = splits_host.to(input.device(), /*non_blocking=*/true);
   args.splits = splits_dev.data_ptr<int32_t>();
-  if (on_host && run_host_splits(args, splits_host.data_ptr<int32_t>(), nullptr)) return out;
+  if (run_host_splits(args, splits_host, nullptr)) return out;
   check_status(fluxmi_grouped_gemm(&args, nullptr, 0, current_stream()), "fluxmi_grouped_gemm");
   return out;
 }

@@ -71,10 +71,12 @@ struct DistEnvTPWithEP {  // include/flux/ths_op/ths_op.h:117-130; only world si
   }
 };
 
-// The GEMM of `args` for row counts known on the host: one kernel is launched.  With args.splits unset that takes a form for few rows
-// per expert, with the counts in its arguments and no copy to the device.  False: nothing was launched, and always while the current
-// stream is being captured (a replay reads the counts again from where the copy reads them).
-bool run_host_splits(const fluxmi_grouped_gemm_args &args, const int32_t *splits_host, const float *row_scale2,
+// The GEMM of `args` for row counts known on the host (int32, contiguous): one kernel is launched.  With args.splits unset that takes a
+// form for few rows per expert, with the counts in its arguments and no copy to the device.  False: nothing was launched.  Always so
+//  - while the current stream is being captured (a replay reads the counts again from where the copy reads them), and
+//  - for counts in pinned memory: a copy that the stream has yet to run may be about to write them (`splits.copy_(on_device,
+//    non_blocking=True)` without a synchronisation), and only what the stream does after it, such as a copy back, sees them.
+bool run_host_splits(const fluxmi_grouped_gemm_args &args, const torch::Tensor &splits, const float *row_scale2,
                      const float *a_scale = nullptr, int32_t a_layout = 0, const float *b_scale = nullptr, int32_t b_layout = 0);
 
 // Launch tuning of a grouped GEMM: CUs to leave free (Flux's sm_margin) and the tile schedule registered

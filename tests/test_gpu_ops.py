@@ -360,6 +360,44 @@ def test_sm_margin_through_the_ops(c1):
         op0.forward(x, w1, sp, si, sm_margin=-1)
 
 
+@pytest.mark.parametrize("stale,fresh,n,k", [([0, 0, 40, 0], [20, 8, 0, 12], 256, 512), ([60] * 24, [600, 620] + [10] * 22, 1408, 1152),
+                                             ([50] * 130, [3017] + [27] * 129, 640, 512)])
+@pytest.mark.parametrize("op", ["layer1", "grouped", "blockscale"])
+def test_row_counts_in_pinned_memory_that_the_stream_has_yet_to_write(op, stale, fresh, n, k):
+    """A non-blocking copy into the pinned counts is ordered before the call by the stream alone: the call must not use what the host
+    sees in them."""
+    print(f"[case] pinned row counts {op} {fresh[:4]}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    m, e = sum(fresh), len(fresh)
+    x = torch.randn(m, k, generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn(e, n, k, generator=g, device="cuda") * 0.05).to(torch.bfloat16)
+    routing_idx = torch.randperm(m, generator=g, device="cuda").to(torch.int32)
+    factors = [torch.rand(m, generator=g, device="cuda") + 0.5 for _ in range(2)]
+    if op == "layer1":
+        layer = flux_amd.GemmGroupedV3GatherRS(e, m, n, 2, 0, 1, 1, 1)
+        run = lambda counts: layer.forward_gather_rs(x, w, counts, routing_idx, input_scale=factors[0], output_vec_scale=factors[1])
+    elif op == "grouped":
+        gemm = flux_amd.GemmGroupedV3(w, e)
+        run = lambda counts: gemm.forward(x, counts)
+    else:
+        q = flux_amd.Quantization(torch.bfloat16, torch.float8_e4m3fn)
+        qx, sx, _, _ = q.quantize_vector_blockwise(x, return_tranpose=False)
+        qw, sw = w.to(torch.float8_e4m3fn), torch.ones(e, n // 128, k // 128, device="cuda")
+        gemm = flux_amd.BlockScaleGemm(torch.float8_e4m3fn, torch.float8_e4m3fn, torch.bfloat16)
+        run = lambda counts: gemm.forward_grouped(qx, counts, qw, input_scale=sx, weight_scale=sw)
+    want = run(torch.tensor(fresh, dtype=torch.int32))
+    on_device = torch.tensor(fresh, dtype=torch.int32, device="cuda")
+    pinned = torch.empty(e, dtype=torch.int32, pin_memory=True)
+    pinned.copy_(torch.tensor(stale, dtype=torch.int32))
+    busy = torch.ones(8192, 8192, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(4):  # (about 40 ms on the stream)
+        torch.mm(busy, busy)
+    pinned.copy_(on_device, non_blocking=True)
+    got = run(pinned)
+    assert torch.equal(got, want)
+
+
 def test_blockscale_gemm_op_dense_and_grouped():
     """BlockScaleGemm.forward / forward_grouped / forward_multistream / reference (src/pybind/gemm_only.cc:77-160) fed by the Quantization op, the way
     test/python/gemm_only/test_blockwise_scale_gemm_only.py drives them: both scale layouts of forward_grouped."""
