@@ -584,7 +584,8 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
   } else {
     return PanelPlan{};
   }
-  if (most_items(p, dtype, 64, plan.chunk_rows, plan.any_splits, kMaxWeightGroups) > kMostItems) return PanelPlan{};
+  // Counted in the streaming form's narrowest columns and the most weight groups: where that form gives up the macro tiles run.
+  if (most_items(p, dtype, 32, plan.chunk_rows, plan.any_splits, kMaxWeightGroups) > kMostItems) return PanelPlan{};
   finish(p, dtype, cus, leave_cus, plan);
   return plan;
 }

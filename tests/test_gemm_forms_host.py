@@ -74,6 +74,7 @@ def test_a_launch_stays_below_the_grid_limit(dtype, k, block_scaled, groups):
         assert 1 <= info.stream_workgroups <= ((1 << 32) - 1) // (info.stream_waves * 64)
     assert capi.gemm_launch_info(dtype, 1024, 1024, 1 << 20, k, block_scaled=block_scaled).stream_workgroups == 256
     assert capi.gemm_launch_info(dtype, 1024, 1024, 1 << 24, k, block_scaled=block_scaled).form == capi.GEMM_MACRO_TILES
+    assert capi.gemm_launch_info(dtype, 1024, 1024, 1 << 24, k, block_scaled=block_scaled, panel=True).cols == 0
 
 
 @pytest.mark.parametrize("dtype", [BF16, F16, FP8])
