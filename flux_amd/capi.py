@@ -55,7 +55,7 @@ class GemmLaunchInfo(ctypes.Structure):
 
 
 class GemmPanelInfo(ctypes.Structure):
-    _fields_ = [(n, ctypes.c_int32) for n in ("cols", "chunk_rows", "workgroups", "lds_bytes", "macro_tiles_too", "computes")]
+    _fields_ = [(n, ctypes.c_int32) for n in ("cols", "chunk_rows", "workgroups", "lds_bytes", "macro_tiles_too", "computes", "sums")]
 
 
 def lib_path():
@@ -240,7 +240,7 @@ def grouped_gemm(a, b, splits, out=None, gather_a=None, scatter_d=None, alpha=No
     return out
 
 
-GEMM_GENERIC, GEMM_MACRO_TILES, GEMM_STREAM, GEMM_BY_SPLITS = 0, 1, 2, 3
+GEMM_GENERIC, GEMM_MACRO_TILES, GEMM_STREAM, GEMM_BY_SPLITS, GEMM_PANEL = range(5)
 
 
 def gemm_launch_info(dtype, nexperts, max_rows, n, k, ngroups=1, block_scaled=False, splits=None, cu_count=256, cu_margin=0,

@@ -1,6 +1,6 @@
 // Grouped GEMM entry point: argument checks, choice between the MFMA kernels and the generic kernel, and
 // the generic kernel itself.  The MFMA kernels are the macro tiles (grouped_gemm_kernel.hpp) and, for few rows per
-// expert, the streaming form (grouped_gemm_stream.hip).
+// expert, the panel tiles (grouped_gemm_panel.hip) and the streaming form (grouped_gemm_stream.hip).
 #include "grouped_gemm_panel.hpp"
 #include "grouped_gemm_stream.hpp"
 
@@ -242,7 +242,7 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   p.by_splits = 0;
   int cus = dry_run ? dry_run->cus : fluxmi_device_cu_count();
   FLUXMI_REQUIRE(cus > 0 || dry_run, FLUXMI_ERR_HIP, "grouped_gemm: cannot query the device");
-  // CUs left to other work of the caller (Flux's sm_margin): both MFMA forms launch fewer workgroups.
+  // CUs left to other work of the caller (Flux's sm_margin): every MFMA form launches fewer workgroups.
   cus = cus - args->cu_margin > 1 ? cus - args->cu_margin : 1;
   const bool leave_cus = args->cu_margin > 0;
   PanelPlan panel = {};
@@ -472,15 +472,14 @@ extern "C" int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *a
   DryRun dry;
   const int kind = describe_launch(args, ngroups, a_scale, cu_count, dry);
   if (kind < 0) return kind;
-  info->form = kind == 0 ? FLUXMI_GEMM_GENERIC : (!dry.stream ? FLUXMI_GEMM_MACRO_TILES : (args->max_rows > kStreamRows ? FLUXMI_GEMM_BY_SPLITS : FLUXMI_GEMM_STREAM));
-  if (info->form == FLUXMI_GEMM_BY_SPLITS && splits_host != nullptr)
-    info->form = few_chunks(args, splits_host, kStreamRows) ? FLUXMI_GEMM_STREAM : FLUXMI_GEMM_MACRO_TILES;
-  if (dry.stream && dry.panel.cols != 0) {
-    info->stream_cols = dry.panel.cols;
-    info->stream_waves = 4;
-    info->stream_workgroups = static_cast<int32_t>(dry.panel.workgroups);
-    info->stream_lds_bytes = dry.panel.lds_bytes;
-  } else if (dry.stream) {
+  const bool panel = dry.panel.cols != 0;
+  const int32_t few_rows_form = panel ? FLUXMI_GEMM_PANEL : FLUXMI_GEMM_STREAM;
+  if (kind == 0) info->form = FLUXMI_GEMM_GENERIC;
+  else if (!panel && !dry.stream) info->form = FLUXMI_GEMM_MACRO_TILES;
+  else if (!dry.macro) info->form = few_rows_form;
+  else if (splits_host == nullptr) info->form = FLUXMI_GEMM_BY_SPLITS;
+  else info->form = few_chunks(args, splits_host, panel ? dry.panel.chunk_rows : kStreamRows) ? few_rows_form : FLUXMI_GEMM_MACRO_TILES;
+  if (dry.stream && !panel) {
     info->stream_cols = dry.plan.cols;
     info->stream_waves = dry.plan.waves;
     info->stream_workgroups = static_cast<int32_t>(dry.plan.workgroups);
@@ -504,6 +503,7 @@ extern "C" int fluxmi_grouped_gemm_panel_info(const fluxmi_grouped_gemm_args *ar
   info->lds_bytes = dry.panel.lds_bytes;
   info->macro_tiles_too = dry.macro ? 1 : 0;
   info->computes = !dry.macro || (splits_host != nullptr && few_chunks(args, splits_host, dry.panel.chunk_rows)) ? 1 : 0;
+  info->sums = dry.panel.sums;
   return FLUXMI_OK;
 }
 

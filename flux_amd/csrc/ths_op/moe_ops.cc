@@ -76,7 +76,7 @@ float time_calls(F &&run) {
 // Times `run` (one whole forward) under every candidate schedule on the current stream, 5 warm-up and 10
 // timed calls each like the reference's profiling loops (gemm_grouped_v3_ag_scatter.cc:540-590), records
 // them in `ctx` and registers the fastest for `key`.  `args`: the launch that `run` makes; splits: its row counts on the host.  The
-// schedules are the macro tiles'; where the streaming form runs the launch they are all one, and only the default is timed.
+// schedules are the macro tiles'; where another form computes the launch they are all one, and only the default is timed.
 template <class F>
 void profile_schedules(const GemmShapeKey &key, ProfilingContext *ctx, const fluxmi_grouped_gemm_args &args, const torch::Tensor &splits,
                        F &&run) {
@@ -86,7 +86,7 @@ void profile_schedules(const GemmShapeKey &key, ProfilingContext *ctx, const flu
   for (const GemmLaunchTuning &cand : gemm_tuning_candidates()) {
     ScopedTuningOverride scope(&cand);
     ctx->add(key, cand, time_calls(run));
-    if (info.form == FLUXMI_GEMM_STREAM) break;
+    if (info.form == FLUXMI_GEMM_STREAM || info.form == FLUXMI_GEMM_PANEL) break;
   }
   TuningTable::instance().add(key, ctx->record_best(key));
 }

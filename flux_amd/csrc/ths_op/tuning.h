@@ -4,7 +4,7 @@
 // The reference's records pick one of its generated kernel variants; here a record picks the tile
 // schedule of the persistent macro-tile kernel (height of the raster groups, whether the last round is cut into
 // pieces, whether an expert's last row tile may run half height).  No choice changes a result bit.  Launches that the
-// streaming form computes (few rows per expert) have no such schedule: a record changes nothing there.
+// streaming form or the panel tiles compute (few rows per expert) have no such schedule: a record changes nothing there.
 #pragma once
 #include <cstdint>
 #include <map>

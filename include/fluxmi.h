@@ -114,7 +114,7 @@ int fluxmi_moe_gather_index(const int32_t *scatter_index, int32_t nrows, int32_t
  *   - N % 4 == 0; a, b 16-byte aligned; d 8-byte (bf16) / 16-byte (fp32) aligned; col_scale 16-byte aligned;
  *   - one expert's weights below 4 GiB (N * K * element size), and with `gather_a`: a_rows > 0 and the whole
  *     of A below 4 GiB (its rows are addressed with 32-bit byte offsets).
- * With few rows per expert it has a second form that streams the weights (fluxmi_grouped_gemm_launch_info).
+ * With few rows per expert it has other forms that read the weights at the memory's rate (fluxmi_grouped_gemm_launch_info).
  * Any other shape runs a generic kernel (one thread per output element, roughly 100 times slower, meant for
  * correctness only).  fluxmi_grouped_gemm_kernel_kind() tells which of the two a call would take.
  * ---------------------------------------------------------------------------------------------- */
@@ -138,7 +138,8 @@ typedef struct fluxmi_grouped_gemm_args {
   int32_t d_fp32;           /* 0: D is bf16 (fp16 for FLUXMI_FP16); 1: D is fp32 [max_rows, N] (unrounded layer1 intermediate) */
   const float *scalar_scale_dev; /* device [1] or NULL; multiplied in if given */
   /* Launch tuning; all zero = defaults.  None of them changes a result bit.  raster_rows and sched_flags steer the macro-tile
-   * kernel; launches that the streaming form computes (fluxmi_grouped_gemm_launch_info) take no notice of them. */
+   * kernel; launches that another form computes (fluxmi_grouped_gemm_launch_info: the streaming form, the panel tiles) take no notice
+   * of them, whether they are left out or force something. */
   int32_t cu_margin;     /* compute units left free for other work (Flux `sm_margin`) */
   int32_t raster_rows;   /* row tiles of an expert walked together over all weight panels; 0 = 8 */
   int32_t sched_flags;   /* FLUXMI_SCHED_* */
@@ -174,28 +175,30 @@ int fluxmi_grouped_gemm_host_splits(const fluxmi_grouped_gemm_args *args, const 
                                     const float *a_scale, int32_t a_scale_layout, const float *b_scale, int32_t b_scale_layout,
                                     void *stream);
 
-/* Which form of the MFMA kernels a launch takes and how the streaming form is launched.  Host only: nothing is
+/* Which form of the kernels computes a launch and how the streaming form is launched.  Host only: nothing is
  * launched, no device is needed, and pointers in `args` are only looked at for their alignment (b and d stand for every
  * weight group).  a_scale: non-NULL for fluxmi_grouped_gemm_blockscale with MFMA-kernel layouts.  splits_host: host copy of
  * args->splits, or NULL.  cu_count: compute units of the device asked about.  Returns FLUXMI_OK or the status the call
  * itself would return. */
 #define FLUXMI_GEMM_GENERIC 0
 #define FLUXMI_GEMM_MACRO_TILES 1
-#define FLUXMI_GEMM_STREAM 2    /* few rows per expert: weights streamed into MFMA registers */
-#define FLUXMI_GEMM_BY_SPLITS 3 /* 2 or 1, decided on the device from `splits`: 2 while few experts have more than 32 rows */
+#define FLUXMI_GEMM_STREAM 2    /* few rows per expert: weights streamed into MFMA registers, K split over waves */
+#define FLUXMI_GEMM_BY_SPLITS 3 /* splits_host was not given and `splits` decides on the device: the macro tiles, or while few experts have
+                                 * more rows than one work item holds, the panel tiles (where fluxmi_grouped_gemm_panel_info has cols
+                                 * != 0) or the streaming form */
+#define FLUXMI_GEMM_PANEL 4     /* up to about a hundred rows per expert: the panel tiles (fluxmi_grouped_gemm_panel_info) */
 typedef struct fluxmi_gemm_launch_info {
   int32_t form;              /* FLUXMI_GEMM_* */
-  int32_t stream_cols;       /* the streaming form: columns per workgroup, */
+  int32_t stream_cols;       /* the streaming form, where it is launched: columns per workgroup, */
   int32_t stream_waves;      /* waves per workgroup (K is split over them), */
   int32_t stream_workgroups; /* workgroups launched, */
-  int32_t stream_lds_bytes;  /* LDS per workgroup; all 0 for the other forms */
+  int32_t stream_lds_bytes;  /* LDS per workgroup; all 0 where it is not */
 } fluxmi_gemm_launch_info;
 int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
                                     const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_launch_info *info);
 
-/* The panel tiles: what launches of up to about 96 rows per expert run on where the streaming form above is not the one that
- * splits K over waves.  They compute FLUXMI_GEMM_STREAM launches with stream_waves == 4 and, with more rows per expert, launches
- * that fluxmi_grouped_gemm_launch_info calls FLUXMI_GEMM_MACRO_TILES; arguments as there. */
+/* How the panel tiles are launched: on up to about 96 rows per expert (192 where the weights are small), where the streaming form is not
+ * the faster one.  Arguments as for fluxmi_grouped_gemm_launch_info, whose form is FLUXMI_GEMM_PANEL where they compute the launch. */
 typedef struct fluxmi_gemm_panel_info {
   int32_t cols;            /* columns per workgroup; 0 (and everything else 0): not for these tiles */
   int32_t chunk_rows;      /* most rows of a work item; an expert with more is several */
@@ -203,6 +206,8 @@ typedef struct fluxmi_gemm_panel_info {
   int32_t lds_bytes;       /* LDS per workgroup */
   int32_t macro_tiles_too; /* 1: the macro tiles are launched as well and the splits decide on the device which of the two computes */
   int32_t computes;        /* 1: these tiles compute the launch (with macro_tiles_too: for splits_host; 0 without it) */
+  int32_t sums;            /* partial sums over K that make up a result, line l of 128 bytes in sum l % sums: 4 or 8, with the bits of the
+                            * streaming form that splits K over as many waves, or 1, with those of the macro tiles (16-bit operands) */
 } fluxmi_gemm_panel_info;
 int fluxmi_grouped_gemm_panel_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
                                    const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_panel_info *info);

@@ -1,4 +1,4 @@
-"""Which form of the MFMA kernels a grouped GEMM takes, and how the streaming form is launched (host code only, no GPU)."""
+"""Which form of the MFMA kernels a grouped GEMM takes, and how those for few rows per expert are launched (host code only, no GPU)."""
 import pytest
 import torch
 
@@ -9,12 +9,20 @@ BF16, F16, FP8 = torch.bfloat16, torch.float16, torch.float8_e4m3fn
 
 @pytest.mark.parametrize("dtype,block_scaled,line", [(BF16, False, 32), (F16, False, 32), (FP8, False, 24), (FP8, True, 24)])
 def test_form_by_rows(dtype, block_scaled, line):
+    k = 4096 if dtype == FP8 else 2048  # rows of 4 KiB and many columns: the streaming form's up to 16 rows per expert
+
     def form(rows, splits=None):
-        return capi.gemm_launch_info(dtype, 8, rows, 4096, 1024, block_scaled=block_scaled, splits=splits).form
+        return capi.gemm_launch_info(dtype, 8, rows, 16384, k, block_scaled=block_scaled, splits=splits).form
+
+    def panel(rows):
+        return capi.gemm_launch_info(dtype, 8, rows, 16384, k, block_scaled=block_scaled, panel=True)
 
     assert form(1) == form(32) == capi.GEMM_STREAM  # no expert can have more than one chunk of 32 rows
-    assert form(33) == form(8 * line) == capi.GEMM_BY_SPLITS
-    assert form(8 * line + 1) == form(100000) == capi.GEMM_MACRO_TILES
+    assert form(33) == form(128) == capi.GEMM_BY_SPLITS and panel(33).cols == panel(128).cols == 0
+    assert form(129) == form(768) == capi.GEMM_BY_SPLITS and panel(129).cols > 0 and panel(768).cols > 0
+    assert form(769) == form(100000) == capi.GEMM_MACRO_TILES
+    # up to `line` rows per expert both forms for few rows take a launch, with the same sums over K
+    assert [panel(rows).sums for rows in (129, 8 * line, 8 * line + 1, 768)] == [4, 4, 1, 1]
     # under 16 experts with rows: one chunk each
     assert form(80, [32, 0, 10, 0, 0, 30, 8, 0]) == capi.GEMM_STREAM
     assert form(80, [33, 0, 10, 0, 0, 29, 8, 0]) == capi.GEMM_MACRO_TILES
@@ -24,11 +32,31 @@ def test_form_by_rows(dtype, block_scaled, line):
 
     # from 16 on a quarter more chunks of 32 rows than experts with rows
     def form_of(splits):
-        return capi.gemm_launch_info(dtype, len(splits), 200, 4096, 1024, block_scaled=block_scaled, splits=splits).form
+        return capi.gemm_launch_info(dtype, len(splits), 200, 16384, k, block_scaled=block_scaled, splits=splits).form
 
     assert form_of([33] * 4 + [0] * 5 + [3] * 12) == form_of([129] + [0] * 5 + [3] * 15) == capi.GEMM_STREAM
     assert form_of([33] * 5 + [0] * 5 + [2] * 11) == form_of([129, 33] + [0] * 5 + [2] * 14) == capi.GEMM_MACRO_TILES
     assert form_of([33] + [0] * 5 + [3] * 14) == capi.GEMM_MACRO_TILES  # 15 experts with rows
+
+
+@pytest.mark.parametrize("dtype,splits,n,k,form,without", [
+    (BF16, [0, 0, 0, 240, 0, 0, 0, 0], 1024, 2048, capi.GEMM_PANEL, capi.GEMM_PANEL),  # small weights: whatever the splits
+    (BF16, [60] * 4 + [0] * 4, 14336, 4096, capi.GEMM_PANEL, capi.GEMM_BY_SPLITS),
+    (BF16, [40, 40, 20, 20, 10, 10, 10, 10], 14336, 4096, capi.GEMM_PANEL, capi.GEMM_BY_SPLITS),
+    (F16, [100] + [20] * 7, 14336, 4096, capi.GEMM_PANEL, capi.GEMM_BY_SPLITS),
+    (F16, [240] + [0] * 7, 14336, 4096, capi.GEMM_MACRO_TILES, capi.GEMM_BY_SPLITS),
+    (FP8, [66, 66] + [13] * 14, 4096, 4096, capi.GEMM_MACRO_TILES, capi.GEMM_BY_SPLITS),
+    (FP8, [66] + [13] * 15, 4096, 4096, capi.GEMM_PANEL, capi.GEMM_BY_SPLITS),
+    (BF16, [129] + [90] * 7, 14336, 4096, capi.GEMM_PANEL, capi.GEMM_BY_SPLITS),
+    (BF16, [400] + [50] * 7, 14336, 4096, capi.GEMM_MACRO_TILES, capi.GEMM_BY_SPLITS),
+    (BF16, [120] * 8, 14336, 4096, capi.GEMM_MACRO_TILES, capi.GEMM_MACRO_TILES)])
+def test_form_is_that_of_the_kernel_that_computes(dtype, splits, n, k, form, without):
+    info = capi.gemm_launch_info(dtype, len(splits), sum(splits), n, k, splits=splits)
+    panel = capi.gemm_launch_info(dtype, len(splits), sum(splits), n, k, splits=splits, panel=True)
+    assert info.form == form and panel.computes == (form == capi.GEMM_PANEL)
+    assert capi.gemm_launch_info(dtype, len(splits), sum(splits), n, k).form == without
+    assert (panel.cols > 0) == (form == capi.GEMM_PANEL or without == capi.GEMM_BY_SPLITS)
+    assert (info.stream_cols, info.stream_waves, info.stream_workgroups, info.stream_lds_bytes) == (0, 0, 0, 0)
 
 
 def test_generic_shapes_have_no_streaming_form():
@@ -40,13 +68,16 @@ def test_generic_shapes_have_no_streaming_form():
 
 
 @pytest.mark.parametrize("dtype", [BF16, F16, FP8])
-@pytest.mark.parametrize("experts,rows,n,k", [(8, 74, 2048, 4096), (8, 20, 2048, 8192), (64, 90, 400, 8192), (1, 8, 16384, 8192), (16, 200, 1408, 2048)])
+@pytest.mark.parametrize("experts,rows,n,k", [(8, 74, 2048, 4096), (8, 20, 2048, 8192), (64, 90, 400, 8192), (1, 8, 16384, 8192), (16, 200, 1408, 2048),
+                                              (64, 576, 1408, 2048), (64, 576, 1408, 4096), (32, 256, 2048, 2048), (64, 1500, 1408, 2048)])
 def test_weight_groups_do_not_change_how_k_is_split(dtype, experts, rows, n, k):
-    """A launch of several weight groups adds K up in the order of a launch per group: the same number of waves."""
-    alone = capi.gemm_launch_info(dtype, experts, rows, n, k)
-    for groups in (2, 3, 4):
-        together = capi.gemm_launch_info(dtype, experts, rows, n, k, ngroups=groups)
-        assert (together.form, together.stream_waves) == (alone.form, alone.stream_waves)
+    """A launch of several weight groups adds K up in the order of a launch per group: as many waves, or sums of the panel tiles, and the
+    same choice between these forms and the macro tiles."""
+    def split(groups):
+        info, panel = (capi.gemm_launch_info(dtype, experts, rows, n, k, ngroups=groups, panel=p) for p in (False, True))
+        return (panel.sums if panel.cols else info.stream_waves, info.form == capi.GEMM_BY_SPLITS, panel.chunk_rows if panel.cols else 32)
+
+    assert split(2) == split(3) == split(4) == split(1)
 
 
 @pytest.mark.parametrize("dtype,block_scaled", [(BF16, False), (FP8, False), (FP8, True)])
@@ -55,11 +86,16 @@ def test_weight_groups_do_not_change_how_k_is_split(dtype, experts, rows, n, k):
 def test_margin_leaves_whole_compute_units(dtype, block_scaled, experts, rows, n, k, margin):
     """With a margin every workgroup has a compute unit for itself (more than half of its 160 KiB of LDS), and there are no more
     of them than units that may be used."""
-    info = capi.gemm_launch_info(dtype, experts, rows, n, k, block_scaled=block_scaled, cu_margin=margin)
-    assert 80 * 1024 < info.stream_lds_bytes <= 160 * 1024
-    assert 1 <= info.stream_workgroups <= max(1, 256 - margin)
-    free = capi.gemm_launch_info(dtype, experts, rows, n, k, block_scaled=block_scaled)
-    assert (free.form, free.stream_cols, free.stream_waves) == (info.form, info.stream_cols, info.stream_waves)  # same bits
+    def launch(margin):
+        info, panel = (capi.gemm_launch_info(dtype, experts, rows, n, k, block_scaled=block_scaled, cu_margin=margin, panel=p) for p in (False, True))
+        if panel.cols > 0:
+            return panel.workgroups, panel.lds_bytes, (info.form, panel.cols, panel.sums)
+        return info.stream_workgroups, info.stream_lds_bytes, (info.form, info.stream_cols, info.stream_waves)
+
+    workgroups, lds_bytes, form = launch(margin)
+    assert 80 * 1024 < lds_bytes <= 160 * 1024
+    assert 1 <= workgroups <= max(1, 256 - margin)
+    assert launch(0)[2] == form  # same bits
 
 
 @pytest.mark.parametrize("dtype,k,block_scaled", [(BF16, 8, False), (FP8, 16, False), (FP8, 128, True)])

@@ -2,7 +2,8 @@
 
 Operands are small integers, so every product and every partial sum is a whole number below 2^24 and the fp32 result is the
 same in any order of summation: the outputs have to equal an int64 matmul exactly, no tolerance.  The form computes launches
-of up to 24 (fp8) or 32 rows per expert on average in which few experts have more than 32 rows; `gemm_launch_info` tells."""
+of few rows per expert, up to four on average or where the panel tiles are not the faster ones, in which few experts have more than 32
+rows; `gemm_launch_info` tells, and each test asks it."""
 import ctypes
 
 import pytest
@@ -28,13 +29,29 @@ def expected(a, w, splits, rows_of=None):
     return out
 
 
+def sparse(splits):
+    """As many experts without rows as make it four rows per expert on average, which no other form for few rows takes."""
+    return splits + [0] * ((sum(splits) + 3) // 4 - len(splits))
+
+
+def streams(dtype, splits, n, k, block_scaled=False, **kw):
+    """The launch's description; no panel tiles, and the streaming form computes it unless too many experts have more than 32 rows."""
+    about = dict(block_scaled=block_scaled, **kw)
+    assert capi.gemm_launch_info(DT[dtype], len(splits), sum(splits), n, k, panel=True, **about).cols == 0
+    info = capi.gemm_launch_info(DT[dtype], len(splits), sum(splits), n, k, splits=splits, **about)
+    active, chunks = sum(r > 0 for r in splits), sum((r + 31) // 32 for r in splits)
+    few = chunks <= active + (active // 4 if active >= 16 else 0)
+    assert info.form == (capi.GEMM_STREAM if few else capi.GEMM_MACRO_TILES) and info.stream_cols in (32, 64)
+    return info
+
+
 # (splits, N, K), all of them on 32-column tiles: one row; 15, 16 and 17 rows; empty experts and more than 64 of them; column tiles
 # cut off at 4 columns; K shorter than a line, ending inside one, and over many lines per wave (eight waves).  The macro tiles
 # compute the cases with an expert of more than 32 rows: same results where the two forms meet.
 CASES = [
-    ([1], 4, 16), ([1, 0, 2], 64, 128), ([15, 16, 17], 100, 272), ([33, 0, 64, 65, 2], 132, 1040),
+    ([1], 4, 16), ([1, 0, 2], 64, 128), (sparse([15, 16, 17]), 100, 272), (sparse([33, 0, 64, 65, 2]), 132, 1040),
     ([0] * 70 + [3, 1] + [0] * 8 + [9], 68, 400), ([7, 5], 1028, 8192 + 48), ([2, 3, 1, 4, 2, 0, 1, 5], 4224, 2064),
-    ([40, 1, 22, 30], 704, 176),
+    (sparse([40, 1, 22, 30]), 704, 176),
 ]
 
 
@@ -42,6 +59,7 @@ CASES = [
 @pytest.mark.parametrize("splits,n,k", CASES)
 def test_stream_form_is_exact_on_integers(dtype, splits, n, k):
     print(f"[case] stream gemm {dtype} splits={splits[:6]} n={n} k={k}", flush=True)
+    assert streams(dtype, splits, n, k).stream_cols == 32
     g = torch.Generator().manual_seed(n + k)
     m, e = sum(splits), len(splits)
     a, w = small_ints(g, m, k), small_ints(g, e, n, k)
@@ -67,11 +85,12 @@ def test_stream_form_is_exact_on_integers(dtype, splits, n, k):
     assert torch.equal(two[1].cpu().long(), expected(a, w.flip(0) if dtype != "fp8" else w, splits))
 
 
-@pytest.mark.parametrize("splits,n,k", [([1], 128, 128), ([16, 0, 17, 2], 256, 384), ([33, 31, 5], 384, 2048), ([2, 1], 132, 8192)])
+@pytest.mark.parametrize("splits,n,k", [([1], 128, 128), (sparse([16, 0, 17, 2]), 256, 384), (sparse([33, 31, 5]), 384, 2048), ([2, 1], 132, 8192)])
 @pytest.mark.parametrize("a_layout", [capi.ASCALE_BLOCK128, capi.ASCALE_EXPERT_K_M])
 @pytest.mark.parametrize("b_layout", [capi.BSCALE_N_K, capi.BSCALE_K_N])
 def test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b_layout):
     print(f"[case] stream gemm block-scaled splits={splits} n={n} k={k} layouts {a_layout} {b_layout}", flush=True)
+    streams("fp8", splits, n, k, block_scaled=True)
     g = torch.Generator().manual_seed(n + k)
     m, e, kb, nb = sum(splits), len(splits), k // 128, (n + 127) // 128
     a, w = small_ints(g, m, k), small_ints(g, e, n, k)
@@ -99,27 +118,51 @@ def test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b
         at += r
 
 
-# The 64-column form: more than four rows per expert on average (block-scaled: any) and at least 512 column tiles in all.  One block
-# and two blocks of 16 rows, rows that do not fill them, experts of several chunks of 32 rows; columns cut off at 4; K that ends inside a line and numbers of lines that
-# four waves with two lines in flight do not divide; more than 64 experts.
-WIDE = [([32, 0, 31, 17, 16, 1, 2, 9], 4164, 272), ([32, 32, 32, 32, 5, 0, 31, 20], 4096, 1040), ([17] * 70 + [0, 32, 1], 516, 2064 + 16),
-        ([65, 7, 9, 5, 3, 30, 1, 8, 2, 64, 17] + [2] * 8, 2052, 400), ([3] * 66 + [70, 33, 0, 96], 580, 272)]
+# The 64-column form: more than four rows per expert on average (block-scaled: any), at least 512 column tiles in all, and rows of 4 KiB in
+# at least 1024 tiles of 128 columns or too few columns for the panel tiles.  One block and two blocks of 16 rows, rows that do not fill
+# them, experts of several chunks of 32 rows; columns cut off at 4; K that ends inside a line and numbers of lines that four waves with
+# two lines in flight do not divide; more than 64 experts.  (splits, N, bytes of K)
+WIDE = [([32, 0, 31, 17, 16, 1, 2, 9] * 8, 2052, 4096), (([65, 7, 9, 5, 3, 30, 1, 8, 2, 64, 17] + [2] * 8) * 4, 1732, 4096),
+        ([32, 0, 31, 17, 16, 1, 2, 9, 5, 20] * 52, 60, 544), ([16, 0, 31, 17, 16, 1, 2, 9, 5, 33] * 52, 60, 4112)]
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
-@pytest.mark.parametrize("splits,n,k", WIDE)
-def test_stream_form_64_columns(dtype, splits, n, k):
-    info = capi.gemm_launch_info(DT[dtype], len(splits), sum(splits), n, k, splits=splits)
-    assert (info.form, info.stream_cols) == (capi.GEMM_STREAM, 64)
-    test_stream_form_is_exact_on_integers(dtype, splits, n, k)
+@pytest.mark.parametrize("splits,n,kbytes", WIDE)
+def test_stream_form_64_columns(dtype, splits, n, kbytes):
+    k = kbytes // (1 if dtype == "fp8" else 2)
+    print(f"[case] stream gemm, 64 columns {dtype} splits={splits[:6]} n={n} k={k}", flush=True)
+    info = streams(dtype, splits, n, k)
+    assert (info.form, info.stream_cols, info.stream_waves) == (capi.GEMM_STREAM, 64, 4)
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    m, e = sum(splits), len(splits)
+    a = torch.randint(-3, 4, (m, k), generator=g, device="cuda").float().to(DT[dtype])
+    w = torch.randint(-3, 4, (e, n, k), generator=g, device="cuda", dtype=torch.int8).float().to(DT[dtype])
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    perm = torch.randperm(m, generator=g, device="cuda").to(torch.int32)
+    ends = torch.tensor(splits).cumsum(0).tolist()
+
+    def product(a, reverse=False):
+        rows = [(end - r, end, i) for r, end, i in zip(splits, ends, range(e)) if r > 0]
+        return torch.cat([a[lo:hi].double() @ w[e - 1 - i if reverse else i].double().t().contiguous() for lo, hi, i in rows])
+
+    want = product(a)
+    assert torch.equal(capi.grouped_gemm(a, w, sp, out_dtype=torch.float32).double(), want)
+    row_scale = 2.0 ** torch.randint(-1, 2, (m,), generator=g, device="cuda").float()
+    picked = product(a[perm.long()]) * row_scale.double()[:, None]
+    for margin in (0, 40, 1000):
+        out = torch.full((m, n), -7.0, device="cuda")
+        capi.grouped_gemm(a, w, sp, out=out, gather_a=perm, scatter_d=perm, row_scale=row_scale, cu_margin=margin)
+        assert torch.equal(out[perm.long()].double(), picked), f"margin {margin}"
+    two = capi.grouped_gemm_multi(a, [w, w.view(torch.uint8).flip(0).contiguous().view(w.dtype)], sp, out_dtype=torch.float32)
+    assert torch.equal(two[0].double(), want) and torch.equal(two[1].double(), product(a, reverse=True))
 
 
-@pytest.mark.parametrize("splits,n,k", [([32, 0, 31, 17, 16, 1, 2, 9], 4160, 384), ([3] * 70 + [0, 32, 1], 516, 1152),
+@pytest.mark.parametrize("splits,n,k", [([32, 0, 31, 17, 16, 1, 2, 9], 4164, 384), ([3] * 70 + [0, 32, 1], 516, 1152),
                                         ([65, 7, 9, 5, 3, 30, 1, 8, 2, 64, 17] + [2] * 8, 2052, 384), ([3] * 66 + [70, 33, 0, 96], 580, 256)])
 @pytest.mark.parametrize("a_layout", [capi.ASCALE_BLOCK128, capi.ASCALE_EXPERT_K_M])
 @pytest.mark.parametrize("b_layout", [capi.BSCALE_N_K, capi.BSCALE_K_N])
 def test_stream_form_64_columns_block_scaled(splits, n, k, a_layout, b_layout):
-    info = capi.gemm_launch_info(DT["fp8"], len(splits), sum(splits), n, k, splits=splits, block_scaled=True)
+    info = streams("fp8", splits, n, k, block_scaled=True)
     assert (info.form, info.stream_cols) == (capi.GEMM_STREAM, 64)
     test_stream_form_block_scaled_is_exact_on_integers(splits, n, k, a_layout, b_layout)
 
@@ -131,8 +174,10 @@ def test_stream_form_64_columns_block_scaled(splits, n, k, a_layout, b_layout):
 def test_one_form_computes_a_launch(dtype, splits, form):
     """Which form runs is decided on the device; every result is computed, and added to a sum, exactly once."""
     print(f"[case] form by splits {dtype} {splits[-6:]}", flush=True)
+    splits = sparse(splits)
     n, k, m, e = 260, 272, sum(splits), len(splits)
-    assert capi.gemm_launch_info(DT[dtype], e, m, n, k, splits=splits).form == form
+    assert streams(dtype, splits, n, k).form == form
+    assert capi.gemm_launch_info(DT[dtype], e, m, n, k).form == (capi.GEMM_BY_SPLITS if m > 32 else capi.GEMM_STREAM)
     g = torch.Generator().manual_seed(m)
     a, w = small_ints(g, m, k), small_ints(g, e, n, k)
     ad, wd = a.float().to(DT[dtype]).cuda(), w.float().to(DT[dtype]).cuda()
@@ -149,15 +194,16 @@ def test_form_follows_the_splits_of_each_replay():
     """A captured launch holds both forms; every replay runs the one that its row counts ask for, as an eager call does."""
     g = torch.Generator().manual_seed(7)
     x = torch.randn(90, 400, generator=g).to(torch.bfloat16).cuda()
-    w = (torch.randn(6, 516, 400, generator=g) * 0.05).to(torch.bfloat16).cuda()
-    sp, out = torch.zeros(6, dtype=torch.int32, device="cuda"), torch.zeros(90, 516, device="cuda")
+    w = (torch.randn(24, 516, 400, generator=g) * 0.05).to(torch.bfloat16).cuda()
+    sp, out = torch.zeros(24, dtype=torch.int32, device="cuda"), torch.zeros(90, 516, device="cuda")
     capi.grouped_gemm(x, w, sp, out=out)
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         capi.grouped_gemm(x, w, sp, out=out)
     for splits in ([32, 0, 8, 20, 30, 0], [33, 0, 7, 20, 30, 0], [15] * 6, [0, 0, 90, 0, 0, 0], [32, 0, 8, 20, 30, 0]):
-        sp.copy_(torch.tensor(splits, dtype=torch.int32))
+        streams("bf16", splits + [0] * 18, 516, 400)
+        sp[:6].copy_(torch.tensor(splits, dtype=torch.int32))
         want = capi.grouped_gemm(x, w, sp, out_dtype=torch.float32)
         out.fill_(-1)
         graph.replay()
@@ -181,12 +227,13 @@ def test_stream_form_weight_groups_have_the_bits_of_one_launch_each(dtype, split
 
 
 @pytest.mark.parametrize("kblocks,rows,n,experts", [(1, 3, 128, 1), (3, 3, 128, 1), (7, 3, 256, 2), (8, 3, 128, 1), (9, 3, 128, 1),
-                                                    (65, 3, 128, 1), (3, 7, 2176, 24), (9, 7, 2176, 24)])
+                                                    (65, 3, 128, 1), (3, 4, 2176, 24), (9, 4, 2176, 24)])
 def test_stream_form_block_scaled_infinite_scales(kblocks, rows, n, experts):
     """An infinite product of scales (each of them finite, or one infinite) makes a result infinite, not NaN, whatever K is
     padded to inside the kernel.  Codes 1 ... 3, so every block's sum is positive; fp32 results, exact integers or +inf."""
     print(f"[case] stream gemm infinite scales kblocks={kblocks} rows={rows} n={n} experts={experts}", flush=True)
     k, m = kblocks * 128, rows * experts
+    streams("fp8", [rows] * experts, n, k, block_scaled=True)
     g = torch.Generator().manual_seed(kblocks)
     a, w = torch.randint(1, 4, (m, k), generator=g), torch.randint(1, 4, (experts, n, k), generator=g)
     sa, sb = torch.ones(m, kblocks), torch.ones(experts, n // 128, kblocks)
@@ -210,7 +257,7 @@ def test_stream_form_block_scaled_infinite_scales(kblocks, rows, n, experts):
 @pytest.mark.parametrize("margin", [1, 100, 255, 1000])
 @pytest.mark.parametrize("splits,n,k", [([2, 3, 1, 4, 2, 0, 1, 5], 4224, 2064), ([33, 0, 64, 65, 2], 4096, 528), ([1] * 80, 1028, 400)])
 def test_stream_form_leaves_compute_units_and_changes_no_bit(splits, n, k, margin):
-    """With `cu_margin` few workgroups walk all items (down to one workgroup); the second case is the macro tiles'."""
+    """With `cu_margin` few workgroups walk all items (down to one workgroup); the second case is the panel tiles'."""
     print(f"[case] stream gemm margin={margin} splits={splits[:6]} n={n} k={k}", flush=True)
     g = torch.Generator().manual_seed(n + k)
     a = torch.randn(sum(splits), k, generator=g).to(torch.bfloat16).cuda()

@@ -269,7 +269,7 @@ def test_profiling_registers_a_schedule_and_keeps_results(c1):
     rec = ctx.get_latest_record()
     assert f"experts={e} n={f} k={h} rows={t * k} groups=1" in rec.shape
     assert rec.raster_rows in (4, 8, 16) and rec.sched_flags in (0, 1, 2, 3, 4, 8, 16, 32)
-    assert ctx.get_latest_prof_result().count("TopK=") == 5
+    assert ctx.get_latest_prof_result().count("TopK=") == 1  # the panel tiles compute this launch: no schedule to choose
     assert torch.equal(op0.forward(x, w1, splits_gpu, scatter_index), ref0)  # now under the registered schedule
 
     op1 = flux_amd.GemmGroupedV3GatherRS(e, t * k, h, k, 0, 1, 1, 1)
@@ -301,10 +301,11 @@ def test_profiling_registers_a_schedule_and_keeps_results(c1):
     m.clear_tuning_records()
 
 
-@pytest.mark.parametrize("cnt,timed", [([9, 0, 30, 32, 5, 1, 0, 3], 1), ([0, 0, 40, 35, 2, 1, 0, 2], 5)])
+@pytest.mark.parametrize("cnt,timed", [([2, 0, 30, 0, 0, 0, 0, 0], 1), ([9, 0, 30, 32, 5, 1, 0, 3], 1), ([0, 0, 40, 35, 2, 1, 0, 2], 1),
+                                       ([300, 200, 0, 500, 400, 180, 100, 36], 5)])
 def test_profiling_times_one_schedule_where_none_has_an_effect(cnt, timed):
-    """With few rows in every expert the streaming form computes the launch, whatever the schedule; with several experts of more
-    than 32 rows the macro tiles do, and all schedules are timed."""
+    """With few rows per expert the streaming form or the panel tiles compute the launch, whatever the schedule; with more the macro
+    tiles do, and all schedules are timed."""
     m = flux_amd.flux_ths_pybind
     m.clear_tuning_records()
     g = torch.Generator().manual_seed(3)
