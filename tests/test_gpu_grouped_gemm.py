@@ -482,7 +482,7 @@ def test_skinny_tail_pieces_same_bits_as_in_place(dtype, ksteps):
     k = ksteps * 64 // elt
     print(f"[case] grouped_gemm {dtype} skinny tail pieces K={k} ({ksteps} k-steps)", flush=True)
     g = torch.Generator().manual_seed(100 + ksteps)
-    split = np.array([300, 30, 257, 64, 65, 1, 0, 513, 256], dtype=np.int32)  # skinny: 300, 30, 257, 64, 1, 513
+    split = np.array([300, 30, 257, 64, 65, 1, 0, 513, 512], dtype=np.int32)  # skinny: 300, 30, 257, 64, 1, 513
     rows, n = int(split.sum()), 328
     src_rows = rows + 37
     gi = torch.randint(0, src_rows, (rows,), generator=g, dtype=torch.int32)
@@ -492,6 +492,7 @@ def test_skinny_tail_pieces_same_bits_as_in_place(dtype, ksteps):
     else:
         a = torch.randn(src_rows, k, generator=g).to(torch.float8_e4m3fn)
         w = (torch.randn(len(split), n, k, generator=g) * 0.25).to(torch.float8_e4m3fn)
+    assert capi.gemm_launch_info(a.dtype, len(split), rows, n, k).form == capi.GEMM_MACRO_TILES
     rs = torch.rand(rows, generator=g) + 0.5
     cs = torch.rand(len(split), n, generator=g) + 0.5
     ref = layers.grouped_gemm_fp32(a.float()[gi.long()], w.float(), split, row_scale=rs, col_scale=cs)
