@@ -35,6 +35,9 @@ CASES = [
     ("128 columns, 128 rows", spread(1, 128, 24, 3), 1412, 1040, 128, 128),
     ("64 columns, 128 rows", [32, 33, 64, 65, 96, 97, 128, 0], 1092, 8192 + 16, 64, 128),
 ]
+# In none of these K is whole lines of 128 bytes; in the same ones with K cut to a multiple of 128 (one line at least) it is, in every type, and
+# the weights' loads are the non-temporal ones.
+LINES = [(name + ", whole lines", splits, n, max(128, k // 128 * 128), cols, chunk) for name, splits, n, k, cols, chunk in CASES]
 
 
 def made(splits, n, k, dtype, seed):
@@ -54,13 +57,13 @@ def product(a, w, splits):
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
-@pytest.mark.parametrize("name,splits,n,k,cols,chunk", CASES, ids=[c[0] for c in CASES])
+@pytest.mark.parametrize("name,splits,n,k,cols,chunk", CASES + LINES, ids=[c[0] for c in CASES + LINES])
 def test_panel_tiles_are_exact_on_integers(name, splits, n, k, cols, chunk, dtype):
     print(f"[case] panel gemm {dtype} {name} n={n} k={k}", flush=True)
+    assert (k * DT[dtype].itemsize % 128 == 0) == name.endswith("whole lines")
     m, e = sum(splits), len(splits)
     info = capi.gemm_launch_info(DT[dtype], e, m, n, k, splits=splits, panel=True)
-    if dtype != "fp8" or name != "64 columns, 128 rows":  # (fp8: half the bytes, so the small launches' 64 rows)
-        assert (info.cols, info.chunk_rows, info.computes) == (cols, chunk, 1)
+    assert (info.cols, info.chunk_rows, info.computes) == (cols, chunk, 1)
     a, w, sp, g = made(splits, n, k, dtype, n + k)
     ad, wd = a.to(DT[dtype]), w.to(DT[dtype])
     assert torch.equal(capi.grouped_gemm(ad, wd, sp, out_dtype=torch.float32).double(), product(a, w, splits))
@@ -163,7 +166,7 @@ def test_panel_tiles_infinite_scales(kblocks, rows, n, experts):
     assert torch.equal(torch.isinf(got) & (got > 0), inf.view(m, n))
 
 
-MORE_ROWS = [c for c in CASES if sum(c[1]) > 32 * len(c[1])]  # (with fewer rows they have the streaming form's bits, below)
+MORE_ROWS = [c for c in CASES + LINES if sum(c[1]) > 32 * len(c[1])]  # (with fewer rows they have the streaming form's bits, below)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
@@ -194,6 +197,7 @@ FEW_ROWS = [
     ("64 columns, 64 rows, eight sums, small", [20, 24, 28, 18], 192, 16416, 64, 64, 8),
     ("64 columns, 64 rows, eight sums", [20, 24, 28, 18], 4096, 16416, 64, 64, 8),
 ]
+FEW_ROWS += [(name + ", whole lines", splits, n, kbytes // 128 * 128, *form) for name, splits, n, kbytes, *form in FEW_ROWS]
 
 
 def random_operands(splits, n, k, dtype, groups=1):
@@ -254,11 +258,13 @@ def test_few_rows_several_weight_groups_have_the_bits_of_one_launch_each(dtype, 
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
-@pytest.mark.parametrize("name,splits,n,k,cols,chunk", CASES, ids=[c[0] for c in CASES])
+@pytest.mark.parametrize("name,splits,n,k,cols,chunk", LINES, ids=[c[0] for c in LINES])
 def test_panel_tiles_same_bits_where_weights_do_not_start_on_lines(name, splits, n, k, cols, chunk, dtype):
     """The cache policy of the weights' loads follows their alignment to 128 bytes; results do not."""
+    print(f"[case] panel gemm, weights off a line {dtype} {name} n={n} k={k}", flush=True)
     a, w, sp, _ = made(splits, n, k, dtype, n + k)
     ad, wd = a.to(DT[dtype]), w.to(DT[dtype])
+    assert k * wd.element_size() % 128 == 0 and wd.data_ptr() % 128 == 0
     raw = wd.view(torch.uint8).reshape(-1)
     store = torch.empty(raw.numel() + 128, dtype=torch.uint8, device="cuda")
     store[16:16 + raw.numel()] = raw
