@@ -43,11 +43,13 @@ def test_fp16_grouped_gemm_against_oracle(experts, rows, n, k, seed):
     assert float((out32.cpu() - ref).abs().max()) < 0.1 * float((wrong - ref).abs().max())
 
 
-def test_fp16_gather_scatter_scales_and_weight_groups():
+@pytest.mark.parametrize("tokens,form", [(300, "GEMM_PANEL"), (500, "GEMM_MACRO_TILES")])
+def test_fp16_gather_scatter_scales_and_weight_groups(tokens, form):
     from flux_amd import capi
     rng = np.random.default_rng(31)
     g = torch.Generator().manual_seed(31)
-    tokens, topk, experts, h, n = 300, 3, 6, 256, 520
+    topk, experts, h, n = 3, 6, 256, 520
+    assert capi.gemm_launch_info(torch.float16, experts, tokens * topk, n, h).form == getattr(capi, form)
     choosed = np.stack([rng.permutation(experts)[:topk] for _ in range(tokens)]).astype(np.int32)
     split = routing.splits(choosed, experts)
     si = routing.scatter_index_stable(choosed, experts)

@@ -52,11 +52,13 @@ def test_bf16_plain_against_oracle(experts, rows, n, k, seed, empty):
     assert_close(out, ref, "plain")
 
 
-def test_bf16_gather_scatter_and_scales():
+@pytest.mark.parametrize("tokens,form", [(300, "GEMM_PANEL"), (500, "GEMM_MACRO_TILES")])
+def test_bf16_gather_scatter_and_scales(tokens, form):
     from flux_amd import capi
     rng = np.random.default_rng(21)
     g = torch.Generator().manual_seed(21)
-    tokens, topk, experts, h, n = 300, 3, 6, 256, 520
+    topk, experts, h, n = 3, 6, 256, 520
+    assert capi.gemm_launch_info(torch.bfloat16, experts, tokens * topk, n, h).form == getattr(capi, form)
     choosed = np.stack([rng.permutation(experts)[:topk] for _ in range(tokens)]).astype(np.int32)
     split = routing.splits(choosed, experts)
     si = routing.scatter_index_stable(choosed, experts)
@@ -165,12 +167,14 @@ def test_k_not_a_multiple_of_the_k_step_runs_the_mfma_kernel(dtype, k):
         assert_close(out, ref, f"K={k}")
 
 
-def test_partial_k_step_with_gather_and_last_row_nan_guard():
+@pytest.mark.parametrize("tokens,form", [(200, "GEMM_PANEL"), (400, "GEMM_MACRO_TILES")])
+def test_partial_k_step_with_gather_and_last_row_nan_guard(tokens, form):
     """The partial k-step together with a row gather: the last row of A ends the allocation's payload, and the
     rows are followed by NaN patterns that zero padding must never multiply in."""
     from flux_amd import capi
     g = torch.Generator().manual_seed(5)
-    tokens, topk, experts, k, n = 200, 2, 3, 1000, 264
+    topk, experts, k, n = 2, 3, 1000, 264
+    assert capi.gemm_launch_info(torch.bfloat16, experts, tokens * topk, n, k).form == getattr(capi, form)
     rng = np.random.default_rng(5)
     choosed = np.stack([rng.permutation(experts)[:topk] for _ in range(tokens)]).astype(np.int32)
     split = routing.splits(choosed, experts)
