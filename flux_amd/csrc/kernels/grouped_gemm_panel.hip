@@ -552,10 +552,14 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
   // streaming form's waves are at different lines (64 experts 2816 x 2048, R 8: 115 against 118, fp8 4096 117 against 126; K = 2112
   // 126 against 119, K = 1984 114 against 113).
   if (few_rows && at_most(16) && many_items && !long_k && row_bytes(p, dtype) % 4096 == 0) return PanelPlan{};
-  if (small && at_most(192)) {
+  const int64_t items_one = (p.max_rows + 127) / 128 * ((p.n + 63) / 64);  // all rows on one expert
+  if (small && (at_most(96) || (at_most(192) && items_one <= 512))) {
     // Weights that fit the Infinity Cache in few items: latency counts, so many workgroups, and no second launch whatever the splits
     // (the macro tiles that return at once cost 5).  8 experts of 2048 x 1024, R 16 / 64 / 128: 14.4 -> 11.9, 23 -> 13, 34 -> 20; of
-    // 1024 x 2048: 14.4 -> 12.7, 31 -> 15.6, 47 -> 23; all rows on one expert, R 16 / 128: 19 -> 10 and 22 -> 16.
+    // 1024 x 2048: 14.4 -> 12.7, 31 -> 15.6, 47 -> 23; all rows on one expert, R 16 / 128: 19 -> 10 and 22 -> 16.  With more than 96
+    // rows while even that is one round, two workgroups to a unit (weights that are not in the cache, R 128 and 150, all rows on one
+    // expert: 64 experts 512 x 1024 30 -> 27 and 30 -> 37, fp8 16 experts 2048 x 2048 26 -> 22 and 27 -> 36; 48 experts 512 x 1024, R 170
+    // and 192: 30 -> 27 and 29 -> 37).
     plan.cols = 64;
     plan.chunk_rows = at_most(96) ? 64 : 128;
     plan.any_splits = true;

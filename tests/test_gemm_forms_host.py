@@ -113,6 +113,16 @@ def test_a_launch_stays_below_the_grid_limit(dtype, k, block_scaled, groups):
     assert capi.gemm_launch_info(dtype, 1024, 1024, 1 << 24, k, block_scaled=block_scaled, panel=True).cols == 0
 
 
+@pytest.mark.parametrize("dtype,experts,n,k,most", [(BF16, 64, 512, 1024, 128), (BF16, 128, 256, 1024, 128), (FP8, 16, 2048, 2048, 128),
+                                                     (BF16, 48, 512, 1024, 170), (BF16, 8, 2048, 2048, 192), (FP8, 2, 8192, 4096, 192)])
+def test_small_weights_many_rows_are_panel_tiles_while_one_expert_is_one_round(dtype, experts, n, k, most):
+    """These launches run the panel tiles whatever the splits; with more than 96 rows per expert only while 512 workgroups of 64 columns and
+    128 rows compute them all, also if one expert has every row."""
+    form = [capi.gemm_launch_info(dtype, experts, rows * experts, n, k).form for rows in (96, most, most + 1)]
+    assert form == [capi.GEMM_PANEL, capi.GEMM_PANEL, capi.GEMM_MACRO_TILES]
+    assert (most * experts + 127) // 128 * (n // 64) <= 512 and (most == 192 or (most + 1) * experts / 128 * (n // 64) > 512)
+
+
 @pytest.mark.parametrize("dtype", [BF16, F16, FP8])
 @pytest.mark.parametrize("experts,rows,k", [(64, 64 * 64, 8), (1024, 1024 * 64, 8), (8, 8 * 90, 16)])
 def test_panel_tiles_of_256_columns_have_a_workgroup_per_item(dtype, experts, rows, k):
