@@ -540,7 +540,11 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
   PanelPlan plan = {};
   const int64_t line_count = (row_bytes(p, dtype) + 127) / 128, items64 = even_items(p, 64, 1);
   auto at_most = [&](int64_t rows) { return p.max_rows <= rows * p.nexperts; };
-  const bool small = items64 <= 512 && static_cast<int64_t>(p.nexperts) * p.n * row_bytes(p, dtype) <= (64 << 20);
+  // Weight groups are items and weights as well (two groups of fp8 16 experts 2048 x 2048, R 64 / 80, random: macro tiles 37 and 38, as
+  // small launches 45 and 56).  Not where the streaming form is the other one: whether the macro tiles, with another order of sums, can
+  // compute a launch must not follow from the groups there, and it does not lose (the same at R 23: 34 -> 32).
+  const int groups = few_rows ? 1 : p.ngroups;
+  const bool small = items64 * groups <= 512 && static_cast<int64_t>(groups) * p.nexperts * p.n * row_bytes(p, dtype) <= (64 << 20);
   const bool long_k = line_count >= 48, many_items = even_items(p, 128, p.ngroups) >= 1024;
   if (!shape_ok(p, dtype)) return plan;
   plan.sums = few_rows ? stream_waves(p, dtype) : 1;
@@ -552,7 +556,7 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
   // streaming form's waves are at different lines (64 experts 2816 x 2048, R 8: 115 against 118, fp8 4096 117 against 126; K = 2112
   // 126 against 119, K = 1984 114 against 113).
   if (few_rows && at_most(16) && many_items && !long_k && row_bytes(p, dtype) % 4096 == 0) return PanelPlan{};
-  const int64_t items_one = (p.max_rows + 127) / 128 * ((p.n + 63) / 64);  // all rows on one expert
+  const int64_t items_one = (p.max_rows + 127) / 128 * ((p.n + 63) / 64) * groups;  // all rows on one expert
   if (small && (at_most(96) || (at_most(192) && items_one <= 512))) {
     // Weights that fit the Infinity Cache in few items: latency counts, so many workgroups, and no second launch whatever the splits
     // (the macro tiles that return at once cost 5).  8 experts of 2048 x 1024, R 16 / 64 / 128: 14.4 -> 11.9, 23 -> 13, 34 -> 20; of

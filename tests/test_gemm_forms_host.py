@@ -123,6 +123,16 @@ def test_small_weights_many_rows_are_panel_tiles_while_one_expert_is_one_round(d
     assert (most * experts + 127) // 128 * (n // 64) <= 512 and (most == 192 or (most + 1) * experts / 128 * (n // 64) > 512)
 
 
+@pytest.mark.parametrize("dtype,experts,rows,n,k,forms", [
+    (FP8, 16, 60, 2048, 2048, "PSSS"), (FP8, 16, 20, 2048, 2048, "PPPP"), (BF16, 64, 44, 512, 1024, "PSSS"), (BF16, 8, 60, 1024, 2048, "PPSS"),
+    (BF16, 32, 128, 512, 1024, "PPMM"), (BF16, 8, 150, 1024, 2048, "PPMM")])
+def test_small_launches_count_all_weight_groups(dtype, experts, rows, n, k, forms):
+    """P: panel tiles whatever the splits, S: the splits decide, M: macro tiles, for 1 to 4 weight groups; with few rows per expert the
+    groups do not choose."""
+    names = {capi.GEMM_PANEL: "P", capi.GEMM_BY_SPLITS: "S", capi.GEMM_MACRO_TILES: "M"}
+    assert "".join(names[capi.gemm_launch_info(dtype, experts, rows * experts, n, k, ngroups=g).form] for g in (1, 2, 3, 4)) == forms
+
+
 @pytest.mark.parametrize("dtype", [BF16, F16, FP8])
 @pytest.mark.parametrize("experts,rows,k", [(64, 64 * 64, 8), (1024, 1024 * 64, 8), (8, 8 * 90, 16)])
 def test_panel_tiles_of_256_columns_have_a_workgroup_per_item(dtype, experts, rows, k):

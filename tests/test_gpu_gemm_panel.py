@@ -245,9 +245,10 @@ def test_few_rows_have_the_bits_of_the_streaming_form(name, splits, n, kbytes, c
 
 
 @pytest.mark.parametrize("dtype,splits,n,k", [("bf16", [9] * 64, 1408, 2048), ("bf16", [8] * 32, 2048, 2048), ("fp8", [9] * 64, 1408, 4096),
-                                              ("bf16", [20] * 32, 1024, 512), ("f16", [20, 24, 28, 18], 192, 8208)])
-def test_few_rows_several_weight_groups_have_the_bits_of_one_launch_each(dtype, splits, n, k):
-    """The number of weight groups may choose between panel tiles and the streaming form."""
+                                              ("bf16", [20] * 32, 1024, 512), ("f16", [20, 24, 28, 18], 192, 8208),
+                                              ("fp8", [60] * 16, 2048, 2048), ("fp8", [300] + [30] * 15, 2048, 2048), ("bf16", [44] * 8, 2048, 2048)])
+def test_several_weight_groups_have_the_bits_of_one_launch_each(dtype, splits, n, k):
+    """The number of weight groups may choose between panel tiles and the streaming form, with more rows between them and the macro tiles."""
     print(f"[case] panel gemm groups {dtype} n={n} k={k}", flush=True)
     x, ws, run = random_operands(splits, n, k, dtype, groups=4)
     sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
