@@ -127,7 +127,7 @@ struct DryRun {
 };
 
 // Whether a form for few rows per expert, with chunks of chunk_rows rows, computes a launch with these splits.
-bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, int chunk_rows) {
+bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, int chunk_rows, const PanelPlan &panel) {
   int left = args->max_rows, chunks = 0, active = 0;
   for (int e = 0; e < args->nexperts; ++e) {
     const int rows = splits_host[e] < 0 ? 0 : (splits_host[e] < left ? splits_host[e] : left);
@@ -135,7 +135,7 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
     active += rows > 0 ? 1 : 0;
     chunks += (rows + chunk_rows - 1) / chunk_rows;
   }
-  return chunks <= stream_chunks_limit(active, chunk_rows, args->dtype == FLUXMI_FP8_E4M3);
+  return chunks <= stream_chunks_limit(active, chunk_rows, args->dtype == FLUXMI_FP8_E4M3, panel.chunk_items, panel.round_items);
 }
 
 // Row counts that are known on the host, and a second factor per row.
@@ -250,6 +250,8 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   const StreamPlan plan = stream_form && panel.cols == 0 ? plan_grouped_gemm_stream(p, args->dtype, cus, leave_cus) : StreamPlan{};
   const bool macro = mfma && !panel.any_splits && (!stream_form || args->max_rows > kStreamRows);
   if (macro) p.by_splits = panel.cols != 0 ? panel.chunk_rows : (stream_form ? kStreamRows : 0);
+  p.chunk_items = panel.chunk_items;
+  p.round_items = panel.round_items;
   if (dry_run) {
     dry_run->stream = stream_form;
     dry_run->macro = macro;
@@ -263,7 +265,7 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   few.row_scale2 = nullptr;
   bool run_few = panel.cols != 0 || stream_form, run_macro = macro;
   if (host != nullptr) {
-    const bool computes = run_few && (!macro || few_chunks(args, host->splits, p.by_splits));
+    const bool computes = run_few && (!macro || few_chunks(args, host->splits, p.by_splits, panel));
     p.by_splits = 0;
     if (computes && args->nexperts <= kArgSplits) {
       run_macro = false;
@@ -478,7 +480,7 @@ extern "C" int fluxmi_grouped_gemm_launch_info(const fluxmi_grouped_gemm_args *a
   else if (!panel && !dry.stream) info->form = FLUXMI_GEMM_MACRO_TILES;
   else if (!dry.macro) info->form = few_rows_form;
   else if (splits_host == nullptr) info->form = FLUXMI_GEMM_BY_SPLITS;
-  else info->form = few_chunks(args, splits_host, panel ? dry.panel.chunk_rows : kStreamRows) ? few_rows_form : FLUXMI_GEMM_MACRO_TILES;
+  else info->form = few_chunks(args, splits_host, panel ? dry.panel.chunk_rows : kStreamRows, dry.panel) ? few_rows_form : FLUXMI_GEMM_MACRO_TILES;
   if (dry.stream && !panel) {
     info->stream_cols = dry.plan.cols;
     info->stream_waves = dry.plan.waves;
@@ -502,7 +504,7 @@ extern "C" int fluxmi_grouped_gemm_panel_info(const fluxmi_grouped_gemm_args *ar
   info->workgroups = static_cast<int32_t>(dry.panel.workgroups);
   info->lds_bytes = dry.panel.lds_bytes;
   info->macro_tiles_too = dry.macro ? 1 : 0;
-  info->computes = !dry.macro || (splits_host != nullptr && few_chunks(args, splits_host, dry.panel.chunk_rows)) ? 1 : 0;
+  info->computes = !dry.macro || (splits_host != nullptr && few_chunks(args, splits_host, dry.panel.chunk_rows, dry.panel)) ? 1 : 0;
   info->sums = dry.panel.sums;
   return FLUXMI_OK;
 }

@@ -96,6 +96,7 @@ struct GemmParams {
   // `splits` says which of them computes the launch (stream_chunks_limit) and the other returns at once.  0: the launched one
   // computes it.
   int32_t by_splits;
+  int32_t chunk_items, round_items;  // with by_splits: items of a chunk and items that run at once, 0: do not matter (stream_chunks_limit)
 };
 
 // What a launch of a form for few rows per expert may carry besides GemmParams.  The first argument of those kernels, so that a lane
@@ -117,9 +118,20 @@ constexpr int kStreamRows = 32;
 // macro tiles: bf16 8 experts 14336 x 4096, 64 rows per expert on average, 9 chunks 196 / 225; a layer of 65 experts 5760 x 1792 at
 // 38 rows, a quarter more chunks than experts 646 / 619; all rows on one of 8 experts 95 / 47; fp8 layer of 49 experts 1024 x 1024 at
 // 41 rows 83 / 76; block-scaled 7 experts 6400 x 6912 at 61 rows, one more chunk 255 / 241).
-__host__ __device__ inline int stream_chunks_limit(int active, int chunk_rows, bool fp8) {
+//
+// Block-scaled panel tiles of 128 rows x 128 columns, one workgroup to a unit, take no extra chunks that need another round of the card
+// after the second: their items gain 5 to 25 %, and a round more costs that and more (32 experts 2048 x 7168 with 56 rows on average and
+// square-root skew, 33 chunks: panel tiles 185 us, macro tiles 133; 53 such launches of 26 to 96 rows and random or square-root skew:
+// 1.11 times as fast on the macro tiles).  Not in fp8 and 16 bits, whose macro tiles gain nothing there: 16 and 28 such
+// launches 0.93 and 0.97 times as fast.
+__host__ __device__ inline int stream_chunks_limit(int active, int chunk_rows, bool fp8, int chunk_items, int round_items) {
   if (chunk_rows <= kStreamRows) return active + (active >= 16 ? active / 4 : 0);
-  return fp8 ? active + active / 16 : active + active / 8 + 1;
+  const int limit = fp8 ? active + active / 16 : active + active / 8 + 1;
+  if (round_items == 0) return limit;
+  const uint32_t rounds = (static_cast<uint32_t>(active) * chunk_items + round_items - 1) / round_items;
+  if (rounds < 2) return limit;
+  const int same = static_cast<int>(rounds * round_items / chunk_items);  // chunks that these rounds hold
+  return same < limit ? same : limit;
 }
 
 // One launcher per element type, each in a translation unit of its own (the kernel is a long compile).

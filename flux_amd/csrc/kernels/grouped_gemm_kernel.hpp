@@ -1615,7 +1615,7 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
       acc_cand += cand;
       row_carry += __shfl(incl, 63, 64);
     }
-    if (p.by_splits && chunks <= stream_chunks_limit(active, p.by_splits, ELT == 1)) return;  // the other form runs this launch
+    if (p.by_splits && chunks <= stream_chunks_limit(active, p.by_splits, ELT == 1, p.chunk_items, p.round_items)) return;  // the other form runs this launch
     total_tiles = __builtin_amdgcn_readfirstlane(acc_tiles);
     skinny_experts = __builtin_amdgcn_readfirstlane(acc_cand);
   }

@@ -396,6 +396,7 @@ __device__ __forceinline__ void register_tile(const GemmParams &p, const FewRows
 
 #endif  // __HIP_DEVICE_COMPILE__
 
+constexpr int kUnits = 256;  // compute units
 constexpr int kCuLds = 160 * 1024, kWalkLds = 96 * 1024;
 
 // CH: most 16-row blocks of a chunk; DEPTH: stages of the ring, 0: weights through registers.
@@ -506,7 +507,7 @@ int64_t even_items(const GemmParams &p, int cols, int ngroups) {
 int64_t most_items(const GemmParams &p, int dtype, int cols, int chunk_rows, bool any_splits, int ngroups) {
   const int active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
   int64_t chunks = active + (p.max_rows - active) / chunk_rows;
-  const int limit = stream_chunks_limit(active, chunk_rows, dtype == FLUXMI_FP8_E4M3);
+  const int limit = stream_chunks_limit(active, chunk_rows, dtype == FLUXMI_FP8_E4M3, 0, 0);  // (rounds make it no larger)
   if (!any_splits && chunks > limit) chunks = limit;
   return chunks * ((p.n + cols - 1) / cols) * ngroups;
 }
@@ -524,6 +525,8 @@ bool walks(int64_t blocks, bool leave_cus) { return leave_cus || blocks * 256 > 
 void finish(const GemmParams &p, int dtype, int cus, bool leave_cus, PanelPlan &plan) {
   const int64_t blocks = block_count(p, dtype, plan);
   plan.blocks = static_cast<int>(blocks);
+  plan.chunk_items = (p.n + plan.cols - 1) / plan.cols * p.ngroups;
+  plan.round_items = plan.chunk_rows == 128 && plan.cols == 128 && p.a_scale != nullptr ? kUnits : 0;
   plan.walk = walks(blocks, leave_cus);
   const int64_t most = cus >= 8 ? cus / 8 * 8 : cus;  // whole rounds over the XCDs where there are enough units
   plan.workgroups = static_cast<unsigned>(plan.walk && blocks > most ? most : blocks);

@@ -14,6 +14,8 @@ struct PanelPlan {
   int blocks;           // items the launch is numbered for
   unsigned workgroups;  // workgroups launched; fewer than `blocks`: each walks several items
   bool walk;
+  int chunk_items;      // items of a chunk of rows,
+  int round_items;      // items that run at once: where a round more is not worth it (stream_chunks_limit), otherwise 0
   bool any_splits;      // computes every distribution of the rows; otherwise only those with few chunks (stream_chunks_limit)
   int lds_bytes;        // per workgroup
 };

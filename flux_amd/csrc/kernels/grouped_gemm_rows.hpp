@@ -59,7 +59,7 @@ __device__ __forceinline__ WorkItem locate(const GemmParams &p, int tiles_n, int
   int row_carry = 0, total = 0, active = 0;
   for (int e0 = 0; e0 < p.nexperts; e0 += 64) active += load(e0, row_carry, total);
   WorkItem w = {0, 0, 0, 0, 0, 0};
-  if (p.by_splits && total > stream_chunks_limit(active, chunk_rows, is_fp8(T))) return w;  // the macro tiles run this launch
+  if (p.by_splits && total > stream_chunks_limit(active, chunk_rows, is_fp8(T), p.chunk_items, p.round_items)) return w;  // the macro tiles run this launch
   // Workgroups are dealt to the eight XCDs round-robin.
   const int items = total * tiles_n, per_xcd = (items + 7) / 8, i = block >> 3, item = (block & 7) * per_xcd + i;
   if (i >= per_xcd || item >= items) return w;

@@ -265,7 +265,7 @@ int64_t one_chunk_items(const GemmParams &p, int ngroups, int nb) {
 }
 int64_t most_items(const GemmParams &p, int ngroups, int nb) {
   const int active = p.nexperts < p.max_rows ? p.nexperts : p.max_rows;
-  const int chunks = active + (p.max_rows - active) / kStreamRows, limit = stream_chunks_limit(active, kStreamRows, false);
+  const int chunks = active + (p.max_rows - active) / kStreamRows, limit = stream_chunks_limit(active, kStreamRows, false, 0, 0);
   return static_cast<int64_t>(chunks < limit ? chunks : limit) * ((p.n + 16 * nb - 1) / (16 * nb)) * ngroups;
 }
 

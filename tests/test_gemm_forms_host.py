@@ -133,6 +133,23 @@ def test_small_launches_count_all_weight_groups(dtype, experts, rows, n, k, form
     assert "".join(names[capi.gemm_launch_info(dtype, experts, rows * experts, n, k, ngroups=g).form] for g in (1, 2, 3, 4)) == forms
 
 
+@pytest.mark.parametrize("block_scaled,splits,n,k,form", [
+    (True, [129] + [54] * 31, 2048, 7168, capi.GEMM_MACRO_TILES), (True, [128] + [54] * 31, 2048, 7168, capi.GEMM_PANEL),  # 528 items and 512
+    (True, [129] * 2 + [50] * 30, 2560, 2560, capi.GEMM_PANEL), (True, [129] + [55] * 15, 4096, 5120, capi.GEMM_MACRO_TILES),  # 680 and 544
+    (True, [129] + [60] * 15, 2048, 4096, capi.GEMM_PANEL),  # 272: the first round and the second
+    (True, [129] * 2 + [60] * 23 + [0] * 7, 2560, 4096, capi.GEMM_MACRO_TILES),  # 540, of experts with rows 500; one busy expert less 520, 480
+    (True, [129] + [60] * 23 + [0] * 8, 2560, 4096, capi.GEMM_PANEL), (True, [129] + [60] * 24 + [0] * 7, 2560, 4096, capi.GEMM_MACRO_TILES),
+    (False, [129] + [54] * 31, 2048, 7168, capi.GEMM_PANEL)])
+def test_block_scaled_extra_chunks_take_no_extra_round(block_scaled, splits, n, k, form):
+    """Block-scaled panel tiles of 128 rows and columns, one workgroup to each of 256 units: experts of several chunks must fit the rounds
+    that one chunk each would take, from two on."""
+    rows = max(sum(splits), 41 * len(splits))
+    info = capi.gemm_launch_info(FP8, len(splits), rows, n, k, splits=splits, block_scaled=block_scaled)
+    panel = capi.gemm_launch_info(FP8, len(splits), rows, n, k, splits=splits, block_scaled=block_scaled, panel=True)
+    assert (panel.cols, panel.chunk_rows) == (128, 128)
+    assert info.form == form and panel.computes == (form == capi.GEMM_PANEL)
+
+
 @pytest.mark.parametrize("dtype", [BF16, F16, FP8])
 @pytest.mark.parametrize("experts,rows,k", [(64, 64 * 64, 8), (1024, 1024 * 64, 8), (8, 8 * 90, 16)])
 def test_panel_tiles_of_256_columns_have_a_workgroup_per_item(dtype, experts, rows, k):

@@ -312,6 +312,19 @@ def test_splits_choose_between_panel_and_macro_tiles(dtype, splits, computes):
         assert torch.equal(out[:sum(s)].double(), product(a, w, s)) and bool((out[sum(s):] == -1).all())
 
 
+@pytest.mark.parametrize("splits,computes", [([128] + [50] * 23, 1), ([129] + [50] * 23, 0), ([129] + [50] * 22 + [0], 1)])
+def test_block_scaled_rounds_choose_between_panel_and_macro_tiles(splits, computes):
+    """24 experts of 21 column tiles are two rounds, a chunk more is a third: both launches agree on which of them computes."""
+    n, k, m, e = 2688, 256, sum(splits), len(splits)
+    print(f"[case] panel gemm, rounds {splits[:3]}", flush=True)
+    assert capi.gemm_launch_info(DT["bs"], e, m, n, k, splits=splits, panel=True, block_scaled=True).computes == computes
+    a, w, sp, _ = made(splits, n, k, "bs", m)
+    sad, sbd = torch.ones((m + 127) // 128, k // 128, 128, device="cuda"), torch.ones(e, n // 128, k // 128, device="cuda")
+    out = torch.full((m, n), -1.0, device="cuda")
+    capi.grouped_gemm_blockscale(a.to(DT["bs"]), w.to(DT["bs"]), sp, sad, sbd, out=out)
+    assert torch.equal(out.double(), product(a, w, splits))
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp8", "bs"])
 @pytest.mark.parametrize("splits,n,k,done", [([7, 0, 30, 1], 1024, 8192, 1), ([12, 3, 9, 20, 17, 0, 31, 8], 4160, 384, 1), ([70, 64, 1, 0], 192, 256, 1),
                                              ([-3, 20, 600, 5], 192, 256, 1), ([129] + [40] * 15 + [30] * 8, 1408, 1152, 1),
