@@ -592,6 +592,13 @@ PanelPlan plan_panel(const GemmParams &p, int dtype, bool few_rows, int cus, boo
     plan.cols = 256;
     if (even_items(p, 256, p.ngroups) < 384 || p.a_scale != nullptr || walks(block_count(p, dtype, plan), leave_cus))
       plan.cols = even_items(p, 128, p.ngroups) >= 192 ? 128 : 64;
+    // fp8 with more than 64 rows and short K, two rounds of 128 columns and more: half of a macro tile's columns is no gain any more (770
+    // launches of random, log-normal and square-root-skewed rows, K below 6 KiB, macro tiles / these tiles in the mean: two rounds R 65 to 80
+    // 0.98, R 81 to 96 0.95, more rounds 1.00 and 0.98; at least 0.82; two groups of 16 experts 2048 x 2048, R 80: 38 against 44).  R 41 to 64
+    // 1.04 and 1.11, longer K 1.05, block-scaled 1.00 to 1.17, 16 bits 1.01 to 1.2, one round 1.05 to 1.6.
+    if (dtype == FLUXMI_FP8_E4M3 && p.a_scale == nullptr && !at_most(64) && plan.cols == 128 && even_items(p, 128, p.ngroups) > kUnits &&
+        row_bytes(p, dtype) < 6144)
+      return PanelPlan{};
   } else {
     return PanelPlan{};
   }

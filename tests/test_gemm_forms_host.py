@@ -133,6 +133,17 @@ def test_small_launches_count_all_weight_groups(dtype, experts, rows, n, k, form
     assert "".join(names[capi.gemm_launch_info(dtype, experts, rows * experts, n, k, ngroups=g).form] for g in (1, 2, 3, 4)) == forms
 
 
+@pytest.mark.parametrize("dtype,experts,rows,n,k,ngroups,block_scaled,panel", [
+    (FP8, 16, 64, 4096, 2560, 1, False, True), (FP8, 16, 65, 4096, 2560, 1, False, False), (FP8, 16, 96, 2048, 2560, 1, False, True),
+    (FP8, 16, 96, 2176, 2560, 1, False, False), (FP8, 16, 80, 2048, 2048, 2, False, False), (FP8, 16, 80, 4096, 6144, 1, False, True),
+    (FP8, 32, 80, 4096, 2560, 1, False, True),  # 256 columns
+    (FP8, 16, 80, 4096, 2560, 1, True, True), (BF16, 16, 80, 4096, 2560, 1, False, True)])
+def test_fp8_short_k_in_several_rounds_is_for_the_macro_tiles(dtype, experts, rows, n, k, ngroups, block_scaled, panel):
+    got = capi.gemm_launch_info(dtype, experts, experts * rows, n, k, ngroups=ngroups, block_scaled=block_scaled, panel=True)
+    form = capi.gemm_launch_info(dtype, experts, experts * rows, n, k, ngroups=ngroups, block_scaled=block_scaled).form
+    assert (got.cols > 0) == panel and form == (capi.GEMM_BY_SPLITS if panel else capi.GEMM_MACRO_TILES)
+
+
 @pytest.mark.parametrize("block_scaled,splits,n,k,form", [
     (True, [129] + [54] * 31, 2048, 7168, capi.GEMM_MACRO_TILES), (True, [128] + [54] * 31, 2048, 7168, capi.GEMM_PANEL),  # 528 items and 512
     (True, [129] * 2 + [50] * 30, 2560, 2560, capi.GEMM_PANEL), (True, [129] + [55] * 15, 4096, 5120, capi.GEMM_MACRO_TILES),  # 680 and 544
