@@ -31,7 +31,12 @@
 // 214 / 129 / 159; bf16 64 experts 1408 x 2048, 512 rows 90 / 87 / 123; all 768 rows on eight of the 32 72 / 42 / 33, on
 // one 62 / 34 / 24.
 //
-// Measured (us per launch, the macro tiles -> this form; weights at 6.5 TB/s in brackets), even splits, bf16 8 experts 14336 x
+// The panel tiles (grouped_gemm_panel.hip) take most launches that this form could compute as well, with the same sums; plan_panel says
+// which stay here: up to four rows per expert, few columns at long K, and up to 16 rows per expert in many columns of rows a multiple of
+// 4 KiB apart, and fewer than 64 columns.
+//
+// Measured (us per launch, the macro tiles -> this form; weights at 6.5 TB/s in brackets; with more rows than that by runs without the
+// panel tiles), even splits, bf16 8 experts 14336 x
 // 4096: 64 rows 216 -> 138 [145], 128 rows 216 -> 141, 256 rows 218 -> 165; 4096 x 14336: 64 rows 212 -> 145 [145], 256 rows
 // 218 -> 165; 64 experts 1408 x 2048, 256 rows: 113 -> 57 [57], 2048 rows 116 -> 78; fp8 32 experts 2048 x 7168, 256 rows:
 // 94 -> 72 [72], 768 rows 96 -> 82; 7168 x 2048: 115 -> 80 [72] and 118 -> 98; block-scaled, the same four: 123 -> 74,
@@ -293,7 +298,8 @@ void launch_by_plan(const GemmParams &p, const FewRowsArgs &few, const StreamPla
 
 }  // namespace
 
-// Up to how many rows per expert on average this form is the faster one on even splits (the macro tiles' time hardly depends on
+// Up to how many rows per expert on average this form is faster than the macro tiles on even splits (plan_panel has the line between it and
+// the panel tiles, which up to here sum K as this form does; the macro tiles' time hardly depends on
 // the rows while they are few; this one's grows with them): 16-bit at 32 rows 165 / 218 us on the two 8-expert shapes above,
 // 78 / 116 and 80 / 92 on 64 experts of 1408 x 2048 and 2048 x 1408, 12 / 19 on 8 of 2048 x 1024; fp8 at 24 rows 82 / 96 and 98 /
 // 118, at 32 an earlier build 95 / 97 and 128 / 118; block-scaled at 24 rows 83 / 125 and 104 / 152.  Items are numbered with ints
@@ -301,6 +307,11 @@ void launch_by_plan(const GemmParams &p, const FewRowsArgs &few, const StreamPla
 bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
   const int64_t rows = dtype == FLUXMI_FP8_E4M3 ? 24 : kStreamRows;
   return p.max_rows <= rows * p.nexperts && most_items(p, kMaxWeightGroups, 2) < (int64_t{1} << 31) - (1 << 20);
+}
+
+int stream_waves(const GemmParams &p, int dtype) {
+  const int64_t lines = (static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2) + 127) / 128;
+  return one_chunk_items(p, 1, 4) < 512 && lines >= 64 ? 8 : 4;
 }
 
 // Columns per workgroup: 64 reads the rows' own operand least often (its loads share the queue behind the weights' with them), but
@@ -315,11 +326,6 @@ bool grouped_gemm_stream_takes(const GemmParams &p, int dtype) {
 // / 224 of 256 units, this form and the macro tiles: bf16 8 experts 14336 x 4096, 74 rows 162 / 185 / 255 / 995 and 215 / 238 / 268 /
 // 773; fp8 32 experts 7168 x 2048, 400 rows 97 / 118 / 168 / 642 and 111 / 120 / 147 / 500 (a unit alone streams 30 GB/s here; a
 // ring of three or four lines in place of two changed nothing).
-int stream_waves(const GemmParams &p, int dtype) {
-  const int64_t lines = (static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2) + 127) / 128;
-  return one_chunk_items(p, 1, 4) < 512 && lines >= 64 ? 8 : 4;
-}
-
 StreamPlan plan_grouped_gemm_stream(const GemmParams &p, int dtype, int cus, bool leave_cus) {
   StreamPlan plan;
   const bool few = one_chunk_items(p, p.ngroups, 4) < 512;
