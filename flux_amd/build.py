@@ -35,7 +35,8 @@ HIP_FLAGS = [
 # Per-file additions.  The block-scaled GEMM promotes every MFMA result with vector-ALU instructions right away:
 # its MFMAs must write vector registers (the compiler's default for a kernel that uses both register files is
 # the accumulation registers, which costs a v_accvgpr_read per element and promotion).
-EXTRA_HIP_FLAGS = {"grouped_gemm_fp8_blockscale.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA_HIP_FLAGS = {"grouped_gemm_fp8_blockscale.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                   "grouped_gemm_dual.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 KERNEL_LIB = os.path.join(LIB_DIR, "libfluxmi_kernels.so")
 

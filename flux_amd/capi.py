@@ -29,6 +29,7 @@ EXPORTS = (
     "fluxmi_moe_route_sort_static_max_bytes", "fluxmi_moe_route_sort_static_init", "fluxmi_moe_route_sort_static",
     "fluxmi_grouped_gemm_workspace_bytes", "fluxmi_grouped_gemm", "fluxmi_grouped_gemm_kernel_kind",
     "fluxmi_grouped_gemm_host_splits", "fluxmi_grouped_gemm_launch_info", "fluxmi_grouped_gemm_panel_info",
+    "fluxmi_grouped_gemm_dual_tiles",
     "fluxmi_grouped_gemm_multi", "fluxmi_grouped_gemm_topk_reduce_workspace_bytes",
     "fluxmi_grouped_gemm_topk_reduce", "fluxmi_grouped_gemm_blockscale",
     "fluxmi_topk_gather_reduce", "fluxmi_quant_e4m3_rowwise", "fluxmi_quant_e4m3_square",
@@ -85,6 +86,7 @@ def load():
     lib.fluxmi_grouped_gemm_workspace_bytes.argtypes = [ctypes.POINTER(GroupedGemmArgs)]
     lib.fluxmi_grouped_gemm.argtypes = [ctypes.POINTER(GroupedGemmArgs), vp, sz, vp]
     lib.fluxmi_grouped_gemm_kernel_kind.argtypes = [ctypes.POINTER(GroupedGemmArgs)]
+    lib.fluxmi_grouped_gemm_dual_tiles.argtypes = [ctypes.POINTER(GroupedGemmArgs), i32, vp, i32]
     lib.fluxmi_grouped_gemm_launch_info.argtypes = [ctypes.POINTER(GroupedGemmArgs), i32, vp, vp, i32,
                                                     ctypes.POINTER(GemmLaunchInfo)]
     lib.fluxmi_grouped_gemm_host_splits.argtypes = [ctypes.POINTER(GroupedGemmArgs), vp, vp, vp, i32, vp, i32, vp]
@@ -257,6 +259,16 @@ def gemm_launch_info(dtype, nexperts, max_rows, n, k, ngroups=1, block_scaled=Fa
     _check(call(ctypes.byref(args), ngroups, aligned if block_scaled else None, host, cu_count, ctypes.byref(info)),
            "fluxmi_grouped_gemm_panel_info" if panel else "fluxmi_grouped_gemm_launch_info")
     return info
+
+
+def gemm_dual_tiles(dtype, nexperts, max_rows, n, k, ngroups=1, block_scaled=False, gathered=False, sched_flags=0, d_fp32=False):
+    """Whether the macro tiles' part of a grouped GEMM with aligned operands runs the dual tiles (fluxmi_grouped_gemm_dual_tiles); needs no GPU."""
+    aligned = ctypes.c_void_p(4096)
+    args = GroupedGemmArgs(dtype=_DTYPES[dtype], nexperts=nexperts, max_rows=max_rows, n=n, k=k, a_rows=max_rows, a=aligned, b=aligned, d=aligned,
+                           splits=aligned, gather_a=aligned if gathered else None, scalar_scale=1.0, sched_flags=sched_flags, d_fp32=int(d_fp32))
+    rc = load().fluxmi_grouped_gemm_dual_tiles(ctypes.byref(args), ngroups, aligned if block_scaled else None, 256)
+    _check(min(rc, 0), "fluxmi_grouped_gemm_dual_tiles")
+    return rc == 1
 
 
 ASCALE_BLOCK128, ASCALE_EXPERT_K_M = 0, 1

@@ -212,6 +212,10 @@ typedef struct fluxmi_gemm_panel_info {
 int fluxmi_grouped_gemm_panel_info(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale,
                                    const int32_t *splits_host, int32_t cu_count, fluxmi_gemm_panel_info *info);
 
+/* Whether a launch, or the part of one by splits, that is FLUXMI_GEMM_MACRO_TILES runs the dual tiles, 256 x 256 like the others but on
+ * eight waves that take turns: 1 or 0, or the status the call itself would return.  Arguments as for fluxmi_grouped_gemm_launch_info. */
+int fluxmi_grouped_gemm_dual_tiles(const fluxmi_grouped_gemm_args *args, int32_t ngroups, const float *a_scale, int32_t cu_count);
+
 /* ------------------------------------------------------------------------------------------------
  * Top-k reduction fused into the grouped GEMM's epilogue (layer1 in one pass, no [M, N] intermediate):
  *

@@ -1,0 +1,76 @@
+"""GPU parity of the dual tiles of the grouped GEMM (256 x 256 on eight waves that take turns) at the edges of their tiles.
+
+Operands are small integers and scales powers of two, so every product and every partial sum is a whole multiple of a power of two
+below 2^24 steps: the fp32 result is the same in any order of summation and has to equal a float64 matmul exactly, no tolerance."""
+import ctypes
+
+import pytest
+import torch
+
+from flux_amd import capi
+from test_gpu_gemm_panel import DT, block_scales, made, product
+
+pytestmark = pytest.mark.gpu
+
+# Rows on both sides of a wave's 64, of both halves of a tile and of one, two and more tiles, empty experts, up to 128 experts; columns that end
+# in each group of 32 and after the first half of a tile; the fewest steps of K, odd and even numbers of them, and more than the ring holds;
+# tiles of a last round cut in four, in two and whole, and several rounds.
+CASES = [
+    ("heights", [255, 256, 257, 64, 65, 128, 129, 193, 321, 0, 1, 1000, 190], 392, 384),
+    ("two steps", [300], 136, 256),
+    ("128 experts", [200, 0, 450] + [190] * 124 + [700], 264, 256),
+    ("long K, cut in two", [513, 511, 700, 448, 192], 2312, 2176),
+    ("cut in four", [600, 1], 1032, 1152),
+    ("several rounds", [1100, 900, 1300, 1024], 4104, 640),
+]
+
+
+@pytest.mark.parametrize("name,splits,n,k", CASES, ids=[c[0] for c in CASES])
+@pytest.mark.parametrize("a_layout", [capi.ASCALE_BLOCK128, capi.ASCALE_EXPERT_K_M])
+@pytest.mark.parametrize("b_layout", [capi.BSCALE_N_K, capi.BSCALE_K_N])
+def test_dual_tiles_block_scaled_are_exact_on_integers(name, splits, n, k, a_layout, b_layout):
+    print(f"[case] dual gemm block-scaled {name} n={n} k={k} layouts {a_layout} {b_layout}", flush=True)
+    m, e = sum(splits), len(splits)
+    assert capi.gemm_launch_info(DT["bs"], e, m, n, k, splits=splits, block_scaled=True).form == capi.GEMM_MACRO_TILES
+    assert capi.gemm_dual_tiles(DT["bs"], e, m, n, k, block_scaled=True)
+    a, w, sp, g = made(splits, n, k, "fp8", n + k)
+    sa, sb, sad, sbd = block_scales(m, e, n, k, splits, a_layout, b_layout, g)
+    af = a * torch.repeat_interleave(sa, 128, dim=1)
+    wf = w * torch.repeat_interleave(torch.repeat_interleave(sb, 128, dim=1)[:, :n], 128, dim=2)
+    want = product(af, wf, splits)
+    ad, wd = a.to(DT["bs"]), w.to(DT["bs"])
+    for margin in (0, 40, 253):
+        args, out = capi._gemm_args(ad, wd, sp, None, None, None, None, None, None, 1.0, None, None, torch.float32, margin, 0, 0)
+        capi._check(capi.load().fluxmi_grouped_gemm_blockscale(ctypes.byref(args), capi._ptr(sad), a_layout, capi._ptr(sbd), b_layout, capi._stream()),
+                    "fluxmi_grouped_gemm_blockscale")
+        assert torch.equal(out.double(), want), f"margin {margin}"
+    half = capi.grouped_gemm_blockscale(ad, wd, sp, sad, sbd, a_layout, b_layout)
+    assert torch.equal(half, want.float().to(torch.bfloat16))
+    if a_layout == capi.ASCALE_BLOCK128:  # rows, and their scales, picked by a gather; results put elsewhere, with every factor
+        perm = torch.randperm(m, generator=g, device="cuda").to(torch.int32)
+        to = perm.flip(0).contiguous()
+        row_scale = 2.0 ** torch.randint(-1, 2, (m,), generator=g, device="cuda").float()
+        col_scale = 2.0 ** torch.randint(-1, 2, (e, n), generator=g, device="cuda").float()
+        alpha = 2.0 ** torch.randint(-1, 2, (e,), generator=g, device="cuda").float()
+        expert = torch.repeat_interleave(torch.arange(e, device="cuda"), sp.long())
+        picked = torch.empty_like(want)
+        picked[to.long()] = product(af[perm.long()], wf, splits) * (alpha[expert] * row_scale).double()[:, None] * col_scale[expert].double()
+        got = capi.grouped_gemm_blockscale(ad, wd, sp, sad, sbd, a_layout, b_layout, out_dtype=torch.float32, gather_a=perm, scatter_d=to,
+                                           row_scale=row_scale, col_scale=col_scale, alpha=alpha)
+        assert torch.equal(got.double(), picked)
+
+
+def test_dual_tiles_do_not_touch_rows_past_the_splits():
+    """Rows beyond sum(splits), and negative and too large counts: clamped like everywhere else."""
+    print("[case] dual gemm block-scaled, counts past the rows", flush=True)
+    splits, n, k, m = [400, -7, 300, 5000], 264, 512, 1000
+    a, w, _, g = made([m], n, k, "fp8", 3)
+    w = torch.randint(-3, 4, (4, n, k), generator=g, device="cuda").float()
+    sad, sbd = torch.ones((m + 127) // 128, k // 128, 128, device="cuda"), torch.ones(4, 3, k // 128, device="cuda")
+    out = torch.full((m + 8, n), -5.0, device="cuda")
+    call = lambda s: capi.grouped_gemm_blockscale(a.to(DT["bs"]), w.to(DT["bs"]), torch.tensor(s, dtype=torch.int32, device="cuda"), sad, sbd, out=out)
+    call(splits)
+    assert torch.equal(out[:m].double(), product(a, w, [400, 0, 300, 300])) and bool((out[m:] == -5).all())
+    out.fill_(-5)
+    call([400, 0, 300, 0])
+    assert torch.equal(out[:700].double(), product(a[:700], w, [400, 0, 300, 0])) and bool((out[700:] == -5).all())
