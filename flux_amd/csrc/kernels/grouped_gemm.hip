@@ -140,6 +140,24 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
   return chunks <= stream_chunks_limit(active, chunk_rows, args->dtype == FLUXMI_FP8_E4M3, panel.chunk_items, panel.round_items);
 }
 
+// Whether the dual tiles are the faster ones for a launch that the macro tiles would compute; from 15006 launches of 4 to 96 experts, R = 97
+// to 4000 rows each on average, K 768 to 14336, even, random and Zipf row counts, plain and scaled, weights not in the cache.  Speed
+// against the macro tiles in the mean over ranges of R and K, and how many are slower by more than 3 %:
+//   block-scaled  1.05 to 1.31, 1 %
+//   fp8           R up to 512: 1.05 to 1.25, 2 %.  More rows: K < 3 KiB 1.04 to 1.17, 5 %; K < 4 KiB, R up to 1024 1.04 and 1.05, 12 %, R above
+//                 1.02 to 1.04, up to 27 %; longer K 0.98 to 1.05
+//   16 bits       R up to 320: 1.07 to 1.25, 3 %.  More rows: K < 3 KiB 1.06 to 1.21, 6 %; K < 4 KiB, R up to 768 1.05 to 1.08, 6 %; K < 6 KiB, R up
+//                 to 512 1.05 and 1.06, 8 %; beyond these lines 0.92 to 1.06, up to 76 %
+// The flags of the fill forms name forms of the macro tiles.
+bool dual_is_faster(const fluxmi_grouped_gemm_args *args, bool block_scaled) {
+  if (block_scaled) return true;
+  if ((args->sched_flags & (FLUXMI_SCHED_HALF_LINE_FILLS | FLUXMI_SCHED_WHOLE_LINE_FILLS)) != 0) return false;
+  const bool fp8 = args->dtype == FLUXMI_FP8_E4M3;
+  const int64_t kbytes = static_cast<int64_t>(args->k) * (fp8 ? 1 : 2);
+  auto at_most = [&](int64_t rows) { return args->max_rows <= rows * args->nexperts; };
+  return at_most(fp8 ? 512 : 320) || kbytes < 3072 || (kbytes < 4096 && at_most(fp8 ? 1024 : 768)) || (kbytes < 6144 && at_most(512));
+}
+
 // Row counts that are known on the host, and a second factor per row.
 struct HostSplits {
   const int32_t *splits;
@@ -254,9 +272,7 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   if (macro) p.by_splits = panel.cols != 0 ? panel.chunk_rows : (stream_form ? kStreamRows : 0);
   p.chunk_items = panel.chunk_items;
   p.round_items = panel.round_items;
-  // Block-scaled launches run the dual tiles wherever those take them: 5019 launches of 4 to 96 experts, 97 to 4000 rows each on average,
-  // K 768 to 14336, even, random and Zipf row counts 1.11 times as fast in the mean, 2 % of them slower by more than 3 %.
-  const bool dual = macro && bs != nullptr && dual_takes(p);
+  const bool dual = macro && dual_is_faster(args, bs != nullptr) && dual_takes(p, args->dtype);
   if (dry_run) {
     dry_run->stream = stream_form;
     dry_run->macro = macro;
@@ -307,7 +323,7 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
     const int64_t kbytes = static_cast<int64_t>(args->k) * (args->dtype == FLUXMI_FP8_E4M3 ? 1 : 2);
     const bool lines = (args->sched_flags & FLUXMI_SCHED_WHOLE_LINE_FILLS) != 0 ||
                        ((args->sched_flags & FLUXMI_SCHED_HALF_LINE_FILLS) == 0 && args->gather_a == nullptr && kbytes >= 16384);
-    const int rc = dual ? launch_grouped_gemm_dual(p, grid, s)
+    const int rc = dual ? launch_grouped_gemm_dual(p, args->dtype, grid, s)
                    : bs != nullptr ? launch_grouped_gemm_fp8_blockscale(p, grid, s)
                    : args->dtype == FLUXMI_BF16 ? (lines ? launch_grouped_gemm_bf16_lines(p, grid, s) : launch_grouped_gemm_bf16(p, grid, s))
                    : args->dtype == FLUXMI_FP16 ? launch_grouped_gemm_f16(p, grid, s)  // the half-line form only

@@ -17,9 +17,12 @@
 //  * A lane's four sums of a block are neighbouring columns of one row.  16-bit results: which column an LDS row of B holds is chosen so
 //    that two blocks' sums are eight neighbours, and a store instruction writes 64 bytes of 16 rows straight from registers.
 //
-// us, macro tiles (256 x 128, promotion beside the MFMAs) -> these, block-scaled fp8: 32 experts 2048 x 7168 and 7168 x 2048, 16384 rows
-// in all at random 340 -> 291 and 358 -> 309; 1024 rows each 538 -> 445 and 616 -> 499 (2.16 and 1.93 PFLOP/s); 188 rows each 140 -> 125
-// and 173 -> 147.
+// us, macro tiles -> these.  Block-scaled fp8 (there pieces of 256 x 128): 32 experts 2048 x 7168 and 7168 x 2048, 16384 rows in all at
+// random 309 -> 272 and 330 -> 279; 1024 rows each 523 -> 434 and 593 -> 484 (2.22 and 1.99 PFLOP/s); 188 rows each 146 -> 120 and 166 ->
+// 134.  fp16, 8 experts, 194 rows each: 14336 x 4096 270 -> 247, 4096 x 14336 334 -> 301.  fp8 32 experts 7168 x 2048, 1024 rows each
+// 516 -> 505.  Without block scales long K with many rows stays on the macro tiles: both are at the board's power limit there, and
+// these read half as much again from LDS per MFMA (dense fp8 8192 x 8192 x 8192: 736 k cycles against 771 k, at 1.73 GHz against 1.95;
+// bf16 8 experts 4096 x 14336, 2048 rows each 1361 -> 1540).
 #include "grouped_gemm_dual.hpp"
 #include "grouped_gemm_rows.hpp"
 
@@ -54,12 +57,6 @@ struct DualTile {
   int e_row0, e_rows;  // the expert's rows
 };
 
-__device__ __forceinline__ f32x4 mfma_block(const i32x4 (&w)[2], const i32x4 (&x)[2]) {
-  const i32x8 wa = {w[0][0], w[0][1], w[0][2], w[0][3], w[1][0], w[1][1], w[1][2], w[1][3]};
-  const i32x8 xa = {x[0][0], x[0][1], x[0][2], x[0][3], x[1][0], x[1][1], x[1][2], x[1][3]};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wa, xa, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
-}
-
 template <int FIRST, class F, int... I>
 __device__ __forceinline__ void static_for_seq(F &f, std::integer_sequence<int, I...>) {
   (f(std::integral_constant<int, FIRST + I>{}), ...);
@@ -69,30 +66,62 @@ __device__ __forceinline__ void static_for(F &&f) {
   if constexpr (FIRST < END) static_for_seq<FIRST>(f, std::make_integer_sequence<int, END - FIRST>{});
 }
 
-// 64 rows (four blocks, from I0 on) x 32 columns (two blocks, from J0 on) over 128 bytes of K.
-template <bool FIRST, int I0, int J0>
-__device__ __forceinline__ void quadrant(f32x4 (&acc)[8][4], const i32x4 (&x)[4][2], const i32x4 (&w)[4][2], const float (&scale)[4]) {
-  constexpr int DIST = 3;  // MFMAs between a block's and its promotion (2: the compiler's wait states in between are exposed)
-  f32x4 part[8];
-  auto promote = [&](auto M) {
-    constexpr int m = decltype(M)::value, i = m / 2, j = m % 2;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[I0 + i][J0 + j][v] = fmaf(part[m][v], scale[i], FIRST ? 0.f : acc[I0 + i][J0 + j][v]);
-    asm volatile("" : "+v"(acc[I0 + i][J0 + j]));  // here, not where the sums are next used: the block's registers are needed again
-  };
-  static_for<0, 8>([&](auto M) {
-    constexpr int m = decltype(M)::value;
-    part[m] = mfma_block(w[J0 + m % 2], x[m / 2]);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (m >= DIST) promote(std::integral_constant<int, (m >= DIST ? m - DIST : 0)>{});
-    __builtin_amdgcn_sched_barrier(0);
-  });
-  static_for<8 - DIST, 8>(promote);
+// One block of 16 x 16 over 64 (16-bit elements, half h of a step) or 128 bytes of K, added to c.
+template <Elem T>
+__device__ __forceinline__ f32x4 mfma_block(const i32x4 (&w)[2], const i32x4 (&x)[2], int h, f32x4 c) {
+  if constexpr (is_fp8(T)) {
+    const i32x8 wa = {w[0][0], w[0][1], w[0][2], w[0][3], w[1][0], w[1][1], w[1][2], w[1][3]};
+    const i32x8 xa = {x[0][0], x[0][1], x[0][2], x[0][3], x[1][0], x[1][1], x[1][2], x[1][3]};
+    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wa, xa, c, 0, 0, 0, 0, 0, 0);
+  } else if constexpr (T == Elem::F16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w[h]), __builtin_bit_cast(f16x8, x[h]), c, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[h]), __builtin_bit_cast(bf16x8, x[h]), c, 0, 0, 0);
+  }
 }
 
+// 64 rows (four blocks, from I0 on) x 32 columns (two blocks, from J0 on) over 128 bytes of K.
+template <Elem T, bool FIRST, int I0, int J0>
+__device__ __forceinline__ void quadrant(f32x4 (&acc)[8][4], const i32x4 (&x)[4][2], const i32x4 (&w)[4][2], const float (&scale)[4]) {
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  if constexpr (T == Elem::FP8_BLOCKSCALED) {
+    constexpr int DIST = 3;  // MFMAs between a block's and its promotion (2: the compiler's wait states in between are exposed)
+    f32x4 part[8];
+    auto promote = [&](auto M) {
+      constexpr int m = decltype(M)::value, i = m / 2, j = m % 2;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[I0 + i][J0 + j][v] = fmaf(part[m][v], scale[i], FIRST ? 0.f : acc[I0 + i][J0 + j][v]);
+      asm volatile("" : "+v"(acc[I0 + i][J0 + j]));  // here, not where the sums are next used: the block's registers are needed again
+    };
+    static_for<0, 8>([&](auto M) {
+      constexpr int m = decltype(M)::value;
+      part[m] = mfma_block<T>(w[J0 + m % 2], x[m / 2], 0, zero);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (m >= DIST) promote(std::integral_constant<int, (m >= DIST ? m - DIST : 0)>{});
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    static_for<8 - DIST, 8>(promote);
+  } else {
+    // (16-bit: the halves of a step in ascending order, which are the macro tiles' sums.)
+#pragma unroll
+    for (int h = 0; h < (is_fp8(T) ? 1 : 2); ++h)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[I0 + i][J0 + j] = mfma_block<T>(w[J0 + j], x[i], h, FIRST && h == 0 ? zero : acc[I0 + i][J0 + j]);
+  }
+}
+
+template <Elem T>
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  const f32x2 v = {lo, hi};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+  if constexpr (T == Elem::F16) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    const f16x2 h = {static_cast<_Float16>(lo), static_cast<_Float16>(hi)};
+    return __builtin_bit_cast(uint32_t, h);
+  } else {
+    const f32x2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+  }
 }
 
 // The kernel's argument, read again where it is used; the empty asm keeps the compiler from keeping copies in registers through the loop.
@@ -112,12 +141,15 @@ __device__ __forceinline__ int fresh_lane() {
 
 #endif  // __HIP_DEVICE_COMPILE__
 
+template <Elem T>
 __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(const GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  constexpr bool BS = T == Elem::FP8_BLOCKSCALED;
+  constexpr int ELT = is_fp8(T) ? 1 : 2;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave >> 2, wn = wave & 3;
-  const int kbytes = p.k, steps = kbytes >> 7;
+  const int kbytes = p.k * ELT, steps = kbytes >> 7;
   const int tiles_n1 = (p.n + kTile - 1) / kTile, tiles_n = tiles_n1 * p.ngroups;
   const int grid = gridDim.x, bid = blockIdx.x;
   const int virt = (grid & 7) == 0 ? (bid & 7) * (grid >> 3) + (bid >> 3) : bid;
@@ -149,7 +181,7 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
       tile_carry = __builtin_amdgcn_readlane(tile_end, 63);
     }
     // (another form runs this launch)
-    if (p.by_splits && chunks <= stream_chunks_limit(active, p.by_splits, true, p.chunk_items, p.round_items)) return;
+    if (p.by_splits && chunks <= stream_chunks_limit(active, p.by_splits, is_fp8(T), p.chunk_items, p.round_items)) return;
     total_tiles = tile_carry;
   }
   // Full rounds run whole tiles; the tiles of the last, partly filled round are cut into two or four pieces when they still fit it.
@@ -252,9 +284,11 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
       if (r + 8 < t.rows) nxt1 = src[8];
       if (r + 16 < t.rows) nxt2 = src[16];
       if (r + 24 < t.rows) nxt3 = src[24];
-      const int rs = wn * 64 + fresh_lane();
-      nxts = 0;
-      if (rs < t.rows) nxts = a->gather_a[t.row0 + rs];
+      if constexpr (BS) {
+        const int rs = wn * 64 + fresh_lane();
+        nxts = 0;
+        if (rs < t.rows) nxts = a->gather_a[t.row0 + rs];
+      }
     }
   };
   auto rows_to_offsets = [&](const DualTile &t) {
@@ -274,13 +308,15 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
     nxt1 = offset(nxt1, 1);
     nxt2 = offset(nxt2, 2);
     nxt3 = offset(nxt3, 3);
-    const int rs = wn * 64 + l;
-    int64_t row = t.row0 + rs;
-    if (gathered) row = static_cast<int>(nxts) < 0 ? 0 : (static_cast<int>(nxts) >= a_rows ? a_rows - 1 : static_cast<int>(nxts));
-    const uint32_t off = a->a_scale_layout == FLUXMI_ASCALE_BLOCK128
-                             ? static_cast<uint32_t>(((row >> 7) * steps * 128 + (row & 127)) * 4)
-                             : static_cast<uint32_t>((static_cast<int64_t>(t.e_row0) * (steps - 1) + row) * 4);
-    nxts = rs < t.rows ? off : kNoRow;
+    if constexpr (BS) {
+      const int rs = wn * 64 + l;
+      int64_t row = t.row0 + rs;
+      if (gathered) row = static_cast<int>(nxts) < 0 ? 0 : (static_cast<int>(nxts) >= a_rows ? a_rows - 1 : static_cast<int>(nxts));
+      const uint32_t off = a->a_scale_layout == FLUXMI_ASCALE_BLOCK128
+                               ? static_cast<uint32_t>(((row >> 7) * steps * 128 + (row & 127)) * 4)
+                               : static_cast<uint32_t>((static_cast<int64_t>(t.e_row0) * (steps - 1) + row) * 4);
+      nxts = rs < t.rows ? off : kNoRow;
+    }
   };
   __amdgpu_buffer_rsrc_t xrsrc, wrsrc;
   uint32_t woff0, woff1, woff2, woff3;
@@ -306,11 +342,13 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
   const LdsInt stash = reinterpret_cast<LdsInt>(lds0 + kStash);
   auto put_next = [&]() {
     const int t = wave * 64 + fresh_lane();
-    stash[t] = nxt0, stash[512 + t] = nxt1, stash[1024 + t] = nxt2, stash[1536 + t] = nxt3, stash[2048 + t] = nxts;
+    stash[t] = nxt0, stash[512 + t] = nxt1, stash[1024 + t] = nxt2, stash[1536 + t] = nxt3;
+    if constexpr (BS) stash[2048 + t] = nxts;
   };
   auto get_next = [&]() {
     const int t = wave * 64 + fresh_lane();
-    nxt0 = stash[t], nxt1 = stash[512 + t], nxt2 = stash[1024 + t], nxt3 = stash[1536 + t], nxts = stash[2048 + t];
+    nxt0 = stash[t], nxt1 = stash[512 + t], nxt2 = stash[1024 + t], nxt3 = stash[1536 + t];
+    if constexpr (BS) nxts = stash[2048 + t];
   };
   uint32_t soff = 0;   // block scales: of the scale that this lane of the first group fetches
   int sstep = 0;       // ... and their distance between steps
@@ -380,7 +418,7 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
   rows_to_offsets(cur);
   start_x(cur);
   start_w(cur);
-  start_scales(cur);
+  if constexpr (BS) start_scales(cur);
   DualTile nx = next_tile();
   // Row scales of step st into slot st mod 3 (of the launch's steps).
   auto fill_scales = [&](uint32_t slot, int st) {
@@ -393,7 +431,7 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
     if (wm == 0) {
       fill_w(slot_of(4 * s + 1), s * 128);
       if (s == 0) fill_x(slot_of(3), 0);
-      fill_scales(s, s);
+      if constexpr (BS) fill_scales(s, s);
     } else {
       fill_x(slot_of(4 * s), s * 128);
       fill_w(slot_of(4 * s + 2), s * 128);
@@ -415,8 +453,8 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
     const bool wide = cur.wide;
     const int rows0 = cur.rows - wm * 64;  // rows of the tile from this wave's first on; 128 further on lies its second half
     // B's scales of this wave's columns.
-    int bs_index, bs_step;
-    {
+    int bs_index = 0, bs_step = 0;
+    if constexpr (BS) {
       const KernArgs a = kernel_args();
       const int nblocks = (a->n + 127) >> 7, first = (cur.n0 + (wide ? wn * 64 : 0)) >> 7, nb = first < nblocks ? first : nblocks - 1;
       if (a->b_scale_layout == FLUXMI_BSCALE_N_K) {
@@ -435,7 +473,7 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
         fw -= steps;
         if (fw == 0) {
           start_w(nx);
-          if (wm == 0) {
+          if (BS && wm == 0) {
             get_next();
             start_scales(nx);
           }
@@ -448,35 +486,44 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
           start_x(nx);
         }
       }
-      typedef const __attribute__((address_space(4))) float *ConstF32;
-      const float bscale = ((ConstF32)(kernel_args()->b_scale))[bs_index];
-      bs_index += bs_step;
-      float scale[4];
+      float scale[4], bscale = 1.f;
+      if constexpr (BS) {
+        typedef const __attribute__((address_space(4))) float *ConstF32;
+        bscale = ((ConstF32)(kernel_args()->b_scale))[bs_index];
+        bs_index += bs_step;
+      }
       auto read_scales = [&](int half) {
+        if constexpr (BS) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          scale[i] = *reinterpret_cast<const __attribute__((address_space(3))) float *>(sread + scale_slot * kScaleSlot + half * 512 + i * 64);
+          for (int i = 0; i < 4; ++i)
+            scale[i] = *reinterpret_cast<const __attribute__((address_space(3))) float *>(sread + scale_slot * kScaleSlot + half * 512 + i * 64);
+        }
       };
-      // What the waits count: a unit's fills are four instructions of a wave, and the first group's fills of a step's row scales follow
-      // those of X.  The first steps of a tile were waited for at its start.
+      auto scale_rows = [&]() {
+        if constexpr (BS) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) scale[i] *= bscale;
+        }
+      };
+      // What the waits count: a unit's fills are four instructions of a wave, and with block scales the first group's fills of a step's row
+      // scales, one each, follow those of X.  The first steps of a tile were waited for at its start.
       // Read: the first half's rows, all columns.  Reads before fills: the phase ends when the last of them is issued.
       read_x(slot_of(base));
       read_w(slot_of(base + 1), 0);
       read_w(slot_of(base + 2), 2);
       read_scales(0);
       fill_x(slot_of(base + 7 + wm), fx * 128);
-      if (wm == 0) fill_scales(scale_slot == 0 ? 2 : scale_slot - 1, fw);
+      if (BS && wm == 0) fill_scales(scale_slot == 0 ? 2 : scale_slot - 1, fw);
       FLUXMI_LGKM0();
-#pragma unroll
-      for (int i = 0; i < 4; ++i) scale[i] *= bscale;
+      scale_rows();
       sync();
       __builtin_amdgcn_s_setprio(1);
       if (rows0 > 0) {
-        quadrant<FS, 0, 0>(acc, x, w, scale);
-        if (wide) quadrant<FS, 0, 2>(acc, x, w, scale);
+        quadrant<T, FS, 0, 0>(acc, x, w, scale);
+        if (wide) quadrant<T, FS, 0, 2>(acc, x, w, scale);
       }
       __builtin_amdgcn_s_setprio(0);
-      if (wm == 0 && s > 0) FLUXMI_VMCNT(10);  // X's second half, requested in the step before: a scale fill and two units since
+      if (wm == 0 && s > 0) FLUXMI_VMCNT(BS ? 10 : 8);  // X's second half, requested in the step before: two units, and scales, since
       sync();
       // Read: the second half's rows.
       read_x(slot_of(base + 3));
@@ -484,19 +531,18 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
       fill_w(slot_of(base + wm), fw * 128);
       if (wm != 0 && s > 0) FLUXMI_VMCNT(8);  // the next step's X and W, requested two units ago and before
       FLUXMI_LGKM0();
-#pragma unroll
-      for (int i = 0; i < 4; ++i) scale[i] *= bscale;
+      scale_rows();
       sync();
       __builtin_amdgcn_s_setprio(1);
       if (rows0 > 128) {
-        quadrant<FS, 4, 0>(acc, x, w, scale);
-        if (wide) quadrant<FS, 4, 2>(acc, x, w, scale);
+        quadrant<T, FS, 4, 0>(acc, x, w, scale);
+        if (wide) quadrant<T, FS, 4, 2>(acc, x, w, scale);
       }
       __builtin_amdgcn_s_setprio(0);
-      if (wm == 0 && s > 0) FLUXMI_VMCNT(9);  // the next step's W, requested in the step before: two units and a scale fill since
+      if (wm == 0 && s > 0) FLUXMI_VMCNT(BS ? 9 : 8);  // the next step's W, requested in the step before: the same
       base = base + 4 >= kRing ? base + 4 - kRing : base + 4;
       scale_slot = scale_slot == 2 ? 0 : scale_slot + 1;
-      sync();
+      if (wm == 0 || s + 1 < steps) sync();
     };
     step(std::true_type{}, 0);
     for (int s = 1; s < steps; ++s) step(std::false_type{}, s);
@@ -513,9 +559,11 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
       const int32_t *scatter = a->scatter_d;
       const float tile_scale = scalar * (alpha ? alpha[cur.e] : 1.f);
       const bool f32 = a->d_fp32 != 0, nt = a->nt_stores != 0;
-      const int elt_out = f32 ? 4 : 2, cgrp = lane >> 4;
-      const int col0 = cur.n0 + (wide ? wn * 64 : wn * 32);  // first column of group 0; group 1: 32 further
-      int cols[4];                                            // first column of this lane in block j
+      const int cgrp = lane >> 4, rows = cur.rows - wm * 64 - (lane & 15);  // block i has a row of this lane if its first row is below that
+      const int col0 = cur.n0 + (wide ? wn * 64 : wn * 32);                 // first column of group 0; group 1: 32 further
+      const int first_row = cur.row0 + wm * 64 + (lane & 15);
+      // Everything that is read, before the first store: a load behind stores waits until those have drained.
+      int cols[4];  // first column of this lane in block j
       float4 cs[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -524,78 +572,96 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
         if (col_scale != nullptr && cols[j] < n && (j < 2 || wide))
           cs[j] = *reinterpret_cast<const float4 *>(col_scale + static_cast<int64_t>(cur.e) * n + cols[j]);
       }
+      float rs[8];
+      int out_row[8];  // -1: not stored
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int m = (i >> 2) * 128 + (i & 3) * 16;
+        rs[i] = 1.f;
+        out_row[i] = m < rows ? first_row + m : -1;
+        if (row_scale != nullptr && m < rows) rs[i] = row_scale[first_row + m];
+        if (scatter != nullptr && m < rows) {
+          const int to = scatter[first_row + m];
+          out_row[i] = to < a->d_rows ? to : -1;
+        }
+      }
       uint8_t *const d = static_cast<uint8_t *>(a->d[cur.g]);
+      const int64_t row_bytes = static_cast<int64_t>(n) * (f32 ? 4 : 2);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         if (i >= 4 && rows0 <= 128) break;
-        const int m = (i >> 2) * 128 + wm * 64 + (i & 3) * 16 + (lane & 15);
-        const bool have = m < cur.rows;
-        const int row = cur.row0 + m;
-        float rs = tile_scale;
-        if (row_scale != nullptr && have) rs *= row_scale[row];
-        int64_t drow = row;
-        bool store = have;
-        if (scatter != nullptr && have) {
-          drow = scatter[row];
-          store = drow >= 0 && drow < a->d_rows;
-        }
-        uint8_t *const drowp = d + drow * n * elt_out;
+        const float scale = tile_scale * rs[i];
+        uint8_t *const drow = d + out_row[i] * row_bytes;
 #pragma unroll
         for (int jg = 0; jg < 2; ++jg) {
           if (jg == 1 && !wide) break;
-          float4 v[2];
+          f32x4 v[2];
 #pragma unroll
           for (int j2 = 0; j2 < 2; ++j2) {
             const int j = jg * 2 + j2;
-            v[j2] = make_float4(acc[i][j][0] * rs, acc[i][j][1] * rs, acc[i][j][2] * rs, acc[i][j][3] * rs);
-            if (col_scale != nullptr) v[j2] = make_float4(v[j2].x * cs[j].x, v[j2].y * cs[j].y, v[j2].z * cs[j].z, v[j2].w * cs[j].w);
+            v[j2] = acc[i][j] * scale;
+            if (col_scale != nullptr) v[j2] = f32x4{v[j2][0] * cs[j].x, v[j2][1] * cs[j].y, v[j2][2] * cs[j].z, v[j2][3] * cs[j].w};
           }
+          if (out_row[i] < 0) continue;
           if (f32) {
 #pragma unroll
             for (int j2 = 0; j2 < 2; ++j2) {
               const int j = jg * 2 + j2;
-              if (store && cols[j] < n) {
-                const f32x4 ov = {v[j2].x, v[j2].y, v[j2].z, v[j2].w};
-                f32x4 *const dst = reinterpret_cast<f32x4 *>(drowp + static_cast<int64_t>(cols[j]) * 4);
-                if (nt) __builtin_nontemporal_store(ov, dst);
-                else *dst = ov;
-              }
+              if (cols[j] >= n) continue;
+              f32x4 *const dst = reinterpret_cast<f32x4 *>(drow + static_cast<int64_t>(cols[j]) * 4);
+              if (nt) __builtin_nontemporal_store(v[j2], dst);
+              else *dst = v[j2];
             }
-          } else if (store && cols[jg * 2] < n) {
-            const u32x4 o = {pack2(v[0].x, v[0].y), pack2(v[0].z, v[0].w), pack2(v[1].x, v[1].y), pack2(v[1].z, v[1].w)};
-            *reinterpret_cast<u32x4 *>(drowp + static_cast<int64_t>(cols[jg * 2]) * 2) = o;
+          } else if (cols[jg * 2] < n) {
+            const u32x4 o = {pack2<T>(v[0][0], v[0][1]), pack2<T>(v[0][2], v[0][3]), pack2<T>(v[1][0], v[1][1]), pack2<T>(v[1][2], v[1][3])};
+            *reinterpret_cast<u32x4 *>(drow + static_cast<int64_t>(cols[jg * 2]) * 2) = o;
           }
         }
       }
     }
-    if (nx.rows == 0) break;
+    // The second group ends its last phase with its results stored: the groups' stores are one pause, not two (2 to 4 %).
+    if (nx.rows == 0) {
+      sync();
+      break;
+    }
     cur = nx;
     nx = nx2;
     nx2 = next_tile();
+    if (wm != 0) sync();
   }
-  if (wm == 0) sync();
   FLUXMI_VMCNT(0);
 #endif  // __HIP_DEVICE_COMPILE__
+}
+
+template <Elem T>
+int launch(const GemmParams &p, int grid, hipStream_t s) {
+  static std::atomic<uint64_t> lds_done{0};
+  const int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(grouped_gemm_dual_kernel<T>), kDualLds, lds_done);
+  if (rc != FLUXMI_OK) return rc;
+  hipLaunchKernelGGL(grouped_gemm_dual_kernel<T>, dim3(grid), dim3(kDualThreads), kDualLds, s, p);
+  return FLUXMI_OK;
 }
 
 }  // namespace
 
 // Whole steps of K, at least two; offsets below kNoRow; 16-bit results in stores of 16 bytes.
-bool dual_takes(const GemmParams &p) {
-  const int64_t kbytes = p.k, span = 0x70000000ll;
-  if (p.a_scale == nullptr || p.accumulate || p.nexperts > kDualExperts || kbytes % 128 != 0 || kbytes < 256) return false;
+bool dual_takes(const GemmParams &p, int dtype) {
+  const int64_t kbytes = static_cast<int64_t>(p.k) * (dtype == FLUXMI_FP8_E4M3 ? 1 : 2), span = 0x70000000ll;
+  if (p.accumulate || p.nexperts > kDualExperts || kbytes % 128 != 0 || kbytes < 256) return false;
   if (kTile * kbytes > span || p.n * kbytes > span || (p.gather_a != nullptr && p.a_rows * kbytes > span)) return false;
   const int64_t scale_rows = p.gather_a != nullptr ? p.a_rows : p.max_rows;
-  if ((scale_rows + 127) / 128 * 128 * (kbytes / 128) * 4 > span) return false;
-  return p.d_fp32 || (p.n % 8 == 0 && aligned16(p.d[0]));
+  if (p.a_scale != nullptr && (scale_rows + 127) / 128 * 128 * (kbytes / 128) * 4 > span) return false;
+  if (p.d_fp32) return true;
+  bool aligned = p.n % 8 == 0;
+  for (int g = 0; g < p.ngroups; ++g) aligned = aligned && aligned16(p.d[g]);
+  return aligned;
 }
 
-int launch_grouped_gemm_dual(const GemmParams &p, int grid, hipStream_t s) {
-  static std::atomic<uint64_t> lds_done{0};
-  const int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(grouped_gemm_dual_kernel), kDualLds, lds_done);
-  if (rc != FLUXMI_OK) return rc;
-  hipLaunchKernelGGL(grouped_gemm_dual_kernel, dim3(grid), dim3(kDualThreads), kDualLds, s, p);
-  return FLUXMI_OK;
+int launch_grouped_gemm_dual(const GemmParams &p, int dtype, int grid, hipStream_t s) {
+  if (p.a_scale != nullptr) return launch<Elem::FP8_BLOCKSCALED>(p, grid, s);
+  if (dtype == FLUXMI_FP8_E4M3) return launch<Elem::FP8>(p, grid, s);
+  if (dtype == FLUXMI_FP16) return launch<Elem::F16>(p, grid, s);
+  return launch<Elem::BF16>(p, grid, s);
 }
 
 }  // namespace fluxmi

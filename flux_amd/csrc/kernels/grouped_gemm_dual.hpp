@@ -6,7 +6,7 @@
 namespace fluxmi {
 
 // Whether the dual tiles take a launch that is the macro tiles' otherwise.
-bool dual_takes(const GemmParams &p);
-int launch_grouped_gemm_dual(const GemmParams &p, int grid, hipStream_t s);
+bool dual_takes(const GemmParams &p, int dtype);
+int launch_grouped_gemm_dual(const GemmParams &p, int dtype, int grid, hipStream_t s);
 
 }  // namespace fluxmi

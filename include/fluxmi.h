@@ -137,9 +137,11 @@ typedef struct fluxmi_grouped_gemm_args {
   float scalar_scale;       /* host scalar, 1.0f for none (Flux `input_scale[0]` is passed by pointer below) */
   int32_t d_fp32;           /* 0: D is bf16 (fp16 for FLUXMI_FP16); 1: D is fp32 [max_rows, N] (unrounded layer1 intermediate) */
   const float *scalar_scale_dev; /* device [1] or NULL; multiplied in if given */
-  /* Launch tuning; all zero = defaults.  None of them changes a result bit.  raster_rows and sched_flags steer the macro-tile
-   * kernel; launches that another form computes (fluxmi_grouped_gemm_launch_info: the streaming form, the panel tiles) take no notice
-   * of them, whether they are left out or force something. */
+  /* Launch tuning; all zero = defaults.  None of them changes a result bit, with one exception below.  raster_rows and sched_flags steer
+   * the macro-tile kernel; launches that another form computes (fluxmi_grouped_gemm_launch_info: the streaming form, the panel tiles) take
+   * no notice of them, whether they are left out or force something.  The dual tiles (fluxmi_grouped_gemm_dual_tiles) follow raster_rows
+   * and FLUXMI_SCHED_WHOLE_TAIL_TILES.  The two flags for the ring's fills are about the macro-tile kernel itself and keep a launch on it:
+   * fp8 results can then differ in the last bit of their fp32 sums, as its MFMAs add K by 64 and the dual tiles' by 128. */
   int32_t cu_margin;     /* compute units left free for other work (Flux `sm_margin`) */
   int32_t raster_rows;   /* row tiles of an expert walked together over all weight panels; 0 = 8 */
   int32_t sched_flags;   /* FLUXMI_SCHED_* */

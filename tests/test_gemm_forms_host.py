@@ -177,3 +177,22 @@ def test_panel_tiles_of_256_columns_have_a_workgroup_per_item(dtype, experts, ro
         below, above = info(114912 * 256), info(114912 * 256 + 4)
         assert (below.cols, below.workgroups) == (256, 73 * 114912)
         assert (above.cols, above.workgroups) == (128, 256)
+
+
+@pytest.mark.parametrize("dtype,experts,rows,n,k,block_scaled,dual", [
+    (BF16, 8, 320, 14336, 4096, False, True), (BF16, 8, 321, 14336, 4096, False, False), (F16, 8, 512, 4096, 3072, False, False), (F16, 8, 512, 4096, 3008, False, True), (F16, 64, 1536, 2048, 1408, False, True),
+    (F16, 64, 1536, 1408, 2048, False, False), (BF16, 64, 768, 1408, 1984, False, True), (BF16, 64, 769, 1408, 1984, False, False),
+    (FP8, 32, 512, 2048, 7168, False, True), (FP8, 32, 513, 2048, 7168, False, False), (FP8, 32, 1024, 2048, 3072, False, True),
+    (FP8, 32, 4000, 7168, 2944, False, True), (FP8, 32, 4000, 7168, 7168, True, True),
+    # not whole steps of K, one step, columns that are not in eights, too many experts
+    (BF16, 8, 300, 4096, 4104, False, False), (FP8, 8, 300, 4096, 128, True, False), (BF16, 8, 300, 4100, 4096, False, False),
+    (FP8, 129, 300, 512, 512, True, False)])
+def test_dual_tiles_by_rows_and_k(dtype, experts, rows, n, k, block_scaled, dual):
+    def is_dual(**kw):
+        return capi.gemm_dual_tiles(dtype, experts, rows * experts, n, k, block_scaled=block_scaled, **kw)
+
+    assert capi.gemm_launch_info(dtype, experts, rows * experts, n, k, block_scaled=block_scaled).form == capi.GEMM_MACRO_TILES
+    assert is_dual() == is_dual(gathered=True) == dual
+    assert is_dual(d_fp32=True) == (dual or n % 8 != 0)
+    for flag in (capi.SCHED_HALF_LINE_FILLS, capi.SCHED_WHOLE_LINE_FILLS):
+        assert is_dual(sched_flags=flag) == (dual and block_scaled)

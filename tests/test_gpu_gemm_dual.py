@@ -19,10 +19,59 @@ CASES = [
     ("heights", [255, 256, 257, 64, 65, 128, 129, 193, 321, 0, 1, 1000, 190], 392, 384),
     ("two steps", [300], 136, 256),
     ("128 experts", [200, 0, 450] + [190] * 124 + [700], 264, 256),
-    ("long K, cut in two", [513, 511, 700, 448, 192], 2312, 2176),
+    ("long K, cut in two", [313, 511, 300, 248, 192], 2312, 2176),
     ("cut in four", [600, 1], 1032, 1152),
     ("several rounds", [1100, 900, 1300, 1024], 4104, 640),
 ]
+
+
+def is_dual(dtype, splits, n, k, **kw):
+    m, e = sum(splits), len(splits)
+    info = capi.gemm_launch_info(DT[dtype], e, m, n, k, splits=splits, block_scaled=dtype == "bs")
+    return info.form == capi.GEMM_MACRO_TILES and capi.gemm_dual_tiles(DT[dtype], e, m, n, k, block_scaled=dtype == "bs", **kw)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("name,splits,n,k", CASES, ids=[c[0] for c in CASES])
+def test_dual_tiles_are_exact_on_integers(name, splits, n, k, dtype):
+    print(f"[case] dual gemm {dtype} {name} n={n} k={k}", flush=True)
+    m, e = sum(splits), len(splits)
+    assert is_dual(dtype, splits, n, k)
+    assert not is_dual(dtype, splits, n, k, sched_flags=capi.SCHED_HALF_LINE_FILLS)
+    a, w, sp, g = made(splits, n, k, dtype, n + k)
+    ad, wd = a.to(DT[dtype]), w.to(DT[dtype])
+    want = product(a, w, splits)
+    assert torch.equal(capi.grouped_gemm(ad, wd, sp), want.float().to(capi._half_out(ad.dtype)))
+    perm = torch.randperm(m, generator=g, device="cuda").to(torch.int32)
+    to = perm.flip(0).contiguous()
+    row_scale = 2.0 ** torch.randint(-1, 2, (m,), generator=g, device="cuda").float()
+    col_scale = 2.0 ** torch.randint(-1, 2, (e, n), generator=g, device="cuda").float()
+    alpha = 2.0 ** torch.randint(-1, 2, (e,), generator=g, device="cuda").float()
+    expert = torch.repeat_interleave(torch.arange(e, device="cuda"), sp.long())
+    picked = torch.empty_like(want)
+    picked[to.long()] = product(a[perm.long()], w, splits) * (alpha[expert] * row_scale).double()[:, None] * col_scale[expert].double()
+    for margin, flags in ((0, 0), (40, capi.SCHED_WHOLE_TAIL_TILES), (253, 0)):
+        out = torch.full((m, n), -7.0, device="cuda")
+        capi.grouped_gemm(ad, wd, sp, out=out, gather_a=perm, scatter_d=to, row_scale=row_scale, col_scale=col_scale, alpha=alpha, cu_margin=margin,
+                          sched_flags=flags, raster_rows=margin // 40)
+        assert torch.equal(out.double(), picked), f"margin {margin}"
+    two = capi.grouped_gemm_multi(ad, [wd, wd.flip(0).contiguous()] if dtype != "fp8" else [wd, wd], sp, out_dtype=torch.float32)
+    assert torch.equal(two[0].double(), want)
+    assert torch.equal(two[1].double(), product(a, w.flip(0) if dtype != "fp8" else w, splits))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+@pytest.mark.parametrize("splits,n,k", [([200, 300, 64, 511], 1040, 2112), ([900, 700], 520, 1024), ([128, 470, 77], 2304, 8192)])
+def test_dual_tiles_have_the_macro_tiles_bits(splits, n, k, dtype):
+    print(f"[case] dual gemm bits {dtype} n={n} k={k}", flush=True)
+    assert is_dual(dtype, splits, n, k)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.randn(sum(splits), k, generator=g, device="cuda").to(DT[dtype])
+    w = torch.randn(len(splits), n, k, generator=g, device="cuda").to(DT[dtype])
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    for out in (torch.float32, DT[dtype]):
+        assert torch.equal(capi.grouped_gemm(a, w, sp, out_dtype=out),
+                           capi.grouped_gemm(a, w, sp, out_dtype=out, sched_flags=capi.SCHED_HALF_LINE_FILLS))
 
 
 @pytest.mark.parametrize("name,splits,n,k", CASES, ids=[c[0] for c in CASES])
@@ -31,8 +80,7 @@ CASES = [
 def test_dual_tiles_block_scaled_are_exact_on_integers(name, splits, n, k, a_layout, b_layout):
     print(f"[case] dual gemm block-scaled {name} n={n} k={k} layouts {a_layout} {b_layout}", flush=True)
     m, e = sum(splits), len(splits)
-    assert capi.gemm_launch_info(DT["bs"], e, m, n, k, splits=splits, block_scaled=True).form == capi.GEMM_MACRO_TILES
-    assert capi.gemm_dual_tiles(DT["bs"], e, m, n, k, block_scaled=True)
+    assert is_dual("bs", splits, n, k)
     a, w, sp, g = made(splits, n, k, "fp8", n + k)
     sa, sb, sad, sbd = block_scales(m, e, n, k, splits, a_layout, b_layout, g)
     af = a * torch.repeat_interleave(sa, 128, dim=1)
