@@ -33,7 +33,7 @@ EXPORTS = (
     "fluxmi_grouped_gemm_multi", "fluxmi_grouped_gemm_topk_reduce_workspace_bytes",
     "fluxmi_grouped_gemm_topk_reduce", "fluxmi_grouped_gemm_blockscale",
     "fluxmi_topk_gather_reduce", "fluxmi_quant_e4m3_rowwise", "fluxmi_quant_e4m3_square",
-    "fluxmi_quant_e4m3_block128", "fluxmi_calib_stream_sink_bytes", "fluxmi_calib_stream",
+    "fluxmi_quant_e4m3_block128", "fluxmi_quant_e4m3_block128_filled", "fluxmi_calib_stream_sink_bytes", "fluxmi_calib_stream",
 )
 
 
@@ -100,6 +100,7 @@ def load():
     lib.fluxmi_quant_e4m3_rowwise.argtypes = [vp, i64, i64, i32, f32, vp, vp, i32, vp]
     lib.fluxmi_quant_e4m3_square.argtypes = [vp, i64, i64, i64, f32, vp, vp, vp, vp, vp]
     lib.fluxmi_quant_e4m3_block128.argtypes = [vp, i64, i64, f32, vp, vp, vp, vp, vp]
+    lib.fluxmi_quant_e4m3_block128_filled.argtypes = lib.fluxmi_quant_e4m3_block128.argtypes
     lib.fluxmi_calib_stream_sink_bytes.restype = sz
     lib.fluxmi_calib_stream.argtypes = [vp, vp, sz, i32, vp]
     _lib = lib
@@ -452,14 +453,13 @@ def quant_e4m3_block128(x, eps=0.0, transpose=False):
     rows, cols = x.shape
     nby, nbx = (rows + 127) // 128, (cols + 127) // 128
     q = torch.empty(rows, cols, dtype=torch.float8_e4m3fn, device=x.device)
-    alloc = lambda n, *shape: (torch.zeros if n % 128 else torch.empty)(*shape, dtype=torch.float32, device=x.device)
-    si = alloc(rows, nby, nbx, 128)  # entries past the last row of the last block are not written
+    si = torch.empty(nby, nbx, 128, dtype=torch.float32, device=x.device)  # entries past the last row are 0
     qt = sit = None
     if transpose:
         qt = torch.empty(cols, rows, dtype=torch.float8_e4m3fn, device=x.device)
-        sit = alloc(cols, nbx, nby, 128)
-    _check(lib.fluxmi_quant_e4m3_block128(_ptr(x), rows, cols, float(eps), _ptr(q), _ptr(si), _ptr(qt), _ptr(sit),
-                                          _stream()), "fluxmi_quant_e4m3_block128")
+        sit = torch.empty(nbx, nby, 128, dtype=torch.float32, device=x.device)
+    _check(lib.fluxmi_quant_e4m3_block128_filled(_ptr(x), rows, cols, float(eps), _ptr(q), _ptr(si), _ptr(qt), _ptr(sit),
+                                                 _stream()), "fluxmi_quant_e4m3_block128_filled")
     return q, si, qt, sit
 
 

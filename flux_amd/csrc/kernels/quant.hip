@@ -369,6 +369,9 @@ __global__ __launch_bounds__(256) void quant_square_kernel(const uint16_t *__res
 // Measured, both outputs: 11000 x 7168 186 -> 56 us (5.6 TB/s; a copy of as many bytes takes 53 to 61 us), 4096 x 7168 36.8 -> 24.4, 1000 x 2048 15 -> 7;
 // without the transposed output 16384 x 7168 64.5 -> 60.3, 16384 x 2048 22.6 -> 19.0.  104 registers, four waves per SIMD: held to
 // 96 or 80 the compiler spills (70 and 109 us).
+// `fill` writes 0 to the scales of rows (columns) past the end, which the last tiles hold anyway: a caller that wants
+// them 0 had a fill launch before this one (11000 x 7168 with
+// both outputs as a torch call: 57.3 us with the fill launch, 55.2 without; small matrices 33.0 -> 29.5).
 // Scales are stored as [ceil(rows/128)][ceil(cols/128)][128] (row inside its block fastest), the
 // transposed ones as [ceil(cols/128)][ceil(rows/128)][128].  scale_inv is the fp32 quotient 1.0f / scale:
 // equal to the reference's float(1.0 / double(scale)), since a quotient rounded to 53 bits and then to 24
@@ -384,7 +387,7 @@ __global__ __launch_bounds__(256) void quant_block128_tile_kernel(const uint16_t
                                                                   float eps, uint8_t *__restrict__ q,
                                                                   float *__restrict__ scale_inv,
                                                                   uint8_t *__restrict__ q_t,
-                                                                  float *__restrict__ scale_inv_t) {
+                                                                  float *__restrict__ scale_inv_t, bool fill) {
   __shared__ __attribute__((aligned(16))) uint32_t s_col[TRANSPOSE ? 4 * 64 : 4];  // a pair of columns per word
   __shared__ __attribute__((aligned(16))) float s_scale[TRANSPOSE ? 128 : 4];
   __shared__ __attribute__((aligned(16))) uint8_t s_t[TRANSPOSE ? 128 * 128 : 16];
@@ -424,9 +427,9 @@ __global__ __launch_bounds__(256) void quant_block128_tile_kernel(const uint16_t
     if (((cg >> 1) & 3) == i) key = pair;
   }
   const float row_scale = compute_scale(key_to_float((cg & 1) ? key >> 16 : key & 0xffffu), eps);
-  if (cg < 8 && r0 + cg < rows)
+  if (cg < 8 && (fill || r0 + cg < rows))
     scale_inv[static_cast<int64_t>(tile.by) * (static_cast<int64_t>(nbx) * 128) + static_cast<int64_t>(tile.bx) * 128 + rg * 8 + cg] =
-        1.0f / row_scale;
+        r0 + cg < rows ? 1.0f / row_scale : 0.0f;
   const float sc[8] = {row16_broadcast<0>(row_scale), row16_broadcast<1>(row_scale), row16_broadcast<2>(row_scale),
                        row16_broadcast<3>(row_scale), row16_broadcast<4>(row_scale), row16_broadcast<5>(row_scale),
                        row16_broadcast<6>(row_scale), row16_broadcast<7>(row_scale)};
@@ -437,9 +440,10 @@ __global__ __launch_bounds__(256) void quant_block128_tile_kernel(const uint16_t
       const uint32_t m = max(max(col[0], col[128]), max(col[256], col[384]));  // non-negative keys: unsigned order
       const float scale = compute_scale(key_to_float(m), eps);
       s_scale[threadIdx.x] = scale;
-      if (static_cast<int64_t>(tile.bx) * 128 + threadIdx.x < cols)
+      const bool inside = static_cast<int64_t>(tile.bx) * 128 + threadIdx.x < cols;
+      if (fill || inside)
         scale_inv_t[static_cast<int64_t>(tile.bx) * (static_cast<int64_t>(nby) * 128) + static_cast<int64_t>(tile.by) * 128 +
-                    threadIdx.x] = 1.0f / scale;
+                    threadIdx.x] = inside ? 1.0f / scale : 0.0f;
     }
   }
 #pragma unroll
@@ -582,10 +586,10 @@ extern "C" int fluxmi_quant_e4m3_square(const void *x_bf16, int64_t batch, int64
   return FLUXMI_OK;
 }
 
-extern "C" int fluxmi_quant_e4m3_block128(const void *x_bf16, int64_t rows, int64_t cols, float eps,
-                                          void *q_out, float *scale_inv_out, void *q_t_out,
-                                          float *scale_inv_t_out, void *stream) {
-  using namespace fluxmi;
+namespace fluxmi {
+namespace {
+int quant_block128(const void *x_bf16, int64_t rows, int64_t cols, float eps, void *q_out, float *scale_inv_out,
+                   void *q_t_out, float *scale_inv_t_out, bool fill, void *stream) {
   FLUXMI_REQUIRE(x_bf16 != nullptr && q_out != nullptr && scale_inv_out != nullptr,
                  FLUXMI_ERR_INVALID_ARG, "quant_e4m3_block128: null pointer argument");
   FLUXMI_REQUIRE((q_t_out == nullptr) == (scale_inv_t_out == nullptr), FLUXMI_ERR_INVALID_ARG,
@@ -609,7 +613,7 @@ extern "C" int fluxmi_quant_e4m3_block128(const void *x_bf16, int64_t rows, int6
 #define FLUXMI_B128(V, T, VT)                                                                          \
   hipLaunchKernelGGL((quant_block128_tile_kernel<V, T, VT>), grid, block, 0, s, x, rows, cols,         \
                      static_cast<int32_t>(nbx), static_cast<int32_t>(nby), eps, q, scale_inv_out, qt,  \
-                     scale_inv_t_out)
+                     scale_inv_t_out, fill)
   if (qt == nullptr) {
     if (vec) FLUXMI_B128(true, false, false);
     else FLUXMI_B128(false, false, false);
@@ -623,4 +627,18 @@ extern "C" int fluxmi_quant_e4m3_block128(const void *x_bf16, int64_t rows, int6
 #undef FLUXMI_B128
   FLUXMI_HIP_CHECK(hipGetLastError());
   return FLUXMI_OK;
+}
+}  // namespace
+}  // namespace fluxmi
+
+extern "C" int fluxmi_quant_e4m3_block128(const void *x_bf16, int64_t rows, int64_t cols, float eps,
+                                          void *q_out, float *scale_inv_out, void *q_t_out,
+                                          float *scale_inv_t_out, void *stream) {
+  return fluxmi::quant_block128(x_bf16, rows, cols, eps, q_out, scale_inv_out, q_t_out, scale_inv_t_out, false, stream);
+}
+
+extern "C" int fluxmi_quant_e4m3_block128_filled(const void *x_bf16, int64_t rows, int64_t cols, float eps,
+                                                 void *q_out, float *scale_inv_out, void *q_t_out,
+                                                 float *scale_inv_t_out, void *stream) {
+  return fluxmi::quant_block128(x_bf16, rows, cols, eps, q_out, scale_inv_out, q_t_out, scale_inv_t_out, true, stream);
 }

@@ -360,6 +360,11 @@ int fluxmi_quant_e4m3_square(const void *x_bf16, int64_t batch, int64_t rows, in
 int fluxmi_quant_e4m3_block128(const void *x_bf16, int64_t rows, int64_t cols, float eps, void *q_out,
                                float *scale_inv_out, void *q_t_out, float *scale_inv_t_out, void *stream);
 
+/* The same, and the scale entries of rows (transposed: columns) past the end are written as 0: what
+ * `Quantization::quantize_vector_blockwise` returns, without a fill of the scales before the call. */
+int fluxmi_quant_e4m3_block128_filled(const void *x_bf16, int64_t rows, int64_t cols, float eps, void *q_out,
+                                      float *scale_inv_out, void *q_t_out, float *scale_inv_t_out, void *stream);
+
 /* ------------------------------------------------------------------------------------------------
  * Calibration streams (no counterpart in the reference; for benchmarks): what the memory system of the GPU at
  * hand gives a kernel that only streams.  copy == 0: every byte of src[0, bytes) is read once (16 bytes per lane

@@ -208,6 +208,31 @@ def test_block128_with_transposed_output(rows, cols, eps):
         assert torch.equal(q3.view(torch.uint8), q.view(torch.uint8)) and torch.equal(s3, s)
 
 
+@pytest.mark.parametrize("rows,cols", [(128, 256), (1, 8), (127, 136), (129, 130), (255, 127), (300, 1000)])
+def test_block128_scales_past_the_end(rows, cols):
+    """The filled form writes 0 to the scales of rows and columns past the end and touches nothing behind the
+    scales; the other form leaves those entries as they were.  Everything else is the same."""
+    from flux_amd import capi
+    print(f"[case] quant block128 past the end rows={rows} cols={cols}", flush=True)
+    lib = capi.load()
+    x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows + cols)).to(torch.bfloat16).cuda()
+    nby, nbx = -(-rows // 128), -(-cols // 128)
+    got = {}
+    for name in ("fluxmi_quant_e4m3_block128", "fluxmi_quant_e4m3_block128_filled"):
+        q, qt = (torch.empty(rows * cols, dtype=torch.uint8, device="cuda") for _ in range(2))
+        si, sit = (torch.full((nby * nbx * 128 + 128,), -7.0, device="cuda") for _ in range(2))
+        args = [x.data_ptr(), rows, cols, 0.0, q.data_ptr(), si.data_ptr(), qt.data_ptr(), sit.data_ptr()]
+        assert getattr(lib, name)(*args, torch.cuda.current_stream().cuda_stream) == 0
+        got[name] = [t.cpu() for t in (q, qt, si, sit)]
+    plain, filled = got.values()
+    assert torch.equal(plain[0], filled[0]) and torch.equal(plain[1], filled[1])
+    for p, f, n, a, b in ((plain[2], filled[2], rows, nby, nbx), (plain[3], filled[3], cols, nbx, nby)):
+        assert bool((p[-128:] == -7.0).all()) and bool((f[-128:] == -7.0).all())
+        p, f = (t[:-128].view(a, b, 128).transpose(1, 2).reshape(a * 128, b) for t in (p, f))
+        assert torch.equal(p[:n], f[:n]) and bool((p[:n] > 0).all())
+        assert bool((p[n:] == -7.0).all()) and bool((f[n:] == 0.0).all())
+
+
 def test_block128_all_bit_patterns_both_directions():
     """All 65536 bf16 patterns as a 256 x 256 matrix through the fused kernel: tiny amax (scale saturates at the
     bf16 maximum, scale_inv denormal), inf (scale 0) and NaN, along rows and along columns."""
