@@ -28,7 +28,7 @@ EXPORTS = (
     "fluxmi_moe_route_sort_workspace_bytes", "fluxmi_moe_route_sort", "fluxmi_moe_gather_index",
     "fluxmi_moe_route_sort_static_max_bytes", "fluxmi_moe_route_sort_static_init", "fluxmi_moe_route_sort_static",
     "fluxmi_grouped_gemm_workspace_bytes", "fluxmi_grouped_gemm", "fluxmi_grouped_gemm_kernel_kind",
-    "fluxmi_grouped_gemm_host_splits", "fluxmi_grouped_gemm_launch_info", "fluxmi_grouped_gemm_panel_info",
+    "fluxmi_grouped_gemm_host_splits", "fluxmi_grouped_gemm_host_counts", "fluxmi_grouped_gemm_launch_info", "fluxmi_grouped_gemm_panel_info",
     "fluxmi_grouped_gemm_dual_tiles",
     "fluxmi_grouped_gemm_multi", "fluxmi_grouped_gemm_topk_reduce_workspace_bytes",
     "fluxmi_grouped_gemm_topk_reduce", "fluxmi_grouped_gemm_blockscale",
@@ -90,6 +90,7 @@ def load():
     lib.fluxmi_grouped_gemm_launch_info.argtypes = [ctypes.POINTER(GroupedGemmArgs), i32, vp, vp, i32,
                                                     ctypes.POINTER(GemmLaunchInfo)]
     lib.fluxmi_grouped_gemm_host_splits.argtypes = [ctypes.POINTER(GroupedGemmArgs), vp, vp, vp, i32, vp, i32, vp]
+    lib.fluxmi_grouped_gemm_host_counts.argtypes = lib.fluxmi_grouped_gemm_host_splits.argtypes
     lib.fluxmi_grouped_gemm_panel_info.argtypes = [ctypes.POINTER(GroupedGemmArgs), i32, vp, vp, i32, ctypes.POINTER(GemmPanelInfo)]
     lib.fluxmi_grouped_gemm_topk_reduce_workspace_bytes.restype = sz
     lib.fluxmi_grouped_gemm_topk_reduce_workspace_bytes.argtypes = [i32, i32]

@@ -14,7 +14,7 @@ void set_error(const char *fmt, ...) {
 }
 }  // namespace fluxmi
 
-extern "C" int fluxmi_version(void) { return 115; }
+extern "C" int fluxmi_version(void) { return 116; }
 
 extern "C" const char *fluxmi_last_error(void) { return fluxmi::g_last_error; }
 

@@ -41,6 +41,11 @@ constexpr int kTables = kUnit * kRing + 3 * kScaleSlot, kStash = kTables + 2 * k
 constexpr int kDualLds = kStash + 5 * 4 * kDualThreads;
 constexpr uint32_t kNoRow = 0x80000000u;  // a byte offset past every operand, with offsets along K still below 2^32
 
+struct DualArgs {
+  GemmParams p;
+  FewRowsArgs few;
+};
+
 #if defined(__HIP_DEVICE_COMPILE__)
 
 #define FLUXMI_VMCNT(vm) __builtin_amdgcn_s_waitcnt(((vm)&15) | (((vm) >> 4) << 14) | (7 << 4) | (15 << 8))
@@ -125,12 +130,16 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
 }
 
 // The kernel's argument, read again where it is used; the empty asm keeps the compiler from keeping copies in registers through the loop.
+typedef const __attribute__((address_space(4))) DualArgs *DualArgSegment;
 typedef const __attribute__((address_space(4))) GemmParams *KernArgs;
-__device__ __forceinline__ KernArgs kernel_args() {
-  KernArgs k = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+typedef const __attribute__((address_space(4))) FewRowsArgs *FewArgs;
+__device__ __forceinline__ DualArgSegment all_args() {
+  DualArgSegment k = (DualArgSegment)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(k));
   return k;
 }
+__device__ __forceinline__ KernArgs kernel_args() { return &all_args()->p; }
+__device__ __forceinline__ FewArgs few_args() { return &all_args()->few; }
 
 // The lane, opaque to the compiler: what is computed from it is not moved out of the tile loop, where it would occupy registers.
 __device__ __forceinline__ int fresh_lane() {
@@ -142,8 +151,9 @@ __device__ __forceinline__ int fresh_lane() {
 #endif  // __HIP_DEVICE_COMPILE__
 
 template <Elem T>
-__global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(const GemmParams p) {
+__global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(const DualArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  const GemmParams &p = args.p;
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   constexpr bool BS = T == Elem::FP8_BLOCKSCALED;
   constexpr int ELT = is_fp8(T) ? 1 : 2;
@@ -164,7 +174,8 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int ee = c * 64 + lane;
-      int r = ee < p.nexperts ? p.splits[ee] : 0;
+      int r = 0;
+      if (ee < p.nexperts) r = few_args()->count > 0 ? few_args()->splits[ee] : p.splits[ee];
       if (r < 0) r = 0;
       const int incl = wave_inclusive_scan(r);
       int begin = row_carry + incl - r, end = row_carry + incl;
@@ -564,7 +575,7 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
     {
       const KernArgs a = kernel_args();
       const int lane = fresh_lane(), n = a->n;
-      const float *alpha = a->alpha[cur.g], *row_scale = a->row_scale, *col_scale = a->col_scale;
+      const float *alpha = a->alpha[cur.g], *row_scale = a->row_scale, *row_scale2 = few_args()->row_scale2, *col_scale = a->col_scale;
       const int32_t *scatter = a->scatter_d;
       const float tile_scale = scalar * (alpha ? alpha[cur.e] : 1.f);
       const bool f32 = a->d_fp32 != 0, nt = a->nt_stores != 0;
@@ -589,6 +600,7 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
         rs[i] = 1.f;
         out_row[i] = m < rows ? first_row + m : -1;
         if (row_scale != nullptr && m < rows) rs[i] = row_scale[first_row + m];
+        if (row_scale2 != nullptr && m < rows) rs[i] *= row_scale2[first_row + m];
         if (scatter != nullptr && m < rows) {
           const int to = scatter[first_row + m];
           out_row[i] = to < a->d_rows ? to : -1;
@@ -643,11 +655,11 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
 }
 
 template <Elem T>
-int launch(const GemmParams &p, int grid, hipStream_t s) {
+int launch(const GemmParams &p, const FewRowsArgs &few, int grid, hipStream_t s) {
   static std::atomic<uint64_t> lds_done{0};
   const int rc = ensure_dynamic_lds(reinterpret_cast<const void *>(grouped_gemm_dual_kernel<T>), kDualLds, lds_done);
   if (rc != FLUXMI_OK) return rc;
-  hipLaunchKernelGGL(grouped_gemm_dual_kernel<T>, dim3(grid), dim3(kDualThreads), kDualLds, s, p);
+  hipLaunchKernelGGL(grouped_gemm_dual_kernel<T>, dim3(grid), dim3(kDualThreads), kDualLds, s, DualArgs{p, few});
   return FLUXMI_OK;
 }
 
@@ -666,11 +678,11 @@ bool dual_takes(const GemmParams &p, int dtype) {
   return aligned;
 }
 
-int launch_grouped_gemm_dual(const GemmParams &p, int dtype, int grid, hipStream_t s) {
-  if (p.a_scale != nullptr) return launch<Elem::FP8_BLOCKSCALED>(p, grid, s);
-  if (dtype == FLUXMI_FP8_E4M3) return launch<Elem::FP8>(p, grid, s);
-  if (dtype == FLUXMI_FP16) return launch<Elem::F16>(p, grid, s);
-  return launch<Elem::BF16>(p, grid, s);
+int launch_grouped_gemm_dual(const GemmParams &p, const FewRowsArgs &few, int dtype, int grid, hipStream_t s) {
+  if (p.a_scale != nullptr) return launch<Elem::FP8_BLOCKSCALED>(p, few, grid, s);
+  if (dtype == FLUXMI_FP8_E4M3) return launch<Elem::FP8>(p, few, grid, s);
+  if (dtype == FLUXMI_FP16) return launch<Elem::F16>(p, few, grid, s);
+  return launch<Elem::BF16>(p, few, grid, s);
 }
 
 }  // namespace fluxmi

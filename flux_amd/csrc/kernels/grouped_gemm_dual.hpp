@@ -7,6 +7,7 @@ namespace fluxmi {
 
 // Whether the dual tiles take a launch that is the macro tiles' otherwise.
 bool dual_takes(const GemmParams &p, int dtype);
-int launch_grouped_gemm_dual(const GemmParams &p, int dtype, int grid, hipStream_t s);
+// few: row counts in the arguments (count > 0) and a second factor per row, as the forms for few rows take them.
+int launch_grouped_gemm_dual(const GemmParams &p, const FewRowsArgs &few, int dtype, int grid, hipStream_t s);
 
 }  // namespace fluxmi

@@ -156,8 +156,8 @@ bool run_host_splits(const fluxmi_grouped_gemm_args &args, const torch::Tensor &
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
   if (splits.is_cuda() || splits.is_pinned()) return false;
-  const int rc = fluxmi_grouped_gemm_host_splits(&args, splits.data_ptr<int32_t>(), row_scale2, a_scale, a_layout, b_scale, b_layout, stream);
-  if (rc < 0) check_status(rc, "fluxmi_grouped_gemm_host_splits");
+  const int rc = fluxmi_grouped_gemm_host_counts(&args, splits.data_ptr<int32_t>(), row_scale2, a_scale, a_layout, b_scale, b_layout, stream);
+  if (rc < 0) check_status(rc, "fluxmi_grouped_gemm_host_counts");
   return rc == 1;
 }
 
@@ -451,7 +451,7 @@ torch::Tensor GemmGroupedV3GatherRS::forward_impl(
       else if (is.numel() == m) row_factors[row_factors[0] != nullptr ? 1 : 0] = is.data_ptr<float>();
       else TORCH_CHECK(false, "input_scale must be [1] or [M]");
     }
-    // With few rows per expert one kernel takes the row counts and both factors of a row as they are.
+    // With few rows per expert, and on the dual tiles, one kernel takes the row counts and both factors of a row as they are.
     if (!fused) {
       const fluxmi_grouped_gemm_args args = gemm_args(inputs[g], weights[g], nullptr, inter_[g], nullptr, m, alpha, row_factors[0], col, scalar,
                                                       sm_margin);

@@ -177,6 +177,12 @@ int fluxmi_grouped_gemm_host_splits(const fluxmi_grouped_gemm_args *args, const 
                                     const float *a_scale, int32_t a_scale_layout, const float *b_scale, int32_t b_scale_layout,
                                     void *stream);
 
+/* fluxmi_grouped_gemm_host_splits, and launches that the dual tiles compute (fluxmi_grouped_gemm_dual_tiles) take the counts and row_scale2 in the
+ * kernel's arguments as well: returns 1 for them without args->splits, too. */
+int fluxmi_grouped_gemm_host_counts(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, const float *row_scale2,
+                                    const float *a_scale, int32_t a_scale_layout, const float *b_scale, int32_t b_scale_layout,
+                                    void *stream);
+
 /* Which form of the kernels computes a launch and how the streaming form is launched.  Host only: nothing is
  * launched, no device is needed, and pointers in `args` are only looked at for their alignment (b and d stand for every
  * weight group).  a_scale: non-NULL for fluxmi_grouped_gemm_blockscale with MFMA-kernel layouts.  splits_host: host copy of

@@ -122,3 +122,44 @@ def test_dual_tiles_do_not_touch_rows_past_the_splits():
     out.fill_(-5)
     call([400, 0, 300, 0])
     assert torch.equal(out[:700].double(), product(a[:700], w, [400, 0, 300, 0])) and bool((out[700:] == -5).all())
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8", "bs"])
+@pytest.mark.parametrize("splits,n,k,done", [([600, 0, 500, 557], 392, 384, 1), ([-3, 700, 900, 1], 264, 256, 1), ([600, 500, 700], 136, 256, 1),
+                                             ([250] * 128, 264, 256, 1), ([250] * 129, 264, 256, 0), ([700, 600], 264, 320, 0)])
+def test_dual_tiles_take_row_counts_from_the_host(dtype, splits, n, k, done):
+    """Counts and a second factor per row in the kernel's arguments: the bits of the ordinary call with the factors' product.  Not for more
+    experts than the arguments hold nor (K = 320, in fp8 no whole lines) for other forms; nothing is launched then."""
+    if dtype == "bs" and k % 128:
+        pytest.skip("block scales have whole blocks of K")
+    print(f"[case] dual gemm, counts in the arguments {dtype} {splits[:4]} n={n} k={k}", flush=True)
+    if dtype != "fp8" and k == 320:
+        done = 1
+    if dtype == "bs":
+        n = (n + 127) // 128 * 128
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    m, e = sum(max(0, r) for r in splits) - (100 if splits == [600, 500, 700] else 0), len(splits)  # or fewer rows than the counts say
+    x = torch.randn(m, k, generator=g, device="cuda").to(DT[dtype])
+    w = (torch.randn(e, n, k, generator=g, device="cuda") * 0.05).to(DT[dtype])
+    sa, sb = torch.rand((m + 127) // 128, k // 128, 128, generator=g, device="cuda"), torch.rand(e, (n + 127) // 128, k // 128, generator=g, device="cuda")
+    r1, r2 = (torch.rand(m, generator=g, device="cuda") + 0.5 for _ in range(2))
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    want = torch.full((m, n), -1.0, device="cuda")
+    if dtype == "bs": capi.grouped_gemm_blockscale(x, w, sp, sa, sb, out=want)
+    else: capi.grouped_gemm(x, w, sp, out=want, row_scale=r1 * r2)
+    args, out = capi._gemm_args(x, w, sp, None, None, None, None, None if dtype == "bs" else r1, None, 1.0, None, None, torch.float32, 0, 0, 0)
+    host, on_device = (ctypes.c_int32 * e)(*splits), args.splits
+    scales = [capi._ptr(sa), capi.ASCALE_BLOCK128, capi._ptr(sb), capi.BSCALE_N_K] if dtype == "bs" else [None, 0, None, 0]
+    call = lambda entry, second: getattr(capi.load(), entry)(ctypes.byref(args), host, second, *scales, capi._stream())
+    args.splits = None
+    out.fill_(-1)
+    second = None if dtype == "bs" else capi._ptr(r2)
+    assert call("fluxmi_grouped_gemm_host_splits", second) == 0
+    assert bool((out == -1).all())
+    assert call("fluxmi_grouped_gemm_host_counts", second) == done
+    assert torch.equal(out, want) if done else bool((out == -1).all())
+    args.splits, r12 = on_device, r1 * r2  # with the counts on the device as well
+    if dtype != "bs": args.row_scale = r12.data_ptr()
+    out.fill_(-1)
+    assert call("fluxmi_grouped_gemm_host_counts", None) == 1
+    assert torch.equal(out, want)
