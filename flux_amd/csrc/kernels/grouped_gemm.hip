@@ -128,15 +128,23 @@ struct DryRun {
   PanelPlan panel = {};
 };
 
-// Whether a form for few rows per expert, with chunks of chunk_rows rows, computes a launch with these splits.
-bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, int chunk_rows, const PanelPlan &panel) {
-  int left = args->max_rows, chunks = 0, active = 0;
+// Chunks of up to chunk_rows rows of a launch with these splits, and the experts that have rows.
+int count_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, int chunk_rows, int &active) {
+  int left = args->max_rows, chunks = 0;
+  active = 0;
   for (int e = 0; e < args->nexperts; ++e) {
     const int rows = splits_host[e] < 0 ? 0 : (splits_host[e] < left ? splits_host[e] : left);
     left -= rows;
     active += rows > 0 ? 1 : 0;
     chunks += (rows + chunk_rows - 1) / chunk_rows;
   }
+  return chunks;
+}
+
+// Whether a form for few rows per expert, with chunks of chunk_rows rows, computes a launch with these splits.
+bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host, int chunk_rows, const PanelPlan &panel) {
+  int active;
+  const int chunks = count_chunks(args, splits_host, chunk_rows, active);
   return chunks <= stream_chunks_limit(active, chunk_rows, args->dtype == FLUXMI_FP8_E4M3, panel.chunk_items, panel.round_items);
 }
 
@@ -300,6 +308,10 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
       few.row_scale2 = host->row_scale2;
       few.count = args->nexperts;
       for (int e = 0; e < args->nexperts; ++e) few.splits[e] = host->splits[e];
+      if (computes && panel.cols != 0) {
+        int active;
+        set_chunks(p, count_chunks(args, host->splits, panel.chunk_rows, active), cus, panel);
+      }
     } else {
       if (args->splits == nullptr) return 0;
       FLUXMI_REQUIRE(host->row_scale2 == nullptr, FLUXMI_ERR_UNSUPPORTED, "grouped_gemm_host_splits: row_scale2 with splits on the device");

@@ -504,6 +504,10 @@ int launch_by_plan(const GemmParams &p, const FewRowsArgs &few, const PanelPlan 
     return plan.pairs ? launch<T, 2, 1, 6, 4>(p, few, plan, s) : launch<T, 2, 1, 4, 4>(p, few, plan, s);
   }
   if (wide) return plan.sums == 4 ? launch<T, 4, 2, 3, 4>(p, few, plan, s) : launch<T, 4, 2, 3, 1>(p, few, plan, s);
+  if constexpr (T != Elem::FP8_BLOCKSCALED)
+    if (plan.deep)
+      return plan.sums == 8 ? launch<T, 4, 1, 6, 8>(p, few, plan, s)
+                            : (plan.sums == 4 ? launch<T, 4, 1, 6, 4>(p, few, plan, s) : launch<T, 4, 1, 6, 1>(p, few, plan, s));
   return plan.sums == 8 ? launch<T, 4, 1, 4, 8>(p, few, plan, s)
                         : (plan.sums == 4 ? launch<T, 4, 1, 4, 4>(p, few, plan, s) : launch<T, 4, 1, 4, 1>(p, few, plan, s));
 }
@@ -514,6 +518,7 @@ int lds_of(const PanelPlan &plan) {
   if (plan.cols == 256) return lds_bytes<T, 8, 4, 0>();
   if (plan.cols == 128) return blocks16 <= 2 ? lds_bytes<T, 2, 2, kDepth32<T>>() : (blocks16 <= 4 ? lds_bytes<T, 4, 2, 3>() : lds_bytes<T, 8, 2, 3>());
   if (blocks16 <= 2 && plan.pairs) return lds_bytes<T, 2, 1, 6>();
+  if (plan.deep) return lds_bytes<T, 4, 1, 6>();
   return blocks16 <= 2 ? lds_bytes<T, 2, 1, 4>() : (blocks16 <= 4 ? lds_bytes<T, 4, 1, 4>() : lds_bytes<T, 8, 1, 3>());
 }
 
@@ -547,6 +552,15 @@ int64_t block_count(const GemmParams &p, int dtype, const PanelPlan &plan) {
 // Whether the workgroups of a launch walk several items: compute units are to be left free, or it would have 2^31 threads and more.
 bool walks(int64_t blocks, bool leave_cus) { return leave_cus || blocks * 256 > 0x7fffffffll; }
 
+// A ring of six stages, lines in pairs: 96 KiB, so one workgroup to a unit, which is all there is where no unit gets two.  A line then costs its wait, barrier
+// and chain of reads and MFMAs (0.2 us), and pairs halve the waits.  us per launch, weights not in the cache, four stages line by line / six in
+// pairs / eight in pairs: bf16 8 experts 1024 x 2048, R 16 13.6 / 12.3 / 12.0, R 64 16.0 / 15.1 / 15.7; 4 experts 2048 x 1024, R 48 10.2 / 9.7 / 10.1; fp8 8
+// experts 1024 x 2048, R 64 11.0 / 10.4 / 11.1; fp16 4 experts 1024 x 4096, R 80 24.9 / 22.3 / 22.6.  Eight stages line by line 17.5, 11.6, 12.1, 26.2: more to
+// ask for before the first line.  Block-scaled 13.4 / 13.4 / 14.1: four stages.
+bool is_deep(const PanelPlan &plan, int64_t blocks, bool block_scaled, int cus) {
+  return plan.cols == 64 && plan.chunk_rows == 64 && !plan.walk && !block_scaled && blocks <= cus;
+}
+
 // Sizes of the launch of a plan whose columns and chunks are decided.
 void finish(const GemmParams &p, int dtype, int cus, bool leave_cus, PanelPlan &plan) {
   const int64_t blocks = block_count(p, dtype, plan);
@@ -554,6 +568,7 @@ void finish(const GemmParams &p, int dtype, int cus, bool leave_cus, PanelPlan &
   plan.chunk_items = (p.n + plan.cols - 1) / plan.cols * p.ngroups;
   plan.round_items = plan.chunk_rows == 128 && plan.cols == 128 && p.a_scale != nullptr ? kUnits : 0;
   plan.walk = walks(blocks, leave_cus);
+  plan.deep = is_deep(plan, blocks, p.a_scale != nullptr, cus);
   const int64_t most = cus >= 8 ? cus / 8 * 8 : cus;  // whole rounds over the XCDs where there are enough units
   plan.workgroups = static_cast<unsigned>(plan.walk && blocks > most ? most : blocks);
   plan.lds_bytes = p.a_scale != nullptr ? lds_of<Elem::FP8_BLOCKSCALED>(plan) : lds_of<Elem::FP8>(plan);
@@ -562,6 +577,16 @@ void finish(const GemmParams &p, int dtype, int cus, bool leave_cus, PanelPlan &
 }
 
 }  // namespace
+
+void set_chunks(const GemmParams &p, int64_t chunks, int cus, PanelPlan &plan) {
+  if (plan.walk) return;
+  const int64_t blocks = (chunks > 0 ? chunks * plan.chunk_items + 7 : 8) / 8 * 8;
+  if (blocks >= plan.blocks) return;
+  plan.blocks = static_cast<int>(blocks);
+  plan.workgroups = static_cast<unsigned>(blocks);
+  plan.deep = is_deep(plan, blocks, p.a_scale != nullptr, cus);
+  plan.lds_bytes = p.a_scale != nullptr ? lds_of<Elem::FP8_BLOCKSCALED>(plan) : lds_of<Elem::FP8>(plan);
+}
 
 // Rules by rows per expert on average (R), items and bytes of the weights; us are bf16 unless they say otherwise, before (streaming
 // form or macro tiles) -> these tiles.  The sums of a result follow from the launch of one weight group, whatever its margin.

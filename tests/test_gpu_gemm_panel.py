@@ -357,3 +357,22 @@ def test_row_counts_known_on_the_host(dtype, splits, n, k, done):
     out.fill_(-1)
     assert call(None) == 1
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("splits,n,kbytes", [([64, 0, 33, 17], 192, b) for b in (64, 128, 256, 384, 640, 720, 896, 1664)] +
+                         [([30, 34, 20, 17, 30, 0, 3, 26], 64, 8192), ([20, 17, 30, 0], 256, 768), ([96, 80, 1, 64], 1024, 1152), ([0, 0, 0], 192, 256)])
+def test_a_ring_in_pairs_for_one_workgroup_to_a_unit(dtype, splits, n, kbytes):
+    """Launches with no more items than compute units, as the host's row counts say: odd and even numbers of lines of K, fewer than the ring holds,
+    a part of a line, one, four and eight sums, no rows at all.  Integers, so any order of summation is exact."""
+    k, m, e = kbytes // DT[dtype].itemsize, max(1, sum(splits)), len(splits)
+    print(f"[case] panel gemm in pairs {dtype} {splits} n={n} k={k}", flush=True)
+    a, w, sp, _ = made(splits, n, k, dtype, n + k) if sum(splits) else made([1] + splits[1:], n, k, dtype, n + k)
+    ad, wd = a.to(DT[dtype]), w.to(DT[dtype])
+    args, out = capi._gemm_args(ad, wd, sp, None, None, None, None, None, None, 1.0, None, None, torch.float32, 0, 0, 0)
+    args.splits = None
+    out.fill_(-1)
+    host = (ctypes.c_int32 * e)(*splits)
+    assert capi.load().fluxmi_grouped_gemm_host_splits(ctypes.byref(args), host, None, None, 0, None, 0, capi._stream()) == 1
+    if sum(splits): assert torch.equal(out.double(), product(a, w, splits))
+    else: assert bool((out == -1).all())
