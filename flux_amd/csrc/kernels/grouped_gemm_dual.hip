@@ -204,6 +204,12 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
     const KernArgs a = kernel_args();
     const int n = a->n, raster = a->raster_rows;
     DualTile t = {0, 0, 0, 0, 0, false, false, 0, 0};
+    // A launch of one round that is not full deals its items to the eight XCDs evenly.
+    if (full_items == 0 && (grid & 7) == 0) {
+      const int per_xcd = (total_items + 7) >> 3, xcd = item / (grid >> 3), i = item - xcd * (grid >> 3);
+      if (xcd > 7 || i >= per_xcd) return t;
+      item = __builtin_amdgcn_readfirstlane(xcd * per_xcd + i);
+    }
     if (item >= total_items) return t;
     int tile = item, piece = 0;
     if (item >= full_items) {
