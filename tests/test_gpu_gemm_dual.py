@@ -161,3 +161,19 @@ def test_dual_tiles_take_row_counts_from_the_host(dtype, splits, n, k, done):
     out.fill_(-1)
     assert call("fluxmi_grouped_gemm_host_counts", None) == 1
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("splits,n,k", [([700], 264, 384), ([300, 257, 512], 520, 512), ([513, 0, 470, 256, 300], 1032, 640), ([290] * 9, 1800, 256)])
+def test_fewer_tiles_than_compute_units(splits, n, k, dtype):
+    """Grids of more workgroups than tiles: one to four tiles to an XCD, cut in four, in two and whole, grids off the eight XCDs, in both forms of
+    256 x 256 tiles.  Integers, exact."""
+    print(f"[case] few tiles {dtype} {splits[:4]} n={n} k={k}", flush=True)
+    assert is_dual(dtype, splits, n, k)
+    a, w, sp, _ = made(splits, n, k, dtype, n + k)
+    ad, wd, want = a.to(DT[dtype]), w.to(DT[dtype]), product(a, w, splits)
+    for flags in (0, capi.SCHED_WHOLE_TAIL_TILES, capi.SCHED_HALF_LINE_FILLS, capi.SCHED_HALF_LINE_FILLS | capi.SCHED_NO_SKINNY_TAIL):
+        for margin in (0, 100, 219):
+            out = torch.full((sum(splits), n), -7.0, device="cuda")
+            capi.grouped_gemm(ad, wd, sp, out=out, sched_flags=flags, cu_margin=margin)
+            assert torch.equal(out.double(), want), f"flags {flags} margin {margin}"
