@@ -329,12 +329,11 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
     // Workgroups: the upper bound of the tile count, or up to four for each of those where there are too few tiles for the card: the kernels cut the
     // tiles of a round that is not full into two or four pieces when these still fit the grid.  us, one workgroup to a tile -> up to four: dual
     // tiles fp16 8 experts 4096 x 14336, 194 rows each 299 -> 267; bf16 2 experts 4096 x 8192, 200 rows 154 -> 117; block-scaled 4 experts 1024 x 4096, 500
-    // rows 61 -> 44; macro tiles bf16 4 experts 2048 x 4096, 500 rows 105 -> 70; fp8 one expert 2048 x 4096, 2000 rows 48 -> 29.  The macro tiles only
-    // where all tiles are cut: whole tiles in a grid that they do not fill occupy few XCDs (192 tiles, 208 workgroups 88, 256 workgroups 96; the
-    // dual tiles deal such a round to all of them).
+    // rows 61 -> 44; macro tiles bf16 4 experts 2048 x 4096, 500 rows 105 -> 70; fp8 one expert 2048 x 4096, 2000 rows 48 -> 29.  Both deal a round
+    // that is not full to all XCDs (bf16 8 experts 2048 x 4096, 600 rows, 192 whole tiles: 88, in 256 workgroups without that 96, with it 87; 360 rows 77 -> 71).
     const int64_t tiles_n = (args->n + BN - 1) / BN * ngroups;
     const int64_t max_tiles = (static_cast<int64_t>(args->max_rows) / BM + args->nexperts) * tiles_n;
-    const int64_t most = dual || max_tiles * 2 <= cus ? max_tiles * 4 : max_tiles;
+    const int64_t most = max_tiles * 4;
     const int grid = static_cast<int>(most < cus ? most : cus);
     // Form of the ring fills.  Whole 128-byte lines cost the memory pipeline less per byte and need one barrier per
     // pair of k-steps, but a pair's 64 KiB stay in LDS for both of its steps, so fewer fills are in flight: faster

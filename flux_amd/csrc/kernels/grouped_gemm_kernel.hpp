@@ -1742,6 +1742,10 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
   typename std::conditional<kLineFills, LinePrefetch, TilePrefetch>::type pf;
   pf.valid = false;
   int item = virt;
+  if (skinny_items == 0 && total_items < grid && grid % 8 == 0) {  // a single round that is not full: an even share for each XCD
+    const int per_xcd = (total_items + 7) >> 3;
+    item = (bid >> 3) < per_xcd ? (bid & 7) * per_xcd + (bid >> 3) : total_items;
+  }
   TileDesc cur = locate(item);
   while (cur.kind != -2) {
     item += grid;
