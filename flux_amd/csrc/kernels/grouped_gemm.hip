@@ -148,14 +148,27 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
   return chunks <= stream_chunks_limit(active, chunk_rows, args->dtype == FLUXMI_FP8_E4M3, panel.chunk_items, panel.round_items);
 }
 
-// Whether the dual tiles are the faster ones for a launch that the macro tiles would compute; from 15006 launches of 4 to 96 experts, R = 97
-// to 4000 rows each on average, K 768 to 14336, even, random and Zipf row counts, plain and scaled, weights not in the cache.  Speed
-// against the macro tiles in the mean over ranges of R and K, and how many are slower by more than 3 %:
-//   block-scaled  1.05 to 1.31, 1 %
-//   fp8           R up to 512: 1.05 to 1.25, 2 %.  More rows: K < 3 KiB 1.04 to 1.17, 5 %; K < 4 KiB, R up to 1024 1.04 and 1.05, 12 %, R above
-//                 1.02 to 1.04, up to 27 %; longer K 0.98 to 1.05
-//   16 bits       R up to 320: 1.07 to 1.25, 3 %.  More rows: K < 3 KiB 1.06 to 1.21, 6 %; K < 4 KiB, R up to 768 1.05 to 1.08, 6 %; K < 6 KiB, R up
-//                 to 512 1.05 and 1.06, 8 %; beyond these lines 0.92 to 1.06, up to 76 %
+// Whether the dual tiles are the faster ones for a launch that the macro tiles would compute.  Speed against the macro tiles in the mean, and how
+// many launches are slower by more than 3 %: 19125 launches of 1 to 128 experts with more than 128 tiles, R = 97 to 4000 rows each on average,
+// rows of K of 0.5 to 28 KiB, even, random and Zipf row counts, plain and scaled, gathered and not, weights not in the cache.  fp32 results have
+// lines of their own: a tile's stores drain ahead of the next tile's fills, and these are twice as many.
+//                                         16-bit results                      fp32 results
+//   16 bits  R up to 320                  1.20,  2 %                          1.16,  3 %
+//            R up to 512, K < 6 KiB       1.17,  1 %                          1.09,  5 %
+//            more rows, K < 1 KiB         1.42,  none                         1.27,  none
+//                       K < 2 KiB         1.20,  none                         R up to 1500 1.15,  3 %; more 1.09, 14 %: not taken
+//                       K < 3 KiB         1.12,  none                         R up to 1024 1.06, 10 %; more 1.02, 25 %: not taken
+//                       K < 4 KiB         R up to 768 1.09, 2 %; 1.06, 5 %    1.02, 21 %: not taken
+//            the rest                     1.00, 34 %: not taken               0.99, 44 %: not taken
+//   fp8      R up to 512                  1.20,  2 %                          1.16,  4 %
+//            more rows, K < 1 KiB         1.30,  none                         1.19,  6 %
+//                       K < 2 KiB         1.15,  none                         R up to 1500 1.09,  6 %; more 1.05, 19 %: not taken
+//                       K < 3 KiB         1.07,  4 %                          R up to 1024 1.05, 11 %; more 1.03, 15 %: not taken
+//                       K < 4 KiB         R up to 1024 1.05, 9 %; 1.03, 13 %  1.02, 20 %: not taken
+//            the rest                     1.00, 30 %: not taken               0.99, 38 %: not taken
+//   block-scaled                          1.21,  2 %                          1.12,  5 %
+// Launches of fewer tiles, which both forms cut into pieces, are not told apart here: up to 192 rows 0.92 to 1.06, more rows 0.74 to 1.14, so the
+// macro tiles would be the faster ones for many (both gain on one workgroup to a tile, these 1.06 to 1.47).
 // The flags of the fill forms name forms of the macro tiles.
 bool dual_is_faster(const fluxmi_grouped_gemm_args *args, bool block_scaled) {
   if (block_scaled) return true;
@@ -163,7 +176,9 @@ bool dual_is_faster(const fluxmi_grouped_gemm_args *args, bool block_scaled) {
   const bool fp8 = args->dtype == FLUXMI_FP8_E4M3;
   const int64_t kbytes = static_cast<int64_t>(args->k) * (fp8 ? 1 : 2);
   auto at_most = [&](int64_t rows) { return args->max_rows <= rows * args->nexperts; };
-  return at_most(fp8 ? 512 : 320) || kbytes < 3072 || (kbytes < 4096 && at_most(fp8 ? 1024 : 768)) || (kbytes < 6144 && at_most(512));
+  if (at_most(fp8 ? 512 : 320) || (kbytes < 6144 && at_most(512))) return true;
+  if (args->d_fp32 != 0) return kbytes < 1024 || (kbytes < 2048 && at_most(1500)) || (kbytes < 3072 && at_most(1024));
+  return kbytes < 3072 || (kbytes < 4096 && at_most(fp8 ? 1024 : 768));
 }
 
 // Row counts that are known on the host, and a second factor per row.

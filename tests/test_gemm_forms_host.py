@@ -179,20 +179,26 @@ def test_panel_tiles_of_256_columns_have_a_workgroup_per_item(dtype, experts, ro
         assert (above.cols, above.workgroups) == (128, 256)
 
 
-@pytest.mark.parametrize("dtype,experts,rows,n,k,block_scaled,dual", [
-    (BF16, 8, 320, 14336, 4096, False, True), (BF16, 8, 321, 14336, 4096, False, False), (F16, 8, 512, 4096, 3072, False, False), (F16, 8, 512, 4096, 3008, False, True), (F16, 64, 1536, 2048, 1408, False, True),
-    (F16, 64, 1536, 1408, 2048, False, False), (BF16, 64, 768, 1408, 1984, False, True), (BF16, 64, 769, 1408, 1984, False, False),
-    (FP8, 32, 512, 2048, 7168, False, True), (FP8, 32, 513, 2048, 7168, False, False), (FP8, 32, 1024, 2048, 3072, False, True),
-    (FP8, 32, 4000, 7168, 2944, False, True), (FP8, 32, 4000, 7168, 7168, True, True),
+# dual32: the same with fp32 results
+@pytest.mark.parametrize("dtype,experts,rows,n,k,block_scaled,dual,dual32", [
+    (BF16, 8, 320, 14336, 4096, False, True, True), (BF16, 8, 321, 14336, 4096, False, False, False), (F16, 8, 512, 4096, 3072, False, False, False),
+    (F16, 8, 512, 4096, 3008, False, True, True), (F16, 8, 513, 4096, 3008, False, False, False), (F16, 64, 1536, 2048, 1408, False, True, False),
+    (F16, 64, 1536, 1408, 2048, False, False, False), (BF16, 64, 768, 1408, 1984, False, True, False), (BF16, 64, 769, 1408, 1984, False, False, False),
+    (BF16, 64, 1024, 2048, 1472, False, True, True), (BF16, 64, 1025, 2048, 1472, False, True, False), (F16, 64, 1500, 2048, 960, False, True, True),
+    (F16, 64, 1501, 2048, 960, False, True, False), (BF16, 64, 4000, 2048, 448, False, True, True),
+    (FP8, 32, 512, 2048, 7168, False, True, True), (FP8, 32, 513, 2048, 7168, False, False, False), (FP8, 32, 1024, 2048, 3072, False, True, False),
+    (FP8, 32, 1024, 2048, 2944, False, True, True), (FP8, 32, 1025, 2048, 2944, False, True, False), (FP8, 32, 1500, 2048, 1920, False, True, True),
+    (FP8, 32, 1501, 2048, 1920, False, True, False), (FP8, 32, 4000, 2048, 896, False, True, True),
+    (FP8, 32, 4000, 7168, 2944, False, True, False), (FP8, 32, 4000, 7168, 7168, True, True, True),
     # not whole steps of K, one step, columns that are not in eights, too many experts
-    (BF16, 8, 300, 4096, 4104, False, False), (FP8, 8, 300, 4096, 128, True, False), (BF16, 8, 300, 4100, 4096, False, False),
-    (FP8, 129, 300, 512, 512, True, False)])
-def test_dual_tiles_by_rows_and_k(dtype, experts, rows, n, k, block_scaled, dual):
+    (BF16, 8, 300, 4096, 4104, False, False, False), (FP8, 8, 300, 4096, 128, True, False, False), (BF16, 8, 300, 4100, 4096, False, False, True),
+    (FP8, 129, 300, 512, 512, True, False, False)])
+def test_dual_tiles_by_rows_and_k(dtype, experts, rows, n, k, block_scaled, dual, dual32):
     def is_dual(**kw):
         return capi.gemm_dual_tiles(dtype, experts, rows * experts, n, k, block_scaled=block_scaled, **kw)
 
     assert capi.gemm_launch_info(dtype, experts, rows * experts, n, k, block_scaled=block_scaled).form == capi.GEMM_MACRO_TILES
     assert is_dual() == is_dual(gathered=True) == dual
-    assert is_dual(d_fp32=True) == (dual or n % 8 != 0)
+    assert is_dual(d_fp32=True) == is_dual(d_fp32=True, gathered=True) == dual32
     for flag in (capi.SCHED_HALF_LINE_FILLS, capi.SCHED_WHOLE_LINE_FILLS):
         assert is_dual(sched_flags=flag) == (dual and block_scaled)
