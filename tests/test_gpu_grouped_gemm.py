@@ -528,6 +528,27 @@ def test_skinny_tail_pieces_same_bits_as_in_place(dtype, ksteps):
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+@pytest.mark.parametrize("margin", [0, 232, 244, 250, 252])
+def test_skinny_tails_in_launches_of_one_round(dtype, margin):
+    """Seven row tiles of long K (enough for skinny tails), three of them with at most 64 rows, on 256, 24, 12, 6 and 4 compute units: in place,
+    where all tiles are cut as small as the others alone would be; behind the others, where these are cut in four or two without them; and
+    in launches of two rounds.  The bits of the schedule without skinny tails, and the dense product."""
+    from flux_amd import capi
+    split, n, k = [300, 257, 513], 200, 8192 + 64
+    m, t = sum(split), torch.bfloat16 if dtype == "bf16" else torch.float8_e4m3fn
+    print(f"[case] grouped_gemm {dtype} skinny tails, one round, margin {margin}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(margin)
+    a = torch.randint(-3, 4, (m, k), generator=g, device="cuda").float()
+    w = torch.randint(-3, 4, (len(split), n, k), generator=g, device="cuda").float()
+    want = torch.cat([x.double() @ w[e].double().t().contiguous() for e, x in enumerate(a.split(split))])  # integers: exact in fp32
+    sp = torch.tensor(split, dtype=torch.int32).cuda()
+    for flags in (capi.SCHED_NO_SKINNY_TAIL, 0, capi.SCHED_FORCE_SKINNY_TAIL):
+        out = torch.full((m, n), -7.0, device="cuda")
+        capi.grouped_gemm(a.to(t), w.to(t), sp, out=out, sched_flags=flags, cu_margin=margin)
+        assert torch.equal(out.double(), want), f"flags {flags}"
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
 @pytest.mark.parametrize("k", [128, 1024, 1040, 4096])
 def test_both_fill_forms_give_the_same_bits(dtype, k):
     """Half-line and whole-line ring fills walk K in the same order with the same MFMAs: ragged experts (whole,
