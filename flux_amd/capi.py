@@ -184,7 +184,8 @@ SCHED_WHOLE_LINE_FILLS = 32
 
 
 # Form of the MFMA kernel's ring fills for calls that name none themselves: 0 (the library's rule by shape),
-# SCHED_HALF_LINE_FILLS or SCHED_WHOLE_LINE_FILLS.  Results are bit-identical either way.
+# SCHED_HALF_LINE_FILLS or SCHED_WHOLE_LINE_FILLS.  Results are bit-identical between the two; without block scales both keep a launch off
+# the dual tiles, whose fp8 sums can differ from them in the last bit.
 default_fill_form = 0
 
 

@@ -76,14 +76,16 @@ float time_calls(F &&run) {
 // Times `run` (one whole forward) under every candidate schedule on the current stream, 5 warm-up and 10
 // timed calls each like the reference's profiling loops (gemm_grouped_v3_ag_scatter.cc:540-590), records
 // them in `ctx` and registers the fastest for `key`.  `args`: the launch that `run` makes; splits: its row counts on the host.  The
-// schedules are the macro tiles'; where another form computes the launch they are all one, and only the default is timed.
+// schedules are the macro tiles' and the dual tiles'; where another form computes the launch they are all one, and only the default is timed.
 template <class F>
 void profile_schedules(const GemmShapeKey &key, ProfilingContext *ctx, const fluxmi_grouped_gemm_args &args, const torch::Tensor &splits,
                        F &&run) {
   fluxmi_gemm_launch_info info;
   check_status(fluxmi_grouped_gemm_launch_info(&args, key.ngroups, nullptr, splits.data_ptr<int32_t>(), fluxmi_device_cu_count(), &info),
                "fluxmi_grouped_gemm_launch_info");
-  for (const GemmLaunchTuning &cand : gemm_tuning_candidates()) {
+  const int dual = fluxmi_grouped_gemm_dual_tiles(&args, key.ngroups, nullptr, fluxmi_device_cu_count());
+  if (dual < 0) check_status(dual, "fluxmi_grouped_gemm_dual_tiles");
+  for (const GemmLaunchTuning &cand : gemm_tuning_candidates(dual == 1, key.dtype == FLUXMI_FP8_E4M3)) {
     ScopedTuningOverride scope(&cand);
     ctx->add(key, cand, time_calls(run));
     if (info.form == FLUXMI_GEMM_STREAM || info.form == FLUXMI_GEMM_PANEL) break;

@@ -28,15 +28,20 @@ std::string GemmLaunchTuning::to_string() const {
 
 std::string TuningRecord::to_string() const { return "fluxmi_gemm_tuning " + key.to_string() + " " + best.to_string(); }
 
-std::vector<GemmLaunchTuning> gemm_tuning_candidates() {
+std::vector<GemmLaunchTuning> gemm_tuning_candidates(bool dual_tiles, bool fp8) {
   std::vector<GemmLaunchTuning> out;
   for (int32_t flags : {0, FLUXMI_SCHED_WHOLE_TAIL_TILES, FLUXMI_SCHED_NO_HALF_TILES,
-                        FLUXMI_SCHED_WHOLE_TAIL_TILES | FLUXMI_SCHED_NO_HALF_TILES})
+                        FLUXMI_SCHED_WHOLE_TAIL_TILES | FLUXMI_SCHED_NO_HALF_TILES}) {
+    if (dual_tiles && (flags & FLUXMI_SCHED_NO_HALF_TILES) != 0) continue;  // the same launch again
     for (int32_t rows : {8, 4, 16}) out.push_back(GemmLaunchTuning{rows, flags});
+  }
   // where the few last rows of an expert run: as 64 x 64 pieces behind all other tiles, or in place
-  out.push_back(GemmLaunchTuning{8, FLUXMI_SCHED_NO_SKINNY_TAIL});
-  out.push_back(GemmLaunchTuning{8, FLUXMI_SCHED_FORCE_SKINNY_TAIL});
-  // both forms of the ring fills, whatever the default picks for the shape
+  if (!dual_tiles) {
+    out.push_back(GemmLaunchTuning{8, FLUXMI_SCHED_NO_SKINNY_TAIL});
+    out.push_back(GemmLaunchTuning{8, FLUXMI_SCHED_FORCE_SKINNY_TAIL});
+  }
+  // both forms of the macro tiles' ring fills, whatever the default picks for the shape; in fp8 their sums are not the dual tiles'
+  if (dual_tiles && fp8) return out;
   out.push_back(GemmLaunchTuning{8, FLUXMI_SCHED_HALF_LINE_FILLS});
   out.push_back(GemmLaunchTuning{8, FLUXMI_SCHED_WHOLE_LINE_FILLS});
   return out;

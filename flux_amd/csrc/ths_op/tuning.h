@@ -3,8 +3,11 @@
 // (include/flux/ths_op/ths_op.h:64-113, src/ths_op/ths_op.cc:217-320) and its TuningConfigRegistry.
 // The reference's records pick one of its generated kernel variants; here a record picks the tile
 // schedule of the persistent macro-tile kernel (height of the raster groups, whether the last round is cut into
-// pieces, whether an expert's last row tile may run half height).  No choice changes a result bit.  Launches that the
-// streaming form or the panel tiles compute (few rows per expert) have no such schedule: a record changes nothing there.
+// pieces, whether an expert's last row tile may run half height).  Launches that the streaming form or the panel tiles compute
+// (few rows per expert) have no such schedule: a record changes nothing there.  The dual tiles follow the first two choices.
+// No choice that profiling() makes among the schedules changes a result bit.  One that it does not try can: a record that names a form of the ring's
+// fills, made by hand or where no dual tiles were, keeps an fp8 launch on the macro tiles, whose MFMAs add K by 64 and not by 128.  (Layer1's fused
+// reduction is another form of the sums as well, by atomic additions.)
 #pragma once
 #include <cstdint>
 #include <map>
@@ -43,8 +46,8 @@ struct TuningRecord {
   std::string to_string() const;  // one line of the text form read by TuningTable::load_text
 };
 
-// Every schedule the profiler tries.
-std::vector<GemmLaunchTuning> gemm_tuning_candidates();
+// Every schedule the profiler tries.  dual_tiles: the launch runs the dual tiles unless a form of the fills is named.
+std::vector<GemmLaunchTuning> gemm_tuning_candidates(bool dual_tiles, bool fp8);
 
 // Process-wide table consulted by every grouped-GEMM launch of the ops.
 class TuningTable {

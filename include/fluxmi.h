@@ -140,8 +140,9 @@ typedef struct fluxmi_grouped_gemm_args {
   /* Launch tuning; all zero = defaults.  None of them changes a result bit, with one exception below.  raster_rows and sched_flags steer
    * the macro-tile kernel; launches that another form computes (fluxmi_grouped_gemm_launch_info: the streaming form, the panel tiles) take
    * no notice of them, whether they are left out or force something.  The dual tiles (fluxmi_grouped_gemm_dual_tiles) follow raster_rows
-   * and FLUXMI_SCHED_WHOLE_TAIL_TILES.  The two flags for the ring's fills are about the macro-tile kernel itself and keep a launch on it:
-   * fp8 results can then differ in the last bit of their fp32 sums, as its MFMAs add K by 64 and the dual tiles' by 128. */
+   * and FLUXMI_SCHED_WHOLE_TAIL_TILES.  The two flags for the ring's fills are about the macro-tile kernel itself and keep a launch without
+   * block scales on it: fp8 results can then differ in the last bit of their fp32 sums, as its MFMAs add K by 64 and the dual tiles' by
+   * 128.  Block-scaled launches, which have one form of the fills, take no notice of them. */
   int32_t cu_margin;     /* compute units left free for other work (Flux `sm_margin`) */
   int32_t raster_rows;   /* row tiles of an expert walked together over all weight panels; 0 = 8 */
   int32_t sched_flags;   /* FLUXMI_SCHED_* */

@@ -330,6 +330,31 @@ def test_profiling_times_one_schedule_where_none_has_an_effect(cnt, timed):
     m.clear_tuning_records()
 
 
+@pytest.mark.parametrize("dtype,flags", [(torch.bfloat16, {0, 1, 16, 32}), (torch.float8_e4m3fn, {0, 1})])
+def test_profiling_on_the_dual_tiles(dtype, flags):
+    """Where the dual tiles compute a launch, profiling() tries what they follow and, where the results are the same bits, the macro tiles'
+    two forms of fills (16, 32): a schedule that it picks never changes a result bit."""
+    from flux_amd import capi
+    m = flux_amd.flux_ths_pybind
+    m.clear_tuning_records()
+    g = torch.Generator().manual_seed(4)
+    e, h, f, t, k = 4, 512, 1536, 500, 2
+    cnt = [300, 200, 257, 243]
+    assert capi.gemm_dual_tiles(dtype, e, t * k, f, h, gathered=True)
+    x = torch.randn(t, h, generator=g).to(dtype).cuda()
+    w1 = (torch.randn(e, f, h, generator=g) * 0.5).to(dtype).cuda()
+    splits = torch.tensor(cnt, dtype=torch.int32).cuda()
+    scatter = torch.randperm(t * k, generator=g).to(torch.int32).view(t, k).cuda()
+    op0 = flux_amd.GemmGroupedV3AGScatter(flux_amd.DistEnvTPWithEP(None, 1, None), flux_amd.MoeArguments(t, h, f, e, k, dtype, torch.bfloat16))
+    y = op0.forward(x, w1, splits, scatter)
+    ctx = flux_amd.ProfilingContext("dual tiles")
+    assert torch.equal(op0.profiling(x, w1, splits, scatter, prof_ctx=ctx), y)
+    tried = {int(word.split("=")[1]) for word in ctx.get_latest_prof_result().split() if word.startswith("sched_flags=")}  # of the five fastest
+    assert tried and tried <= flags
+    assert torch.equal(op0.forward(x, w1, splits, scatter), y)
+    m.clear_tuning_records()
+
+
 @pytest.mark.parametrize("raster_rows,flags,margin", [(4, 0, 0), (16, 1, 0), (8, 2, 0), (1, 3, 0), (8, 0, 40), (8, 0, 255),
                                                        (8, 0, 1000), (8, 4, 0), (8, 8, 0), (2, 9, 5)])
 def test_tile_schedules_and_cu_margin_do_not_change_a_bit(raster_rows, flags, margin):
