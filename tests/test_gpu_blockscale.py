@@ -198,3 +198,61 @@ def test_blockscale_last_rows_of_an_expert(split, n, k):
     wide_s = torch.ones(sum(whole), k // 128)
     wide_s[at] = sa
     assert torch.equal(run(wide_a.view(torch.float8_e4m3fn), wide_s, whole)[at], out)
+
+
+# Launches that the dual tiles do not take: 16-bit results in columns that are not in eights, and more than 128 experts; one and two blocks of K,
+# six, seven and thirteen (the last pair of an unrolled trip of the k loop and the first of the next); last row tiles 64, 128 and 256 rows high.
+@pytest.mark.parametrize("split,n,f32", [([129, 192, 193, 64, 65, 128, 1, 320, 321, 384, 385, 255], 268, False), ([513, 576, 0, 577, 640, 641], 132, False),
+                                         ([300], 516, False), ([97, 200, 300, 0] + [97] * 125 + [260], 136, True)])
+@pytest.mark.parametrize("k", [128, 256, 768, 896, 1664])
+def test_blockscale_macro_tiles_are_exact_on_integers(split, n, f32, k):
+    """The macro tiles' kernel, with every factor; operands are small integers and scales powers of two, so the fp32 sums are exact."""
+    import ctypes
+    from flux_amd import capi
+    print(f"[case] blockscale macro tiles {split[:6]} N={n} K={k}", flush=True)
+    m, e, kb = sum(split), len(split), k // 128
+    assert capi.gemm_launch_info(torch.float8_e4m3fn, e, m, n, k, splits=split, block_scaled=True).form == capi.GEMM_MACRO_TILES
+    assert not capi.gemm_dual_tiles(torch.float8_e4m3fn, e, m, n, k, block_scaled=True, d_fp32=f32)
+    g = torch.Generator(device="cuda").manual_seed(k + n)
+    power = lambda *shape: 2.0 ** torch.randint(-1, 2, shape, generator=g, device="cuda").float()
+    a = torch.randint(-3, 4, (m, k), generator=g, device="cuda").float()
+    w = torch.randint(-3, 4, (e, n, k), generator=g, device="cuda").float()
+    sa, sb, row_scale, alpha = power(m, kb), power(e, (n + 127) // 128, kb), power(m), power(e)
+    full = w * torch.repeat_interleave(torch.repeat_interleave(sb, 128, dim=1)[:, :n], 128, dim=2)
+    rows = (a * torch.repeat_interleave(sa, 128, dim=1)).double().split(split)
+    want = torch.cat([r @ full[i].double().t().contiguous() for i, r in enumerate(rows)])
+    want *= (row_scale * alpha[torch.repeat_interleave(torch.arange(e, device="cuda"), torch.tensor(split, device="cuda"))]).double()[:, None]
+    qa, qw, sp = a.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn), torch.tensor(split, dtype=torch.int32, device="cuda")
+    pad = torch.zeros((m + 127) // 128 * 128, kb, device="cuda")
+    pad[:m] = sa
+    block = pad.view(-1, 128, kb).permute(0, 2, 1).contiguous()
+    by_expert = torch.cat([s.t().contiguous().flatten() for s in sa.split(split)])
+    kind = torch.float32 if f32 else torch.bfloat16
+    for scales, weights, a_layout, b_layout in ((block, sb, capi.ASCALE_BLOCK128, capi.BSCALE_N_K),
+                                                (by_expert, sb.transpose(1, 2).contiguous(), capi.ASCALE_EXPERT_K_M, capi.BSCALE_K_N)):
+        for margin in (0, 100, 254):  # a workgroup to every piece and to fewer, walking
+            args, out = capi._gemm_args(qa, qw, sp, None, None, None, alpha, row_scale, None, 1.0, None, None, kind, margin, 0, 0)
+            capi._check(capi.load().fluxmi_grouped_gemm_blockscale(ctypes.byref(args), capi._ptr(scales), a_layout, capi._ptr(weights), b_layout,
+                                                                   capi._stream()), "fluxmi_grouped_gemm_blockscale")
+            assert torch.equal(out, want.to(torch.float32).to(kind)), f"layouts {a_layout} {b_layout} margin {margin}"
+
+
+@pytest.mark.parametrize("k", [256, 896, 4096])
+def test_blockscale_macro_and_dual_tiles_have_the_same_bits(k):
+    """A block of K after the other, each scaled by the product of its two scales: the same fp32 sums in both kernels, from operands and scales
+    of any value.  129 experts run the macro tiles, the first 128 of them the dual tiles."""
+    from flux_amd import capi
+    split, n = [97, 200, 300, 0] + [110] * 124 + [64], 264
+    print(f"[case] blockscale bits of macro and dual tiles K={k}", flush=True)
+    assert [capi.gemm_dual_tiles(torch.float8_e4m3fn, e, sum(split[:e]), n, k, block_scaled=True, d_fp32=True) for e in (129, 128)] == [False, True]
+    m, kb = sum(split), k // 128
+    g = torch.Generator(device="cuda").manual_seed(k)
+    qa = torch.randn(m, k, generator=g, device="cuda").to(torch.float8_e4m3fn)
+    qw = torch.randn(len(split), n, k, generator=g, device="cuda").to(torch.float8_e4m3fn)
+    sa = torch.rand((m + 127) // 128, kb, 128, generator=g, device="cuda") + 0.1
+    sb = torch.rand(len(split), (n + 127) // 128, kb, generator=g, device="cuda") + 0.1
+    sp = torch.tensor(split, dtype=torch.int32, device="cuda")
+    some = m - split[-1]
+    macro = capi.grouped_gemm_blockscale(qa, qw, sp, sa, sb, out_dtype=torch.float32)
+    dual = capi.grouped_gemm_blockscale(qa[:some], qw[:128], sp[:128].contiguous(), sa, sb, out_dtype=torch.float32)
+    assert torch.equal(macro[:some], dual)
