@@ -55,9 +55,83 @@ def test_dual_tiles_are_exact_on_integers(name, splits, n, k, dtype):
         capi.grouped_gemm(ad, wd, sp, out=out, gather_a=perm, scatter_d=to, row_scale=row_scale, col_scale=col_scale, alpha=alpha, cu_margin=margin,
                           sched_flags=flags, raster_rows=margin // 40)
         assert torch.equal(out.double(), picked), f"margin {margin}"
-    two = capi.grouped_gemm_multi(ad, [wd, wd.flip(0).contiguous()] if dtype != "fp8" else [wd, wd], sp, out_dtype=torch.float32)
+    other = -w.flip(0)  # (negated too: a single expert flipped is itself)
+    two = capi.grouped_gemm_multi(ad, [wd, other.to(DT[dtype])], sp, out_dtype=torch.float32)
     assert torch.equal(two[0].double(), want)
-    assert torch.equal(two[1].double(), product(a, w.flip(0) if dtype != "fp8" else w, splits))
+    assert torch.equal(two[1].double(), product(a, other, splits))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("out_dtype", ["half", "fp32"])
+def test_dual_tiles_odd_indices_scalars_and_weights_off_lines(dtype, out_dtype):
+    """Gathered rows outside A are its first or last row, scattered rows outside D are not stored; a scalar from the host and one from the
+    device; weights that start 16 bytes past a line.  Experts of one row tile and of two."""
+    splits, n, k = [250, 256, 0, 300, 230], 392, 384
+    print(f"[case] dual gemm odd indices {dtype} {out_dtype}", flush=True)
+    m, e, a_rows = sum(splits), len(splits), 77
+    assert is_dual(dtype, splits, n, k, gathered=True) and is_dual(dtype, splits, n, k, gathered=True, d_fp32=True)
+    a, w, sp, g = made(splits, n, k, dtype, 11)
+    a = a[:a_rows]
+    raw = torch.zeros(w.numel() * DT[dtype].itemsize + 256, dtype=torch.uint8, device="cuda")
+    at = -raw.data_ptr() % 128 + 16
+    wd = raw[at:at + w.numel() * DT[dtype].itemsize].view(DT[dtype]).view(e, n, k)
+    wd.copy_(w.to(DT[dtype]))
+    assert wd.data_ptr() % 128 == 16
+    gather = torch.randint(-90, 200, (m,), generator=g, device="cuda").to(torch.int32)
+    to = torch.randperm(m, generator=g, device="cuda").to(torch.int32)
+    outside = torch.randperm(m, generator=g, device="cuda")[:200]
+    to[outside[:100]] = torch.randint(-(1 << 31), 0, (100,), generator=g, device="cuda").to(torch.int32)
+    to[outside[100:]] = torch.randint(m, (1 << 31) - 1, (100,), generator=g, device="cuda").to(torch.int32)
+    kept = (to >= 0) & (to < m)
+    want = torch.full((m, n), -7.0, device="cuda", dtype=torch.float64)
+    rows = product(a[gather.long().clamp(0, a_rows - 1)], w, splits) * (0.5 * 4.0)
+    want[to[kept].long()] = rows[kept]
+    kind = torch.float32 if out_dtype == "fp32" else capi._half_out(DT[dtype])
+    out = torch.full((m, n), -7.0, device="cuda", dtype=kind)
+    capi.grouped_gemm(a.to(DT[dtype]), wd, sp, out=out, gather_a=gather, scatter_d=to, scalar_scale=0.5,
+                      scalar_scale_dev=torch.tensor([4.0], device="cuda"), max_rows=m)
+    assert torch.equal(out, want.to(torch.float32).to(kind))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp8"])
+def test_dual_tiles_fp32_results_beyond_half_a_gigabyte(dtype):
+    """Such launches store non-temporally.  Most rows are not any expert's: they keep what they held."""
+    splits, n, k, m = [300, 0, 256, 129, 64, 700] + [0] * 10, 5640, 256, 24000
+    print(f"[case] dual gemm non-temporal stores {dtype}", flush=True)
+    assert m * n * 4 > 512 << 20 and capi.gemm_dual_tiles(DT[dtype], len(splits), m, n, k, d_fp32=True)
+    a, w, sp, _ = made([sum(splits)] + [0] * 15, n, k, dtype, 5)
+    wide = torch.zeros(m, k, device="cuda", dtype=DT[dtype])
+    wide[:a.shape[0]] = a.to(DT[dtype])
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    out = torch.full((m, n), -7.0, device="cuda")
+    capi.grouped_gemm(wide, w.to(DT[dtype]), sp, out=out)
+    assert torch.equal(out[:a.shape[0]].double(), product(a, w, splits)) and bool((out[a.shape[0]:] == -7).all())
+
+
+@pytest.mark.parametrize("k", [256, 384, 1152])
+def test_dual_tiles_block_scaled_infinite_and_nan_scales(k):
+    """A scale that is infinite or not a number reaches the results of its row, or of its 128 columns of one expert, and no others; in the
+    first block of K, where nothing has been summed yet, and in the last.  Positive operands: no infinity meets its opposite or a zero."""
+    splits, n = [300, 129, 64, 250], 392
+    print(f"[case] dual gemm block-scaled, scales that are not finite K={k}", flush=True)
+    m, e, kb = sum(splits), len(splits), k // 128
+    assert is_dual("bs", splits, n, k)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.randint(1, 4, (m, k), generator=g, device="cuda").float()
+    w = torch.randint(1, 4, (e, n, k), generator=g, device="cuda").float()
+    sp = torch.tensor(splits, dtype=torch.int32, device="cuda")
+    sa, sb, _, _ = block_scales(m, e, n, k, splits, capi.ASCALE_BLOCK128, capi.BSCALE_N_K, g)
+    sa[5, 0], sa[70, kb - 1], sa[310, 0], sa[440, kb - 1] = float("inf"), float("inf"), float("nan"), float("nan")
+    sb[1, 1, 0], sb[3, 3, kb - 1] = float("inf"), float("nan")
+    pad = torch.zeros((m + 127) // 128 * 128, kb, device="cuda")
+    pad[:m] = sa
+    want = product(a * torch.repeat_interleave(sa, 128, dim=1),
+                   w * torch.repeat_interleave(torch.repeat_interleave(sb, 128, dim=1)[:, :n], 128, dim=2), splits)
+    got = capi.grouped_gemm_blockscale(a.to(DT["bs"]), w.to(DT["bs"]), sp, pad.view(-1, 128, kb).permute(0, 2, 1).contiguous(), sb,
+                                       out_dtype=torch.float32).double()
+    assert torch.isnan(want).any() and torch.isinf(want).any() and torch.isfinite(want).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(want))
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16"])
