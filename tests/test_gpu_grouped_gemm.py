@@ -12,11 +12,11 @@ FP8_FROB = 3e-2
 
 
 
-@pytest.fixture(autouse=True, params=["half_line_fills", "whole_line_fills"])
+@pytest.fixture(autouse=True, params=["half_line_fills", "whole_line_fills", "default"])
 def fill_form(request):
-    """Every test of this module runs with both forms of the MFMA kernel's ring fills."""
+    """Every test of this module runs with both forms of the macro tiles' ring fills, and with what the library picks (the dual tiles for many)."""
     from flux_amd import capi
-    capi.default_fill_form = capi.SCHED_HALF_LINE_FILLS if request.param == "half_line_fills" else capi.SCHED_WHOLE_LINE_FILLS
+    capi.default_fill_form = {"half_line_fills": capi.SCHED_HALF_LINE_FILLS, "whole_line_fills": capi.SCHED_WHOLE_LINE_FILLS, "default": 0}[request.param]
     yield request.param
     capi.default_fill_form = 0
 
