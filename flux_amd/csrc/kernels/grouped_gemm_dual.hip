@@ -393,9 +393,11 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
   };
 #undef FLUXMI_FILL_UNIT
   auto fill_x = [&](uint32_t slot, int kb) { fill_unit(false, xrsrc, fill0 + slot, xoff0, xoff1, xoff2, xoff3, kb); };
-  // Weights that no other tile reads come non-temporally, where rows start on lines (a load that covers parts of two lines needs the
+  // Weights of an expert that is one row tile come non-temporally, where rows start on lines (a load that covers parts of two lines needs the
   // second again): 3 to 5 % up to 256 rows per expert (fp16 32 experts 2048 x 4096, 194 rows each 145 -> 127 us, 8 experts 14336 x 4096 250 ->
   // 237, 4096 x 14336 312 -> 297; fp8 32 experts 2048 x 7168 110 -> 91).  Block-scaled launches gain nothing and lose 1 % by the branch.
+  // Where the tile of such an expert is cut in four, two workgroups read each weight, and still do so non-temporally: ordinary loads there are 0.4 %
+  // slower (8003 launches of up to 64 tiles, 120 to 260 rows per expert; 199 slower by more than 3 %, 47 as much faster).
   auto fill_w = [&](uint32_t slot, int kb) { fill_unit(!BS && w_once, wrsrc, fill0 + slot, woff0, woff1, woff2, woff3, kb); };
 
   // ---- fragments -------------------------------------------------------------------------------------------
@@ -430,7 +432,7 @@ __global__ __launch_bounds__(kDualThreads, 2) void grouped_gemm_dual_kernel(cons
       w[j0 + j][1] = *reinterpret_cast<LdsFrag>(b + j * 2048);
     }
   };
-  // Unit U lies in slot U mod 10.  base: unit number of the current step's first unit, mod 10.
+  // Unit U lies in slot U mod 9.  base: unit number of the current step's first unit, mod 9.
   auto slot_of = [&](int u) { return static_cast<uint32_t>(u >= kRing ? u - kRing : u) * kUnit; };
   auto sync = [&]() {
     __builtin_amdgcn_sched_barrier(0);
