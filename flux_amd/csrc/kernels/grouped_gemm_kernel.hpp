@@ -1628,11 +1628,10 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
   // is short (under 128 k-steps a piece is mostly its own start and end: measured 2-3 % slower on 64 experts at
   // K = 2048).
   const int skinny_tiles_all = skinny_experts * tiles_n;
-  auto pieces_of = [&](int tiles) { return !cut_tail ? 1 : (tiles * 4 <= grid ? 4 : (tiles * 2 <= grid ? 2 : 1)); };  // of a round of so many tiles
-  // In a launch of one round these tiles have compute units of their own; behind the other tiles they can be a second round.  So there only
-  // where the others are cut smaller without them.  (K of 8 KiB and more, up to 256 tiles, in place against behind in the mean of 967 launches:
-  // 1.05, 1 in 100 slower by more than 3 %; fp16 2 experts 2920 x 11008, 1793 rows each, 192 tiles: 298 us -> 268.)
-  const bool own_units = total_tiles <= grid && pieces_of(total_tiles) == pieces_of(total_tiles - skinny_tiles_all);
+  // In a launch of one round these tiles have compute units of their own, and behind the other tiles they would be a second one.  (K of 8 KiB
+  // and more, up to 256 tiles, in place against behind: 8423 launches 1.20 in the mean, 51 slower by more than 3 %, all of them where the other
+  // tiles are cut smaller without these; there, 2515 launches, 1.16.  fp8 9 experts 2920 x 14336, 192 tiles, 108 of them skinny: 225 us -> 137.)
+  const bool own_units = total_tiles <= grid;
   const bool skinny_on = !BS && half_tiles && (p.sched_flags & FLUXMI_SCHED_NO_SKINNY_TAIL) == 0 && skinny_tiles_all > 0 &&
                          ((p.sched_flags & FLUXMI_SCHED_FORCE_SKINNY_TAIL) != 0 || (skinny_tiles_all * 4 <= 2 * grid && c.nk >= 128 && !own_units));
   const int skinny_items = skinny_on ? skinny_tiles_all * 4 : 0;
@@ -1643,7 +1642,7 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
   // Block-scaled launches run every tile as two 256 x 128 pieces (one column block of B's scales each).
   const int full_items = BS ? 0 : (reg_tiles / grid) * grid;
   const int rem_tiles = reg_tiles - full_items;
-  const int pieces = BS ? 2 : pieces_of(rem_tiles);
+  const int pieces = BS ? 2 : (!cut_tail ? 1 : (rem_tiles * 4 <= grid ? 4 : (rem_tiles * 2 <= grid ? 2 : 1)));
   const int skinny_first = full_items + rem_tiles * pieces;  // first work item of the skinny pieces
   const int total_items = skinny_first + skinny_items;
 

@@ -531,8 +531,7 @@ def test_skinny_tail_pieces_same_bits_as_in_place(dtype, ksteps):
 @pytest.mark.parametrize("margin", [0, 232, 244, 250, 252])
 def test_skinny_tails_in_launches_of_one_round(dtype, margin):
     """Seven row tiles of long K (enough for skinny tails), three of them with at most 64 rows, on 256, 24, 12, 6 and 4 compute units: in place,
-    where all tiles are cut as small as the others alone would be; behind the others, where these are cut in four or two without them; and
-    in launches of two rounds.  The bits of the schedule without skinny tails, and the dense product."""
+    whole or cut, in launches of one round, and behind the others in launches of two.  The bits of the schedule without skinny tails, and the dense product."""
     from flux_amd import capi
     split, n, k = [300, 257, 513], 200, 8192 + 64
     m, t = sum(split), torch.bfloat16 if dtype == "bf16" else torch.float8_e4m3fn
