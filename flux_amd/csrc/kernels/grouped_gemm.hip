@@ -148,6 +148,23 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
   return chunks <= stream_chunks_limit(active, chunk_rows, args->dtype == FLUXMI_FP8_E4M3, panel.chunk_items, panel.round_items);
 }
 
+// Launches that leave most of the dual tiles' waves or phases without work; tiles: the most that a launch can have.  Dual tiles against macro
+// tiles, both with up to four workgroups to a tile, in the mean, and launches slower by more than 3 %; where macro tiles had one workgroup to
+// a tile, before the dual tiles were there, is the third figure:
+//   up to 128 columns, up to 128 tiles, rows of K of 1 KiB and more   0.73, 88 %; 0.94  (5 experts 32 x 12672, 104 rows each: fp8 90 us, 42, 36)
+//     the same with shorter K                                         1.16,  9 %; 1.27, taken
+//   block-scaled, few rows that no form for few rows takes (columns not in 64s):
+//     R up to 64, up to 128 tiles                                     0.65, 99 %; 1.01  (one expert 1904 x 13696, 51 rows: 112 us, 46, 86)
+//                 129 to 256 tiles                                    1.02, 26 %; 1.09, taken
+//                 257 to 448 tiles                                    1.00, 43 %; 0.99
+//     R up to 96, more than 256 tiles, K of 4 KiB and more            1.00, 38 %; 1.00  (shorter K 1.12,  5 %; 1.12, taken)
+bool dual_tiles_idle(const fluxmi_grouped_gemm_args *args, bool block_scaled, int64_t kbytes, int64_t tiles) {
+  auto at_most = [&](int64_t rows) { return args->max_rows <= rows * args->nexperts; };
+  if (args->n <= 128 && tiles <= 128 && kbytes >= 1024) return true;
+  if (!block_scaled) return false;
+  return (at_most(64) && (tiles <= 128 || (tiles > 256 && tiles <= 448))) || (at_most(96) && tiles > 256 && kbytes >= 4096);
+}
+
 // Whether the dual tiles are the faster ones for a launch that the macro tiles would compute.  Speed against the macro tiles in the mean, and how
 // many launches are slower by more than 3 %: 19125 launches of 1 to 128 experts with more than 128 tiles, R = 97 to 4000 rows each on average,
 // rows of K of 0.5 to 28 KiB, even, random and Zipf row counts, plain and scaled, gathered and not, weights not in the cache.  fp32 results have
@@ -170,11 +187,12 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
 // Launches of fewer tiles, which both forms cut into pieces, are not told apart here: up to 192 rows 0.92 to 1.06, more rows 0.74 to 1.14, so the
 // macro tiles would be the faster ones for many (both gain on one workgroup to a tile, these 1.06 to 1.47).
 // The flags of the fill forms name forms of the macro tiles.
-bool dual_is_faster(const fluxmi_grouped_gemm_args *args, bool block_scaled) {
-  if (block_scaled) return true;
-  if ((args->sched_flags & (FLUXMI_SCHED_HALF_LINE_FILLS | FLUXMI_SCHED_WHOLE_LINE_FILLS)) != 0) return false;
+bool dual_is_faster(const fluxmi_grouped_gemm_args *args, bool block_scaled, bool by_splits, int64_t tiles) {
   const bool fp8 = args->dtype == FLUXMI_FP8_E4M3;
   const int64_t kbytes = static_cast<int64_t>(args->k) * (fp8 ? 1 : 2);
+  if (!by_splits && dual_tiles_idle(args, block_scaled, kbytes, tiles)) return false;
+  if (block_scaled) return true;
+  if ((args->sched_flags & (FLUXMI_SCHED_HALF_LINE_FILLS | FLUXMI_SCHED_WHOLE_LINE_FILLS)) != 0) return false;
   auto at_most = [&](int64_t rows) { return args->max_rows <= rows * args->nexperts; };
   if (at_most(fp8 ? 512 : 320) || (kbytes < 6144 && at_most(512))) return true;
   if (args->d_fp32 != 0) return kbytes < 1024 || (kbytes < 2048 && at_most(1500)) || (kbytes < 3072 && at_most(1024));
@@ -296,7 +314,9 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
   if (macro) p.by_splits = panel.cols != 0 ? panel.chunk_rows : (stream_form ? kStreamRows : 0);
   p.chunk_items = panel.chunk_items;
   p.round_items = panel.round_items;
-  const bool dual = macro && dual_is_faster(args, bs != nullptr) && dual_takes(p, args->dtype);
+  const int64_t tiles_n = (args->n + BN - 1) / BN * ngroups;
+  const int64_t max_tiles = (static_cast<int64_t>(args->max_rows) / BM + args->nexperts) * tiles_n;  // whatever the splits
+  const bool dual = macro && dual_is_faster(args, bs != nullptr, p.by_splits != 0, max_tiles) && dual_takes(p, args->dtype);
   if (dry_run) {
     dry_run->stream = stream_form;
     dry_run->macro = macro;
@@ -346,8 +366,6 @@ int run_grouped_gemm(const fluxmi_grouped_gemm_args *args, int ngroups, const vo
     // tiles fp16 8 experts 4096 x 14336, 194 rows each 299 -> 267; bf16 2 experts 4096 x 8192, 200 rows 154 -> 117; block-scaled 4 experts 1024 x 4096, 500
     // rows 61 -> 44; macro tiles bf16 4 experts 2048 x 4096, 500 rows 105 -> 70; fp8 one expert 2048 x 4096, 2000 rows 48 -> 29.  Both deal a round
     // that is not full to all XCDs (bf16 8 experts 2048 x 4096, 600 rows, 192 whole tiles: 88, in 256 workgroups without that 96, with it 87; 360 rows 77 -> 71).
-    const int64_t tiles_n = (args->n + BN - 1) / BN * ngroups;
-    const int64_t max_tiles = (static_cast<int64_t>(args->max_rows) / BM + args->nexperts) * tiles_n;
     const int64_t most = max_tiles * 4;
     const int grid = static_cast<int>(most < cus ? most : cus);
     // Form of the ring fills.  Whole 128-byte lines cost the memory pipeline less per byte and need one barrier per

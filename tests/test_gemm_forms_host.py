@@ -202,3 +202,31 @@ def test_dual_tiles_by_rows_and_k(dtype, experts, rows, n, k, block_scaled, dual
     assert is_dual(d_fp32=True) == is_dual(d_fp32=True, gathered=True) == dual32
     for flag in (capi.SCHED_HALF_LINE_FILLS, capi.SCHED_WHOLE_LINE_FILLS):
         assert is_dual(sched_flags=flag) == (dual and block_scaled)
+
+
+@pytest.mark.parametrize("experts,rows,n,k,dual", [
+    # up to 128 tiles whatever the splits: macro tiles up to 64 rows
+    (1, 59, 416, 13056, False), (1, 64, 416, 256, False), (1, 65, 416, 13056, True), (3, 45, 272, 7168, False), (64, 64, 264, 256, True),
+    (8, 64, 3064, 512, False), (8, 64, 3336, 512, True),
+    # more than 256: macro tiles up to 448 and 64 rows, and up to 96 rows with K of 4 KiB and more
+    (64, 64, 1032, 256, False), (64, 64, 1544, 256, True), (64, 64, 1544, 4096, False), (64, 65, 1032, 2048, True), (64, 96, 1032, 4096, False),
+    (64, 96, 1032, 3968, True), (64, 97, 1032, 4096, True),
+    # columns in 64s: the panel tiles take them, and what is left by splits stays with the dual tiles
+    (64, 64, 4096, 4096, True)])
+def test_block_scaled_launches_of_few_rows_run_the_macro_tiles(experts, rows, n, k, dual):
+    kind = capi.gemm_launch_info(FP8, experts, rows * experts, n, k, block_scaled=True).form
+    assert kind == (capi.GEMM_MACRO_TILES if n % 64 else capi.GEMM_BY_SPLITS)
+    for d_fp32 in (False, True):
+        assert capi.gemm_dual_tiles(FP8, experts, rows * experts, n, k, block_scaled=True, d_fp32=d_fp32) == dual
+
+
+@pytest.mark.parametrize("dtype,block_scaled", [(BF16, False), (F16, False), (FP8, False), (FP8, True)])
+@pytest.mark.parametrize("experts,rows,n,kbytes,dual", [
+    # up to 128 columns, up to 128 tiles whatever the splits, rows of K of 1 KiB and more: macro tiles
+    (5, 300, 32, 2048, False), (5, 300, 128, 1024, False), (5, 300, 128, 896, True), (5, 300, 136, 2048, True),
+    (64, 256, 128, 2048, False), (64, 260, 128, 2048, True)])
+def test_few_tiles_of_few_columns_run_the_macro_tiles(dtype, block_scaled, experts, rows, n, kbytes, dual):
+    k = kbytes // (1 if dtype == FP8 else 2)
+    assert capi.gemm_launch_info(dtype, experts, rows * experts, n, k, block_scaled=block_scaled).form == capi.GEMM_MACRO_TILES
+    for d_fp32 in (False, True):
+        assert capi.gemm_dual_tiles(dtype, experts, rows * experts, n, k, block_scaled=block_scaled, d_fp32=d_fp32) == dual
