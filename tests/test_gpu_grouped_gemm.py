@@ -547,6 +547,27 @@ def test_skinny_tails_in_launches_of_one_round(dtype, margin):
         assert torch.equal(out.double(), want), f"flags {flags}"
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("n", [8, 132, 392])
+def test_low_tiles_cut_in_two(dtype, n):
+    """Launches whose tiles are cut in two pieces of 128 columns, several of them with at most 128 rows; in one round and in the last of two.
+    Integers: the exact product."""
+    from flux_amd import capi
+    split, k = [300, 90, 257, 0, 128, 129, 384, 385, 1, 100], 1024
+    tiles = sum((r + 255) // 256 for r in split) * ((n + 255) // 256)
+    print(f"[case] grouped_gemm {dtype} low tiles cut in two n={n}", flush=True)
+    t = {"bf16": torch.bfloat16, "f16": torch.float16, "fp8": torch.float8_e4m3fn}[dtype]
+    g = torch.Generator(device="cuda").manual_seed(n)
+    a = torch.randint(-3, 4, (sum(split), k), generator=g, device="cuda").float()
+    w = torch.randint(-3, 4, (len(split), n, k), generator=g, device="cuda").float()
+    want = torch.cat([x.double() @ w[e].double().t().contiguous() for e, x in enumerate(a.split(split))])
+    sp = torch.tensor(split, dtype=torch.int32).cuda()
+    for units in (tiles * 2, tiles * 3, tiles * 4 // 5):
+        out = torch.full((sum(split), n), -7.0, device="cuda")
+        capi.grouped_gemm(a.to(t), w.to(t), sp, out=out, cu_margin=256 - units)
+        assert torch.equal(out.double(), want), f"{units} compute units"
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "fp8"])
 @pytest.mark.parametrize("k", [128, 1024, 1040, 4096])
 def test_both_fill_forms_give_the_same_bits(dtype, k):
