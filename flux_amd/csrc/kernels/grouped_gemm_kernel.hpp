@@ -1639,10 +1639,12 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
   // Full rounds run whole macro tiles.  The tiles of the last, partly filled round are cut into
   // `pieces` parts (2 pieces of 256x128, or 4 of 128x128) when that still fits one round, so that the
   // chip does not idle while a fraction of the CUs finishes whole tiles.
-  // Block-scaled launches run every tile as two 256 x 128 pieces (one column block of B's scales each).
+  // Block-scaled launches run every tile as two 256 x 128 pieces (one column block of B's scales each); with up to 128 columns the second ones would
+  // have none, and every other workgroup of an even grid no work (139 experts 24 x 9088, 156 rows each: 145 us, one piece 80; one
+  // workgroup to a tile, an odd grid, 86).
   const int full_items = BS ? 0 : (reg_tiles / grid) * grid;
   const int rem_tiles = reg_tiles - full_items;
-  const int pieces = BS ? 2 : (!cut_tail ? 1 : (rem_tiles * 4 <= grid ? 4 : (rem_tiles * 2 <= grid ? 2 : 1)));
+  const int pieces = BS ? (p.n <= 128 ? 1 : 2) : (!cut_tail ? 1 : (rem_tiles * 4 <= grid ? 4 : (rem_tiles * 2 <= grid ? 2 : 1)));
   const int skinny_first = full_items + rem_tiles * pieces;  // first work item of the skinny pieces
   const int total_items = skinny_first + skinny_items;
 
@@ -1724,14 +1726,14 @@ __global__ __launch_bounds__(NTHREADS) void grouped_gemm_mfma_kernel(const GemmP
     const int g = p.ngroups > 1 ? nt / tiles_n1 : 0;
     const int gcol = g * tiles_n1 * BN;  // first virtual column of the weight group
     t.n0 = (nt - g * tiles_n1) * BN;
-    if (item < full_items || pieces == 1) {
+    if (!BS && (item < full_items || pieces == 1)) {
       // The last row tile of an expert is run 128 rows high when that covers its rows, the last column
       // tile 128 columns wide when that covers its columns (N = 1408: the sixth tile holds 128 columns).
       // With at most 64 rows left (and the skinny tail not in use for them) it runs 64 rows high.
       const bool low = half_tiles && rows_e - t.m0 <= 128;
       const bool narrow = half_tiles && p.n - t.n0 <= 128;
       t.kind = low ? (narrow ? 3 : (rows_e - t.m0 <= 64 ? 5 : 1)) : (narrow ? 2 : 0);
-    } else if (pieces == 2) {
+    } else if (BS || pieces == 2) {
       // 128 rows high where that covers the rows, as whole tiles are (bf16 8 experts 3584 x 4096, 300 rows each: 127 us -> 101; fp8 117
       // experts 8 x 12544, 106 rows each 84 -> 52).  Block-scaled tiles find their height themselves.
       t.n0 += piece * 128;

@@ -203,7 +203,7 @@ def test_blockscale_last_rows_of_an_expert(split, n, k):
 # Launches that the dual tiles do not take: 16-bit results in columns that are not in eights, and more than 128 experts; one and two blocks of K,
 # six, seven and thirteen (the last pair of an unrolled trip of the k loop and the first of the next); last row tiles 64, 128 and 256 rows high.
 @pytest.mark.parametrize("split,n,f32", [([129, 192, 193, 64, 65, 128, 1, 320, 321, 384, 385, 255], 268, False), ([513, 576, 0, 577, 640, 641], 132, False),
-                                         ([300], 516, False), ([97, 200, 300, 0] + [97] * 125 + [260], 136, True)])
+                                         ([300], 516, False), ([129, 192, 0, 193, 64, 65, 128, 1, 320], 100, False), ([97, 200, 300, 0] + [97] * 125 + [260], 136, True)])
 @pytest.mark.parametrize("k", [128, 256, 768, 896, 1664])
 def test_blockscale_macro_tiles_are_exact_on_integers(split, n, f32, k):
     """The macro tiles' kernel, with every factor; operands are small integers and scales powers of two, so the fp32 sums are exact."""
