@@ -153,6 +153,9 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
 // a tile, before the dual tiles were there, is the third figure:
 //   up to 128 columns, up to 128 tiles, rows of K of 1 KiB and more   0.73, 88 %; 0.94  (5 experts 32 x 12672, 104 rows each: fp8 90 us, 42, 36)
 //     the same with shorter K                                         1.16,  9 %; 1.27, taken
+//     129 to 256 tiles, K of 4 KiB and more                           1.02,  9 %; 1.06  (bf16 107 experts 32 x 5888, 118 rows each 86 us, 58, 59)
+//     the same with shorter K                                         1.27,  1 %; 1.29, taken
+//     block-scaled, 129 to 256 tiles, rows of K of 1 KiB and more     0.97, 58 %; 1.29
 //   block-scaled, few rows that no form for few rows takes (columns not in 64s):
 //     R up to 64, up to 128 tiles                                     0.65, 99 %; 1.01  (one expert 1904 x 13696, 51 rows: 112 us, 46, 86)
 //                 129 to 256 tiles                                    1.02, 26 %; 1.09, taken
@@ -160,7 +163,7 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
 //     R up to 96, more than 256 tiles, K of 4 KiB and more            1.00, 38 %; 1.00  (shorter K 1.12,  5 %; 1.12, taken)
 bool dual_tiles_idle(const fluxmi_grouped_gemm_args *args, bool block_scaled, int64_t kbytes, int64_t tiles) {
   auto at_most = [&](int64_t rows) { return args->max_rows <= rows * args->nexperts; };
-  if (args->n <= 128 && tiles <= 128 && kbytes >= 1024) return true;
+  if (args->n <= 128 && kbytes >= 1024 && (tiles <= 128 || (tiles <= 256 && (block_scaled || kbytes >= 4096)))) return true;
   if (!block_scaled) return false;
   return (at_most(64) && (tiles <= 128 || (tiles > 256 && tiles <= 448))) || (at_most(96) && tiles > 256 && kbytes >= 4096);
 }
