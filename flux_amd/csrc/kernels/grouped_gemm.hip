@@ -155,6 +155,7 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
 //     the same with shorter K                                         1.16,  9 %; 1.27, taken
 //     129 to 256 tiles, K of 4 KiB and more                           1.02,  9 %; 1.06  (bf16 107 experts 32 x 5888, 118 rows each 86 us, 58, 59)
 //     the same with shorter K                                         1.27,  1 %; 1.29, taken
+//     block-scaled, up to 128 tiles, any K                            0.99, 16 %; 1.29  (3 experts 88 x 896, 64 rows each: 16.2 us; before 11.5)
 //     block-scaled, 129 to 256 tiles, rows of K of 1 KiB and more     0.97, 58 %; 1.29
 //   block-scaled, few rows that no form for few rows takes (columns not in 64s):
 //     R up to 64, up to 128 tiles                                     0.65, 99 %; 1.01  (one expert 1904 x 13696, 51 rows: 112 us, 46, 86)
@@ -163,7 +164,8 @@ bool few_chunks(const fluxmi_grouped_gemm_args *args, const int32_t *splits_host
 //     R up to 96, more than 256 tiles, K of 4 KiB and more            1.00, 38 %; 1.00  (shorter K 1.12,  5 %; 1.12, taken)
 bool dual_tiles_idle(const fluxmi_grouped_gemm_args *args, bool block_scaled, int64_t kbytes, int64_t tiles) {
   auto at_most = [&](int64_t rows) { return args->max_rows <= rows * args->nexperts; };
-  if (args->n <= 128 && kbytes >= 1024 && (tiles <= 128 || (tiles <= 256 && (block_scaled || kbytes >= 4096)))) return true;
+  if (args->n <= 128 && tiles <= 128 && (block_scaled || kbytes >= 1024)) return true;
+  if (args->n <= 128 && tiles <= 256 && kbytes >= (block_scaled ? 1024 : 4096)) return true;
   if (!block_scaled) return false;
   return (at_most(64) && (tiles <= 128 || (tiles > 256 && tiles <= 448))) || (at_most(96) && tiles > 256 && kbytes >= 4096);
 }
@@ -186,9 +188,10 @@ bool dual_tiles_idle(const fluxmi_grouped_gemm_args *args, bool block_scaled, in
 //                       K < 3 KiB         1.07,  4 %                          R up to 1024 1.05, 11 %; more 1.03, 15 %: not taken
 //                       K < 4 KiB         R up to 1024 1.05, 9 %; 1.03, 13 %  1.02, 20 %: not taken
 //            the rest                     1.00, 30 %: not taken               0.99, 38 %: not taken
-//   block-scaled                          1.21,  2 %                          1.12,  5 %
+//   block-scaled                          1.21,  2 %                          1.12,  5 %; of these with K < 1 KiB, more than 1024 columns and 256
+//                                                                             rows, up to 512 tiles 1.02, 31 %, taken: the macro tiles are no safer
 // Launches of fewer tiles, which both forms cut into pieces, are not told apart here: up to 192 rows 0.92 to 1.06, more rows 0.74 to 1.14, so the
-// macro tiles would be the faster ones for many (both gain on one workgroup to a tile, these 1.06 to 1.47).
+// macro tiles would be the faster ones for many.  None of them loses against macro tiles with one workgroup to a tile (1.28 to 1.49 in the mean).
 // The flags of the fill forms name forms of the macro tiles.
 bool dual_is_faster(const fluxmi_grouped_gemm_args *args, bool block_scaled, bool by_splits, int64_t tiles) {
   const bool fp8 = args->dtype == FLUXMI_FP8_E4M3;

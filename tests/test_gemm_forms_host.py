@@ -222,8 +222,8 @@ def test_block_scaled_launches_of_few_rows_run_the_macro_tiles(experts, rows, n,
 
 @pytest.mark.parametrize("dtype,block_scaled", [(BF16, False), (F16, False), (FP8, False), (FP8, True)])
 @pytest.mark.parametrize("experts,rows,n,kbytes,dual", [  # dual: None for "but for block scales"
-    # up to 128 columns, rows of K of 1 KiB and more: macro tiles up to 128 tiles whatever the splits, up to 256 with 4 KiB and more or block scales
-    (5, 300, 32, 2048, False), (5, 300, 128, 1024, False), (5, 300, 128, 896, True), (5, 300, 136, 2048, True),
+    # up to 128 columns, rows of K of 1 KiB and more or block scales: macro tiles up to 128 tiles whatever the splits; up to 256 with 4 KiB (1 KiB) and more
+    (5, 300, 32, 2048, False), (5, 300, 128, 1024, False), (5, 300, 128, 896, None), (5, 300, 136, 2048, True),
     (64, 256, 128, 2048, False), (64, 260, 128, 2048, None), (64, 260, 128, 4096, False), (64, 260, 128, 3968, None), (64, 260, 128, 896, True),
     (100, 500, 128, 4096, True)])
 def test_few_tiles_of_few_columns_run_the_macro_tiles(dtype, block_scaled, experts, rows, n, kbytes, dual):
